@@ -56,8 +56,9 @@ static int check_common(int hq, int hkv, int d, int bs, int max_blocks, int64_t 
 
 // shapes the balanced schedule and the matrix-core grid schedule both take
 static bool streamk_shape(int batch, int hq, int hkv, int d, int bs, int q_dtype, int kv_dtype) {
-    return ((d == 128 && hq / hkv <= 16) || (d == 64 && hq / hkv <= 8)) && bs == 16 && is_16bit_float(q_dtype) &&
-           (kv_dtype == q_dtype || kv_dtype == AICOMP_KV_FP8_E4M3) && batch <= 1024;
+    const bool half = is_16bit_float(q_dtype) && (kv_dtype == q_dtype || kv_dtype == AICOMP_KV_FP8_E4M3);
+    const bool f32 = q_dtype == AICOMP_KV_F32 && kv_dtype == AICOMP_KV_F32;
+    return (d == 128 || d == 64) && hq / hkv <= (half && d == 64 ? 8 : 16) && bs == 16 && (half || f32) && batch <= 1024;
 }
 
 // A decode call over few, short rows is a chain of launch and memory latencies, not a stream: the
@@ -276,8 +277,8 @@ static int decode_impl(void* out, const void* query, const void* new_key, const 
     a.num_parts = resolve_parts(batch, num_kv_heads, block_size, max_blocks_per_seq, matrix_shape, a.partition_size);
     a.stream = (hipStream_t)stream;
     // the matrix-core kernels append the new rows themselves when they can read them 16 bytes at a time
-    const bool injectable = fused && is_16bit_float(q_dtype) && kv_token_stride % 8 == 0 &&
-                            kv_head_stride % 8 == 0 && (uintptr_t)new_key % 16 == 0 &&
+    const int64_t vec = 16 / dtype_size(q_dtype);
+    const bool injectable = fused && kv_token_stride % vec == 0 && kv_head_stride % vec == 0 && (uintptr_t)new_key % 16 == 0 &&
                             (uintptr_t)new_value % 16 == 0;
     if (partition_size == 0 && decode_streamk_supported(a) && !small_call(batch, block_size, max_blocks_per_seq)) {
         // balanced schedule: equal tile counts per wave, merged by a second kernel

@@ -143,6 +143,7 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 struct Bf16Fmt {
     typedef bf16_t elem;
+    typedef uint16_t raw;
     static constexpr int DT = AICOMP_KV_BF16;
     // D[16x16] += A[16x32] * B[32x16]: v_mfma_f32_16x16x32_bf16
     __device__ __forceinline__ static f32x4_t mfma(const uint4& a, const uint4& b, const f32x4_t& c) {
@@ -175,6 +176,7 @@ struct Bf16Fmt {
 
 struct F16Fmt {
     typedef f16_t elem;
+    typedef uint16_t raw;
     static constexpr int DT = AICOMP_KV_F16;
     __device__ __forceinline__ static f32x4_t mfma(const uint4& a, const uint4& b, const f32x4_t& c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
@@ -199,6 +201,12 @@ struct F16Fmt {
         return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, pp), one, acc, false);
     }
     static constexpr uint32_t SIGN_PAIR = 0x80008000u;
+};
+
+// float32 tensors: outputs are stored as they are
+struct F32Fmt {
+    typedef float raw;
+    __device__ __forceinline__ static float from_f32(float f) { return f; }
 };
 
 // --------------------------------------- order of query tiles in a prefill grid ---

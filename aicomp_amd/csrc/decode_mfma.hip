@@ -11,7 +11,9 @@
 // one 128-element row: every head takes two B-operand columns, one per token
 // parity, with the query in the matching half of the row and zeros in the other,
 // and the two columns' partial softmaxes are merged at the end.  Same instruction
-// stream per byte as head_dim 128.  Everything else goes to the vector-ALU kernel.
+// stream per byte as head_dim 128.  Float32 queries over float32 pools, head_dim 128 and
+// 64, up to 16 heads per KV head, run the same two schedules on the float32 matrix
+// instruction (decode_tile_f32.h).  Everything else goes to the vector-ALU kernel.
 //
 // HBM-bound: per sequence 2 * L * Hkv * D * e_kv bytes of K/V are streamed and
 // used exactly once; 4 * G flop per byte (bf16), far below the MFMA roof, so
@@ -74,8 +76,8 @@ struct MfmaParams {
     float* ws_acc;
     float* ws_ml;
     // fused append (optional): row b of new_key / new_value is token context_lens[b]-1
-    const uint16_t* new_key;
-    const uint16_t* new_value;
+    const void* new_key;
+    const void* new_value;
     int64_t new_token_stride, new_head_stride;     // elements
 };
 
@@ -182,10 +184,18 @@ __device__ __forceinline__ KTileOffsets k_tile_offsets(int lane) {
 }
 
 // Per-wave running state of the online softmax and the output accumulators.
-struct WaveState {
+template <int NO>
+struct WaveStateT {
     float m, lsum;
-    f32x4_t O[8];
+    f32x4_t O[NO];
 };
+typedef WaveStateT<8> WaveState;
+template <int NO>
+__device__ __forceinline__ void clear_state(WaveStateT<NO>& st) {
+    st.m = NEG_BIG; st.lsum = 0.f;
+#pragma unroll
+    for (int j = 0; j < NO; ++j) st.O[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+}
 
 // One 32-token tile: K registers -> LDS -> S^T = K Q^T -> online softmax -> O^T += V^T P^T.
 // NEXT: prefetch the wave's next tile (blocks nb0/nb1) into the same registers.
@@ -304,12 +314,12 @@ __device__ __forceinline__ uint2 quant8_fp8(const uint4& x, float scale) {
     return make_uint2((uint32_t)lo, (uint32_t)hi);
 }
 
-// Fused append for the grid-scheduled kernel: the tile that holds the sequence's newest token
-// (context_lens - 1) takes its K/V row from new_key / new_value instead of what was loaded from
-// the pool, and writes it to the pool (the append itself).  No other wave of the launch reads
-// that token.  A tile row is one token (16 lanes of 8 elements), or with PAIR half a row (8 lanes).
+// Fused append: the tile that holds the sequence's newest token (context_lens - 1) takes its K/V
+// row from new_key / new_value instead of what was loaded from the pool, and writes it to the pool
+// (the append itself).  No other wave of the launch reads that token, so no cross-wave ordering is
+// needed.  A tile row is one token (16 lanes of 8 elements), or with PAIR half a row (8 lanes).
 template <typename E, bool FP8, bool PAIR, typename Params>
-__device__ __forceinline__ void inject_new_row_grid(TileRegs<FP8>& kr, TileRegs<FP8>& vr, const Params& p,
+__device__ __forceinline__ void inject_new_row(TileRegs<FP8>& kr, TileRegs<FP8>& vr, const Params& p,
                                                     int seq, int kvh, int lane, int tile_start, int len,
                                                     const int64_t (&bb)[4]) {
     constexpr int DQ = PAIR ? 64 : D;
@@ -321,8 +331,8 @@ __device__ __forceinline__ void inject_new_row_grid(TileRegs<FP8>& kr, TileRegs<
     const bool mine = (lane >> 4) == (row & 3) && (!PAIR || ((lane >> 3) & 1) == (tau & 1));
     const int slot = row >> 2;
     const int64_t src = (int64_t)seq * p.new_token_stride + (int64_t)kvh * p.new_head_stride + 8 * c;
-    const uint4 nk = *(const uint4*)(p.new_key + src);
-    const uint4 nv = *(const uint4*)(p.new_value + src);
+    const uint4 nk = *(const uint4*)((const uint16_t*)p.new_key + src);
+    const uint4 nv = *(const uint4*)((const uint16_t*)p.new_value + src);
     const int64_t blk = bb[blk_i];
     const int64_t dst = ((blk * p.hkv + kvh) * BS + tb) * (DQ / 8) + c;        // 8-element chunks
     if constexpr (FP8) {
@@ -340,14 +350,87 @@ __device__ __forceinline__ void inject_new_row_grid(TileRegs<FP8>& kr, TileRegs<
     }
 }
 
-template <typename E, bool FP8, bool PAIR>
+// ---------------------------------------------------------------------------------------
+// What a schedule needs to know about the tiles it walks: the two kernels below are written over
+// one of these.  A tile is TT tokens of one KV head, BPT blocks, 8 KB of K and 8 KB of V per wave
+// (half of that for fp8), loaded with eight loads of each.
+// Tile16: 16-bit queries E over pools of E or fp8, head_dim 128, or 64 as rows of token pairs.
+template <typename E, bool FP8_, bool PAIR_>
+struct Tile16 {
+    typedef E Fmt;
+    static constexpr bool FP8 = FP8_, PAIR = PAIR_;
+    static constexpr int DQ = PAIR ? 64 : D;             // head_dim of the tensors
+    static constexpr int TT = PAIR ? 2 * TILE : TILE;    // tokens per tile
+    static constexpr int BPT = TT / BS;                  // blocks per tile
+    static constexpr int OROW = D;                       // floats per B column of the accumulators
+    static constexpr int NPAR = PAIR ? 2 : 1;            // B columns per query head
+    typedef WaveState State;
+    typedef KTileOffsets Offsets;
+    struct Q { uint4 r[4]; };
+    struct Regs { TileRegs<FP8> k, v; };
+    __device__ __forceinline__ static Offsets offsets(int lane) { return k_tile_offsets(lane); }
+
+    // raw query rows of (sequence, KV head); columns beyond the group are zeroed by q_operand only
+    // when the rows are used, so that issuing the loads never waits for them.
+    // PAIR: column c = (head c / 2, parity c % 2): k-slot s covers row elements 32s + 8 g4 .., which are
+    // the query's elements (32s + 8 g4) % 64 when the slot lies in the column's own half of the row.
+    template <typename Params>
+    __device__ __forceinline__ static void load_q(Q& q, const Params& p, int seq, int kvh, int lane) {
+        const int r16 = lane & 15, g4 = lane >> 4, h = PAIR ? (r16 >> 1) : r16;
+        const uint16_t* row = (const uint16_t*)p.query + ((int64_t)seq * p.hq + kvh * p.group + min(h, p.group - 1)) * DQ;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) q.r[s] = *(const uint4*)(row + (PAIR ? ((32 * s + 8 * g4) & 63) : 32 * s + 8 * g4));
+    }
+    __device__ __forceinline__ static void q_operand(Q& q, const Q& raw, int group, int lane) {
+        const int r16 = lane & 15, g4 = lane >> 4;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            bool use = r16 < NPAR * group;
+            if constexpr (PAIR) use = use && ((32 * s + 8 * g4 >= 64) == ((r16 & 1) != 0));
+            q.r[s] = use ? raw.r[s] : make_uint4(0, 0, 0, 0);
+        }
+    }
+    template <typename Params>
+    __device__ __forceinline__ static void load(Regs& t, const Params& p, const int64_t (&bb)[4], int kvh, int lane) {
+        if constexpr (PAIR) {
+            load_tile_pair<FP8>(t.k, p.k_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kvh, lane);
+            load_tile_pair<FP8>(t.v, p.v_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kvh, lane);
+        } else {
+            load_tile<FP8>(t.k, p.k_pool, bb[0], bb[1], p.hkv, kvh, lane);
+            load_tile<FP8>(t.v, p.v_pool, bb[0], bb[1], p.hkv, kvh, lane);
+        }
+    }
+    template <bool NEXT, bool MASK, typename Params>
+    __device__ __forceinline__ static void process(State& st, Regs& t, const Q& q, unsigned char* kt, const Offsets& ko,
+                                                   const Params& p, const int64_t (&nb)[4], int kvh_next, int lane,
+                                                   int tile_start, int end, float cmul) {
+        process_tile<E, FP8, NEXT, MASK, PAIR>(st, t.k, t.v, q.r, kt, ko, p.k_pool, p.v_pool, nb[0], nb[1], p.hkv,
+                                               kvh_next, lane, lane >> 4, tile_start, end, cmul, nb[2], nb[3]);
+    }
+    template <typename Params>
+    __device__ __forceinline__ static void inject(Regs& t, const Params& p, int seq, int kvh, int lane, int tile_start,
+                                                  int len, const int64_t (&bb)[4]) {
+        inject_new_row<E, FP8, PAIR>(t.k, t.v, p, seq, kvh, lane, tile_start, len, bb);
+    }
+    // this lane's accumulators into the row of its column: elements 32 g4 + 8 i + j from O[j][i]
+    __device__ __forceinline__ static void store_acc(float* row, const State& st, int g4) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float* dst = row + 32 * g4 + 8 * i;
+            *(float4*)dst = make_float4(st.O[0][i], st.O[1][i], st.O[2][i], st.O[3][i]);
+            *(float4*)(dst + 4) = make_float4(st.O[4][i], st.O[5][i], st.O[6][i], st.O[7][i]);
+        }
+    }
+};
+
+#include "decode_tile_f32.h"
+
+template <typename T>
 __global__ void __launch_bounds__(256, 2)
 paged_decode_mfma_kernel(MfmaParams p) {
     // KV head fastest: the workgroups launched together read the Hkv slices of the same
     // physical blocks, i.e. one contiguous Hkv*4 KB piece of each pool
-    constexpr int DQ = PAIR ? 64 : D;            // head_dim of the tensors
-    constexpr int TT = PAIR ? 2 * TILE : TILE;   // tokens per tile
-    constexpr int BPT = TT / BS;                 // blocks per tile
+    constexpr int DQ = T::DQ, TT = T::TT, BPT = T::BPT, NPAR = T::NPAR;
     const int kvh = blockIdx.x;
     const int part = blockIdx.y;
     const int seq = blockIdx.z;
@@ -357,7 +440,7 @@ paged_decode_mfma_kernel(MfmaParams p) {
     const int r16 = lane & 15;      // MFMA row / column index of this lane
     const int g4 = lane >> 4;       // MFMA k-group of this lane
     const int G = p.group;
-    const int ncol = PAIR ? 2 * G : G;           // B-operand columns in use
+    const int ncol = NPAR * G;      // B-operand columns in use
     const int start = part * p.partition_size;
     const int blk_base = start / BS;
 
@@ -369,32 +452,17 @@ paged_decode_mfma_kernel(MfmaParams p) {
     int tab_first = 0;                       // first entry (relative to blk_base) held in `tab`
     int tab = (blk_base + lane < p.max_blocks) ? table[blk_base + lane] : 0;
 
-    // Q as the B operand of S^T = K Q^T: column = head r16, k-slots = dims 32s + 8*g4 ..
-    // PAIR: column c is (head c/2, parity c%2); a row of the K tile is [token 2r | token 2r+1], so
-    // the column carries the query in elements 0..63 (parity 0) or 64..127 (parity 1), zeros elsewhere.
-    uint4 qf[4];
+    typename T::Q qf;
     {
-        const int h = PAIR ? (r16 >> 1) : r16;
-        const uint16_t* qrow = (const uint16_t*)p.query + ((int64_t)seq * p.hq + kvh * G + min(h, G - 1)) * DQ;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int e0 = 32 * s + 8 * g4;                       // first element of this k-slot in the row
-            bool use = r16 < ncol;
-            int src = e0;
-            if constexpr (PAIR) {
-                use = use && ((e0 >= 64) == ((r16 & 1) != 0));
-                src = e0 & 63;
-            }
-            uint4 v = *(const uint4*)(qrow + src);
-            if (!use) v = make_uint4(0, 0, 0, 0);
-            qf[s] = v;
-        }
+        typename T::Q raw;
+        T::load_q(raw, p, seq, kvh, lane);
+        T::q_operand(qf, raw, G, lane);
     }
 
     const int len = min(p.context_lens[seq], p.max_blocks * BS);   // never read past the table row
     if (start >= len) {
         if (len <= 0 && part == 0) {   // nothing to attend to: the output row is defined as zero
-            uint16_t* o = (uint16_t*)p.out + ((int64_t)seq * p.hq + kvh * G) * DQ;
+            auto* o = (typename T::Fmt::raw*)p.out + ((int64_t)seq * p.hq + kvh * G) * DQ;
             for (int i = tid; i < G * DQ; i += blockDim.x) o[i] = 0;
         }
         return;
@@ -407,12 +475,10 @@ paged_decode_mfma_kernel(MfmaParams p) {
     __shared__ float sm_l[NWAVES][16];
     unsigned char* kt = lds + w * KTILE_BYTES;
 
-    const float cmul = p.qk_mul * (FP8 ? p.k_scale[kvh] : 1.f);
+    const float cmul = p.qk_mul * (T::FP8 ? p.k_scale[kvh] : 1.f);
 
-    WaveState st;
-    st.m = NEG_BIG; st.lsum = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) st.O[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    typename T::State st;
+    clear_state(st);
 
     // physical blocks of tile tt (wave-uniform); the held table slice is refilled every 64 blocks
     int64_t bb[4] = {0, 0, 0, 0};
@@ -428,27 +494,19 @@ paged_decode_mfma_kernel(MfmaParams p) {
             bb[j] = clamp_block(__builtin_amdgcn_readlane(tab, i0 + j - tab_first), p.num_blocks);
     };
 
-    const KTileOffsets ko = k_tile_offsets(lane);
+    const typename T::Offsets ko = T::offsets(lane);
 
     if (w < ntiles) {
-        TileRegs<FP8> kr, vr;
+        typename T::Regs kv;
         tile_blocks(w);
         // Q must have landed before the tile loads are issued: the loop's waits then count
         // only tile loads, so a wave computes on tile t while tile t+1 is still in flight.
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-        if constexpr (PAIR) {
-            load_tile_pair<FP8>(kr, p.k_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kvh, lane);
-            load_tile_pair<FP8>(vr, p.v_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kvh, lane);
-        } else {
-            load_tile<FP8>(kr, p.k_pool, bb[0], bb[1], p.hkv, kvh, lane);
-            load_tile<FP8>(vr, p.v_pool, bb[0], bb[1], p.hkv, kvh, lane);
-        }
+        T::load(kv, p, bb, kvh, lane);
         int tt = w;
         for (; tt + NWAVES < ntiles; tt += NWAVES) {      // steady state: never the partition's last tile
             tile_blocks(tt + NWAVES);
-            process_tile<E, FP8, true, false, PAIR>(st, kr, vr, qf, kt, ko, p.k_pool, p.v_pool, bb[0],
-                                                 bb[1], p.hkv, kvh, lane, g4, start + tt * TT, end, cmul,
-                                                 bb[2], bb[3]);
+            T::template process<true, false>(st, kv, qf, kt, ko, p, bb, kvh, lane, start + tt * TT, end, cmul);
         }
         const int tile_start = start + tt * TT;
         // the sequence's newest token lives in this tile (bb still holds its blocks: the last lookup
@@ -459,41 +517,30 @@ paged_decode_mfma_kernel(MfmaParams p) {
             // (and attends over what the clamped table entry holds, like the unfused sequence of calls).
             const int raw_blk = __builtin_amdgcn_readlane(tab, BPT * tt + ((len - 1 - tile_start) >> 4) - tab_first);
             if (p.context_lens[seq] == len && raw_blk >= 0 && raw_blk < p.num_blocks)
-                inject_new_row_grid<E, FP8, PAIR>(kr, vr, p, seq, kvh, lane, tile_start, len, bb);
+                T::inject(kv, p, seq, kvh, lane, tile_start, len, bb);
         }
         if (tile_start + TT > end)
-            process_tile<E, FP8, false, true, PAIR>(st, kr, vr, qf, kt, ko, p.k_pool, p.v_pool, 0, 0,
-                                                 p.hkv, kvh, lane, g4, tile_start, end, cmul);
+            T::template process<false, true>(st, kv, qf, kt, ko, p, bb, kvh, lane, tile_start, end, cmul);
         else
-            process_tile<E, FP8, false, false, PAIR>(st, kr, vr, qf, kt, ko, p.k_pool, p.v_pool, 0, 0,
-                                                  p.hkv, kvh, lane, g4, tile_start, end, cmul);
+            T::template process<false, false>(st, kv, qf, kt, ko, p, bb, kvh, lane, tile_start, end, cmul);
     }
     const float m = st.m;
     float lsum = st.lsum;
-    f32x4_t (&O)[8] = st.O;
 
-    // ---- wave result: lane (column r16, g4) holds O^T[element 32*g4 + 8*i + j][column] in O[j][i]
+    // ---- wave result: the accumulators of column r16 into its row of the wave's own K tile region
     lsum += __shfl_xor(lsum, 16);
     lsum += __shfl_xor(lsum, 32);
-    float* osm = (float*)kt;        // this wave's own K tile region, 16 columns * 128 floats = 8192 bytes, the whole tile
+    float* osm = (float*)kt;        // 16 columns of at most 128 floats: 8192 bytes, the whole tile
     if (r16 < ncol) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float4 a = make_float4(O[0][i], O[1][i], O[2][i], O[3][i]);
-            float4 b = make_float4(O[4][i], O[5][i], O[6][i], O[7][i]);
-            float* dst = osm + r16 * D + 32 * g4 + 8 * i;
-            *(float4*)dst = a;
-            *(float4*)(dst + 4) = b;
-        }
+        T::store_acc(osm + r16 * T::OROW, st, g4);
         if (g4 == 0) { sm_m[w][r16] = m; sm_l[w][r16] = lsum; }
     }
     __syncthreads();
 
     // merge of the waves (PAIR: and of the two parity columns of a head, whose useful halves are
     // elements 0..63 and 64..127 of their accumulators)
-    const float vs = FP8 ? p.v_scale[kvh] : 1.f;
+    const float vs = T::FP8 ? p.v_scale[kvh] : 1.f;
     const bool direct = p.num_parts == 1;     // unsplit call: no merge needed
-    constexpr int NPAR = PAIR ? 2 : 1;
     for (int idx = tid; idx < G * DQ; idx += 256) {
         const int h = idx / DQ, dd = idx % DQ;
         float mxw = NEG_BIG;
@@ -508,14 +555,14 @@ paged_decode_mfma_kernel(MfmaParams p) {
             for (int par = 0; par < NPAR; ++par) {
                 const int c = NPAR * h + par;
                 const float f = exp2f(sm_m[ww][c] - mxw);
-                num = fmaf(f, ((const float*)(lds + ww * KTILE_BYTES))[c * D + dd + 64 * par], num);
+                num = fmaf(f, ((const float*)(lds + ww * KTILE_BYTES))[c * T::OROW + dd + 64 * par], num);
                 den = fmaf(f, sm_l[ww][c], den);
             }
         }
         const int head = kvh * G + h;
         if (direct) {
-            ((uint16_t*)p.out)[((int64_t)seq * p.hq + head) * DQ + dd] =
-                E::from_f32(den > 0.f ? vs * num / den : 0.f);
+            ((typename T::Fmt::raw*)p.out)[((int64_t)seq * p.hq + head) * DQ + dd] =
+                T::Fmt::from_f32(den > 0.f ? vs * num / den : 0.f);
         } else {
             const int64_t slot = ((int64_t)seq * p.hq + head) * p.num_parts + part;
             p.ws_acc[slot * DQ + dd] = num;
@@ -562,41 +609,10 @@ struct StreamKParams {
     float* ws_ml;       // [slots][G][2]
     int* ws_rows;       // [rows][2]: first and last part (wave of the row's head) holding a partial of the row
     // fused append (optional): row b of new_key / new_value is token context_lens[b]-1
-    const uint16_t* new_key;
-    const uint16_t* new_value;
+    const void* new_key;
+    const void* new_value;
     int64_t new_token_stride, new_head_stride;     // elements
 };
-
-// Fused append: the row's last tile holds the sequence's newest token, whose K/V are not in
-// the pool yet.  The 16 lanes that own that row take it from new_key / new_value instead of
-// what they loaded, and write it to the pool (the append itself).  No other wave of this
-// launch reads that token, so no cross-wave ordering is needed.
-template <typename E, bool FP8>
-__device__ __forceinline__ void inject_new_row(TileRegs<FP8>& kr, TileRegs<FP8>& vr,
-                                               const StreamKParams& p, int seq, int kvh, int lane,
-                                               int tile_start, int len, int64_t b0, int64_t b1) {
-    const int tau = len - 1 - tile_start;              // 0..31, wave-uniform
-    const int c = lane & 15, q = lane >> 4;
-    const int64_t src = (int64_t)seq * p.new_token_stride + (int64_t)kvh * p.new_head_stride + 8 * c;
-    const uint4 nk = *(const uint4*)(p.new_key + src);
-    const uint4 nv = *(const uint4*)(p.new_value + src);
-    const bool mine = (tau & 3) == q;
-    const int64_t blk = tau < 16 ? b0 : b1;
-    const int64_t dst = ((blk * p.hkv + kvh) * BS + (tau & 15)) * (D / 8) + c;   // 8-element chunks
-    if constexpr (FP8) {
-        const uint2 ck = quant8_fp8<E>(nk, p.k_scale[kvh]);
-        const uint2 cv = quant8_fp8<E>(nv, p.v_scale[kvh]);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (mine && i == (tau >> 2)) { kr.r[i] = ck; vr.r[i] = cv; }
-        if (mine) { ((uint2*)p.k_pool)[dst] = ck; ((uint2*)p.v_pool)[dst] = cv; }
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (mine && i == (tau >> 2)) { kr.r[i] = nk; vr.r[i] = nv; }
-        if (mine) { ((uint4*)p.k_pool)[dst] = nk; ((uint4*)p.v_pool)[dst] = nv; }
-    }
-}
 
 template <int TT>
 __device__ __forceinline__ int sk_tiles(int len, int max_blocks) {
@@ -605,21 +621,18 @@ __device__ __forceinline__ int sk_tiles(int len, int max_blocks) {
 }
 
 
-// PAIR: head_dim 64 as rows of token pairs (see paged_decode_mfma_kernel): a tile is 64 tokens in
-// four blocks, every head takes two B-operand columns (one per token parity), and a flush merges
-// the two columns of a head inside the wave and writes one partial of 64 floats per head.
-template <typename E, bool FP8, bool PAIR>
+// Token pairs (Tile16 with PAIR): every head takes two B-operand columns, one per token parity, and a
+// flush merges the two columns of a head inside the wave and writes one partial of 64 floats per head.
+template <typename T>
 __global__ void __launch_bounds__(256, 1)     // one workgroup per CU: a wave may use the whole register file
 streamk_decode_kernel(StreamKParams p) {
-    constexpr int DQ = PAIR ? 64 : D;            // head_dim of the tensors
-    constexpr int TT = PAIR ? 2 * TILE : TILE;   // tokens per tile
-    constexpr int BPT = TT / BS;                 // blocks per tile
+    constexpr int DQ = T::DQ, TT = T::TT, BPT = T::BPT;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g4 = lane >> 4;
     const int G = p.group, B = p.num_seqs;
-    const int ncol = PAIR ? 2 * G : G;           // B-operand columns in use
+    const int ncol = T::NPAR * G;                // B-operand columns in use
 
     __shared__ __attribute__((aligned(16))) unsigned char lds[NWAVES * KTILE_BYTES];
     __shared__ int prefix[SK_MAX_SEQS + 1];     // prefix[s] = tiles of the sequences before s
@@ -695,67 +708,33 @@ streamk_decode_kernel(StreamKParams p) {
     int kvh = __builtin_amdgcn_readfirstlane(kvh_mine);
     int t = __builtin_amdgcn_readfirstlane((int)(g0 - prefix[seq]));
 
-    const KTileOffsets ko = k_tile_offsets(lane);
+    const typename T::Offsets ko = T::offsets(lane);
 
     // ---- segments.  A segment is the part of one (sequence, KV head) row that falls into this
     // wave's tile range.  The next segment's query rows and table slice are requested while the
     // current one streams, and its first K/V tile is prefetched by the current segment's last
     // tile, so the loads never drain at a row boundary.
-    // raw query rows of (sequence, KV head); columns beyond the group are zeroed by q_operand
-    // only when the rows are used, so that issuing the loads never waits for them
-    auto load_q = [&](int sq, int kh, uint4 (&q)[4]) {
-        if constexpr (PAIR) {
-            // column c = (head c / 2, parity c % 2): k-slot s covers row elements 32s + 8 g4 .., which are
-            // the query's elements (32s + 8 g4) % 64 when the slot lies in the column's own half of the row
-            const uint16_t* qrow = (const uint16_t*)p.query + ((int64_t)sq * p.hq + kh * G + min(r16 >> 1, G - 1)) * DQ;
-#pragma unroll
-            for (int s = 0; s < 4; ++s) q[s] = *(const uint4*)(qrow + ((32 * s + 8 * g4) & 63));
-        } else {
-            const uint4* qp = (const uint4*)((const uint16_t*)p.query +
-                                             ((int64_t)sq * p.hq + kh * G + min(r16, G - 1)) * D + 8 * g4);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) q[s] = qp[s * 4];
-        }
-    };
-    auto q_operand = [&](const uint4 (&raw)[4], uint4 (&q)[4]) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            bool use = r16 < ncol;
-            if constexpr (PAIR) use = use && ((32 * s + 8 * g4 >= 64) == ((r16 & 1) != 0));
-            q[s] = use ? raw[s] : make_uint4(0, 0, 0, 0);
-        }
-    };
     auto load_tab = [&](int sq, int first_block) {
         const int32_t* table = p.block_table + (int64_t)sq * p.block_table_stride;
         return (first_block + lane < p.max_blocks) ? table[first_block + lane] : 0;
     };
 
     int nt = (int)min((int64_t)(row_tiles - t), g1 - g0);          // tiles of the current segment (>= 1)
-    uint4 qf[4];
-    uint4 qraw[4];
-    load_q(seq, kvh, qraw);
+    typename T::Q qf, qraw;
+    T::load_q(qraw, p, seq, kvh, lane);
     int tab = load_tab(seq, BPT * t);
-    TileRegs<FP8> kr, vr;
+    typename T::Regs kv;
     // the blocks of a tile out of a table slice held one entry per lane
     auto slice_blocks = [&](int slice, int first, int64_t (&bb)[4]) {
 #pragma unroll
         for (int j = 0; j < BPT; ++j) bb[j] = clamp_block(__builtin_amdgcn_readlane(slice, first + j), p.num_blocks);
     };
-    auto load_kv = [&](const int64_t (&bb)[4], int kh) {
-        if constexpr (PAIR) {
-            load_tile_pair<FP8>(kr, p.k_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kh, lane);
-            load_tile_pair<FP8>(vr, p.v_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kh, lane);
-        } else {
-            load_tile<FP8>(kr, p.k_pool, bb[0], bb[1], p.hkv, kh, lane);
-            load_tile<FP8>(vr, p.v_pool, bb[0], bb[1], p.hkv, kh, lane);
-        }
-    };
     {
         __builtin_amdgcn_s_waitcnt(0x0F70);                        // Q and table have landed
-        q_operand(qraw, qf);
+        T::q_operand(qf, qraw, G, lane);
         int64_t bb[4] = {0, 0, 0, 0};
         slice_blocks(tab, 0, bb);
-        load_kv(bb, kvh);
+        T::load(kv, p, bb, kvh, lane);
     }
 
     for (int64_t g = g0; g < g1 && seq < B;) {
@@ -763,7 +742,7 @@ streamk_decode_kernel(StreamKParams p) {
         const int blk_base = BPT * t;
         const int32_t* table = p.block_table + (int64_t)seq * p.block_table_stride;
         int tab_first = 0;
-        const float cmul = p.qk_mul * (FP8 ? p.k_scale[kvh] : 1.f);
+        const float cmul = p.qk_mul * (T::FP8 ? p.k_scale[kvh] : 1.f);
         auto tile_blocks = [&](int k, int64_t (&bb)[4]) {              // k-th tile of the segment
             const int i0 = BPT * k;
             if (i0 - tab_first >= 64) {
@@ -783,23 +762,20 @@ streamk_decode_kernel(StreamKParams p) {
         }
         const bool has_next = more && nseq < B;
         int tabn = 0;
-        uint4 qn[4];
+        typename T::Q qn;
         if (has_next) {
-            load_q(nseq, nkvh, qraw);
+            T::load_q(qraw, p, nseq, nkvh, lane);
             tabn = load_tab(nseq, 0);
         }
 
-        WaveState st;
-        st.m = NEG_BIG; st.lsum = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) st.O[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        typename T::State st;
+        clear_state(st);
 
         int64_t bb[4] = {0, 0, 0, 0};
         int k = 0;
         for (; k + 1 < nt; ++k) {
             tile_blocks(k + 1, bb);
-            process_tile<E, FP8, true, false, PAIR>(st, kr, vr, qf, kt, ko, p.k_pool, p.v_pool, bb[0], bb[1],
-                                                    p.hkv, kvh, lane, g4, (t + k) * TT, len, cmul, bb[2], bb[3]);
+            T::template process<true, false>(st, kv, qf, kt, ko, p, bb, kvh, lane, (t + k) * TT, len, cmul);
         }
         const int tile_start = (t + k) * TT;
         if (p.new_key != nullptr && t + k == row_tiles - 1) {       // the row's newest token lives here
@@ -808,10 +784,8 @@ streamk_decode_kernel(StreamKParams p) {
             // block of the pool and the length fits the table; otherwise the call leaves the pools alone
             // (and attends over what the clamped table entry holds, like the unfused sequence of calls).
             const int raw_blk = __builtin_amdgcn_readlane(tab, BPT * k + ((len - 1 - tile_start) >> 4) - tab_first);
-            if (p.context_lens[seq] == len && raw_blk >= 0 && raw_blk < p.num_blocks) {
-                if constexpr (PAIR) inject_new_row_grid<E, FP8, true>(kr, vr, p, seq, kvh, lane, tile_start, len, bb);
-                else inject_new_row<E, FP8>(kr, vr, p, seq, kvh, lane, tile_start, len, bb[0], bb[1]);
-            }
+            if (p.context_lens[seq] == len && raw_blk >= 0 && raw_blk < p.num_blocks)
+                T::inject(kv, p, seq, kvh, lane, tile_start, len, bb);
         }
         // The segment's last tile always runs the masked body (a full tile simply masks nothing):
         // one prefetching call site, so the prefetched registers need no merging afterwards.
@@ -819,22 +793,20 @@ streamk_decode_kernel(StreamKParams p) {
         if (has_next) {
             // prefetch the first tile of the next segment
             __builtin_amdgcn_s_waitcnt(0x0F70);      // next Q rows and table slice (and this tile) have landed
-            q_operand(qraw, qn);
+            T::q_operand(qn, qraw, G, lane);
             tab_ready = tabn;
             slice_blocks(tab_ready, 0, bb);
-            process_tile<E, FP8, true, true, PAIR>(st, kr, vr, qf, kt, ko, p.k_pool, p.v_pool, bb[0], bb[1],
-                                                   p.hkv, nkvh, lane, g4, tile_start, len, cmul, bb[2], bb[3]);
+            T::template process<true, true>(st, kv, qf, kt, ko, p, bb, nkvh, lane, tile_start, len, cmul);
         } else {
-            process_tile<E, FP8, false, true, PAIR>(st, kr, vr, qf, kt, ko, p.k_pool, p.v_pool, 0, 0,
-                                                    p.hkv, kvh, lane, g4, tile_start, len, cmul);
+            T::template process<false, true>(st, kv, qf, kt, ko, p, bb, kvh, lane, tile_start, len, cmul);
         }
 
-        // ---- flush: lane (head r16, g4) holds O^T[dim 32*g4 + 8*i + j][head] in O[j][i]
+        // ---- flush
         float lsum = st.lsum;
         lsum += __shfl_xor(lsum, 16);
         lsum += __shfl_xor(lsum, 32);
         const int64_t slot = (int64_t)kvh * (p.waves_per_head + B) + part + seq;
-        if constexpr (PAIR) {
+        if constexpr (T::PAIR) {
             // Column (head, parity) holds its own token's half of the pair rows: parity 0 elements 0..63 of
             // its accumulator (lanes g4 = 0, 1), parity 1 elements 64..127 (lanes g4 = 2, 3).  The two are
             // partial softmaxes over the even and the odd tokens of the same segment: merged here, inside the
@@ -858,12 +830,7 @@ streamk_decode_kernel(StreamKParams p) {
                 if (g4 == 0) *(float2*)(p.ws_ml + (slot * G + (r16 >> 1)) * 2) = make_float2(mm, f0 * lsum + f1 * l1);
             }
         } else if (r16 < ncol) {
-            float* dst = p.ws_acc + (slot * G + r16) * DQ + 32 * g4;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                *(float4*)(dst + 8 * i) = make_float4(st.O[0][i], st.O[1][i], st.O[2][i], st.O[3][i]);
-                *(float4*)(dst + 8 * i + 4) = make_float4(st.O[4][i], st.O[5][i], st.O[6][i], st.O[7][i]);
-            }
+            T::store_acc(p.ws_acc + (slot * G + r16) * DQ, st, g4);
             if (g4 == 0) *(float2*)(p.ws_ml + (slot * G + r16) * 2) = make_float2(st.m, lsum);
         }
         // the waves holding a row's first and last tile tell the merge kernel where its partials are
@@ -879,8 +846,7 @@ streamk_decode_kernel(StreamKParams p) {
         seq = nseq; kvh = nkvh; row_tiles = nrow_tiles; t = 0;
         nt = (int)min((int64_t)row_tiles, g1 - g);
         tab = tab_ready;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) qf[s] = qn[s];
+        qf = qn;
     }
 }
 
@@ -896,7 +862,7 @@ streamk_decode_kernel(StreamKParams p) {
 constexpr int RED_WGT = 256;       // weights parked in LDS per wave; rows with more partials recompute the rest
 template <typename E, int DQ>
 __global__ void __launch_bounds__(1024)
-streamk_reduce_kernel(uint16_t* __restrict__ out, const float* __restrict__ ws_acc,
+streamk_reduce_kernel(typename E::raw* __restrict__ out, const float* __restrict__ ws_acc,
                       const float* __restrict__ ws_ml, const int* __restrict__ ws_rows,
                       const int32_t* __restrict__ context_lens, int hq, int hkv, int group,
                       const float* __restrict__ v_scale, int head_slots) {
@@ -909,7 +875,7 @@ streamk_reduce_kernel(uint16_t* __restrict__ out, const float* __restrict__ ws_a
     __shared__ float part[16][DQ];
     float* wgt = wgt_all[wv];
     const int64_t row = (int64_t)seq * hkv + kvh;
-    uint16_t* o = out + ((int64_t)seq * hq + kvh * group + h) * DQ;
+    auto* o = out + ((int64_t)seq * hq + kvh * group + h) * DQ;
     // the length and the row's record are requested together (the record of an empty row was never
     // written and is not used)
     const int ctx = context_lens[seq];
@@ -1007,11 +973,13 @@ streamk_reduce_kernel(uint16_t* __restrict__ out, const float* __restrict__ ws_a
 // hence groups up to 8 and partitions of whole 64-token tiles)
 bool decode_mfma_supported(const DecodeArgs& a) {
     const int group = a.hkv > 0 ? a.hq / a.hkv : 0;
-    const bool shape = (a.d == D && group <= 16 && a.partition_size % TILE == 0) ||
-                       (a.d == 64 && group <= 8 && a.partition_size % (2 * TILE) == 0);
-    return a.cu_q_lens == nullptr && shape && a.bs == BS && is_16bit_float(a.q_dtype) &&
-           (a.kv_dtype == a.q_dtype || a.kv_dtype == AICOMP_KV_FP8_E4M3) && group >= 1 &&
-           a.scale > 0.f && a.rows <= 65535 &&
+    const bool f32 = a.q_dtype == AICOMP_KV_F32 && a.kv_dtype == AICOMP_KV_F32;
+    const bool half = is_16bit_float(a.q_dtype) && (a.kv_dtype == a.q_dtype || a.kv_dtype == AICOMP_KV_FP8_E4M3);
+    // tokens per tile: what a partition must be a multiple of
+    const int tile = f32 ? (a.d == D ? TILE / 2 : TILE) : (a.d == D ? TILE : 2 * TILE);
+    const bool shape = (a.d == D || a.d == 64) && group >= 1 && group <= (half && a.d == 64 ? 8 : 16) &&
+                       a.partition_size % tile == 0;
+    return a.cu_q_lens == nullptr && shape && a.bs == BS && (half || f32) && a.scale > 0.f && a.rows <= 65535 &&
            a.num_parts <= 65535 && ((uintptr_t)a.query % 16 == 0) && ((uintptr_t)a.k_pool % 16 == 0) &&
            ((uintptr_t)a.v_pool % 16 == 0);
 }
@@ -1063,15 +1031,18 @@ int launch_decode_streamk(const DecodeArgs& a, void* workspace) {
     p.ws_acc = (float*)workspace;
     p.ws_ml = p.ws_acc + slots * ncol * a.d;
     p.ws_rows = (int*)(p.ws_ml + slots * ncol * 2);
-    p.new_key = (const uint16_t*)a.new_key; p.new_value = (const uint16_t*)a.new_value;
+    p.new_key = a.new_key; p.new_value = a.new_value;
     p.new_token_stride = a.new_token_stride; p.new_head_stride = a.new_head_stride;
-    const bool fp8 = a.kv_dtype == AICOMP_KV_FP8_E4M3, f16 = a.q_dtype == AICOMP_KV_F16;
+    const bool fp8 = a.kv_dtype == AICOMP_KV_FP8_E4M3, f16 = a.q_dtype == AICOMP_KV_F16, f32 = a.q_dtype == AICOMP_KV_F32;
 #define AICOMP_LAUNCH_SK(E, PAIR)                                                                                  \
     do {                                                                                                           \
-        if (fp8) hipLaunchKernelGGL((streamk_decode_kernel<E, true, PAIR>), dim3(wgs), dim3(256), 0, a.stream, p);  \
-        else hipLaunchKernelGGL((streamk_decode_kernel<E, false, PAIR>), dim3(wgs), dim3(256), 0, a.stream, p);    \
+        if (fp8) hipLaunchKernelGGL((streamk_decode_kernel<Tile16<E, true, PAIR>>), dim3(wgs), dim3(256), 0, a.stream, p);  \
+        else hipLaunchKernelGGL((streamk_decode_kernel<Tile16<E, false, PAIR>>), dim3(wgs), dim3(256), 0, a.stream, p);    \
     } while (0)
-    if (pair) { if (f16) AICOMP_LAUNCH_SK(F16Fmt, true); else AICOMP_LAUNCH_SK(Bf16Fmt, true); }
+    if (f32) {
+        if (a.d == 64) hipLaunchKernelGGL((streamk_decode_kernel<TileF32<64>>), dim3(wgs), dim3(256), 0, a.stream, p);
+        else hipLaunchKernelGGL((streamk_decode_kernel<TileF32<128>>), dim3(wgs), dim3(256), 0, a.stream, p);
+    } else if (pair) { if (f16) AICOMP_LAUNCH_SK(F16Fmt, true); else AICOMP_LAUNCH_SK(Bf16Fmt, true); }
     else { if (f16) AICOMP_LAUNCH_SK(F16Fmt, false); else AICOMP_LAUNCH_SK(Bf16Fmt, false); }
 #undef AICOMP_LAUNCH_SK
     AICOMP_HIP_LAUNCH_CHECK();
@@ -1080,9 +1051,10 @@ int launch_decode_streamk(const DecodeArgs& a, void* workspace) {
     const int sub = per_row > 8 ? 16 / group : 1;
 #define AICOMP_LAUNCH_RED(E, DQ)                                                                                  \
     hipLaunchKernelGGL((streamk_reduce_kernel<E, DQ>), dim3(a.hkv, (unsigned)a.rows), dim3(64 * group * sub), 0,  \
-                       a.stream, (uint16_t*)a.out, p.ws_acc, p.ws_ml, p.ws_rows, a.context_lens, a.hq, a.hkv,     \
+                       a.stream, (E::raw*)a.out, p.ws_acc, p.ws_ml, p.ws_rows, a.context_lens, a.hq, a.hkv,     \
                        group, a.v_scale, p.waves_per_head + (int)a.rows)
-    if (pair) { if (f16) AICOMP_LAUNCH_RED(F16Fmt, 64); else AICOMP_LAUNCH_RED(Bf16Fmt, 64); }
+    if (f32) { if (a.d == 64) AICOMP_LAUNCH_RED(F32Fmt, 64); else AICOMP_LAUNCH_RED(F32Fmt, 128); }
+    else if (pair) { if (f16) AICOMP_LAUNCH_RED(F16Fmt, 64); else AICOMP_LAUNCH_RED(Bf16Fmt, 64); }
     else { if (f16) AICOMP_LAUNCH_RED(F16Fmt, 128); else AICOMP_LAUNCH_RED(Bf16Fmt, 128); }
 #undef AICOMP_LAUNCH_RED
     AICOMP_HIP_LAUNCH_CHECK();
@@ -1100,21 +1072,24 @@ int launch_decode_mfma(const DecodeArgs& a) {
     p.k_scale = a.k_scale; p.v_scale = a.v_scale;
     p.partition_size = a.partition_size; p.num_parts = a.num_parts;
     p.ws_acc = a.ws.acc; p.ws_ml = a.ws.ml;
-    p.new_key = (const uint16_t*)a.new_key; p.new_value = (const uint16_t*)a.new_value;
+    p.new_key = a.new_key; p.new_value = a.new_value;
     p.new_token_stride = a.new_token_stride; p.new_head_stride = a.new_head_stride;
     dim3 grid((unsigned)a.hkv, (unsigned)a.num_parts, (unsigned)a.rows);
     const bool fp8 = a.kv_dtype == AICOMP_KV_FP8_E4M3;
 #define AICOMP_LAUNCH_GRID(E)                                                                                       \
     do {                                                                                                            \
         if (a.d == 64) {                                                                                            \
-            if (fp8) hipLaunchKernelGGL((paged_decode_mfma_kernel<E, true, true>), grid, dim3(256), 0, a.stream, p); \
-            else hipLaunchKernelGGL((paged_decode_mfma_kernel<E, false, true>), grid, dim3(256), 0, a.stream, p);   \
+            if (fp8) hipLaunchKernelGGL((paged_decode_mfma_kernel<Tile16<E, true, true>>), grid, dim3(256), 0, a.stream, p); \
+            else hipLaunchKernelGGL((paged_decode_mfma_kernel<Tile16<E, false, true>>), grid, dim3(256), 0, a.stream, p);   \
         } else {                                                                                                    \
-            if (fp8) hipLaunchKernelGGL((paged_decode_mfma_kernel<E, true, false>), grid, dim3(256), 0, a.stream, p); \
-            else hipLaunchKernelGGL((paged_decode_mfma_kernel<E, false, false>), grid, dim3(256), 0, a.stream, p);  \
+            if (fp8) hipLaunchKernelGGL((paged_decode_mfma_kernel<Tile16<E, true, false>>), grid, dim3(256), 0, a.stream, p); \
+            else hipLaunchKernelGGL((paged_decode_mfma_kernel<Tile16<E, false, false>>), grid, dim3(256), 0, a.stream, p);  \
         }                                                                                                           \
     } while (0)
-    if (a.q_dtype == AICOMP_KV_F16) AICOMP_LAUNCH_GRID(F16Fmt);
+    if (a.q_dtype == AICOMP_KV_F32) {
+        if (a.d == 64) hipLaunchKernelGGL((paged_decode_mfma_kernel<TileF32<64>>), grid, dim3(256), 0, a.stream, p);
+        else hipLaunchKernelGGL((paged_decode_mfma_kernel<TileF32<128>>), grid, dim3(256), 0, a.stream, p);
+    } else if (a.q_dtype == AICOMP_KV_F16) AICOMP_LAUNCH_GRID(F16Fmt);
     else AICOMP_LAUNCH_GRID(Bf16Fmt);
 #undef AICOMP_LAUNCH_GRID
     AICOMP_HIP_LAUNCH_CHECK();

@@ -64,8 +64,8 @@ static bool streamk_shape(int batch, int hq, int hkv, int d, int bs, int q_dtype
 // A decode call over few, short rows is a chain of launch and memory latencies, not a stream: the
 // balanced schedule (set up for 256 CUs of work, always followed by its merge kernel) then loses to
 // one workgroup per (row, KV head, partition) on the grid schedule, without any merge kernel when
-// no row can be longer than 640 tokens (measured on 1 to 16 rows of 512 and 2048 tokens: 5.4-8.5
-// against 9-13 us, 8-15 against 11-17 us).  "Small" is rows x (table width x block size) at or
+// no row can be longer than 768 (head_dim 128) or 1280 (64) tokens of a 16-bit pool, 640 of another (measured on 1 to 16 rows of 512
+// and 2048 tokens: 5.4-8.5 against 9-13 us, 8-15 against 11-17 us).  "Small" is rows x (table width x block size) at or
 // below a process-wide threshold: 32768 by default, or the value of the environment variable
 // AICOMP_KV_SMALL_DECODE_TOKENS when the library first needs it (read once, never again), or what
 // aicomp_kv_set_small_decode_tokens() stored last (0 keeps every automatic call of a supported
@@ -82,14 +82,20 @@ static bool small_call(int64_t rows, int bs, int max_blocks) {
     return rows * (int64_t)max_blocks * bs <= small_decode_tokens().load(std::memory_order_relaxed);
 }
 
-static int auto_partition(int64_t rows, int hkv, int bs, int max_blocks, bool matrix_shape) {
+static int auto_partition(int64_t rows, int hkv, int d, int bs, int max_blocks, int kv_dtype, bool matrix_shape) {
     // Longer partitions amortise a workgroup's start-up and merge; shorter ones give the
     // 256 CUs enough workgroups when there are few (sequence, KV head) rows.
     const int64_t max_ctx = (int64_t)max_blocks * bs;
     int ps;
     if (matrix_shape && small_call(rows, bs, max_blocks)) {
-        // matrix-core grid schedule: whole rows (a whole number of its 64-token tiles), or 256 tokens
-        ps = max_ctx <= 640 ? (int)((max_ctx + 63) / 64 * 64) : 256;
+        // Matrix-core grid schedule: whole rows (a whole number of its 64-token tiles) and no merge
+        // launch, or partitions of 256 tokens.  The line lies where the merge's launch (about 3 us of
+        // device and 3 us of host time) costs what the longer chain of one workgroup does: 1000 and
+        // 1200 tokens at D 64 whole 7.2 and 7.4 us, split 8.0 us, 2000 tokens 9.7 and 7.9; D 128: 760
+        // tokens 7.7 and 8.8, 1000 tokens 9.2 and 8.2 us.  Other pools keep 640: float32 rows are bound by
+        // the matrix instruction of their one CU (640 tokens, D 128: 18.0 whole, 14.9 split in 256).
+        const int64_t whole = !is_16bit_float(kv_dtype) ? 640 : d == 64 ? 1280 : 768;
+        ps = max_ctx <= whole ? (int)((max_ctx + 63) / 64 * 64) : 256;
     } else {
         ps = 64;       // vector-ALU kernel on few short rows: spread the call wide
         for (int cand : {1024, 512, 256, 128}) {
@@ -208,12 +214,13 @@ int aicomp_paged_decode_partition_size(int batch, int num_q_heads, int num_kv_he
                                        int block_size, int max_blocks_per_seq, int q_dtype,
                                        int kv_dtype) {
     if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || block_size <= 0 || max_blocks_per_seq <= 0) return 0;
-    return auto_partition(batch, num_kv_heads, block_size, max_blocks_per_seq,
+    return auto_partition(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype,
                           streamk_shape(batch, num_q_heads, num_kv_heads, head_dim, block_size, q_dtype, kv_dtype));
 }
 
-static int resolve_parts(int64_t rows, int hkv, int bs, int max_blocks, bool matrix_shape, int& partition_size) {
-    if (partition_size <= 0) partition_size = auto_partition(rows, hkv, bs, max_blocks, matrix_shape);
+static int resolve_parts(int64_t rows, int hkv, int d, int bs, int max_blocks, int kv_dtype, bool matrix_shape,
+                         int& partition_size) {
+    if (partition_size <= 0) partition_size = auto_partition(rows, hkv, d, bs, max_blocks, kv_dtype, matrix_shape);
     const int64_t max_ctx = (int64_t)max_blocks * bs;
     int64_t parts = (max_ctx + partition_size - 1) / partition_size;
     return (int)(parts < 1 ? 1 : parts);
@@ -227,7 +234,7 @@ size_t aicomp_paged_decode_workspace_bytes(int batch, int num_q_heads, int num_k
         return 0;
     const bool automatic = partition_size <= 0;
     const bool matrix_shape = streamk_shape(batch, num_q_heads, num_kv_heads, head_dim, block_size, q_dtype, kv_dtype);
-    const int parts = resolve_parts(batch, num_kv_heads, block_size, max_blocks_per_seq, matrix_shape, partition_size);
+    const int parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, matrix_shape, partition_size);
     size_t need = parts <= 1 ? 0 : split_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, parts);
     if (automatic && matrix_shape && !small_call(batch, block_size, max_blocks_per_seq)) {
         const size_t sk = decode_streamk_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim);
@@ -274,7 +281,7 @@ static int decode_impl(void* out, const void* query, const void* new_key, const 
     a.v_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? v_scale : nullptr;
     a.partition_size = partition_size;
     const bool matrix_shape = streamk_shape(batch, num_q_heads, num_kv_heads, head_dim, block_size, q_dtype, kv_dtype);
-    a.num_parts = resolve_parts(batch, num_kv_heads, block_size, max_blocks_per_seq, matrix_shape, a.partition_size);
+    a.num_parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, matrix_shape, a.partition_size);
     a.stream = (hipStream_t)stream;
     // the matrix-core kernels append the new rows themselves when they can read them 16 bytes at a time
     const int64_t vec = 16 / dtype_size(q_dtype);

@@ -425,8 +425,8 @@ struct Tile16 {
 
 #include "decode_tile_f32.h"
 
-template <typename T>
-__global__ void __launch_bounds__(256, 2)
+template <typename T, int NW>
+__global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1)
 paged_decode_mfma_kernel(MfmaParams p) {
     // KV head fastest: the workgroups launched together read the Hkv slices of the same
     // physical blocks, i.e. one contiguous Hkv*4 KB piece of each pool
@@ -453,11 +453,7 @@ paged_decode_mfma_kernel(MfmaParams p) {
     int tab = (blk_base + lane < p.max_blocks) ? table[blk_base + lane] : 0;
 
     typename T::Q qf;
-    {
-        typename T::Q raw;
-        T::load_q(raw, p, seq, kvh, lane);
-        T::q_operand(qf, raw, G, lane);
-    }
+    T::load_q(qf, p, seq, kvh, lane);
 
     const int len = min(p.context_lens[seq], p.max_blocks * BS);   // never read past the table row
     if (start >= len) {
@@ -470,9 +466,9 @@ paged_decode_mfma_kernel(MfmaParams p) {
     const int end = min(len, start + p.partition_size);
     const int ntiles = (end - start + TT - 1) / TT;
 
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NWAVES * KTILE_BYTES];
-    __shared__ float sm_m[NWAVES][16];
-    __shared__ float sm_l[NWAVES][16];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[NW * KTILE_BYTES];
+    __shared__ float sm_m[NW][16];
+    __shared__ float sm_l[NW][16];
     unsigned char* kt = lds + w * KTILE_BYTES;
 
     const float cmul = p.qk_mul * (T::FP8 ? p.k_scale[kvh] : 1.f);
@@ -499,13 +495,11 @@ paged_decode_mfma_kernel(MfmaParams p) {
     if (w < ntiles) {
         typename T::Regs kv;
         tile_blocks(w);
-        // Q must have landed before the tile loads are issued: the loop's waits then count
-        // only tile loads, so a wave computes on tile t while tile t+1 is still in flight.
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
         T::load(kv, p, bb, kvh, lane);
+        T::q_operand(qf, qf, G, lane);
         int tt = w;
-        for (; tt + NWAVES < ntiles; tt += NWAVES) {      // steady state: never the partition's last tile
-            tile_blocks(tt + NWAVES);
+        for (; tt + NW < ntiles; tt += NW) {      // steady state: never the partition's last tile
+            tile_blocks(tt + NW);
             T::template process<true, false>(st, kv, qf, kt, ko, p, bb, kvh, lane, start + tt * TT, end, cmul);
         }
         const int tile_start = start + tt * TT;
@@ -541,16 +535,16 @@ paged_decode_mfma_kernel(MfmaParams p) {
     // elements 0..63 and 64..127 of their accumulators)
     const float vs = T::FP8 ? p.v_scale[kvh] : 1.f;
     const bool direct = p.num_parts == 1;     // unsplit call: no merge needed
-    for (int idx = tid; idx < G * DQ; idx += 256) {
+    for (int idx = tid; idx < G * DQ; idx += 64 * NW) {
         const int h = idx / DQ, dd = idx % DQ;
         float mxw = NEG_BIG;
 #pragma unroll
-        for (int ww = 0; ww < NWAVES; ++ww)
+        for (int ww = 0; ww < NW; ++ww)
 #pragma unroll
             for (int par = 0; par < NPAR; ++par) mxw = fmaxf(mxw, sm_m[ww][NPAR * h + par]);
         float num = 0.f, den = 0.f;
 #pragma unroll
-        for (int ww = 0; ww < NWAVES; ++ww) {
+        for (int ww = 0; ww < NW; ++ww) {
 #pragma unroll
             for (int par = 0; par < NPAR; ++par) {
                 const int c = NPAR * h + par;
@@ -1075,22 +1069,27 @@ int launch_decode_mfma(const DecodeArgs& a) {
     p.new_key = a.new_key; p.new_value = a.new_value;
     p.new_token_stride = a.new_token_stride; p.new_head_stride = a.new_head_stride;
     dim3 grid((unsigned)a.hkv, (unsigned)a.num_parts, (unsigned)a.rows);
-    const bool fp8 = a.kv_dtype == AICOMP_KV_FP8_E4M3;
-#define AICOMP_LAUNCH_GRID(E)                                                                                       \
-    do {                                                                                                            \
-        if (a.d == 64) {                                                                                            \
-            if (fp8) hipLaunchKernelGGL((paged_decode_mfma_kernel<Tile16<E, true, true>>), grid, dim3(256), 0, a.stream, p); \
-            else hipLaunchKernelGGL((paged_decode_mfma_kernel<Tile16<E, false, true>>), grid, dim3(256), 0, a.stream, p);   \
-        } else {                                                                                                    \
-            if (fp8) hipLaunchKernelGGL((paged_decode_mfma_kernel<Tile16<E, true, false>>), grid, dim3(256), 0, a.stream, p); \
-            else hipLaunchKernelGGL((paged_decode_mfma_kernel<Tile16<E, false, false>>), grid, dim3(256), 0, a.stream, p);  \
-        }                                                                                                           \
+    const bool fp8 = a.kv_dtype == AICOMP_KV_FP8_E4M3, d64 = a.d == 64;
+    // Eight waves instead of four per workgroup once a partition is more than sixteen tiles: such a call
+    // has few workgroups, each a chain of rounds of one tile per wave at memory latency, and half the
+    // rounds outweigh the longer merge (1 row of 600 tokens, D 128: 7.9 -> 6.5 us; 500 tokens, D 64,
+    // eight tiles: 5.72 us with four waves, 5.84 with eight; 16 rows of 500, D 128, sixteen: 8.70 and 8.88).
+    const int tile = a.q_dtype == AICOMP_KV_F32 ? (d64 ? TILE : TILE / 2) : (d64 ? 2 * TILE : TILE);
+    const bool wide = a.partition_size > 16 * tile;
+#define AICOMP_LAUNCH_GRID(...)                                                                                        \
+    do {                                                                                                               \
+        if (wide) hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 8>), grid, dim3(512), 0, a.stream, p);     \
+        else hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 4>), grid, dim3(256), 0, a.stream, p);          \
     } while (0)
-    if (a.q_dtype == AICOMP_KV_F32) {
-        if (a.d == 64) hipLaunchKernelGGL((paged_decode_mfma_kernel<TileF32<64>>), grid, dim3(256), 0, a.stream, p);
-        else hipLaunchKernelGGL((paged_decode_mfma_kernel<TileF32<128>>), grid, dim3(256), 0, a.stream, p);
-    } else if (a.q_dtype == AICOMP_KV_F16) AICOMP_LAUNCH_GRID(F16Fmt);
-    else AICOMP_LAUNCH_GRID(Bf16Fmt);
+#define AICOMP_LAUNCH_GRID16(E)                                                                     \
+    do {                                                                                            \
+        if (d64) { if (fp8) AICOMP_LAUNCH_GRID(Tile16<E, true, true>); else AICOMP_LAUNCH_GRID(Tile16<E, false, true>); } \
+        else { if (fp8) AICOMP_LAUNCH_GRID(Tile16<E, true, false>); else AICOMP_LAUNCH_GRID(Tile16<E, false, false>); }   \
+    } while (0)
+    if (a.q_dtype == AICOMP_KV_F32) { if (d64) AICOMP_LAUNCH_GRID(TileF32<64>); else AICOMP_LAUNCH_GRID(TileF32<128>); }
+    else if (a.q_dtype == AICOMP_KV_F16) AICOMP_LAUNCH_GRID16(F16Fmt);
+    else AICOMP_LAUNCH_GRID16(Bf16Fmt);
+#undef AICOMP_LAUNCH_GRID16
 #undef AICOMP_LAUNCH_GRID
     AICOMP_HIP_LAUNCH_CHECK();
     if (a.num_parts > 1) return launch_split_reduce(a);

@@ -125,8 +125,8 @@ int aicomp_kv_append(const void* key, const void* value,
  *                   (batch * max_blocks_per_seq * block_size at or below the process-wide
  *                   threshold of aicomp_kv_set_small_decode_tokens(), default 32768) runs one workgroup per (row, KV head,
  *                   256-token partition) instead, and no merge kernel at all when
- *                   max_blocks_per_seq * block_size <= 640: such a call is bound by
- *                   launch and memory latency, not by bandwidth.  The result is the
+ *                   max_blocks_per_seq * block_size <= 768 (head_dim 128) or 1280 (64) over a
+ *                   16-bit pool, 640 over another: such a call is bound by launch and memory latency, not by bandwidth.  The result is the
  *                   same to within the tolerance between split sizes (2e-3).
  *   workspace       device scratch of at least
  *                   aicomp_paged_decode_workspace_bytes(...) bytes (may be NULL

@@ -1,0 +1,26 @@
+"""The grid schedule's workgroups of eight waves (partitions of more than sixteen tiles) and its whole-row
+calls, around the lengths where the choice changes, against the float64 oracle at the bf16 bound."""
+import numpy as np
+import pytest
+import torch
+
+import test_gpu_prefill as tp
+from aicomp_amd import ops
+from helpers import assert_close_attn, to_f64
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d,kv,dtype,limit", [(128, None, torch.bfloat16, 768), (64, None, torch.float16, 1280),
+                                             (128, torch.float8_e4m3fn, torch.bfloat16, 640), (64, None, torch.float32, 640)])
+def test_rows_around_the_one_workgroup_limit(device, d, kv, dtype, limit):
+    ops.set_small_decode_tokens(1 << 40)                    # the grid schedule; restored by the suite's fixture
+    for longest in (limit - 255, limit - 16, limit, limit + 1):
+        ctx = [longest, 1, longest - 17, 40]
+        c = tp.build_case(device, [n - 1 for n in ctx], [1] * 4, 8, 2, d, dtype=dtype, kv_dtype=kv, seed=longest)
+        ps = ops.decode_partition_size(4, 8, 2, d, 16, c["table"].shape[1], dtype, kv or dtype)
+        assert ps == (-(-longest // 64) * 64 if longest <= limit else 256)
+        got = to_f64(ops.paged_decode_attn(torch.full_like(c["q"], float("nan")), c["q"], c["k_pool"], c["v_pool"], c["table"],
+                                           c["ctx"], c["scale"], c["ks"], c["vs"]))
+        assert_close_attn(got, tp.oracle(c), *((1e-5, 1e-5) if dtype == torch.float32 else (1e-2, 2e-2)), f"{d} {dtype} {longest}")
+        assert np.isfinite(got).all()

@@ -17,8 +17,15 @@
 // With an fp8 pool the rotated K and the V row are quantised like the plain append does.
 //
 // HBM-bound and small.  One lane owns 8 columns j .. j+7 of the low half and the matching
-// 8 of the high half of one (token, head) row: both halves of a rotation pair are in
-// the same lane, every access is a 16-byte (bf16) or 2 x 16-byte (fp32) vector.
+// 8 of the high half of one or two (token, head) rows: both halves of a rotation pair are in
+// the same lane, every access is a 16-byte (bf16) or 2 x 16-byte (fp32) vector.  A workgroup
+// holds one token: its position and slot are scalar loads, the row loads are on their way before
+// either has arrived, and the chain to the first store is two memory latencies instead of three.
+// Per-lane index division, one head per lane and a position test before the row loads took, for 2108
+// and 8192 tokens of 32 / 8 heads, D 128, bf16: 11.9 and 39.9 us; this 10.4 and 34.7 us (5.1 and
+// 5.9 TB/s of input read and output written); 2000 tokens of 64 / 8 heads into fp8 19.4 -> 15.9 us;
+// one token 2.7 -> 2.4 us.  Non-temporal row loads are slower at 2108 tokens (12.1 us): the projection
+// that made the rows left them in the memory-side cache.
 #include "common.h"
 
 namespace aicomp {
@@ -93,18 +100,119 @@ __device__ __forceinline__ uint2 quant8(const float* f, float scale) {
     return make_uint2((uint32_t)lo, (uint32_t)hi);
 }
 
-// out = round(round(x * c) + round(r * s)), products and sum as separate roundings
-template <typename T>
+// out = round(round(x * c) + round(r * s)), products and sum as separate roundings; NEG: -r in r's place
+// (rounding is symmetric, so the sign moves to the sum)
+template <typename T, bool NEG = false>
 __device__ __forceinline__ float rot1(float x, float r, float c, float s) {
 #pragma clang fp contract(off)
     const float p1 = Row8<T>::round(x * c);
     const float p2 = Row8<T>::round(r * s);
-    return Row8<T>::round(p1 + p2);
+    return Row8<T>::round(NEG ? p1 - p2 : p1 + p2);
 }
 
-template <typename T, bool FP8POOL>
+// 8 elements as they lie in memory
+template <typename T> struct Raw8 {
+    static constexpr int V16 = 8 * sizeof(T) / 16;
+    uint4 v[V16];
+    __device__ __forceinline__ void load(const T* p) {
+#pragma unroll
+        for (int k = 0; k < V16; ++k) v[k] = ((const uint4*)p)[k];
+    }
+    __device__ __forceinline__ void store(T* p) const {
+#pragma unroll
+        for (int k = 0; k < V16; ++k) ((uint4*)p)[k] = v[k];
+    }
+    __device__ __forceinline__ void unpack(float* f) const { Row8<T>::load((const T*)v, f); }
+};
+
+// One workgroup per token (and slice of its heads, blockIdx.y): position and slot are scalar loads, a
+// lane keeps its column chunk over its NI heads, so the cos / sin chunks are read once per lane, and
+// every Q / K / V load is issued before the position has arrived.  CH = chunks per row (head_dim / 16).
+template <typename T, bool FP8POOL, int CH, int NI>
 __global__ void __launch_bounds__(256)
 rope_kv_append_kernel(RopeParams p) {
+    const int64_t t = blockIdx.x;
+    const int c = (int)threadIdx.x & (CH - 1);
+    const int rows_it = (int)blockDim.x / CH;                         // heads per pass of the workgroup
+    const int hs0 = blockIdx.y * (NI * rows_it) + (int)threadIdx.x / CH;
+    const int nh = p.hq + 2 * p.hkv;
+    constexpr int D = 16 * CH, HALF = 8 * CH;
+    const int lo_col = 8 * c, hi_col = HALF + 8 * c;
+
+    Raw8<T> lo[NI], hi[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int hs = hs0 + i * rows_it;
+        if (hs < nh) {
+            const bool is_q = hs < p.hq, is_k = hs < p.hq + p.hkv;
+            const T* src = is_q ? (const T*)p.q_in + t * p.q_ts + hs * p.q_hs
+                                : (is_k ? (const T*)p.key + t * p.kv_ts + (hs - p.hq) * p.kv_hs
+                                        : (const T*)p.value + t * p.kv_ts + (hs - p.hq - p.hkv) * p.kv_hs);
+            lo[i].load(src + lo_col);
+            hi[i].load(src + hi_col);
+        }
+    }
+    const int64_t pos = p.positions ? p.positions[t] : t;
+    const int64_t slot = p.slot_mapping[t];
+    if (pos < 0 || pos >= p.tab_rows) return;                 // no table row: the token is left alone
+    const bool stored = slot >= 0 && slot < p.num_slots;      // otherwise a padding row: Q alone is rotated
+    const uint32_t blk = stored ? (uint32_t)slot / (uint32_t)p.bs : 0u;
+    const uint32_t off = stored ? (uint32_t)slot - blk * (uint32_t)p.bs : 0u;
+    const T* cr = (const T*)p.cos_tab + pos * p.tab_stride;
+    const T* sr = (const T*)p.sin_tab + pos * p.tab_stride;
+    Raw8<T> cl, ch, sl, sh;
+    cl.load(cr + lo_col); ch.load(cr + hi_col); sl.load(sr + lo_col); sh.load(sr + hi_col);
+
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int hs = hs0 + i * rows_it;
+        if (hs >= nh) break;
+        const bool is_q = hs < p.hq, is_k = !is_q && hs < p.hq + p.hkv;
+        if (!is_q && !stored) break;
+        const int h = is_q ? hs : (is_k ? hs - p.hq : hs - p.hq - p.hkv);
+        const int64_t row = ((int64_t)blk * p.hkv + h) * p.bs + off;          // pool row of D elements
+        if constexpr (!FP8POOL) {
+            if (!is_q && !is_k) {                             // V into a pool of its own type: raw bytes
+                T* dst = (T*)p.v_pool + row * D;
+                lo[i].store(dst + lo_col);
+                hi[i].store(dst + hi_col);
+                break;
+            }
+        }
+        float xl[8], xh[8];
+        lo[i].unpack(xl);
+        hi[i].unpack(xh);
+        if (is_q || is_k) {
+            float fcl[8], fch[8], fsl[8], fsh[8];
+            cl.unpack(fcl); ch.unpack(fch); sl.unpack(fsl); sh.unpack(fsh);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float ol = rot1<T, true>(xl[j], xh[j], fcl[j], fsl[j]);     // rotate_half: (-x2, x1)
+                xh[j] = rot1<T>(xh[j], xl[j], fch[j], fsh[j]);
+                xl[j] = ol;
+            }
+        }
+        if (is_q) {
+            T* dst = (T*)p.q_out + t * p.qo_ts + h * p.qo_hs;
+            Row8<T>::store(dst + lo_col, xl);
+            Row8<T>::store(dst + hi_col, xh);
+        } else if constexpr (FP8POOL) {
+            const float sc = (is_k ? p.k_scale : p.v_scale)[h];
+            uint8_t* dst = (uint8_t*)(is_k ? p.k_pool : p.v_pool) + row * D;
+            *(uint2*)(dst + lo_col) = quant8(xl, sc);
+            *(uint2*)(dst + hi_col) = quant8(xh, sc);
+        } else {
+            T* dst = (T*)p.k_pool + row * D;
+            Row8<T>::store(dst + lo_col, xl);
+            Row8<T>::store(dst + hi_col, xh);
+        }
+    }
+}
+
+// Any other head_dim (a multiple of 16): one lane per chunk of one (token, head) row.
+template <typename T, bool FP8POOL>
+__global__ void __launch_bounds__(256)
+rope_kv_append_any_kernel(RopeParams p) {
     // 32-bit index arithmetic throughout (the launcher bounds the lane count and the slot range)
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= (uint32_t)p.total) return;
@@ -161,7 +269,7 @@ rope_kv_append_kernel(RopeParams p) {
         Row8<T>::load(sr + hi_col, sh);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            ol[j] = rot1<T>(lo[j], -hi[j], cl[j], sl[j]);     // rotate_half: (-x2, x1)
+            ol[j] = rot1<T, true>(lo[j], hi[j], cl[j], sl[j]);     // rotate_half: (-x2, x1)
             oh[j] = rot1<T>(hi[j], lo[j], ch[j], sh[j]);
         }
 #pragma unroll
@@ -207,19 +315,49 @@ int launch_rope_kv_append(const void* q_in, void* q_out, int64_t q_ts, int64_t q
     AICOMP_REQUIRE(p.total < (int64_t)1 << 31 && p.num_slots < (int64_t)1 << 31, AICOMP_KV_EINVAL,
                    "rope_kv_append: %lld tokens / %lld slots exceed one launch's 32-bit index range",
                    (long long)num_tokens, (long long)p.num_slots);
-    const int64_t blocks = (p.total + 255) / 256;
     const bool fp8 = pool_dtype == AICOMP_KV_FP8_E4M3;
-    dim3 grid((unsigned)blocks), block(256);
-    if (in_dtype == AICOMP_KV_BF16) {
-        if (fp8) hipLaunchKernelGGL((rope_kv_append_kernel<bf16_t, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((rope_kv_append_kernel<bf16_t, false>), grid, block, 0, stream, p);
-    } else if (in_dtype == AICOMP_KV_F16) {
-        if (fp8) hipLaunchKernelGGL((rope_kv_append_kernel<f16_t, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((rope_kv_append_kernel<f16_t, false>), grid, block, 0, stream, p);
+#define AICOMP_ROPE(T, CH, NI)                                                                                       \
+    do {                                                                                                             \
+        if (fp8) hipLaunchKernelGGL((rope_kv_append_kernel<T, true, CH, NI>), grid, block, 0, stream, p);            \
+        else hipLaunchKernelGGL((rope_kv_append_kernel<T, false, CH, NI>), grid, block, 0, stream, p);               \
+    } while (0)
+#define AICOMP_ROPE_NI(T, CH)                                                                                        \
+    do {                                                                                                             \
+        if (ni == 1) AICOMP_ROPE(T, CH, 1); else AICOMP_ROPE(T, CH, 2);                                              \
+    } while (0)
+#define AICOMP_ROPE_T(T)                                                                                             \
+    do {                                                                                                             \
+        if (d == 64) AICOMP_ROPE_NI(T, 4); else AICOMP_ROPE_NI(T, 8);                                                \
+    } while (0)
+    if ((d == 64 || d == 128) && num_tokens <= INT32_MAX) {
+        const int items = (hq + 2 * hkv) * (d / 16);
+        // Two heads per lane (one read of the cos / sin chunks for both) once there are tokens enough to
+        // fill the chip, one below: 2108 tokens, 32 / 8 heads, D 128: 10.4 and 10.8 us; 64 tokens 2.79 and
+        // 2.55.  Workgroups of at most 128 lanes: of 256, 10.8 us; four heads per lane, 11.2 us.
+        constexpr int LANES = 128, TOKENS_TWO = 256;
+        const int ni = items > LANES && num_tokens >= TOKENS_TWO ? 2 : 1;
+        const int slices = (items + ni * LANES - 1) / (ni * LANES);
+        const int threads = (items + ni * slices * 64 - 1) / (ni * slices * 64) * 64;
+        dim3 grid((unsigned)num_tokens, (unsigned)slices), block(threads);
+        if (in_dtype == AICOMP_KV_BF16) AICOMP_ROPE_T(bf16_t);
+        else if (in_dtype == AICOMP_KV_F16) AICOMP_ROPE_T(f16_t);
+        else AICOMP_ROPE_T(float);
     } else {
-        if (fp8) hipLaunchKernelGGL((rope_kv_append_kernel<float, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((rope_kv_append_kernel<float, false>), grid, block, 0, stream, p);
+        const int64_t blocks = (p.total + 255) / 256;
+        dim3 grid((unsigned)blocks), block(256);
+#define AICOMP_ROPE_ANY(T)                                                                                           \
+    do {                                                                                                             \
+        if (fp8) hipLaunchKernelGGL((rope_kv_append_any_kernel<T, true>), grid, block, 0, stream, p);                \
+        else hipLaunchKernelGGL((rope_kv_append_any_kernel<T, false>), grid, block, 0, stream, p);                   \
+    } while (0)
+        if (in_dtype == AICOMP_KV_BF16) AICOMP_ROPE_ANY(bf16_t);
+        else if (in_dtype == AICOMP_KV_F16) AICOMP_ROPE_ANY(f16_t);
+        else AICOMP_ROPE_ANY(float);
+#undef AICOMP_ROPE_ANY
     }
+#undef AICOMP_ROPE_T
+#undef AICOMP_ROPE_NI
+#undef AICOMP_ROPE
     AICOMP_HIP_LAUNCH_CHECK();
     return AICOMP_KV_OK;
 }

@@ -1,0 +1,39 @@
+"""Rotary + append at the edges of the launch shapes: head counts that do not fill a workgroup's passes or
+need several slices, the token count where a lane takes two heads, head dims of both kernels, against the
+oracle bit for bit."""
+import pytest
+import torch
+
+from aicomp_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(1, 1, 64), (3, 1, 128), (16, 2, 128), (5, 5, 64), (32, 8, 128), (64, 8, 128), (7, 1, 96)])
+@pytest.mark.parametrize("T", [1, 255, 256])
+@pytest.mark.parametrize("kv", [None, torch.float8_e4m3fn])
+def test_launch_shapes(device, hq, hkv, d, T, kv):
+    dtype = torch.bfloat16
+    g = torch.Generator().manual_seed(hq + d + T)
+    qkv = torch.randn(T, hq + 2 * hkv, d, generator=g).to(dtype).to(device)
+    q, k, v = qkv[:, :hq], qkv[:, hq:hq + hkv], qkv[:, hq + hkv:]
+    cos, sin = ops.rotary_tables(1.0 / 10000.0 ** (torch.arange(0, d, 2) / d), 512, dtype, device=device)
+    pos = torch.randint(0, 512, (T,), generator=g).to(device)
+    blocks = T // 16 + 3
+    slots = torch.randperm(blocks * 16, generator=g)[:T]
+    slots[T // 2] = -1                                             # a padding row: Q is rotated, nothing is stored
+    slots = slots.to(device)
+    ks = vs = None
+    if kv is not None:
+        ks, vs = (torch.rand(hkv, generator=g).to(device) * 0.01 + 0.005 for _ in range(2))
+    kp, vp = (torch.zeros(blocks, hkv, 16, d, dtype=kv or dtype, device=device) for _ in range(2))
+    out = torch.empty(T, hq, d, dtype=dtype, device=device)
+    ops.rope_kv_append(q, k, v, cos, sin, pos, kp, vp, slots, ks, vs, query_out=out)
+    # torch's own evaluation of the same expression, one rounding per product and sum
+    half = lambda x: torch.cat((-x[..., d // 2:], x[..., :d // 2]), -1)
+    rot = lambda x: x * cos[pos][:, None] + half(x) * sin[pos][:, None]
+    kp2, vp2 = torch.zeros_like(kp), torch.zeros_like(vp)
+    ops.kv_append(rot(k).contiguous(), v.contiguous(), kp2, vp2, slots, ks, vs)
+    bits = lambda t: t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t.view(torch.int16)
+    assert torch.equal(bits(out), bits(rot(q)))
+    assert torch.equal(bits(kp), bits(kp2)) and torch.equal(bits(vp), bits(vp2))

@@ -100,8 +100,19 @@ def load() -> C.CDLL:
             if lib.aicomp_kv_version() < MIN_VERSION:
                 raise LibraryMissing(f"{LIB_PATH} is version {lib.aicomp_kv_version()}, this package needs "
                                      f">= {MIN_VERSION}: rebuild it with `python -m aicomp_amd.build`")
+            _entries.update((n, getattr(lib, n)) for n in SYMBOLS)
             _lib = lib
         return _lib
+
+
+_entries = {}
+
+
+def untouched(entry: str) -> bool:
+    """Whether the library's ctypes function is the one ``load`` found: a caller that put a wrapper in
+    its place (to count or trace calls) goes on seeing every call, by the ctypes route."""
+    lib = _lib or load()
+    return lib.__dict__.get(entry) is _entries[entry]
 
 
 TORCH_LIB_PATH = os.path.join(_HERE, "libaicomp_kv_torch.so")

@@ -185,8 +185,9 @@ class StepPlan:
     host_cu_q_lens: np.ndarray = None
     host_slot_mapping: np.ndarray = None
     host_positions: np.ndarray = None
-    # order of the prompt chunks' query tiles per (tile size, head groups): one list serves every layer of the step
+    # order of the prompt chunks' query tiles per head geometry and types: one list serves every layer of the step
     _prefill_items: dict = None
+    _only_chunks: Optional[bool] = None
 
     def prefill_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:
         """The (sequence, query tile) pairs of this step's prompt chunks, most expensive first, as the
@@ -197,19 +198,20 @@ class StepPlan:
         npre = self.num_prefill_seqs
         if npre < 2:
             return None
-        hq, hkv, d, bs = query.shape[1], k_pool.shape[1], k_pool.shape[3], k_pool.shape[2]
-        tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
-        if tile <= 0:
-            return None
-        group = hq // hkv
-        hgroups = hq // (group if 16 % group == 0 else 1)
-        key = (tile, hgroups, query.device)
+        (_, hq, _), (_, hkv, bs, d) = query.shape, k_pool.shape
         if self._prefill_items is None:
             self._prefill_items = {}
-        if key not in self._prefill_items:
-            cus = torch.cuda.get_device_properties(query.device).multi_processor_count if query.is_cuda else 0
-            items = ops.prefill_items(self.host_context_lens[:npre], self.new_lens[:npre], tile, hgroups, cus)
-            self._prefill_items[key] = torch.from_numpy(items).to(query.device, non_blocking=True)
+        key = ("chunks", hq, hkv, bs, d, query.dtype, k_pool.dtype, query.device)
+        if key not in self._prefill_items:         # (a layer's lookup costs 1 us, the library's tile size 4)
+            tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
+            items = None
+            if tile > 0:
+                group = hq // hkv
+                hgroups = hq // (group if 16 % group == 0 else 1)
+                cus = torch.cuda.get_device_properties(query.device).multi_processor_count if query.is_cuda else 0
+                items = ops.prefill_items(self.host_context_lens[:npre], self.new_lens[:npre], tile, hgroups, cus)
+                items = torch.from_numpy(items).to(query.device, non_blocking=True)
+            self._prefill_items[key] = items
         return self._prefill_items[key]
 
     # Longest decode row and largest decode batch for which a mixed step goes through one launch
@@ -233,22 +235,26 @@ class StepPlan:
             return None
         if query.dtype not in (torch.bfloat16, torch.float16) or k_pool.dtype != query.dtype:
             return None
-        if int(self.host_context_lens[npre:].max()) > self.ONE_LAUNCH_MAX_CONTEXT:
-            return None
-        hq, hkv, d, bs = query.shape[1], k_pool.shape[1], k_pool.shape[3], k_pool.shape[2]
-        tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
-        group = hq // hkv
-        gpack = group if 16 % group == 0 else 1
-        if tile * gpack != 128:                   # (0: no list; 64: the one-column-group kernel)
-            return None
-        hgroups = hq // gpack
-        key = ("step", tile, hgroups, query.device)
         if self._prefill_items is None:
             self._prefill_items = {}
+        longest = self._prefill_items.get("longest row")
+        if longest is None:
+            longest = self._prefill_items["longest row"] = int(self.host_context_lens[npre:].max())
+        if longest > self.ONE_LAUNCH_MAX_CONTEXT:
+            return None
+        (_, hq, _), (_, hkv, bs, d) = query.shape, k_pool.shape
+        key = ("step", hq, hkv, bs, d, query.dtype, query.device)
         if key not in self._prefill_items:
-            cus = torch.cuda.get_device_properties(query.device).multi_processor_count if query.is_cuda else 0
-            items = ops.step_items(self.host_context_lens, self.new_lens, npre, tile, hgroups, cus)
-            self._prefill_items[key] = torch.from_numpy(items).to(query.device, non_blocking=True)
+            tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
+            group = hq // hkv
+            gpack = group if 16 % group == 0 else 1
+            items = None
+            if tile * gpack == 128:               # (0: no list; 64: the one-column-group kernel)
+                hgroups = hq // gpack
+                cus = torch.cuda.get_device_properties(query.device).multi_processor_count if query.is_cuda else 0
+                items = ops.step_items(self.host_context_lens, self.new_lens, npre, tile, hgroups, cus)
+                items = torch.from_numpy(items).to(query.device, non_blocking=True)
+            self._prefill_items[key] = items
         return self._prefill_items[key]
 
     @property
@@ -258,6 +264,16 @@ class StepPlan:
     @property
     def num_decode_seqs(self) -> int:
         return len(self.seq_ids) - self.num_prefill_seqs
+
+    @property
+    def only_chunks(self) -> bool:
+        """Prompt chunks and nothing else, and device tensors of exactly their sizes."""
+        if self._only_chunks is None:
+            S, T = self.num_seqs, self.num_prefill_tokens
+            self._only_chunks = (0 < S == self.num_prefill_seqs and self.block_table.shape[0] == S
+                                 and self.context_lens.shape[0] == S and self.cu_q_lens.shape[0] == S + 1
+                                 and self.slot_mapping.shape[0] == T)
+        return self._only_chunks
 
     @property
     def num_prefill_tokens(self) -> int:
@@ -623,6 +639,15 @@ def paged_attention_step(plan: StepPlan, out: torch.Tensor, query: torch.Tensor,
         return ops.paged_prefill_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens,
                                       plan.cu_q_lens, scale, max_q_len=plan.max_q_len, k_scale=k_scale,
                                       v_scale=v_scale, items=items)
+    if plan.only_chunks and t_pre == query.shape[0] == out.shape[0] == key.shape[0] == value.shape[0]:
+        # chunks alone: the tensors as they are (a slice costs a microsecond)
+        ops.kv_append(key, value, k_pool, v_pool, plan.slot_mapping, k_scale, v_scale)
+        return ops.paged_prefill_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens, plan.cu_q_lens,
+                                      scale, max_q_len=plan.max_q_len, k_scale=k_scale, v_scale=v_scale,
+                                      items=plan.prefill_items(query, k_pool))
+    if S and npre == 0:
+        return ops.paged_decode_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens, scale, k_scale,
+                                     v_scale, new_key=key, new_value=value)
     if npre:
         ops.kv_append(key[:t_pre], value[:t_pre], k_pool, v_pool, plan.slot_mapping[:t_pre], k_scale, v_scale)
         ops.paged_prefill_attn(out[:t_pre], query[:t_pre], k_pool, v_pool, plan.block_table[:npre],

@@ -11,6 +11,11 @@
 //   out   = _aicomp_fast.decode_step(layer, query, key, value, position, group, scale)
 //
 // Same checks, same errors (RuntimeError), same results as the registered operator.
+//
+// Beside it, the plain calls of aicomp_amd.ops (kv_append, rope_kv_append, paged_decode_attn,
+// paged_prefill_attn, sample_tokens): the same checks made here instead of in Python.  A call that
+// passes them all is launched and returns true; any other returns false without having touched
+// anything, and the Python function goes on to convert what may be converted or to name what is wrong.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -20,6 +25,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
+#include <climits>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -53,7 +59,7 @@ void layer_free(PyObject* cap) { delete (Layer*)PyCapsule_GetPointer(cap, "aicom
 
 // scratch of calls that need a merge: one growing buffer per (device, stream), never destroyed
 // (tensors freed at interpreter exit, after the allocator, would fault)
-at::Tensor& cached_scratch(const c10::Device& dev, void* stream, size_t bytes) {
+at::Tensor cached_scratch(const c10::Device& dev, void* stream, size_t bytes) {
     static std::mutex mu;
     static auto* table = new std::map<std::pair<int, void*>, at::Tensor>();
     std::lock_guard<std::mutex> lock(mu);
@@ -140,10 +146,11 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         void* stream = (void*)c10::hip::getCurrentHIPStream(L->dev.index()).stream();
         size_t ws_bytes = aicomp_paged_decode_workspace_bytes(L->B, hq, L->hkv, L->d, L->bs, width, L->dt, L->dt, 0);
         void* ws = nullptr;
+        at::Tensor scratch;
         if (ws_bytes) {
-            at::Tensor& t = cached_scratch(L->dev, stream, ws_bytes);
-            ws = t.data_ptr();
-            ws_bytes = (size_t)t.numel();
+            scratch = cached_scratch(L->dev, stream, ws_bytes);
+            ws = scratch.data_ptr();
+            ws_bytes = (size_t)scratch.numel();
         }
         // (the allocator's own entry: at::empty goes through the dispatcher for the same result)
         at::Tensor out(at::detail::empty_cuda(query.sizes(), L->st, L->dev, c10::MemoryFormat::Contiguous));
@@ -158,14 +165,298 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
 }
 
+// ---------------------------------------------------------------- the plain calls of aicomp_amd.ops
+// Host time was what bounded these calls: their checks alone, a few dozen attribute reads of Python
+// tensors, cost 15 to 20 us a call, where the kernels of a decode or rotary call of ordinary size
+// need 3 to 12 (measured per call: see the wrappers in ops.py).
+
+int any_dtype_code(at::ScalarType t) { return t == at::kFloat8_e4m3fn ? AICOMP_KV_FP8_E4M3 : dtype_code(t); }
+
+// The tensor behind an argument, or null unless it is a plain strided tensor on a GPU with storage of
+// its own (no subclass, no wrapper of a transform): those go the Python way.
+const at::Tensor* plain(PyObject* o) {
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() ? &t : nullptr;
+}
+
+bool on(const at::Tensor& t, const at::Tensor& ref) { return t.device() == ref.device(); }
+
+struct Pools {
+    const at::Tensor *k, *v;
+    int64_t nb;
+    int hkv, bs, d, dt;
+    const float *ks = nullptr, *vs = nullptr;
+
+    bool get(PyObject* ko, PyObject* vo) {
+        k = plain(ko); v = plain(vo);
+        if (!k || !v || k->dim() != 4 || v->sizes() != k->sizes() || k->scalar_type() != v->scalar_type() ||
+            !k->is_contiguous() || !v->is_contiguous() || !on(*v, *k))
+            return false;
+        dt = any_dtype_code(k->scalar_type());
+        nb = k->size(0); hkv = (int)k->size(1); bs = (int)k->size(2); d = (int)k->size(3);
+        return dt >= 0;
+    }
+    // the scales of an fp8 pool; other pools have none, whatever is passed
+    bool scales(PyObject* kso, PyObject* vso) {
+        if (dt != AICOMP_KV_FP8_E4M3) return true;
+        const at::Tensor *a = plain(kso), *b = plain(vso);
+        for (const at::Tensor* s : {a, b})
+            if (!s || s->scalar_type() != at::kFloat || !s->is_contiguous() || s->numel() != hkv || !on(*s, *k)) return false;
+        ks = (const float*)a->data_ptr(); vs = (const float*)b->data_ptr();
+        return true;
+    }
+};
+
+bool vector_of(const at::Tensor* t, at::ScalarType st, int64_t n, const at::Tensor& ref) {
+    return t && t->scalar_type() == st && t->numel() == n && t->is_contiguous() && on(*t, ref);
+}
+
+bool as_double(PyObject* o, double& x) {
+    if (!PyFloat_CheckExact(o) && !PyLong_CheckExact(o)) return false;
+    x = PyFloat_AsDouble(o);
+    if (x == -1.0 && PyErr_Occurred()) { PyErr_Clear(); return false; }
+    return true;
+}
+
+bool as_int(PyObject* o, int& x) {
+    if (!PyLong_CheckExact(o)) return false;
+    int overflow = 0;
+    const long v = PyLong_AsLongAndOverflow(o, &overflow);
+    if (overflow || v < INT_MIN || v > INT_MAX) return false;
+    x = (int)v;
+    return true;
+}
+
+void* stream_of(const at::Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// runs a library call without the interpreter lock (a launch waits while the stream's queue is full)
+template <typename F> int unlocked(F call) {
+    PyThreadState* state = PyEval_SaveThread();
+    const int rc = call();
+    PyEval_RestoreThread(state);
+    return rc;
+}
+
+#define DONE(rc)                                                                                     \
+    do {                                                                                             \
+        if ((rc) != AICOMP_KV_OK) FAIL("aicomp_kv error %d: %s", (rc), aicomp_kv_last_error());      \
+        Py_RETURN_TRUE;                                                                              \
+    } while (0)
+
+PyObject* kv_append(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        Pools p;
+        if (nargs != 7) FAIL("kv_append(key, value, k_pool, v_pool, slot_mapping, k_scale, v_scale)");
+        const at::Tensor *key = plain(args[0]), *value = plain(args[1]), *slots = plain(args[4]);
+        if (!key || !value || !p.get(args[2], args[3]) || key->dim() != 3 || value->sizes() != key->sizes() ||
+            value->scalar_type() != key->scalar_type() || key->size(1) != p.hkv || key->size(2) != p.d ||
+            !slots || slots->dim() != 1 || !vector_of(slots, at::kLong, key->size(0), *key) || !on(*value, *key) ||
+            !on(*p.k, *key) || key->stride(2) != 1 || key->strides() != value->strides())
+            Py_RETURN_FALSE;
+        const int dt = any_dtype_code(key->scalar_type());
+        if (dt < 0 || (dt != p.dt && !p.scales(args[5], args[6]))) Py_RETURN_FALSE;
+        const c10::DeviceGuard guard(key->device());
+        void* stream = stream_of(*key);
+        const int rc = unlocked([&] {
+            return aicomp_kv_append(key->data_ptr(), value->data_ptr(), key->stride(0), key->stride(1), p.k->data_ptr(),
+                                    p.v->data_ptr(), (const int64_t*)slots->data_ptr(), key->size(0), p.hkv, p.d, p.bs,
+                                    p.nb, dt, p.dt, p.ks, p.vs, stream);
+        });
+        DONE(rc);
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
+PyObject* rope_kv_append(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        Pools p;
+        if (nargs != 12)
+            FAIL("rope_kv_append(query, key, value, cos, sin, positions, k_pool, v_pool, slot_mapping, k_scale, v_scale, out)");
+        const at::Tensor *q = plain(args[0]), *key = plain(args[1]), *value = plain(args[2]), *cos = plain(args[3]),
+                         *sin = plain(args[4]), *slots = plain(args[8]), *out = plain(args[11]);
+        const bool by_row = args[5] == Py_None;
+        const at::Tensor* pos = by_row ? nullptr : plain(args[5]);
+        if (!q || !key || !value || !cos || !sin || !out || (!by_row && !pos) || !p.get(args[6], args[7]) ||
+            q->dim() != 3 || key->dim() != 3 || value->sizes() != key->sizes() || out->sizes() != q->sizes())
+            Py_RETURN_FALSE;
+        const int64_t T = q->size(0);
+        const at::ScalarType st = q->scalar_type();
+        const int dt = dtype_code(st);
+        if (T == 0 || dt < 0 || key->size(0) != T || key->size(1) != p.hkv || key->size(2) != p.d || q->size(2) != p.d ||
+            key->scalar_type() != st || value->scalar_type() != st || out->scalar_type() != st || q->stride(2) != 1 ||
+            out->stride(2) != 1 || key->stride(2) != 1 || key->strides() != value->strides() || cos->dim() != 2 ||
+            cos->size(1) != p.d || sin->sizes() != cos->sizes() || cos->scalar_type() != st || sin->scalar_type() != st ||
+            cos->stride(1) != 1 || cos->strides() != sin->strides())
+            Py_RETURN_FALSE;
+        if (by_row ? cos->size(0) < T : !vector_of(pos, at::kLong, T, *q)) Py_RETURN_FALSE;
+        if (!vector_of(slots, at::kLong, T, *q) || !on(*key, *q) || !on(*value, *q) || !on(*out, *q) || !on(*cos, *q) ||
+            !on(*sin, *q) || !on(*p.k, *q) || (p.dt != dt && p.dt != AICOMP_KV_FP8_E4M3) || !p.scales(args[9], args[10]))
+            Py_RETURN_FALSE;
+        const c10::DeviceGuard guard(q->device());
+        void* stream = stream_of(*q);
+        const int rc = unlocked([&] {
+            return aicomp_rope_kv_append(
+                q->data_ptr(), out->data_ptr(), q->stride(0), q->stride(1), out->stride(0), out->stride(1),
+                key->data_ptr(), value->data_ptr(), key->stride(0), key->stride(1), cos->data_ptr(), sin->data_ptr(),
+                cos->stride(0), cos->size(0), pos ? (const int64_t*)pos->data_ptr() : nullptr, p.k->data_ptr(),
+                p.v->data_ptr(), (const int64_t*)slots->data_ptr(), T, (int)q->size(1), p.hkv, p.d, p.bs, p.nb, dt, p.dt,
+                p.ks, p.vs, stream);
+        });
+        DONE(rc);
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
+// what a decode and a prefill call share
+bool attention_args(PyObject* const* args, const at::Tensor*& out, const at::Tensor*& q, Pools& p, const at::Tensor*& table,
+                    const at::Tensor*& ctx, int& dt, int64_t& rows) {
+    out = plain(args[0]); q = plain(args[1]); table = plain(args[4]); ctx = plain(args[5]);
+    if (!out || !q || !table || !ctx || !p.get(args[2], args[3]) || q->dim() != 3 || out->sizes() != q->sizes() ||
+        out->scalar_type() != q->scalar_type() || q->size(2) != p.d || !q->is_contiguous() || !out->is_contiguous())
+        return false;
+    dt = any_dtype_code(q->scalar_type());
+    rows = ctx->numel();
+    return dt >= 0 && vector_of(ctx, at::kInt, rows, *q) && table->scalar_type() == at::kInt && table->dim() == 2 &&
+           table->size(0) == rows && table->stride(1) == 1 && on(*table, *q) && on(*out, *q) && on(*p.k, *q);
+}
+
+PyObject* paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        Pools p;
+        const at::Tensor *out, *q, *table, *ctx;
+        int dt, partition;
+        int64_t B;
+        double scale;
+        if (nargs != 13)
+            FAIL("paged_decode_attn(out, query, k_pool, v_pool, block_table, context_lens, scale, k_scale, v_scale, "
+                 "partition_size, workspace, new_key, new_value)");
+        if (!attention_args(args, out, q, p, table, ctx, dt, B) || B != q->size(0) || !as_double(args[6], scale) ||
+            !p.scales(args[7], args[8]) || !as_int(args[9], partition))
+            Py_RETURN_FALSE;
+        const at::Tensor *nk = nullptr, *nv = nullptr;
+        if (args[11] != Py_None) {
+            nk = plain(args[11]); nv = plain(args[12]);
+            if (!nk || !nv || nk->dim() != 3 || nk->size(0) != B || nk->size(1) != p.hkv || nk->size(2) != p.d ||
+                nv->sizes() != nk->sizes() || nk->scalar_type() != q->scalar_type() ||
+                nv->scalar_type() != q->scalar_type() || !on(*nk, *q) || !on(*nv, *q) || nk->stride(2) != 1 ||
+                nk->strides() != nv->strides())
+                Py_RETURN_FALSE;
+        }
+        const int hq = (int)q->size(1), width = (int)table->size(1);
+        const c10::DeviceGuard guard(q->device());
+        void* stream = stream_of(*q);
+        at::Tensor scratch;
+        if (args[10] != Py_None) {
+            const at::Tensor* w = plain(args[10]);
+            if (!w) Py_RETURN_FALSE;
+            scratch = *w;
+        } else {
+            const size_t need = aicomp_paged_decode_workspace_bytes((int)B, hq, p.hkv, p.d, p.bs, width, dt, p.dt, partition);
+            if (need) scratch = cached_scratch(q->device(), stream, need);
+        }
+        void* ws = scratch.defined() ? scratch.data_ptr() : nullptr;
+        const size_t ws_bytes = scratch.defined() ? (size_t)(scratch.numel() * scratch.element_size()) : 0;
+        const int rc = unlocked([&] {
+            const int32_t *bt = (const int32_t*)table->data_ptr(), *cl = (const int32_t*)ctx->data_ptr();
+            if (nk)
+                return aicomp_paged_decode_attn_append(
+                    out->data_ptr(), q->data_ptr(), nk->data_ptr(), nv->data_ptr(), nk->stride(0), nk->stride(1),
+                    p.k->data_ptr(), p.v->data_ptr(), bt, table->stride(0), cl, (int)B, hq, p.hkv, p.d, p.bs, width, p.nb,
+                    (float)scale, dt, p.dt, p.ks, p.vs, partition, ws, ws_bytes, stream);
+            return aicomp_paged_decode_attn(out->data_ptr(), q->data_ptr(), p.k->data_ptr(), p.v->data_ptr(), bt,
+                                            table->stride(0), cl, (int)B, hq, p.hkv, p.d, p.bs, width, p.nb, (float)scale,
+                                            dt, p.dt, p.ks, p.vs, partition, ws, ws_bytes, stream);
+        });
+        DONE(rc);
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
+PyObject* paged_prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        Pools p;
+        const at::Tensor *out, *q, *table, *ctx;
+        int dt, max_q_len;
+        int64_t S;
+        double scale;
+        if (nargs != 12)
+            FAIL("paged_prefill_attn(out, query, k_pool, v_pool, block_table, context_lens, cu_q_lens, scale, max_q_len, "
+                 "k_scale, v_scale, items)");
+        if (!attention_args(args, out, q, p, table, ctx, dt, S) || !as_double(args[7], scale) ||
+            !as_int(args[8], max_q_len) || !p.scales(args[9], args[10]))
+            Py_RETURN_FALSE;
+        const at::Tensor* cu = plain(args[6]);
+        if (!vector_of(cu, at::kInt, S + 1, *q)) Py_RETURN_FALSE;
+        const at::Tensor* items = nullptr;
+        if (args[11] != Py_None) {
+            items = plain(args[11]);
+            if (!items || items->numel() == 0 || items->scalar_type() != at::kInt || items->dim() != 2 ||
+                items->size(1) != 2 || items->size(0) > INT_MAX || !items->is_contiguous() || !on(*items, *q))
+                Py_RETURN_FALSE;
+        }
+        const c10::DeviceGuard guard(q->device());
+        void* stream = stream_of(*q);
+        const int rc = unlocked([&] {
+            return aicomp_paged_prefill_attn_items(
+                out->data_ptr(), q->data_ptr(), p.k->data_ptr(), p.v->data_ptr(), (const int32_t*)table->data_ptr(),
+                table->stride(0), (const int32_t*)ctx->data_ptr(), (const int32_t*)cu->data_ptr(), (int)S, q->size(0),
+                max_q_len, (int)q->size(1), p.hkv, p.d, p.bs, (int)table->size(1), p.nb, (float)scale, dt, p.dt, p.ks, p.vs,
+                items ? (const int32_t*)items->data_ptr() : nullptr, items ? (int)items->size(0) : 0, stream);
+        });
+        DONE(rc);
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
+// (tokens come back as a new tensor; None: take the Python way)
+PyObject* sample_tokens(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        if (nargs != 6) FAIL("sample_tokens(logits, temperature, top_k, top_p, do_sample, uniforms)");
+        const at::Tensor *x = plain(args[0]), *u = nullptr;
+        double temperature, top_p;
+        int top_k;
+        if (!x || x->dim() != 2 || x->size(0) == 0 || x->size(0) > INT_MAX || x->size(1) > INT_MAX || x->stride(1) != 1 ||
+            dtype_code(x->scalar_type()) < 0 || !as_double(args[1], temperature) || !as_int(args[2], top_k) ||
+            !as_double(args[3], top_p) || !PyBool_Check(args[4]))
+            Py_RETURN_NONE;
+        const bool sample = args[4] == Py_True;
+        if (sample && !vector_of(u = plain(args[5]), at::kFloat, x->size(0), *x)) Py_RETURN_NONE;
+        const c10::DeviceGuard guard(x->device());
+        void* stream = stream_of(*x);
+        at::Tensor out(at::detail::empty_cuda({x->size(0)}, at::kLong, x->device(), c10::MemoryFormat::Contiguous));
+        const int rc = unlocked([&] {
+            return aicomp_sample_tokens((int64_t*)out.data_ptr(), x->data_ptr(), x->stride(0), nullptr,
+                                        sample ? (const float*)u->data_ptr() : nullptr, (int)x->size(0), (int)x->size(1),
+                                        (float)temperature, top_k, (float)top_p, sample ? 0 : 1,
+                                        dtype_code(x->scalar_type()), stream);
+        });
+        if (rc != AICOMP_KV_OK) FAIL("aicomp_kv error %d: %s", rc, aicomp_kv_last_error());
+        return THPVariable_Wrap(std::move(out));
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
+#define FAST(f) (PyCFunction)(void (*)(void))f, METH_FASTCALL
+
 PyMethodDef methods[] = {
     {"layer", (PyCFunction)(void (*)(void))layer_new, METH_FASTCALL,
      "layer(k_pool, v_pool, block_table, ctx_rows) -> handle: a layer's static tensors, checked once"},
     {"decode_step", (PyCFunction)(void (*)(void))decode_step, METH_FASTCALL,
      "decode_step(layer, query, key, value, position, group, scale) -> out [B, Hq, 1, D]"},
+    {"kv_append", FAST(kv_append), "ops.kv_append of a plain call: True once launched, False if it is not one"},
+    {"rope_kv_append", FAST(rope_kv_append), "ops.rope_kv_append of a plain call, out given"},
+    {"paged_decode_attn", FAST(paged_decode_attn), "ops.paged_decode_attn of a plain call"},
+    {"paged_prefill_attn", FAST(paged_prefill_attn), "ops.paged_prefill_attn of a plain call, max_q_len given"},
+    {"sample_tokens", FAST(sample_tokens), "ops.sample_tokens of a plain call: the tokens, or None if it is not one"},
     {nullptr, nullptr, 0, nullptr}};
 
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "_aicomp_fast", "decode step of the paged KV-cache operator, lean host route",
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_aicomp_fast", "lean host routes into the paged KV-cache library",
                       -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

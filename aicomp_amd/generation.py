@@ -83,6 +83,12 @@ class PagedAttentionBackend:
         if items is not None:                      # mixed step: chunks and decode rows in one launch
             return ops.paged_prefill_attn(out, q, kp, vp, plan.block_table, plan.context_lens, plan.cu_q_lens,
                                           self.scale, max_q_len=plan.max_q_len, k_scale=ks, v_scale=vs, items=items)
+        if plan.only_chunks and t_pre == query.shape[0]:     # chunks alone, rows alone: the plan's tensors as they are
+            return ops.paged_prefill_attn(out, q, kp, vp, plan.block_table, plan.context_lens, plan.cu_q_lens, self.scale,
+                                          max_q_len=plan.max_q_len, k_scale=ks, v_scale=vs,
+                                          items=plan.prefill_items(q, kp))
+        if S and npre == 0:
+            return ops.paged_decode_attn(out, q, kp, vp, plan.block_table, plan.context_lens, self.scale, ks, vs)
         if npre:
             ops.paged_prefill_attn(out[:t_pre], q[:t_pre], kp, vp, plan.block_table[:npre], plan.context_lens[:npre],
                                    plan.cu_q_lens[:npre + 1], self.scale, max_q_len=plan.max_q_len,

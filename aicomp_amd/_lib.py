@@ -27,10 +27,12 @@ SYMBOLS = (
     "aicomp_paged_prefill_tile_positions",
     "aicomp_rope_kv_append",
     "aicomp_sample_tokens",
+    "aicomp_sample_tokens_split",
+    "aicomp_sample_workspace_bytes",
 )
 
 F32, BF16, FP8_E4M3, F16 = 0, 1, 2, 3
-MIN_VERSION = 200            # 0.2.0: the entry points of SYMBOLS above
+MIN_VERSION = 300            # 0.3.0: the entry points of SYMBOLS above
 
 _lock = threading.RLock()       # torch_ops() loads the HIP library while holding it
 _lib = None
@@ -81,6 +83,10 @@ def _declare(lib: C.CDLL) -> None:
                                           vp, vp, vp, i64, i32, i32, i32, i32, i64, i32, i32, vp, vp, vp]
     lib.aicomp_sample_tokens.restype = i32
     lib.aicomp_sample_tokens.argtypes = [vp, vp, i64, vp, vp, i32, i32, f32, i32, f32, i32, i32, vp]
+    lib.aicomp_sample_tokens_split.restype = i32
+    lib.aicomp_sample_tokens_split.argtypes = [vp, vp, i64, vp, vp, i32, i32, f32, i32, f32, i32, i32, vp, sz, vp]
+    lib.aicomp_sample_workspace_bytes.restype = sz
+    lib.aicomp_sample_workspace_bytes.argtypes = [i32, i32, i64, f32, i32, i32, i32]
 
 
 def load() -> C.CDLL:

@@ -112,7 +112,7 @@ using namespace aicomp;
 
 extern "C" {
 
-int aicomp_kv_version(void) { return 200; }
+int aicomp_kv_version(void) { return 300; }
 
 const char* aicomp_kv_last_error(void) { return g_err; }
 
@@ -190,11 +190,13 @@ int aicomp_rope_kv_append(const void* q_in, void* q_out, int64_t q_token_stride,
                                  in_dtype, pool_dtype, k_scale, v_scale, (hipStream_t)stream);
 }
 
-int aicomp_sample_tokens(int64_t* out, const void* logits, int64_t row_stride, float* probs_out,
-                         const float* uniforms, int batch, int vocab, float temperature, int top_k,
-                         float top_p, int greedy, int logits_dtype, void* stream) {
+int aicomp_sample_tokens_split(int64_t* out, const void* logits, int64_t row_stride, float* probs_out,
+                               const float* uniforms, int batch, int vocab, float temperature, int top_k,
+                               float top_p, int greedy, int logits_dtype, void* workspace,
+                               size_t workspace_bytes, void* stream) {
     AICOMP_REQUIRE(batch >= 0, AICOMP_KV_EINVAL, "sample_tokens: negative batch");
     if (batch == 0) return AICOMP_KV_OK;
+    AICOMP_REQUIRE((uintptr_t)workspace % 8 == 0, AICOMP_KV_EINVAL, "sample_tokens: workspace must be 8-byte aligned");
     AICOMP_REQUIRE(out && logits, AICOMP_KV_EINVAL, "sample_tokens: null pointer");
     AICOMP_REQUIRE(vocab > 0 && row_stride >= vocab, AICOMP_KV_EINVAL,
                    "sample_tokens: bad sizes (vocab %d, row stride %lld)", vocab, (long long)row_stride);
@@ -207,7 +209,20 @@ int aicomp_sample_tokens(int64_t* out, const void* logits, int64_t row_stride, f
         AICOMP_REQUIRE(top_p == top_p, AICOMP_KV_EINVAL, "sample_tokens: top_p is NaN");
     }
     return launch_sample(out, logits, row_stride, probs_out, uniforms, batch, vocab, temperature, top_k,
-                         top_p, greedy ? 1 : 0, logits_dtype, (hipStream_t)stream);
+                         top_p, greedy ? 1 : 0, logits_dtype, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int aicomp_sample_tokens(int64_t* out, const void* logits, int64_t row_stride, float* probs_out,
+                         const float* uniforms, int batch, int vocab, float temperature, int top_k,
+                         float top_p, int greedy, int logits_dtype, void* stream) {
+    return aicomp_sample_tokens_split(out, logits, row_stride, probs_out, uniforms, batch, vocab, temperature, top_k,
+                                      top_p, greedy, logits_dtype, nullptr, 0, stream);
+}
+
+size_t aicomp_sample_workspace_bytes(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy,
+                                     int logits_dtype) {
+    if (batch <= 0 || vocab <= 0) return 0;
+    return sample_workspace_bytes(batch, vocab, row_stride, temperature, top_k, greedy ? 1 : 0, logits_dtype);
 }
 
 int aicomp_paged_decode_partition_size(int batch, int num_q_heads, int num_kv_heads, int head_dim,

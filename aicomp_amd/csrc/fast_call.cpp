@@ -429,11 +429,16 @@ PyObject* sample_tokens(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         const c10::DeviceGuard guard(x->device());
         void* stream = stream_of(*x);
         at::Tensor out(at::detail::empty_cuda({x->size(0)}, at::kLong, x->device(), c10::MemoryFormat::Contiguous));
+        const size_t need = aicomp_sample_workspace_bytes((int)x->size(0), (int)x->size(1), x->stride(0), (float)temperature, top_k,
+                                                          sample ? 0 : 1, dtype_code(x->scalar_type()));
+        at::Tensor scratch;                 // the allocator orders its next user behind this call
+        if (need) scratch = at::detail::empty_cuda({(int64_t)need}, at::kByte, x->device(), c10::MemoryFormat::Contiguous);
         const int rc = unlocked([&] {
-            return aicomp_sample_tokens((int64_t*)out.data_ptr(), x->data_ptr(), x->stride(0), nullptr,
-                                        sample ? (const float*)u->data_ptr() : nullptr, (int)x->size(0), (int)x->size(1),
-                                        (float)temperature, top_k, (float)top_p, sample ? 0 : 1,
-                                        dtype_code(x->scalar_type()), stream);
+            return aicomp_sample_tokens_split((int64_t*)out.data_ptr(), x->data_ptr(), x->stride(0), nullptr,
+                                              sample ? (const float*)u->data_ptr() : nullptr, (int)x->size(0),
+                                              (int)x->size(1), (float)temperature, top_k, (float)top_p, sample ? 0 : 1,
+                                              dtype_code(x->scalar_type()), need ? scratch.data_ptr() : nullptr, need,
+                                              stream);
         });
         if (rc != AICOMP_KV_OK) FAIL("aicomp_kv error %d: %s", rc, aicomp_kv_last_error());
         return THPVariable_Wrap(std::move(out));

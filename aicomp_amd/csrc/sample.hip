@@ -23,9 +23,10 @@
 // exact, order independent and reproducible; ties at the nucleus threshold are kept in
 // index order (what a stable descending sort would do).
 //
-// Not HBM-bound: a row (128 K logits = 512 KB in fp32) belongs to one CU, whose instruction
-// rate bounds a pass; the full-row histogram passes are LDS-atomic bound when many logits
-// share the leading key bits.
+// A row (128 K logits = 512 KB in fp32) on one CU is bound by what that CU can load and compare, two
+// passes of it, with three quarters of the chip idle at 64 rows; the full-row histogram passes are
+// LDS-atomic bound when many logits share the leading key bits.  A caller with scratch memory therefore
+// has greedy and top-k calls cut into parts of a row first (sample_parts_kernel).
 #include "common.h"
 
 #include <type_traits>
@@ -53,7 +54,21 @@ struct SampleParams {
     int top_k;                           // <= 0 or >= V: off
     float top_p;                         // >= 1: off
     int greedy;
+    // rows cut into parts (NULL / 0: not): what sample_parts_kernel leaves for sample_kernel
+    unsigned int* part_count;            // [B, parts] candidates of a part, PART_WHOLE: take the whole row instead
+    uint2* part_list;                    // [B, parts, PART_CAP] (order key of the scaled logit, index)
+    int parts, part_size;                // part_size: a multiple of 4 and at most PART_MAX
 };
+
+constexpr int PART_SLOTS = 16;                      // logits a lane of a part holds in registers
+constexpr int PART_MAX = NT * PART_SLOTS;           // 16384
+constexpr int PART_CAP = 1024;                      // candidates of a part
+constexpr int RAW_CAP = 2048;                       // ... before the exact test
+constexpr int MAX_PARTS = 16;
+constexpr int MERGE_SLOTS = 8;                      // candidates a lane of the merge takes: NT * 8 per row
+constexpr int PART_MAX_K = 256;
+constexpr int PART_MAX_BATCH = 1024;
+constexpr unsigned int PART_WHOLE = 0xffffffffu;
 
 // float -> key with the same order (larger float, larger key).  -0.0 gets the key of +0.0: the
 // reference compares floats (`logits < kth`), for which the two zeros are one value.
@@ -133,15 +148,14 @@ template <> __device__ __forceinline__ float apply_temperature<f16_t>(float x, f
 }
 
 // f(index, scaled logit) over the elements [begin, end) owned by `rank` of `nranks` lanes.
-// With 16-byte aligned rows a lane takes four consecutive elements per load and keeps eight
-// loads in flight; each lane visits its elements in ascending index order.
-template <typename T, typename F>
+// With 16-byte aligned rows a lane takes four consecutive elements per load and keeps U
+// loads in flight (the passes are latency bound); each lane visits its elements in ascending index order.
+template <typename T, int U = 16, typename F>
 __device__ __forceinline__ void for_each_logit(const T* row, int begin, int end, float temperature,
                                                int rank, int nranks, bool vec_ok, F f) {
     int tail = begin;
     if (vec_ok) {
         const int n4 = (end - begin) / 4;              // begin is a multiple of 4 for every caller
-        constexpr int U = 16;                          // loads in flight per lane: the passes are latency bound
         for (int j0 = rank; j0 < n4; j0 += U * nranks) {
             float a[U][4];
 #pragma unroll
@@ -201,6 +215,34 @@ __device__ __forceinline__ uint64_t wave_incl_scan64(uint64_t v, int lane) {
     return v;
 }
 
+// The largest key with its low ten bits clear that at least r lanes of the wave reach (0: fewer do).
+// Bit by bit with a ballot: 22 compares, no LDS and no barrier.
+__device__ __forceinline__ uint32_t wave_rth_bound(uint32_t key, int r) {
+    uint32_t t = 0;
+#pragma unroll
+    for (int bit = 31; bit >= 10; --bit) {
+        const uint32_t cand = t | (1u << bit);
+        if (__popcll(__ballot(key >= cand)) >= r) t = cand;
+    }
+    return t;
+}
+
+// What a raw logit has to reach so that its scaled key can be key_ls = the scaled key of key_l: a
+// prefilter of one compare per element (it lets through whatever the key order would, -0.0 next to +0.0,
+// and everything when the bound lies below -inf, whose key decodes to a NaN).
+template <typename T> __device__ __forceinline__ float raw_bound(uint32_t key_l, uint32_t key_ls, float temperature) {
+    // quotients of neighbouring raw values are more than half a unit in the last place apart where they
+    // are normal, so at most three round to one value; LIST_SLACK covers the subnormal ones
+    const uint32_t steps = fabsf(key_value(key_ls)) >= 2.4e-38f ? 4u : LIST_SLACK;
+    const uint32_t slack = steps * (sizeof(T) == 2 ? 0x10000u : 1u);              // bf16 values are 2^16 keys apart
+    float lo = key_value(key_l > slack ? key_l - slack : 0u);
+    if constexpr (std::is_same<T, f16_t>::value) {
+        const float b = f16_raw_bound<T>(key_value(key_ls), temperature);
+        if (b < lo) lo = b;
+    }
+    return lo;
+}
+
 // Shared state of the radix walks (one row)
 struct Shared {
     alignas(16) unsigned long long mass[BINS];
@@ -222,7 +264,7 @@ struct Shared {
 
 // Wave 0: walking the bins from the top, find the bin that holds the k-th element
 // (by count).  Returns digit and the count strictly above it.
-__device__ void pick_by_count(Shared& s, int nbins, unsigned int k, int lane) {
+__device__ __forceinline__ void pick_by_count(Shared& s, int nbins, unsigned int k, int lane) {
     // lane owns bins [hi - 32*lane - 31, hi - 32*lane], i.e. lane 0 the top 32 bins: read as eight
     // 16-byte vectors (independent loads; a dependent chain of 32 LDS reads costs microseconds)
     constexpr int per = BINS / 64;
@@ -272,7 +314,7 @@ __device__ void pick_by_count(Shared& s, int nbins, unsigned int k, int lane) {
 }
 
 // Wave 0: lowest bin d with mass(bins > d) <= limit.  Returns digit and that mass.
-__device__ void pick_by_mass(Shared& s, int nbins, unsigned long long limit, int lane) {
+__device__ __forceinline__ void pick_by_mass(Shared& s, int nbins, unsigned long long limit, int lane) {
     const int per = BINS / 64;
     unsigned long long local = 0;
     for (int j = 0; j < per; ++j) {
@@ -401,61 +443,281 @@ __device__ __forceinline__ Nucleus nucleus_threshold(Shared& s, Src src, uint32_
     return r;
 }
 
-template <typename T>
+// One part of a row per workgroup: the part is read once, into registers, and what may be among the
+// row's top k leaves it.  Each wave finds the r-th largest of its 64 lane maxima, r = ceil(k / 16); at
+// least 16 r >= k elements of the part reach the smallest of the sixteen, so whatever lies below it (in
+// scaled order, ties stay) is not among the part's top k, nor the row's.  About 2.6 k of 16384 pass at
+// k = 50.  A logit of -inf has no mass and is left out; a part with a NaN, or one
+// with more than PART_CAP candidates (masses of equal logits), sends its row the whole way.  Greedy: the part's
+// argmax is its one candidate.
+//
+// Bound by latency: one round of loads, 22 ballots, three barriers, a few dozen appends.  64 rows of 128256
+// float32, k = 50: 8.8 us here and 11.9 us in sample_merge_kernel as traced, where one launch took 25.5 us.
+template <typename T, bool GREEDY>
 __global__ void __launch_bounds__(NT)
-sample_kernel(SampleParams p) {
-    __shared__ Shared s;
-    const int row_idx = blockIdx.x;
+sample_parts_kernel(SampleParams p) {
+    __shared__ uint32_t red_key[NW];
+    __shared__ unsigned int red_idx[NW];
+    __shared__ unsigned int n_list, n_raw, whole;
+    __shared__ float raw_x[RAW_CAP];
+    __shared__ unsigned int raw_i[RAW_CAP];
+    const int row_idx = blockIdx.x, part = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
+    const int begin = part * p.part_size;
+    const int n = min(p.vocab - begin, p.part_size);              // at least 1
+    if (tid == 0) { n_list = 0; n_raw = 0; whole = 0; }
+
+    // slot 4 u + e: element 4 (tid + NT u) + e of a row with 16-byte alignment, tid + NT (4 u + e) of another
+    const bool vec = ((uintptr_t)row % 16) == 0;
+    const int n4 = vec ? n / 4 : 0;
+    float x[PART_SLOTS], xt = -INFINITY;
+    if (n4 > 0) {
+#pragma unroll
+        for (int u = 0; u < PART_SLOTS / 4; ++u) Load4<T>::get(row + begin + 4 * min(tid + NT * u, n4 - 1), x + 4 * u);
+        if (tid < n - 4 * n4) xt = scaled_logit<T>(row, begin + 4 * n4 + tid, 1.f);
+#pragma unroll
+        for (int i = 0; i < PART_SLOTS; ++i)
+            if (tid + NT * (i / 4) >= n4) x[i] = -INFINITY;
+    } else {
+#pragma unroll
+        for (int i = 0; i < PART_SLOTS; ++i) x[i] = scaled_logit<T>(row, begin + min(tid + NT * i, n - 1), 1.f);
+#pragma unroll
+        for (int i = 0; i < PART_SLOTS; ++i)
+            if (tid + NT * i >= n) x[i] = -INFINITY;
+    }
+    auto index_of = [&](int i) -> unsigned int {
+        return (unsigned int)(begin + (n4 > 0 ? 4 * (tid + NT * (i / 4)) + (i & 3) : tid + NT * i));
+    };
+    const unsigned int tail_idx = (unsigned int)(begin + 4 * n4 + tid);
+    const int64_t slot = (int64_t)row_idx * p.parts + part;
+    uint2* list = p.part_list + slot * PART_CAP;
+
+    if constexpr (GREEDY) {
+        // ascending indices within a lane (the tail's lie above all others), the lowest one wins a tie
+        float best = -INFINITY;
+        unsigned int best_i = 0x7fffffffu;
+#pragma unroll
+        for (int i = 0; i < PART_SLOTS; ++i)
+            if (x[i] > best) { best = x[i]; best_i = index_of(i); }
+        if (xt > best) { best = xt; best_i = tail_idx; }
+        uint32_t key = order_key(best);
+        auto take = [&](uint32_t k2, unsigned int i2) {
+            if (k2 > key || (k2 == key && i2 < best_i)) { key = k2; best_i = i2; }
+        };
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint32_t k2 = __shfl_xor(key, o);
+            const unsigned int i2 = __shfl_xor(best_i, o);
+            take(k2, i2);
+        }
+        if (lane == 0) { red_key[wave] = key; red_idx[wave] = best_i; }
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < NW; ++w) take(red_key[w], red_idx[w]);
+            list[0] = make_uint2(key, best_i);
+            p.part_count[slot] = 1u;
+        }
+        return;
+    }
+
+    float best = xt;
+    bool nan = xt != xt;
+#pragma unroll
+    for (int i = 0; i < PART_SLOTS; ++i) { best = fmaxf(best, x[i]); nan |= x[i] != x[i]; }
+    const uint32_t bound = wave_rth_bound(order_key(best), (p.top_k + NW - 1) / NW);
+    if (lane == 0) red_key[wave] = bound;
+    __syncthreads();
+    if (nan) whole = 1u;
+    uint32_t key_l = red_key[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) key_l = min(key_l, red_key[w]);
+    const uint32_t key_ls = order_key(apply_temperature<T>(key_value(key_l), p.temperature));
+    const float raw_lo = raw_bound<T>(key_l, key_ls, p.temperature);
+    // what passes the prefilter goes through LDS, so that the exact test is made once per candidate
+    unsigned int pass = 0;
+#pragma unroll
+    for (int i = 0; i < PART_SLOTS; ++i) pass |= !(x[i] < raw_lo) && x[i] > -INFINITY ? 1u << i : 0u;
+    pass |= !(xt < raw_lo) && xt > -INFINITY ? 1u << PART_SLOTS : 0u;
+    if (pass) {
+        unsigned int j = atomicAdd(&n_raw, (unsigned int)__popc(pass));
+#pragma unroll
+        for (int i = 0; i <= PART_SLOTS; ++i)
+            if (pass >> i & 1u) {
+                if (j < RAW_CAP) {
+                    raw_x[j] = i < PART_SLOTS ? x[i < PART_SLOTS ? i : 0] : xt;
+                    raw_i[j] = i < PART_SLOTS ? index_of(i) : tail_idx;
+                }
+                ++j;
+            }
+    }
+    __syncthreads();
+    const unsigned int nr = n_raw;
+    for (unsigned int i = tid; i < min(nr, (unsigned int)RAW_CAP); i += NT) {
+        const uint32_t key = order_key(apply_temperature<T>(raw_x[i], p.temperature));
+        if (key >= key_ls) {
+            const unsigned int j = atomicAdd(&n_list, 1u);
+            if (j < PART_CAP) list[j] = make_uint2(key, raw_i[i]);
+        }
+    }
+    __syncthreads();
+    if (tid == 0) p.part_count[slot] = whole || nr > RAW_CAP || n_list > PART_CAP ? PART_WHOLE : n_list;
+}
+
+// Index of the row's maximum, the lowest one among equals (0: nothing above -inf).
+template <typename T, int U>
+__device__ __forceinline__ int block_argmax(Shared& s, const T* row, int V, bool vec_ok) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float best = -INFINITY;
+    int best_i = 0x7fffffff;
+    for_each_logit<T, U>(row, 0, V, 1.f, tid, NT, vec_ok, [&](int i, float x) {
+        if (x > best) { best = x; best_i = i; }       // lowest index wins ties within a lane (ascending i)
+    });
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const float ob = __shfl_xor(best, o);
+        const int oi = __shfl_xor(best_i, o);
+        if (ob > best || (ob == best && oi < best_i)) { best = ob; best_i = oi; }
+    }
+    __syncthreads();
+    if (lane == 0) { s.red_f[wave] = best; s.red_i[wave] = best_i; }
+    __syncthreads();
+    best = s.red_f[0]; best_i = s.red_i[0];
+    for (int w = 1; w < NW; ++w) {
+        const float ob = s.red_f[w];
+        const int oi = s.red_i[w];
+        if (ob > best || (ob == best && oi < best_i)) { best = ob; best_i = oi; }
+    }
+    return best_i == 0x7fffffff ? 0 : best_i;
+}
+
+// A row without finite mass (all -inf, NaN): the argmax, and an all-zero distribution.
+template <typename T, int U>
+__device__ __forceinline__ void no_mass(Shared& s, const SampleParams& p, int row_idx, const T* row, bool vec_ok) {
+    const int best_i = block_argmax<T, U>(s, row, p.vocab, vec_ok);
+    if (threadIdx.x == 0) p.out[row_idx] = best_i;
+    if (p.probs_out)
+        for (int i = threadIdx.x; i < p.vocab; i += NT) p.probs_out[(int64_t)row_idx * p.vocab + i] = 0.f;
+}
+
+// Sum of v over the lanes before this one, and over all.
+__device__ __forceinline__ unsigned long long block_scan(Shared& s, unsigned long long v, unsigned long long& total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long incl = wave_incl_scan64(v, lane);            // -> sum before this lane
+    if (lane == 63) s.seg_mass[wave] = incl;
+    __syncthreads();
+    unsigned long long before = 0;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const unsigned long long x = s.seg_mass[w];
+        before += w < wave ? x : 0ull;
+        total += x;
+    }
+    return before + incl - v;
+}
+
+// At most one candidate per lane.
+// No histograms: every candidate is ranked in the descending order a stable sort would give (key, then
+// index) and in index order, by counting; with top-k the one of rank k-1 holds the k-th largest key;
+// the mass before a candidate in the first order decides the nucleus, a scan in the second
+// order the draw.  Exact 64-bit sums.  Without top-k the list is everything above a cut of the
+// whole row and z_row the mass of the whole row.
+// The counting is n^2 compares: a candidate's are shared by as many lanes as there are for it.  (One lane each and a
+// loop over the list for every mass took 10 of the 25 us of a call over 64 rows, k = 50.)
+template <typename T, int U>
+__device__ __forceinline__ void draw_from_small_list(Shared& s, const SampleParams& p, int row_idx, const T* row, bool vec_ok,
+                                                     float m, bool has_topk, unsigned long long z_row) {
+    const int tid = threadIdx.x, V = p.vocab;
+    const int n = (int)s.n_list;                                    // 1..NT
+    int sh = 6;                                                     // 2^sh lanes per candidate
+    while (sh > 0 && (n << sh) > NT) --sh;
+    const int mine_e = tid >> sh, step = 1 << sh;
+    // (key, ~index) as one number: two compares and two adds per pair.  The zeros behind the list are
+    // above nothing in either order; a lane reads at most 8 * 64 - 1 of them.
+    if (tid < n) s.list_w[tid] = (unsigned long long)s.list_key[tid] << 32 | ~s.list_idx[tid];
+    if (tid < 512) s.list_w[n + tid] = 0;
+    __syncthreads();
+    uint32_t ranks = 0;                                             // rank | rank by index << 16
+    if (mine_e < n) {
+        const unsigned long long me = s.list_w[mine_e];
+        unsigned int by_key = 0, by_index = 0;
+        for (int i0 = tid & (step - 1); i0 < n; i0 += 8 * step) {
+            unsigned long long e[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) e[u] = s.list_w[i0 + u * step];     // eight independent reads
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                by_key += e[u] > me ? 1u : 0u;
+                by_index += (uint32_t)e[u] > (uint32_t)me ? 1u : 0u;
+            }
+        }
+        ranks = by_key | by_index << 16;
+    }
+    for (int o = 1; o < step; o <<= 1) ranks += __shfl_xor(ranks, o);
+    if (mine_e < n && (tid & (step - 1)) == 0) {
+        s.cnt[mine_e] = ranks;
+        if (has_topk && (int)(ranks & 0xffffu) == p.top_k - 1) s.sel_digit = s.list_key[mine_e];   // one writer
+    }
+    __syncthreads();
+    const uint32_t kth = has_topk && n >= p.top_k ? s.sel_digit : 0u;       // fewer than k: all of them stay
+    unsigned int idx = 0, by_index = 0, by_key = 0;
+    uint64_t w = 0;
+    if (tid < n) {
+        const uint32_t key = s.list_key[tid];
+        idx = s.list_idx[tid];
+        by_key = s.cnt[tid] & 0xffffu;
+        by_index = s.cnt[tid] >> 16;
+        if (key >= kth) w = weight_of(key_value(key), m);                   // ties at the k-th value all stay
+    }
+    unsigned long long z = 0;
+    if (p.top_p < 1.f) {
+        // lane t takes the t-th entry of the sorted order
+        __syncthreads();                        // everyone has read keys and indices
+        if (tid < n) { s.list_w[by_key] = w; s.list_idx[by_key] = idx; s.list_key[by_key] = by_index; }
+        __syncthreads();
+        if (tid < n) { w = s.list_w[tid]; idx = s.list_idx[tid]; by_index = s.list_key[tid]; }
+        const unsigned long long before = block_scan(s, w, z);
+        // an entry stays while the mass before it is at most top_p of the total (of the row's total
+        // when the list is a cut of the whole row rather than its top k)
+        const unsigned long long limit = (unsigned long long)((double)fmaxf(p.top_p, 0.f) * (double)(has_topk ? z : z_row));
+        if (before > limit) w = 0;
+    }
+    __syncthreads();
+    if (tid < n) { s.list_w[by_index] = w; s.list_idx[by_index] = idx; }
+    __syncthreads();
+    w = 0;
+    if (tid < n) { w = s.list_w[tid]; idx = s.list_idx[tid]; }
+    const unsigned long long before = block_scan(s, w, z);              // kept mass at lower indices
+    if (z == 0) {                                  // non-finite logits: fall back to the argmax
+        no_mass<T, U>(s, p, row_idx, row, vec_ok);
+        return;
+    }
+    unsigned long long target = (unsigned long long)((double)p.uniforms[row_idx] * (double)z);
+    if (target >= z) target = z - 1;
+    if (before <= target && target < before + w) p.out[row_idx] = idx;
+    if (p.probs_out) {
+        for (int i = tid; i < V; i += NT) p.probs_out[(int64_t)row_idx * V + i] = 0.f;
+        __syncthreads();
+        const double inv_z = 1.0 / (double)z;
+        if (w) p.probs_out[(int64_t)row_idx * V + idx] = (float)((double)w * inv_z);
+    }
+}
+// The whole of a row by one workgroup.  U: loads in flight per lane.
+template <typename T, int U>
+__device__ __forceinline__ void sample_row(const SampleParams& p, Shared& s, int row_idx) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
     const int V = p.vocab;
-    const float temp = p.greedy ? 1.f : p.temperature;
+    const float temp = p.temperature;
 
-    // ---------------------------------------------------------------- 1. maximum (greedy: argmax)
+    // ---------------------------------------------------------------- 1. maximum
     // On the raw logits: dividing by a positive temperature keeps the order, so the maximum of
-    // the scaled row is the scaled maximum and no division is needed in this pass.  Sampling only
-    // needs the value (one v_max per element); the index is found by a second pass in the rare
-    // case that asks for it (greedy decoding, or a row without any finite mass).
+    // the scaled row is the scaled maximum and no division is needed in this pass (one v_max per
+    // element).
     const bool vec_ok = ((uintptr_t)row % 16) == 0;
-    auto block_argmax = [&]() -> int {
-        float best = -INFINITY;
-        int best_i = 0x7fffffff;
-        for_each_logit<T>(row, 0, V, 1.f, tid, NT, vec_ok, [&](int i, float x) {
-            if (x > best) { best = x; best_i = i; }       // lowest index wins ties within a lane (ascending i)
-        });
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ob = __shfl_xor(best, o);
-            const int oi = __shfl_xor(best_i, o);
-            if (ob > best || (ob == best && oi < best_i)) { best = ob; best_i = oi; }
-        }
-        __syncthreads();
-        if (lane == 0) { s.red_f[wave] = best; s.red_i[wave] = best_i; }
-        __syncthreads();
-        best = s.red_f[0]; best_i = s.red_i[0];
-        for (int w = 1; w < NW; ++w) {
-            const float ob = s.red_f[w];
-            const int oi = s.red_i[w];
-            if (ob > best || (ob == best && oi < best_i)) { best = ob; best_i = oi; }
-        }
-        return best_i == 0x7fffffff ? 0 : best_i;
-    };
-    if (p.greedy) {
-        const int best_i = block_argmax();
-        if (tid == 0) p.out[row_idx] = best_i;
-        if (p.probs_out)
-            for (int i = tid; i < V; i += NT) p.probs_out[(int64_t)row_idx * V + i] = i == best_i ? 1.f : 0.f;
-        return;
-    }
-    // a row without finite mass (all -inf, NaN): the argmax, and an all-zero distribution
-    auto no_mass = [&]() {
-        const int best_i = block_argmax();
-        if (tid == 0) p.out[row_idx] = best_i;
-        if (p.probs_out)
-            for (int i = tid; i < V; i += NT) p.probs_out[(int64_t)row_idx * V + i] = 0.f;
-    };
     float lane_best = -INFINITY;                      // raw maximum of this lane's share of the row
-    for_each_logit<T>(row, 0, V, 1.f, tid, NT, vec_ok, [&](int, float x) { lane_best = fmaxf(lane_best, x); });
+    for_each_logit<T, U>(row, 0, V, 1.f, tid, NT, vec_ok, [&](int, float x) { lane_best = fmaxf(lane_best, x); });
     float best = lane_best;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) best = fmaxf(best, __shfl_xor(best, o));
@@ -465,7 +727,7 @@ sample_kernel(SampleParams p) {
     for (int w = 1; w < NW; ++w) best = fmaxf(best, s.red_f[w]);
     const float m = apply_temperature<T>(best, temp);
 
-    auto over_row = [&](auto f) { for_each_logit<T>(row, 0, V, temp, tid, NT, vec_ok, f); };
+    auto over_row = [&](auto f) { for_each_logit<T, U>(row, 0, V, temp, tid, NT, vec_ok, f); };
     auto over_list = [&](auto f) {
         const int n = (int)s.n_list;
         for (int j = tid; j < n; j += NT) f((int)s.list_idx[j], key_value(s.list_key[j]));
@@ -491,19 +753,11 @@ sample_kernel(SampleParams p) {
         // lets in a few more candidates and saves a histogram round
         const uint32_t key_l = select_kth(s, over_lane_max, (unsigned int)p.top_k, tid, lane, wave, 2);
         const uint32_t key_ls = order_key(apply_temperature<T>(key_value(key_l), temp));
-        const uint32_t slack = LIST_SLACK * (sizeof(T) == 2 ? 0x10000u : 1u);     // bf16 values are 2^16 keys apart
-        const uint32_t key_lo = key_l > slack ? key_l - slack : 0u;
         if (tid == 0) s.n_list = 0;
         __syncthreads();
-        // prefilter on the raw float, one compare per element.  It lets through whatever the key
-        // order would (plus -0.0 next to +0.0, and everything when the bound is below -inf, whose
-        // key decodes to a NaN); the exact test on the scaled key follows.
-        float raw_lo = key_value(key_lo);              // may be a NaN (a bound below -inf): lets everything through
-        if constexpr (std::is_same<T, f16_t>::value) {
-            const float b = f16_raw_bound<T>(key_value(key_ls), temp);
-            if (b < raw_lo) raw_lo = b;
-        }
-        for_each_logit<T>(row, 0, V, 1.f, tid, NT, vec_ok, [&](int i, float x) {
+        // the exact test on the scaled key follows the prefilter
+        const float raw_lo = raw_bound<T>(key_l, key_ls, temp);
+        for_each_logit<T, U>(row, 0, V, 1.f, tid, NT, vec_ok, [&](int i, float x) {
             if (!(x < raw_lo)) {
                 const uint32_t key = order_key(apply_temperature<T>(x, temp));
                 if (key >= key_ls) {
@@ -515,89 +769,8 @@ sample_kernel(SampleParams p) {
         __syncthreads();
         use_list = s.n_list <= LIST_CAP;
     }
-    // ---------------------------------------------------------------- at most one candidate per lane
-    // No histograms: every lane ranks its candidate in the descending order a stable sort would give
-    // (key, then index); with top-k the lane of rank k-1 holds the k-th largest key; the mass that
-    // precedes a candidate in that order decides the nucleus; the draw walks the kept candidates in
-    // index order.  Plain loops over the list in LDS, exact 64-bit sums.  Without top-k the list is
-    // everything above a cut of the whole row and z_row the mass of the whole row.
-    auto draw_from_small_list = [&](bool has_topk, unsigned long long z_row) {
-        const int n = (int)s.n_list;
-        const bool mine = tid < n;
-        const uint32_t key = mine ? s.list_key[tid] : 0u;
-        const unsigned int idx = mine ? s.list_idx[tid] : 0xffffffffu;
-        // the loops below read the list eight entries at a time (independent LDS reads; entries past
-        // n are inside the arrays and masked out)
-        unsigned int rank = 0;
-        if (mine)
-            for (int i0 = 0; i0 < n; i0 += 8) {
-                uint32_t kk[8], ii[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) { kk[u] = s.list_key[i0 + u]; ii[u] = s.list_idx[i0 + u]; }
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    rank += (i0 + u < n) && ((kk[u] > key) || (kk[u] == key && ii[u] < idx));
-            }
-        if (has_topk && mine && rank == (unsigned int)p.top_k - 1u) s.sel_digit = key;   // ranks are a permutation: one writer
-        __syncthreads();
-        const uint32_t kth = has_topk ? s.sel_digit : 0u;
-        uint64_t w = (mine && key >= kth) ? weight_of(key_value(key), m) : 0;   // ties at the k-th value all stay
-        if (mine) { s.cnt[tid] = rank; s.list_w[tid] = w; }
-        unsigned long long z = wave_sum64(w);
-        if (lane == 0) s.seg_mass[wave] = z;
-        __syncthreads();
-        z = 0;
-        for (int wv = 0; wv < NW; ++wv) z += s.seg_mass[wv];
-        if (p.top_p < 1.f) {
-            // an entry stays while the mass before it (in sorted order) is at most top_p of the total
-            // (of the row's total when the list is a cut of the whole row rather than its top k)
-            const unsigned long long limit = (unsigned long long)((double)fmaxf(p.top_p, 0.f) * (double)(has_topk ? z : z_row));
-            unsigned long long before = 0;
-            if (w)
-                for (int i0 = 0; i0 < n; i0 += 8) {
-                    uint32_t rr[8];
-                    unsigned long long ww[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) { rr[u] = s.cnt[i0 + u]; ww[u] = s.list_w[i0 + u]; }
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) before += (i0 + u < n && rr[u] < rank) ? ww[u] : 0ull;
-                }
-            if (before > limit) w = 0;
-            __syncthreads();                       // every lane has read the unfiltered weights
-            if (mine) s.list_w[tid] = w;
-            z = wave_sum64(w);
-            if (lane == 0) s.seg_mass[wave] = z;
-            __syncthreads();
-            z = 0;
-            for (int wv = 0; wv < NW; ++wv) z += s.seg_mass[wv];
-        }
-        if (z == 0) {                                  // non-finite logits: fall back to the argmax
-            no_mass();
-            return;
-        }
-        unsigned long long target = (unsigned long long)((double)p.uniforms[row_idx] * (double)z);
-        if (target >= z) target = z - 1;
-        if (p.probs_out) {
-            for (int i = tid; i < V; i += NT) p.probs_out[(int64_t)row_idx * V + i] = 0.f;
-            __syncthreads();
-        }
-        if (w) {
-            unsigned long long before = 0;             // kept mass at lower indices
-            for (int i0 = 0; i0 < n; i0 += 8) {
-                uint32_t ii[8];
-                unsigned long long ww[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) { ii[u] = s.list_idx[i0 + u]; ww[u] = s.list_w[i0 + u]; }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) before += (i0 + u < n && ii[u] < idx) ? ww[u] : 0ull;
-            }
-            if (before <= target && target < before + w) p.out[row_idx] = idx;
-            const double inv_z = 1.0 / (double)z;
-            if (p.probs_out) p.probs_out[(int64_t)row_idx * V + idx] = (float)((double)w * inv_z);
-        }
-    };
     if (use_list && s.n_list <= NT && s.n_list >= (unsigned int)p.top_k) {
-        draw_from_small_list(true, 0ull);
+        draw_from_small_list<T, U>(s, p, row_idx, row, vec_ok, m, true, 0ull);
         return;
     }
 
@@ -630,7 +803,7 @@ sample_kernel(SampleParams p) {
         unsigned long long z_row = 0;
         for (int wv = 0; wv < NW; ++wv) z_row += s.seg_mass[wv];
         if (z_row == 0) {
-            no_mass();
+            no_mass<T, U>(s, p, row_idx, row, vec_ok);
             return;
         }
         const unsigned long long limit = (unsigned long long)((double)fmaxf(p.top_p, 0.f) * (double)z_row);
@@ -657,7 +830,7 @@ sample_kernel(SampleParams p) {
                     const float b = f16_raw_bound<T>(key_value(key_lo_s), temp);
                     if (b < raw_lo) raw_lo = b;
                 }
-                for_each_logit<T>(row, 0, V, 1.f, tid, NT, vec_ok, [&](int i, float x) {
+                for_each_logit<T, U>(row, 0, V, 1.f, tid, NT, vec_ok, [&](int i, float x) {
                     if (!(x < raw_lo)) {
                         const uint32_t key = order_key(apply_temperature<T>(x, temp));
                         if (key >= key_lo_s) {
@@ -668,7 +841,7 @@ sample_kernel(SampleParams p) {
                 });
                 __syncthreads();
                 if (s.n_list <= NT) {
-                    draw_from_small_list(false, z_row);
+                    draw_from_small_list<T, U>(s, p, row_idx, row, vec_ok, m, false, z_row);
                     return;
                 }
             }
@@ -730,7 +903,7 @@ sample_kernel(SampleParams p) {
         unsigned long long z2 = 0;
         for (int w = 0; w < NW; ++w) z2 += s.seg_mass[w];
         if (z2 == 0) {                                 // non-finite logits: fall back to the argmax
-            no_mass();
+            no_mass<T, U>(s, p, row_idx, row, vec_ok);
             return;
         }
         unsigned long long target = (unsigned long long)((double)p.uniforms[row_idx] * (double)z2);
@@ -799,7 +972,7 @@ sample_kernel(SampleParams p) {
     unsigned long long mass_gt = 0;
     unsigned int n_tied = 0;
     uint64_t w_t_val = 0;
-    for_each_logit<T>(row, s0, max(s0, s1), temp, lane, 64, vec_ok, [&](int, float x) {
+    for_each_logit<T, U>(row, s0, max(s0, s1), temp, lane, 64, vec_ok, [&](int, float x) {
         const uint32_t key = order_key(x);
         if (tie_rule ? key > key_t : key >= key_t) mass_gt += weight_of(x, m);
         else if (tie_rule && key == key_t) ++n_tied;
@@ -821,7 +994,7 @@ sample_kernel(SampleParams p) {
         tied_base += nt;
     }
     if (z2 == 0) {                                 // no mass at all (non-finite logits): fall back to the argmax
-        no_mass();
+        no_mass<T, U>(s, p, row_idx, row, vec_ok);
         return;
     }
     unsigned long long target = (unsigned long long)((double)p.uniforms[row_idx] * (double)z2);
@@ -860,7 +1033,7 @@ sample_kernel(SampleParams p) {
     const int c0 = min(s1, s0 + lane * chunk), c1 = min(s1, c0 + chunk);
     unsigned long long lane_mass = 0;
     unsigned int lane_tied = 0;
-    for_each_logit<T>(row, c0, c1, temp, 0, 1, vec_ok, [&](int, float x) {
+    for_each_logit<T, U>(row, c0, c1, temp, 0, 1, vec_ok, [&](int, float x) {
         bool tied;
         lane_mass += weight_or_tie(x, tied);
         lane_tied += tied;
@@ -899,18 +1072,169 @@ sample_kernel(SampleParams p) {
     }
 }
 
+// The draw from the candidates of a row's parts: those of all parts hold the row's top k, with ties (all finite
+// logits if there are fewer).  The same bound once more, over one maximum per lane, leaves a list a few times k
+// long.  A row that its parts gave up, or whose list is longer than the lanes, is done whole.
+template <typename T>
+__global__ void __launch_bounds__(NT)
+sample_merge_kernel(SampleParams p) {
+    __shared__ Shared s;
+    const int row_idx = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
+    const bool vec_ok = ((uintptr_t)row % 16) == 0;
+    const unsigned int* counts = p.part_count + (int64_t)row_idx * p.parts;
+    unsigned int end[MAX_PARTS], total = 0;
+    bool fits = true;
+#pragma unroll
+    for (int q = 0; q < MAX_PARTS; ++q) {
+        const unsigned int c = q < p.parts ? counts[q] : 0u;
+        fits = fits && c <= PART_CAP;
+        total += min(c, (unsigned int)PART_CAP);
+        end[q] = total;
+    }
+    if (fits && total == 0) {                // nothing above -inf
+        no_mass<T, 4>(s, p, row_idx, row, vec_ok);
+        return;
+    }
+    if (fits && total <= (unsigned int)(NT * MERGE_SLOTS)) {
+        // candidate j goes to wave j % 16, so that the waves' shares are alike; lanes without one: key 0
+        const uint2* lists = p.part_list + (int64_t)row_idx * p.parts * PART_CAP;
+        uint2 e[MERGE_SLOTS];
+        uint32_t top = 0;
+#pragma unroll
+        for (int u = 0; u < MERGE_SLOTS; ++u) {
+            const unsigned int j = (unsigned int)(lane * NW + wave + NT * u);
+            e[u] = make_uint2(0u, 0u);
+            if (j < total) {
+                int q = 0;
+                unsigned int start = 0;
+#pragma unroll
+                for (int c = 0; c < MAX_PARTS - 1; ++c)
+                    if (j >= end[c]) { q = c + 1; start = end[c]; }
+                e[u] = lists[(int64_t)q * PART_CAP + (j - start)];
+            }
+            top = max(top, e[u].x);
+        }
+        const uint32_t bound = wave_rth_bound(top, (p.top_k + NW - 1) / NW);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) top = max(top, (uint32_t)__shfl_xor(top, o));
+        if (lane == 0) { s.seg_tied[wave] = bound; s.red_i[wave] = (int)top; }
+        if (tid == 0) s.n_list = 0;
+        __syncthreads();
+        uint32_t key_l = s.seg_tied[0], key_m = (uint32_t)s.red_i[0];
+        for (int w = 1; w < NW; ++w) {
+            key_l = min(key_l, s.seg_tied[w]);
+            key_m = max(key_m, (uint32_t)s.red_i[w]);
+        }
+#pragma unroll
+        for (int u = 0; u < MERGE_SLOTS; ++u)
+            if (e[u].x >= key_l && e[u].x) {
+                const unsigned int j = atomicAdd(&s.n_list, 1u);
+                if (j < NT) { s.list_key[j] = e[u].x; s.list_idx[j] = e[u].y; }
+            }
+        __syncthreads();
+        if (s.n_list <= NT) {
+            draw_from_small_list<T, 4>(s, p, row_idx, row, vec_ok, key_value(key_m), true, 0ull);
+            return;
+        }
+        __syncthreads();
+    }
+    sample_row<T, 4>(p, s, row_idx);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(NT)
+sample_kernel(SampleParams p) {
+    __shared__ Shared s;
+    sample_row<T, 16>(p, s, blockIdx.x);
+}
+
+// Greedy: the argmax, from the parts' candidates if there are any.
+template <typename T>
+__global__ void __launch_bounds__(NT)
+greedy_kernel(SampleParams p) {
+    __shared__ Shared s;
+    const int row_idx = blockIdx.x, tid = threadIdx.x, V = p.vocab;
+    const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
+    int best_i;
+    if (p.parts) {
+        uint2 c = p.part_list[(int64_t)row_idx * p.parts * PART_CAP];
+        for (int q = 1; q < p.parts; ++q) {
+            const uint2 o = p.part_list[((int64_t)row_idx * p.parts + q) * PART_CAP];
+            if (o.x > c.x || (o.x == c.x && o.y < c.y)) c = o;
+        }
+        best_i = c.y == 0x7fffffffu ? 0 : (int)c.y;
+    } else {
+        best_i = block_argmax<T, 16>(s, row, V, ((uintptr_t)row % 16) == 0);
+    }
+    if (tid == 0) p.out[row_idx] = best_i;
+    if (p.probs_out)
+        for (int i = tid; i < V; i += NT) p.probs_out[(int64_t)row_idx * V + i] = i == best_i ? 1.f : 0.f;
+}
+
 }  // namespace
+
+// How many parts the rows of a call are cut into (1: none).  A second launch and the merge cost about 7 us, so it has to save more.
+// Device time in a graph, one launch -> parts, us:
+//   rows whose loads cannot be vectors (a stride that is no multiple of 16 bytes): at once
+//     float32, k 50     50257: 64 rows 23.5 -> 16.9, 512 79.6 -> 47.9;  128255: 64 rows 64.4 -> 22.1, 1024 455 -> 167
+//     bf16              50257: 64 rows 24.4 -> 17.3;  greedy float32 50257: 64 rows 11.4 -> 7.6
+//   other rows from six parts on (65536, four parts: 64 rows 17.4 -> 16.7, 128 rows 18.0 -> 19.3), with k <= 64
+//     float32           128256: 1 row 19.9 -> 15.5, 64 22.9 -> 20.1, 512 88.2 -> 70.8;  262144: 16 rows 29.2 -> 17.6
+//     16-bit            128256: 64 rows 22.3 -> 20.1, but 128 rows 23.3 -> 26.6 (half the bytes to save on): up to 512 parts
+//   k to 256            128256: 1 row 24.3 -> 21.1, 16 25.5 -> 24.6, 64 27.0 -> 30.3: up to 128 parts
+//   greedy              128256: 16 rows 9.1 -> 7.2, 64 10.8 -> 9.8, 128 14.1 -> 17.2: up to 512 parts
+static int sample_parts(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy, int dtype) {
+    const int parts = (int)(((int64_t)vocab + PART_MAX - 1) / PART_MAX);
+    if (parts < 2 || parts > MAX_PARTS || batch > PART_MAX_BATCH) return 1;
+    if (!greedy && (top_k <= 0 || top_k >= vocab || top_k > PART_MAX_K || !(temperature <= LIST_MAX_TEMPERATURE))) return 1;
+    const int per_16 = dtype == AICOMP_KV_F32 ? 4 : 8;
+    if (batch > 1 && row_stride % per_16 != 0) return parts;
+    const int all = batch * parts;
+    if (parts < 6) return 1;
+    if (greedy) return all <= 512 ? parts : 1;
+    if (top_k > 64) return all <= 128 ? parts : 1;
+    return dtype == AICOMP_KV_F32 || all <= 512 ? parts : 1;
+}
+
+size_t sample_workspace_bytes(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy, int dtype) {
+    const int parts = sample_parts(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
+    return parts < 2 ? 0 : (size_t)batch * parts * (PART_CAP * sizeof(uint2) + sizeof(unsigned int));
+}
+
+template <typename T>
+static void launch_rows(const SampleParams& p, int batch, hipStream_t stream) {
+    if (p.greedy) {
+        if (p.parts) hipLaunchKernelGGL((sample_parts_kernel<T, true>), dim3(batch, p.parts), dim3(NT), 0, stream, p);
+        hipLaunchKernelGGL((greedy_kernel<T>), dim3(batch), dim3(NT), 0, stream, p);
+    } else if (p.parts) {
+        hipLaunchKernelGGL((sample_parts_kernel<T, false>), dim3(batch, p.parts), dim3(NT), 0, stream, p);
+        hipLaunchKernelGGL((sample_merge_kernel<T>), dim3(batch), dim3(NT), 0, stream, p);
+    } else {
+        hipLaunchKernelGGL((sample_kernel<T>), dim3(batch), dim3(NT), 0, stream, p);
+    }
+}
 
 int launch_sample(int64_t* out, const void* logits, int64_t row_stride, float* probs_out,
                   const float* uniforms, int batch, int vocab, float temperature, int top_k, float top_p,
-                  int greedy, int dtype, hipStream_t stream) {
+                  int greedy, int dtype, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     SampleParams p;
     p.out = out; p.logits = logits; p.row_stride = row_stride; p.probs_out = probs_out;
     p.uniforms = uniforms; p.vocab = vocab; p.temperature = temperature; p.top_k = top_k;
     p.top_p = top_p; p.greedy = greedy;
-    if (dtype == AICOMP_KV_F32) hipLaunchKernelGGL((sample_kernel<float>), dim3(batch), dim3(NT), 0, stream, p);
-    else if (dtype == AICOMP_KV_F16) hipLaunchKernelGGL((sample_kernel<f16_t>), dim3(batch), dim3(NT), 0, stream, p);
-    else hipLaunchKernelGGL((sample_kernel<bf16_t>), dim3(batch), dim3(NT), 0, stream, p);
+    p.part_count = nullptr; p.part_list = nullptr; p.parts = 0; p.part_size = 0;
+    const size_t need = sample_workspace_bytes(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
+    if (need && workspace && workspace_bytes >= need) {
+        const int parts = sample_parts(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
+        p.part_size = ((vocab + parts - 1) / parts + 3) / 4 * 4;       // parts * part_size < vocab + 4 parts
+        p.parts = (vocab + p.part_size - 1) / p.part_size;             // none is empty
+        p.part_list = (uint2*)workspace;
+        p.part_count = (unsigned int*)(p.part_list + (size_t)batch * p.parts * PART_CAP);
+    }
+    if (dtype == AICOMP_KV_F32) launch_rows<float>(p, batch, stream);
+    else if (dtype == AICOMP_KV_F16) launch_rows<f16_t>(p, batch, stream);
+    else launch_rows<bf16_t>(p, batch, stream);
     AICOMP_HIP_LAUNCH_CHECK();
     return AICOMP_KV_OK;
 }

@@ -578,7 +578,7 @@ def sample_tokens(logits: torch.Tensor, temperature: float = 1.0, top_k: int = 0
     ``uniforms [B]`` (float32 in [0, 1)) makes the draw reproducible; by default they come from
     ``torch.rand`` with ``generator``.  Returns ``tokens [B]`` int64, or ``(tokens, probs [B, V])``.
     """
-    if not return_probs and _native("aicomp_sample_tokens") and (uniforms is not None or not do_sample):
+    if not return_probs and _native("aicomp_sample_tokens_split") and (uniforms is not None or not do_sample):
         tokens = _FAST.sample_tokens(logits, temperature, top_k, top_p, do_sample, uniforms)
         if tokens is not None:
             return tokens
@@ -596,9 +596,13 @@ def sample_tokens(logits: torch.Tensor, temperature: float = 1.0, top_k: int = 0
              "uniforms must be contiguous float32 [B]")
         _dev(uniforms, logits, "uniforms")
     if B:
-        rc = lib.aicomp_sample_tokens(out.data_ptr(), logits.data_ptr(), logits.stride(0), _ptr(probs),
-                                      _ptr(uniforms) if do_sample else None, B, V, float(temperature),
-                                      int(top_k), float(top_p), 0 if do_sample else 1, _dt(logits, "logits"),
-                                      _stream(logits))
+        greedy = 0 if do_sample else 1
+        need = lib.aicomp_sample_workspace_bytes(B, V, logits.stride(0), float(temperature), int(top_k), greedy,
+                                                 _dt(logits, "logits"))
+        scratch = torch.empty(need, dtype=torch.uint8, device=logits.device) if need else None
+        rc = lib.aicomp_sample_tokens_split(out.data_ptr(), logits.data_ptr(), logits.stride(0), _ptr(probs),
+                                            _ptr(uniforms) if do_sample else None, B, V, float(temperature),
+                                            int(top_k), float(top_p), greedy, _dt(logits, "logits"),
+                                            _ptr(scratch), need, _stream(logits))
         _lib.check(rc, lib)
     return (out, probs) if return_probs else out

@@ -46,7 +46,8 @@ extern "C" {
 #define AICOMP_KV_FP8_E4M3  2       /* OCP e4m3 ("e4m3fn"), max finite 448       */
 #define AICOMP_KV_F16       3       /* IEEE binary16                             */
 
-/* Library version (major*10000 + minor*100 + patch).  200 = 0.2.0: added
+/* Library version (major*10000 + minor*100 + patch).  300 = 0.3.0: added
+ * aicomp_sample_tokens_split and aicomp_sample_workspace_bytes.  200 = 0.2.0: added
  * aicomp_kv_set_small_decode_tokens, aicomp_paged_prefill_attn_items and
  * aicomp_paged_prefill_tile_positions; every 0.1 entry point is unchanged. */
 int aicomp_kv_version(void);
@@ -314,7 +315,7 @@ int aicomp_rope_kv_append(const void* q_in, void* q_out,
                           const float* k_scale, const float* v_scale, void* stream);
 
 /*
- * Token sampling, one launch per batch of rows.  Replaces _sample_token
+ * Token sampling of a batch of rows.  Replaces _sample_token
  * (opt_prime/opt_prime/inference.py:786-843): greedy argmax (:806-808), or
  * logits / temperature (:811-812), top-k (:815-818: entries below the k-th largest value are
  * removed, ties at that value stay), top-p (:821-837: in descending order an entry stays while
@@ -336,6 +337,21 @@ int aicomp_sample_tokens(int64_t* out, const void* logits, int64_t row_stride,
                          float* probs_out, const float* uniforms,
                          int batch, int vocab, float temperature, int top_k, float top_p,
                          int greedy, int logits_dtype, void* stream);
+
+/*
+ * The same call, with the same tokens, given scratch memory: greedy and top-k calls over a
+ * large vocabulary are then cut into parts of a row, so that a small batch fills the chip (two launches).
+ *   workspace       device scratch of aicomp_sample_workspace_bytes(...) bytes, 8-byte aligned, needing no
+ *                   initialisation; calls that may overlap need separate ones.  NULL or less: one
+ *                   launch, as aicomp_sample_tokens.
+ */
+int aicomp_sample_tokens_split(int64_t* out, const void* logits, int64_t row_stride,
+                               float* probs_out, const float* uniforms,
+                               int batch, int vocab, float temperature, int top_k, float top_p,
+                               int greedy, int logits_dtype, void* workspace,
+                               size_t workspace_bytes, void* stream);
+size_t aicomp_sample_workspace_bytes(int batch, int vocab, int64_t row_stride, float temperature, int top_k,
+                                     int greedy, int logits_dtype);
 
 #ifdef __cplusplus
 }

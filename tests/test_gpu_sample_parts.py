@@ -1,0 +1,70 @@
+"""Rows cut into parts against the one-launch kernel: the same tokens and kept sets.  The one-launch
+kernel's walk over a whole row (a row with fewer finite logits than k) rounds 1 / mass to float32 before the
+product, its candidate list does not: two roundings of 2^-24 apart at most."""
+import pytest
+import torch
+
+from aicomp_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _one_launch(x, temperature, top_k, top_p, do_sample, u):
+    lib = _lib.load()
+    out = torch.empty(x.shape[0], dtype=torch.int64, device=x.device)
+    probs = torch.empty(x.shape, dtype=torch.float32, device=x.device)
+    rc = lib.aicomp_sample_tokens(out.data_ptr(), x.data_ptr(), x.stride(0), probs.data_ptr(), u.data_ptr(), *x.shape,
+                                  temperature, top_k, top_p, 0 if do_sample else 1, ops._DT[x.dtype],
+                                  torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, lib)
+    return out, probs
+
+
+def _rows(V, dtype, device):
+    """A broad row, a peaked one, ties, few finite values, none, NaN, infinity, most of the row equal."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(10, V, generator=g) * 2.5
+    x[1, torch.randperm(V, generator=g)[:40]] += 12
+    x[2] = (x[2] * 2).round() / 2
+    x[3, torch.randperm(V, generator=g)[:V - 17]] = float("-inf")
+    x[4] = float("-inf")
+    x[5, V // 2] = float("nan")
+    x[6, V - 1] = float("inf")
+    x[7] = -1.25
+    x[7, ::1000] = 1.0
+    x[8, : V // 2] = float("-inf")
+    x[9, V - 1] = x[9, 3] = 40.0
+    return x.to(dtype).to(device)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,stride", [(16385, 16385), (16388, 16391), (32769, 32769), (50257, 50257), (98305, 98312), (81923, 81928),
+                                      (128255, 128255), (128256, 128256), (262144, 262144), (262145, 262145)])
+def test_parts_equal_the_one_launch_kernel(device, V, stride, dtype):
+    x = torch.zeros(10, stride, dtype=dtype, device=device)[:, :V]
+    x.copy_(_rows(V, dtype, device))
+    u = torch.linspace(0.01, 0.99, x.shape[0], device=device)
+    calls = [(0.8, 50, 0.9, True), (1.0, 1, 1.0, True), (1.3, 200, 0.95, True), (0.6, 256, 1.0, True),
+             (1.0, 257, 0.9, True), (40.0, 20, 0.9, True), (1.0, 0, 1.0, False)]
+    assert (_lib.load().aicomp_sample_workspace_bytes(10, V, stride, 0.8, 50, 0, ops._DT[dtype]) > 0) == (V <= 262144)
+    for temperature, top_k, top_p, do_sample in calls:
+        want, dist = _one_launch(x, temperature, top_k, top_p, do_sample, u)
+        got, probs = ops.sample_tokens(x, temperature, top_k, top_p, do_sample, u, return_probs=True)
+        plain = ops.sample_tokens(x, temperature, top_k, top_p, do_sample, u)
+        assert torch.equal(got, want) and torch.equal(plain, want), (temperature, top_k, top_p)
+        assert torch.equal(probs > 0, dist > 0) and torch.allclose(probs, dist, rtol=2.0 ** -22, atol=0.0)
+
+
+def test_parts_in_a_graph(device):
+    x, u = _rows(50257, torch.float32, device), torch.rand(10, device=device)
+    ops.sample_tokens(x, 0.8, 50, 0.9, uniforms=u)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        tokens = ops.sample_tokens(x, 0.8, 50, 0.9, uniforms=u)
+    for seed in range(3):
+        x.copy_(x[torch.randperm(10, device=device)])
+        u.uniform_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(tokens, _one_launch(x, 0.8, 50, 0.9, True, u)[0])

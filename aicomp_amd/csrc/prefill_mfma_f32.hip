@@ -9,19 +9,24 @@
 // softmax and the operand traffic hide under it).  Same mask rule as the 16-bit kernel: query i
 // of a chunk with prior context P sees keys j <= P + i.
 //
-// Work split   one workgroup (4 waves) per (128 query rows, sequence); a row is a (position,
+// Work split   one workgroup (8 waves) per (128 query rows, sequence); a row is a (position,
 //              head) pair, the G heads of one KV head packed per position when G divides 16, so a
-//              K/V tile staged in LDS serves the whole group.  A wave owns two 16-row column groups.
+//              K/V tile staged in LDS serves the whole group.  A wave owns 16 rows: a workgroup that
+//              is alone on its CU, as the last ones of a causal prompt are, still has two waves per
+//              SIMD to run one's softmax beside the other's products.  Four waves of 32 rows read the
+//              LDS tiles half as often and were slower at every size (us, 4 -> 8 waves, 32/8 heads):
+//              one chunk of 24 rows D 128 39.6 -> 14.0, 512 after 2048 275.5 -> 256.5, 2048 389 -> 371,
+//              4096 1311 -> 1304; D 64: 512 after 2048 168.0 -> 135.2, 2048 240.4 -> 192.3, 4096 682 -> 672.
 // K/V tiles    32 tokens, global -> registers (one tile ahead) -> LDS rows of head_dim floats + 16
 //              bytes (the operand reads below are then free of bank conflicts), double-buffered,
 //              one barrier per tile.
 // S^T = K Q^T  A = K rows from LDS, B = the wave's query rows (registers, pre-multiplied by
 //              scale * log2 e).  The k index of MFMA m in lane group g is 16 (m / 4) + 4 g + m % 4:
-//              one 16-byte LDS read supplies the A operands of four MFMAs, for both column groups.
+//              one 16-byte LDS read supplies the A operands of four MFMAs.
 // softmax      online, base 2, per lane one query; the row max crosses the four lanes of a row
 //              with two shuffles; the accumulators are rescaled only when a max moved.
 // O^T += V^T P^T  A = V^T: lane (dim r, g) reads V[token 4 g + m][16 j + r], one 4-byte LDS read per
-//              MFMA and column-group pair; B = P^T is exactly what the lane already holds.
+//              MFMA; B = P^T is exactly what the lane already holds.
 #include "common.h"
 
 #include <atomic>
@@ -32,8 +37,9 @@ namespace {
 
 constexpr int BS = 16;
 constexpr int KT = 32;                  // tokens per LDS tile
-constexpr int R = 2;                    // 16-row column groups per wave
-constexpr int WG_ROWS = 4 * 16 * R;     // query rows per workgroup
+constexpr int WAVES = 8;
+constexpr int NT = 64 * WAVES;
+constexpr int WG_ROWS = 16 * WAVES;     // query rows per workgroup
 constexpr float NEG_BIG = -1.0e30f;
 
 struct PrefillF32Params {
@@ -54,15 +60,15 @@ struct PrefillF32Params {
 };
 
 template <int DH>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(NT, 4)
 paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     constexpr int KROW = DH * 4 + 16;           // LDS row stride in bytes
     constexpr int KROWF = KROW / 4;             // ... in floats
     constexpr int TILE_F = KT * KROWF;          // floats per K (or V) tile
     constexpr int NQ = DH / 16;                 // 16-element chunks of a row (QK: 4 MFMAs each; PV: output tiles)
     constexpr int CPR = DH / 4;                 // float4 chunks per row
-    constexpr int RPL = 256 / CPR;              // rows one load of the workgroup covers (8 or 16)
-    constexpr int NL = KT / RPL;                // loads per tile and pool (4 or 2)
+    constexpr int RPL = NT / CPR;               // rows one load of the workgroup covers (16 or 32)
+    constexpr int NL = KT / RPL;                // loads per tile and pool (2 or 1)
     const int hgroup = blockIdx.x;
     int seq = blockIdx.y;
     int qtile = prefill_tile_of_slice(blockIdx.z, gridDim.z, p.num_cus, gridDim.x * gridDim.y);
@@ -87,9 +93,9 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     if (q0 >= n || n <= 0) return;
     if (prior < 0) {
         // a context shorter than the chunk itself: the rows are defined as zero, as in the other kernels
-        for (int i = tid; i < WG_ROWS * CPR; i += 256) {
-            const int row = i / CPR, chunk = i % CPR;
-            const int pos = q0 + row / p.gpack, hd = hgroup * p.gpack + row % p.gpack;
+        for (int i = tid; i < WG_ROWS * CPR; i += NT) {
+            const int zrow = i / CPR, chunk = i % CPR;
+            const int pos = q0 + zrow / p.gpack, hd = hgroup * p.gpack + zrow % p.gpack;
             if (pos < n)
                 *(float4*)(p.out + ((int64_t)(q_begin + pos) * p.hq + hd) * DH + 4 * chunk) = make_float4(0.f, 0.f, 0.f, 0.f);
         }
@@ -97,44 +103,32 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     }
 
     const int kvh = (hgroup * p.gpack) / p.group;
-    int qpos[R], head[R], qabs[R];
-    bool row_valid[R];
-#pragma unroll
-    for (int c = 0; c < R; ++c) {
-        const int row = 16 * R * w + 16 * c + r16;
-        qpos[c] = q0 + row / p.gpack;
-        head[c] = hgroup * p.gpack + row % p.gpack;
-        row_valid[c] = qpos[c] < n;
-        qabs[c] = row_valid[c] ? prior + qpos[c] : ctx - 1;     // padded rows: computed, never stored
-    }
+    const int row = 16 * w + r16;
+    const int qpos = q0 + row / p.gpack;
+    const int head = hgroup * p.gpack + row % p.gpack;
+    const bool row_valid = qpos < n;
+    const int qabs = row_valid ? prior + qpos : ctx - 1;        // padded rows: computed, never stored
     // (a wave whose rows all lie beyond the chunk's end has nothing to compute: it only takes part in
     // the tile loads and barriers)
-    const int wave_kv_end = q0 + (16 * R * w) / p.gpack >= n ? 0 : min(ctx, prior + q0 + (16 * R * w + 16 * R - 1) / p.gpack + 1);
-    const int wave_kv_min = prior + q0 + (16 * R * w) / p.gpack;
+    const int wave_kv_end = q0 + (16 * w) / p.gpack >= n ? 0 : min(ctx, prior + q0 + (16 * w + 15) / p.gpack + 1);
+    const int wave_kv_min = prior + q0 + (16 * w) / p.gpack;
     const int kv_end = min(ctx, prior + q0 + pos_per_wg);
     const int ntiles = (kv_end + KT - 1) / KT;
 
     // Q as the B operand: MFMA 4 q + e of chunk q takes element 16 q + 4 g4 + e of this lane's row
-    float4 qf[R][NQ];
+    float4 qf[NQ];
+    const float* qrow = p.query + ((int64_t)(q_begin + min(qpos, n - 1)) * p.hq + head) * DH + 4 * g4;
 #pragma unroll
-    for (int c = 0; c < R; ++c) {
-        const float* qrow = p.query + ((int64_t)(q_begin + min(qpos[c], n - 1)) * p.hq + head[c]) * DH + 4 * g4;
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            float4 v = *(const float4*)(qrow + 16 * q);
-            v.x *= p.qk_mul; v.y *= p.qk_mul; v.z *= p.qk_mul; v.w *= p.qk_mul;
-            qf[c][q] = v;
-        }
+    for (int q = 0; q < NQ; ++q) {
+        float4 v = *(const float4*)(qrow + 16 * q);
+        v.x *= p.qk_mul; v.y *= p.qk_mul; v.z *= p.qk_mul; v.w *= p.qk_mul;
+        qf[q] = v;
     }
 
-    float m[R], lsum[R];
-    f32x4_t O[R][NQ];
+    float m = NEG_BIG, lsum = 0.f;
+    f32x4_t O[NQ];
 #pragma unroll
-    for (int c = 0; c < R; ++c) {
-        m[c] = NEG_BIG; lsum[c] = 0.f;
-#pragma unroll
-        for (int j = 0; j < NQ; ++j) O[c][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int j = 0; j < NQ; ++j) O[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     const int32_t* table = p.block_table + (int64_t)seq * p.block_table_stride;
     const int last_blk = (ctx - 1) >> 4;
@@ -146,8 +140,8 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     auto fetch = [&](int t) {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
-            const int row = RPL * i + tid / CPR;
-            const int tok = t * KT + row;
+            const int trow = RPL * i + tid / CPR;
+            const int tok = t * KT + trow;
             const int bi = min(tok >> 4, last_blk);
             const int blk = max(0, min(table[bi], p.num_blocks - 1));
             const int64_t off = (((int64_t)blk * p.hkv + kvh) * BS + (tok & 15)) * DH + 4 * (tid % CPR);
@@ -160,11 +154,11 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
         float* vb = kb + TILE_F;
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
-            const int row = RPL * i + tid / CPR;
+            const int trow = RPL * i + tid / CPR;
             float4 vv = sv[i];
-            if (t * KT + row >= ctx) vv = make_float4(0.f, 0.f, 0.f, 0.f);
-            *(float4*)(kb + row * KROWF + 4 * (tid % CPR)) = sk[i];
-            *(float4*)(vb + row * KROWF + 4 * (tid % CPR)) = vv;
+            if (t * KT + trow >= ctx) vv = make_float4(0.f, 0.f, 0.f, 0.f);
+            *(float4*)(kb + trow * KROWF + 4 * (tid % CPR)) = sk[i];
+            *(float4*)(vb + trow * KROWF + 4 * (tid % CPR)) = vv;
         }
     };
 
@@ -179,92 +173,82 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
         const float* kb = lds + buf * 2 * TILE_F;
         const float* vb = kb + TILE_F;
 
-        // ---- S^T = K Q^T for the two 16-token blocks of the tile
-        f32x4_t sa[2][R];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int c = 0; c < R; ++c) sa[h][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        // ---- S^T = K Q^T for the two 16-token blocks of the tile (two accumulators in turn)
+        f32x4_t sa[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
             float4 a[2];
 #pragma unroll
             for (int h = 0; h < 2; ++h) a[h] = *(const float4*)(kb + (16 * h + r16) * KROWF + 16 * q + 4 * g4);
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h) sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].x, qf[q].x, sa[h], 0, 0, 0);
 #pragma unroll
-                for (int c = 0; c < R; ++c) {
-                    sa[h][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].x, qf[c][q].x, sa[h][c], 0, 0, 0);
-                    sa[h][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].y, qf[c][q].y, sa[h][c], 0, 0, 0);
-                    sa[h][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].z, qf[c][q].z, sa[h][c], 0, 0, 0);
-                    sa[h][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].w, qf[c][q].w, sa[h][c], 0, 0, 0);
-                }
+            for (int h = 0; h < 2; ++h) sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].y, qf[q].y, sa[h], 0, 0, 0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].z, qf[q].z, sa[h], 0, 0, 0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].w, qf[q].w, sa[h], 0, 0, 0);
         }
 
         // ---- online softmax: lane (query r16, g4) holds tokens tile_start + 16 h + 4 g4 + i
         const bool need_mask = tile_start + KT - 1 > wave_kv_min;      // wave-uniform
-        float pr[R][8];
+        float pr[8], sc[8];
 #pragma unroll
-        for (int c = 0; c < R; ++c) {
-            float sc[8];
+        for (int k = 0; k < 8; ++k) sc[k] = sa[k >> 2][k & 3];
+        if (need_mask) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) sc[k] = sa[k >> 2][c][k & 3];
-            if (need_mask) {
+            for (int k = 0; k < 8; ++k)
+                if (tile_start + 16 * (k >> 2) + 4 * g4 + (k & 3) > qabs) sc[k] = NEG_BIG;
+        }
+        float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_new = fmaxf(m, mx);
+        const float alpha = exp2f(m - m_new);
+        float psum = 0.f;
 #pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (tile_start + 16 * (k >> 2) + 4 * g4 + (k & 3) > qabs[c]) sc[k] = NEG_BIG;
-            }
-            float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-            mx = fmaxf(mx, __shfl_xor(mx, 16));
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            const float m_new = fmaxf(m[c], mx);
-            const float alpha = exp2f(m[c] - m_new);
-            float psum = 0.f;
+        for (int k = 0; k < 8; ++k) {
+            float e = exp2f(sc[k] - m_new);
+            if (need_mask && sc[k] == NEG_BIG) e = 0.f;
+            pr[k] = e;
+            psum += e;
+        }
+        lsum = lsum * alpha + psum;
+        m = m_new;
+        if (__any(alpha != 1.f)) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                float e = exp2f(sc[k] - m_new);
-                if (need_mask && sc[k] == NEG_BIG) e = 0.f;
-                pr[c][k] = e;
-                psum += e;
-            }
-            lsum[c] = lsum[c] * alpha + psum;
-            m[c] = m_new;
-            if (__any(alpha != 1.f)) {
-#pragma unroll
-                for (int j = 0; j < NQ; ++j) O[c][j] *= alpha;
-            }
+            for (int j = 0; j < NQ; ++j) O[j] *= alpha;
         }
 
         // ---- O^T += V^T P^T: A = V[token 16 h + 4 g4 + e][16 j + r16], B = this lane's own P values
 #pragma unroll
-        for (int j = 0; j < NQ; ++j) {
+        for (int j = 0; j < NQ; j += 2) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                float a[4];
+                float a[2][4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) a[e] = vb[(16 * h + 4 * g4 + e) * KROWF + 16 * j + r16];
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) a[i][e] = vb[(16 * h + 4 * g4 + e) * KROWF + 16 * (j + i) + r16];
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int c = 0; c < R; ++c)
-                        O[c][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], pr[c][4 * h + e], O[c][j], 0, 0, 0);
+                    for (int i = 0; i < 2; ++i)
+                        O[j + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], pr[4 * h + e], O[j + i], 0, 0, 0);
             }
         }
     }
 
-    // lane (query r16 of column group c, g4) holds O^T[element 16 j + 4 g4 + i][query] in O[c][j][i]
+    // lane (query r16, g4) holds O^T[element 16 j + 4 g4 + i][query] in O[j][i]
+    float l = lsum;
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (row_valid) {
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+        float* o = p.out + ((int64_t)(q_begin + qpos) * p.hq + head) * DH + 4 * g4;
 #pragma unroll
-    for (int c = 0; c < R; ++c) {
-        float l = lsum[c];
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
-        if (row_valid[c]) {
-            const float inv = l > 0.f ? 1.f / l : 0.f;
-            float* o = p.out + ((int64_t)(q_begin + qpos[c]) * p.hq + head[c]) * DH + 4 * g4;
-#pragma unroll
-            for (int j = 0; j < NQ; ++j)
-                *(float4*)(o + 16 * j) = make_float4(O[c][j][0] * inv, O[c][j][1] * inv, O[c][j][2] * inv, O[c][j][3] * inv);
-        }
+        for (int j = 0; j < NQ; ++j)
+            *(float4*)(o + 16 * j) = make_float4(O[j][0] * inv, O[j][1] * inv, O[j][2] * inv, O[j][3] * inv);
     }
 }
 
@@ -284,7 +268,7 @@ hipError_t launch_f32_variant(const PrefillF32Params& p, dim3 grid, hipStream_t 
             if (dev < 64) done.fetch_or(1ull << dev, std::memory_order_release);
         }
     }
-    hipLaunchKernelGGL((paged_prefill_mfma_f32_kernel<DH>), grid, dim3(256), lds_bytes, stream, p);
+    hipLaunchKernelGGL((paged_prefill_mfma_f32_kernel<DH>), grid, dim3(NT), lds_bytes, stream, p);
     return hipSuccess;
 }
 

@@ -187,7 +187,6 @@ class StepPlan:
     host_positions: np.ndarray = None
     # order of the prompt chunks' query tiles per head geometry and types: one list serves every layer of the step
     _prefill_items: dict = None
-    _only_chunks: Optional[bool] = None
 
     def prefill_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:
         """The (sequence, query tile) pairs of this step's prompt chunks, most expensive first, as the
@@ -268,12 +267,10 @@ class StepPlan:
     @property
     def only_chunks(self) -> bool:
         """Prompt chunks and nothing else, and device tensors of exactly their sizes."""
-        if self._only_chunks is None:
-            S, T = self.num_seqs, self.num_prefill_tokens
-            self._only_chunks = (0 < S == self.num_prefill_seqs and self.block_table.shape[0] == S
-                                 and self.context_lens.shape[0] == S and self.cu_q_lens.shape[0] == S + 1
-                                 and self.slot_mapping.shape[0] == T)
-        return self._only_chunks
+        S = self.num_seqs
+        return (0 < S == self.num_prefill_seqs and self.block_table.shape[0] == S
+                and self.context_lens.shape[0] == S and self.cu_q_lens.shape[0] == S + 1
+                and self.slot_mapping.shape[0] == self.num_prefill_tokens)
 
     @property
     def num_prefill_tokens(self) -> int:

@@ -389,6 +389,19 @@ def _mixed_plan(ctx, new, npre, max_q):
                     slot_mapping=None, positions=None, preempted=[], host_context_lens=np.asarray(ctx), host_cu_q_lens=cu)
 
 
+def test_only_chunks_follows_the_plan_as_it_is():
+    import dataclasses
+
+    import torch
+    plan = _mixed_plan([20, 30], [20, 10], 2, 20)
+    plan.slot_mapping = torch.zeros(30, dtype=torch.int64)
+    assert plan.only_chunks
+    wider = dataclasses.replace(plan, context_lens=torch.zeros(4, dtype=torch.int32))
+    assert not wider.only_chunks                  # padded: the call has to slice
+    plan.slot_mapping = torch.zeros(32, dtype=torch.int64)
+    assert not plan.only_chunks
+
+
 def test_step_item_list_orders_a_mixed_step_for_one_launch():
     """ops.step_items: every chunk tile and every decode row exactly once; decode rows that are the
     longer items open the list (one CU-round of them, then one of chunk tiles, then alternating,

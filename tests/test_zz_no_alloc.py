@@ -99,3 +99,50 @@ def test_static_scratch_refuses_shapes_beyond_its_size(device):
     rc = lib.aicomp_paged_decode_attn_append_static(p, p, p, p, 1024, 128, p, p, p, 64, p, 1024, 64, 8, 128, 16,
                                                     64, 4096, 0.1, _lib.BF16, _lib.BF16, None, None, 0, None)
     assert rc == 4 and b"built-in scratch" in lib.aicomp_kv_last_error()
+
+
+@pytest.mark.routing("balanced")
+@pytest.mark.parametrize("B,hq,hkv,longest", [(32, 16, 1, 2048), (1024, 64, 4, 64)])
+def test_static_scratch_takes_float32_batches_whose_balanced_partials_do_not_fit(device, B, hq, hkv, longest):
+    """The balanced schedule's partials (34 and 66 MiB here) are more than the array holds, the grid schedule's
+    (8 MiB, none) are not: the call is accepted, and is the grid schedule's, bit for bit."""
+    import test_gpu_prefill as tp
+    lib, d, F32 = _lib.load(), 128, _lib.F32
+    ctx = [1 + (i * 977) % longest for i in range(B - 1)] + [longest]
+    c = tp.build_case(device, [n - 1 for n in ctx], [1] * B, hq, hkv, d, dtype=torch.float32, seed=B, poison="all")
+    rows = torch.arange(B, device=device)
+    blk, at = c["table"][rows, (c["ctx"] - 1).long() // 16].long(), (c["ctx"] - 1).long() % 16
+    nk, nv = c["k_pool"][blk, :, at].clone(), c["v_pool"][blk, :, at].clone()
+    width = c["table"].shape[1]
+    assert lib.aicomp_paged_decode_workspace_bytes(B, hq, hkv, d, 16, width, F32, F32, 0) > STATIC_SCRATCH_BYTES
+    outs = []
+    for static in (True, False):
+        kp, vp = c["k_pool"].clone(), c["v_pool"].clone()
+        kp[blk, :, at], vp[blk, :, at] = float("nan"), float("nan")
+        out = torch.full_like(c["q"], float("nan"))
+        head = (out.data_ptr(), c["q"].data_ptr(), nk.data_ptr(), nv.data_ptr(), nk.stride(0), nk.stride(1), kp.data_ptr(),
+                vp.data_ptr(), c["table"].data_ptr(), c["table"].stride(0), c["ctx"].data_ptr(), B, hq, hkv, d, 16, width,
+                kp.shape[0], c["scale"], F32, F32, None, None)
+        stream = torch.cuda.current_stream().cuda_stream
+        if static:
+            rc = lib.aicomp_paged_decode_attn_append_static(*head, 0, stream)
+        else:
+            ps = 64 if longest == 2048 else 1024
+            ws = torch.empty(max(16, lib.aicomp_paged_decode_workspace_bytes(B, hq, hkv, d, 16, width, F32, F32, ps)),
+                             dtype=torch.uint8, device=device)
+            rc = lib.aicomp_paged_decode_attn_append(*head, ps, ws.data_ptr(), ws.numel(), stream)
+        _lib.check(rc, lib)
+        torch.cuda.synchronize()
+        outs.append((out, kp, vp))
+    (a, ka, va), (b, kb, vb) = outs
+    assert torch.isfinite(a).all() and _same(a, b) and _same(ka, kb) and _same(va, vb)
+    assert _same(ka, c["k_pool"]) and _same(va, c["v_pool"])                # the new rows are where they were taken from
+    # plain attention of every sixteenth row in float64; 1e-5: the bound of test_gpu_decode_f32
+    for r in range(0, B, 16):
+        n = ctx[r]
+        ids = c["table"][r, :-(-n // 16)].long()
+        k, v = (p[ids].transpose(1, 2).reshape(-1, hkv, d)[:n].double() for p in (c["k_pool"], c["v_pool"]))
+        q = c["q"][r].double().view(hkv, hq // hkv, d)
+        w = torch.softmax((q[:, :, None] * k.transpose(0, 1)[:, None]).sum(-1) * c["scale"], -1)
+        want = (w[..., None] * v.transpose(0, 1)[:, None]).sum(2).view(hq, d)
+        assert (a[r].double() - want).abs().max().item() <= 1e-5

@@ -57,6 +57,15 @@ int dtype_code(at::ScalarType t) {
 
 void layer_free(PyObject* cap) { delete (Layer*)PyCapsule_GetPointer(cap, "aicomp_amd.layer"); }
 
+// A call that uses the scratch below is two launches, and on one stream two of them must not interleave: the
+// second call's partials would replace the first's before their merge reads them.  Two host threads on one
+// stream can get there, one of them inside a plain call, which lets go of the interpreter lock.  Held over the
+// launches alone and never across a wait for the interpreter lock.
+std::mutex& scratch_launches() {
+    static auto* mu = new std::mutex();
+    return *mu;
+}
+
 // scratch of calls that need a merge: one growing buffer per (device, stream), never destroyed
 // (tensors freed at interpreter exit, after the allocator, would fault)
 at::Tensor cached_scratch(const c10::Device& dev, void* stream, size_t bytes) {
@@ -154,10 +163,13 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         }
         // (the allocator's own entry: at::empty goes through the dispatcher for the same result)
         at::Tensor out(at::detail::empty_cuda(query.sizes(), L->st, L->dev, c10::MemoryFormat::Contiguous));
+        std::unique_lock<std::mutex> one_at_a_time(scratch_launches(), std::defer_lock);
+        if (ws) one_at_a_time.lock();
         const int rc = aicomp_paged_decode_attn_append(
             out.data_ptr(), query.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1) * hstep, L->kp, L->vp,
             L->table, L->table_stride, L->ctx + (position + 1) * L->ctx_stride, L->B, hq, L->hkv, L->d, L->bs, width,
             L->nb, (float)scale, L->dt, L->dt, nullptr, nullptr, 0, ws, ws_bytes, stream);
+        if (ws) one_at_a_time.unlock();
         if (rc != AICOMP_KV_OK) FAIL("aicomp_kv error %d: %s", rc, aicomp_kv_last_error());
         return THPVariable_Wrap(std::move(out));
     } catch (const std::exception& e) {
@@ -349,17 +361,21 @@ PyObject* paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
         const c10::DeviceGuard guard(q->device());
         void* stream = stream_of(*q);
         at::Tensor scratch;
+        bool shared = false;                           // the module's own scratch, not the caller's
         if (args[10] != Py_None) {
             const at::Tensor* w = plain(args[10]);
             if (!w) Py_RETURN_FALSE;
             scratch = *w;
         } else {
             const size_t need = aicomp_paged_decode_workspace_bytes((int)B, hq, p.hkv, p.d, p.bs, width, dt, p.dt, partition);
-            if (need) scratch = cached_scratch(q->device(), stream, need);
+            shared = need != 0;
+            if (shared) scratch = cached_scratch(q->device(), stream, need);
         }
         void* ws = scratch.defined() ? scratch.data_ptr() : nullptr;
         const size_t ws_bytes = scratch.defined() ? (size_t)(scratch.numel() * scratch.element_size()) : 0;
         const int rc = unlocked([&] {
+            std::unique_lock<std::mutex> one_at_a_time(scratch_launches(), std::defer_lock);
+            if (shared) one_at_a_time.lock();
             const int32_t *bt = (const int32_t*)table->data_ptr(), *cl = (const int32_t*)ctx->data_ptr();
             if (nk)
                 return aicomp_paged_decode_attn_append(

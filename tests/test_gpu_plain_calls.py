@@ -86,3 +86,41 @@ def test_strided_rows_are_still_converted(device):
     want = _inputs(device)
     ops.kv_append(want["k"], want["v"], want["kp"], want["vp"], want["slots"])
     assert torch.equal(a["kp"], want["kp"]) and torch.equal(a["vp"], want["vp"])
+
+
+@pytest.mark.gpu
+def test_two_threads_on_one_stream_share_the_scratch(device):
+    """Calls of two launches (decode and merge) from two host threads on one stream, one through the operator's
+    lean route and one through the plain call: each gets what it gets alone, bit for bit, every time."""
+    import threading
+
+    from aicomp_amd import kv_cache as akv
+    from aicomp_amd import _aicomp_fast as fast
+    torch.manual_seed(5)
+    B, hq, hkv, d, n, rounds = 4, 8, 2, 64, 2000, 400
+    layer = akv._PagedLayer(B, hkv, d, 2048, BF, device)
+    layer.append(*(torch.randn(B, hkv, n, d, device=device).to(BF) for _ in range(2)), 0, 1)
+    handle = fast.layer(layer.k_pool, layer.v_pool, layer.block_table, layer.ctx_rows)
+    q = torch.randn(B, hq, 1, d, device=device).to(BF)
+    new = [torch.randn(B, hkv, 1, d, device=device).to(BF) for _ in range(2)]
+    other = [t.clone() for t in (layer.k_pool, layer.v_pool)]
+    rows, lens = torch.randn(B, hq, d, device=device).to(BF), torch.tensor([1999, 700, 1300, 1], dtype=torch.int32, device=device)
+    calls = [lambda: fast.decode_step(handle, q, *new, n, 1, 0.125).view(B, hq, d),
+             lambda: ops.paged_decode_attn(torch.empty_like(rows), rows, *other, layer.block_table, lens, 0.125)]
+    assert all(ops.decode_workspace_bytes(B, hq, hkv, d, 16, w, BF, BF) > 0 for w in (126, 128))
+    want = [f() for f in calls]
+    torch.cuda.synchronize()
+    got, go = [[], []], threading.Barrier(2)
+
+    def run(i):
+        go.wait()
+        got[i] += [calls[i]() for _ in range(rounds)]
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == rounds and all(torch.equal(x, want[i]) for x in got[i])

@@ -209,7 +209,8 @@ rope_kv_append_kernel(RopeParams p) {
     }
 }
 
-// Any other head_dim (a multiple of 16): one lane per chunk of one (token, head) row.
+// Any other head_dim (a multiple of 16), and what the launch above cannot hold: one lane per chunk of one
+// (token, head) row.
 template <typename T, bool FP8POOL>
 __global__ void __launch_bounds__(256)
 rope_kv_append_any_kernel(RopeParams p) {
@@ -329,15 +330,17 @@ int launch_rope_kv_append(const void* q_in, void* q_out, int64_t q_ts, int64_t q
     do {                                                                                                             \
         if (d == 64) AICOMP_ROPE_NI(T, 4); else AICOMP_ROPE_NI(T, 8);                                                \
     } while (0)
-    if ((d == 64 || d == 128) && num_tokens <= INT32_MAX) {
-        const int items = (hq + 2 * hkv) * (d / 16);
-        // Two heads per lane (one read of the cos / sin chunks for both) once there are tokens enough to
-        // fill the chip, one below: 2108 tokens, 32 / 8 heads, D 128: 10.4 and 10.8 us; 64 tokens 2.79 and
-        // 2.55.  Workgroups of at most 128 lanes: of 256, 10.8 us; four heads per lane, 11.2 us.
-        constexpr int LANES = 128, TOKENS_TWO = 256;
-        const int ni = items > LANES && num_tokens >= TOKENS_TWO ? 2 : 1;
-        const int slices = (items + ni * LANES - 1) / (ni * LANES);
-        const int threads = (items + ni * slices * 64 - 1) / (ni * slices * 64) * 64;
+    const int items = (hq + 2 * hkv) * (d / 16);
+    // Two heads per lane (one read of the cos / sin chunks for both) once there are tokens enough to
+    // fill the chip, one below: 2108 tokens, 32 / 8 heads, D 128: 10.4 and 10.8 us; 64 tokens 2.79 and
+    // 2.55.  Workgroups of at most 128 lanes: of 256, 10.8 us; four heads per lane, 11.2 us.
+    constexpr int LANES = 128, TOKENS_TWO = 256;
+    const int ni = items > LANES && num_tokens >= TOKENS_TWO ? 2 : 1;
+    const int slices = (items + ni * LANES - 1) / (ni * LANES);
+    const int threads = (items + ni * slices * 64 - 1) / (ni * slices * 64) * 64;
+    // A launch dimension holds less than 2^32 lanes: few heads, rounded up to whole waves, over more than 33
+    // to 67 million tokens go the other way, as do more slices than the second dimension has.
+    if ((d == 64 || d == 128) && num_tokens * threads <= UINT32_MAX && slices <= 65535) {
         dim3 grid((unsigned)num_tokens, (unsigned)slices), block(threads);
         if (in_dtype == AICOMP_KV_BF16) AICOMP_ROPE_T(bf16_t);
         else if (in_dtype == AICOMP_KV_F16) AICOMP_ROPE_T(f16_t);

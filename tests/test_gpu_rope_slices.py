@@ -49,3 +49,22 @@ def _check(device, hq, hkv, d, T, dtype, kv):
     bits = lambda t: t.view({1: torch.uint8, 2: torch.int16, 4: torch.int32}[t.element_size()])
     assert torch.equal(bits(out), bits(rot(q)))
     assert torch.equal(bits(kp), bits(kp2)) and torch.equal(bits(vp), bits(vp2))
+
+
+def test_more_tokens_than_a_launch_of_one_per_workgroup_holds(device):
+    """2^26 + 3 tokens of one head: rounded up to whole waves they are more than the 2^32 lanes of a launch
+    dimension.  The same row for every token (stride 0); the first, a middle and the last one are stored."""
+    T, d, dtype = (1 << 26) + 3, 64, torch.bfloat16
+    g = torch.Generator().manual_seed(1)
+    row = torch.randn(3, 1, 1, d, generator=g).to(dtype).to(device)
+    q, k, v = (row[i].expand(T, 1, d) for i in range(3))
+    cos, sin = ops.rotary_tables(1.0 / 10000.0 ** (torch.arange(0, d, 2) / d), 8, dtype, device=device)
+    slots = torch.full((T,), -1, dtype=torch.int64, device=device)
+    at = [0, (1 << 26) - 1, T - 1]
+    slots[at] = torch.tensor([3, 17, 30], device=device)
+    kp, vp = (torch.zeros(2, 1, 16, d, dtype=dtype, device=device) for _ in range(2))
+    out = torch.zeros(1, 1, d, dtype=dtype, device=device)
+    ops.rope_kv_append(q, k, v, cos, sin, torch.full((T,), 5, device=device), kp, vp, slots, query_out=out.expand(T, 1, d))
+    kp2, vp2, out2 = torch.zeros_like(kp), torch.zeros_like(vp), torch.empty(3, 1, d, dtype=dtype, device=device)
+    ops.rope_kv_append(q[:3], k[:3], v[:3], cos, sin, torch.full((3,), 5, device=device), kp2, vp2, slots[at], query_out=out2)
+    assert torch.equal(out, out2[:1]) and torch.equal(kp, kp2) and torch.equal(vp, vp2) and bool(kp.any())

@@ -1070,12 +1070,15 @@ int launch_decode_mfma(const DecodeArgs& a) {
     p.new_token_stride = a.new_token_stride; p.new_head_stride = a.new_head_stride;
     dim3 grid((unsigned)a.hkv, (unsigned)a.num_parts, (unsigned)a.rows);
     const bool fp8 = a.kv_dtype == AICOMP_KV_FP8_E4M3, d64 = a.d == 64;
-    // Eight waves instead of four per workgroup once a partition is more than sixteen tiles: such a call
-    // has few workgroups, each a chain of rounds of one tile per wave at memory latency, and half the
-    // rounds outweigh the longer merge (1 row of 600 tokens, D 128: 7.9 -> 6.5 us; 500 tokens, D 64,
-    // eight tiles: 5.72 us with four waves, 5.84 with eight; 16 rows of 500, D 128, sixteen: 8.70 and 8.88).
+    // Eight waves instead of four per workgroup for partitions of more than sixteen tiles in at most one
+    // workgroup per CU: each is then a chain of rounds of one tile per wave at memory latency, and half the
+    // rounds outweigh the longer merge (D 128, 576 tokens, 1 to 10 rows of 8 KV heads: 7.8 -> 6.9 us, fp8 9.1 ->
+    // 8.0; float32 448 tokens 16.2 -> 13.9; 500 tokens, D 64, eight tiles: 5.72 us with four waves, 5.84 with
+    // eight; 16 rows of 500, D 128, sixteen: 8.70 and 8.88).  A CU that has two workgroups has eight waves anyway,
+    // and the larger ones are slower: 576 tokens, 256 workgroups 12.5 and 12.4, 320 workgroups 18.2 and 20.5; 1100
+    // rows of 1024 tokens of fp8 406 and 464.
     const int tile = a.q_dtype == AICOMP_KV_F32 ? (d64 ? TILE : TILE / 2) : (d64 ? 2 * TILE : TILE);
-    const bool wide = a.partition_size > 16 * tile;
+    const bool wide = a.partition_size > 16 * tile && a.rows * a.hkv * a.num_parts <= 256;
 #define AICOMP_LAUNCH_GRID(...)                                                                                        \
     do {                                                                                                               \
         if (wide) hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 8>), grid, dim3(512), 0, a.stream, p);     \

@@ -24,3 +24,16 @@ def test_rows_around_the_one_workgroup_limit(device, d, kv, dtype, limit):
                                            c["ctx"], c["scale"], c["ks"], c["vs"]))
         assert_close_attn(got, tp.oracle(c), *((1e-5, 1e-5) if dtype == torch.float32 else (1e-2, 2e-2)), f"{d} {dtype} {longest}")
         assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("rows", [32, 33])
+@pytest.mark.parametrize("d,kv,dtype,longest", [(128, None, torch.bfloat16, 600), (128, torch.float8_e4m3fn, torch.bfloat16, 544),
+                                               (64, None, torch.float16, 1100), (128, None, torch.float32, 288)])
+def test_one_workgroup_per_cu_and_one_more_row(device, d, kv, dtype, longest, rows):
+    """Partitions of more than sixteen tiles in 256 workgroups (eight waves each) and in 264 (four)."""
+    ps = -(-longest // 64) * 64
+    ctx = [longest - 13 * i % (longest - 1) for i in range(rows)]
+    c = tp.build_case(device, [n - 1 for n in ctx], [1] * rows, 8, 8, d, dtype=dtype, kv_dtype=kv, seed=rows)
+    got = to_f64(ops.paged_decode_attn(torch.full_like(c["q"], float("nan")), c["q"], c["k_pool"], c["v_pool"], c["table"],
+                                       c["ctx"], c["scale"], c["ks"], c["vs"], partition_size=ps))
+    assert_close_attn(got, tp.oracle(c), *((1e-5, 1e-5) if dtype == torch.float32 else (1e-2, 2e-2)), f"{d} {dtype} {rows}")

@@ -64,8 +64,9 @@ static bool streamk_shape(int batch, int hq, int hkv, int d, int bs, int q_dtype
 // A decode call over few, short rows is a chain of launch and memory latencies, not a stream: the
 // balanced schedule (set up for 256 CUs of work, always followed by its merge kernel) then loses to
 // one workgroup per (row, KV head, partition) on the grid schedule, without any merge kernel when
-// no row can be longer than 768 (head_dim 128) or 1280 (64) tokens of a 16-bit pool, 640 of another (measured on 1 to 16 rows of 512
-// and 2048 tokens: 5.4-8.5 against 9-13 us, 8-15 against 11-17 us).  "Small" is rows x (table width x block size) at or
+// no row can be longer than 768 (head_dim 128) or 1280 (64) tokens of a 16-bit pool, 640 or 448 of
+// another (measured on 1 to 16 rows of 512 and 2048 tokens: 5.4-8.5 against 9-13 us, 8-15 against
+// 11-17 us).  "Small" is rows x (table width x block size) at or
 // below a process-wide threshold: 32768 by default, or the value of the environment variable
 // AICOMP_KV_SMALL_DECODE_TOKENS when the library first needs it (read once, never again), or what
 // aicomp_kv_set_small_decode_tokens() stored last (0 keeps every automatic call of a supported
@@ -92,9 +93,14 @@ static int auto_partition(int64_t rows, int hkv, int d, int bs, int max_blocks, 
         // launch, or partitions of 256 tokens.  The line lies where the merge's launch (about 3 us of
         // device and 3 us of host time) costs what the longer chain of one workgroup does: 1000 and
         // 1200 tokens at D 64 whole 7.2 and 7.4 us, split 8.0 us, 2000 tokens 9.7 and 7.9; D 128: 760
-        // tokens 7.7 and 8.8, 1000 tokens 9.2 and 8.2 us.  Other pools keep 640: float32 rows are bound by
-        // the matrix instruction of their one CU (640 tokens, D 128: 18.0 whole, 14.9 split in 256).
-        const int64_t whole = !is_16bit_float(kv_dtype) ? 640 : d == 64 ? 1280 : 768;
+        // tokens 7.7 and 8.8, 1000 tokens 9.2 and 8.2 us.  Other pools: 640.  Float32 at D 64: 640 tokens of
+        // one row whole 10.4 us, split 10.5, 768 tokens 12.0 and 10.6.  A float32 row at D 128 is four times the
+        // matrix instructions of a bf16 one on its CU: whole up to 448 tokens where the split has a CU for
+        // each of its workgroups (one row of 448 13.0 whole, 13.2 split; 512 tokens 15.0 and 13.9, 640 17.6
+        // and 13.7; 16 rows of 8 KV heads, 512 tokens 18.0 and 16.9), otherwise up to 640 (those 16 rows,
+        // 576 tokens 19.2 and 22.1, 768 tokens 24.2 and 23.9).
+        const bool f32_few = kv_dtype == AICOMP_KV_F32 && d == 128 && rows * hkv * ((max_ctx + 255) / 256) <= 256;
+        const int64_t whole = f32_few ? 448 : !is_16bit_float(kv_dtype) ? 640 : d == 64 ? 1280 : 768;
         ps = max_ctx <= whole ? (int)((max_ctx + 63) / 64 * 64) : 256;
     } else {
         ps = 64;       // vector-ALU kernel on few short rows: spread the call wide

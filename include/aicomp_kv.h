@@ -127,8 +127,9 @@ int aicomp_kv_append(const void* key, const void* value,
  *                   threshold of aicomp_kv_set_small_decode_tokens(), default 32768) runs one workgroup per (row, KV head,
  *                   256-token partition) instead, and no merge kernel at all when
  *                   max_blocks_per_seq * block_size <= 768 (head_dim 128) or 1280 (64) over a
- *                   16-bit pool, 640 over another: such a call is bound by launch and memory latency, not by bandwidth.  The result is the
- *                   same to within the tolerance between split sizes (2e-3).
+ *                   16-bit pool, 640 over another (448 over a float32 pool of head_dim 128 when
+ *                   the partitions of all rows and KV heads are at most 256): such a call is bound by launch and memory latency, not
+ *                   by bandwidth.  The result is the same to within the tolerance between split sizes (2e-3).
  *   workspace       device scratch of at least
  *                   aicomp_paged_decode_workspace_bytes(...) bytes (may be NULL
  *                   when that returns 0), 16-byte aligned.  Its contents need

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("d,kv,dtype,limit", [(128, None, torch.bfloat16, 768), (64, None, torch.float16, 1280),
-                                             (128, torch.float8_e4m3fn, torch.bfloat16, 640), (64, None, torch.float32, 640)])
+                                             (128, torch.float8_e4m3fn, torch.bfloat16, 640), (64, None, torch.float32, 640),
+                                             (128, None, torch.float32, 448)])
 def test_rows_around_the_one_workgroup_limit(device, d, kv, dtype, limit):
     ops.set_small_decode_tokens(1 << 40)                    # the grid schedule; restored by the suite's fixture
     for longest in (limit - 255, limit - 16, limit, limit + 1):

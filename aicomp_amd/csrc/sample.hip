@@ -56,14 +56,15 @@ struct SampleParams {
     int greedy;
     // rows cut into parts (NULL / 0: not): what sample_parts_kernel leaves for sample_kernel
     unsigned int* part_count;            // [B, parts] candidates of a part, PART_WHOLE: take the whole row instead
-    uint2* part_list;                    // [B, parts, PART_CAP] (order key of the scaled logit, index)
+    uint2* part_list;                    // [B, parts, part_cap] (order key of the scaled logit, index)
     int parts, part_size;                // part_size: a multiple of 4 and at most PART_MAX
+    int part_cap;                        // candidates of a part: part_capacity()
 };
 
 constexpr int PART_SLOTS = 16;                      // logits a lane of a part holds in registers
 constexpr int PART_MAX = NT * PART_SLOTS;           // 16384
-constexpr int PART_CAP = 1024;                      // candidates of a part
-constexpr int RAW_CAP = 2048;                       // ... before the exact test
+constexpr int GREEDY_CAP = 256;                     // room per part of a greedy call, which keeps one: 2 KB apart
+constexpr int RAW_CAP = 2048;                       // candidates of a part before the exact test
 constexpr int MAX_PARTS = 16;
 constexpr int MERGE_SLOTS = 8;                      // candidates a lane of the merge takes: NT * 8 per row
 constexpr int PART_MAX_K = 256;
@@ -448,7 +449,7 @@ __device__ __forceinline__ Nucleus nucleus_threshold(Shared& s, Src src, uint32_
 // least 16 r >= k elements of the part reach the smallest of the sixteen, so whatever lies below it (in
 // scaled order, ties stay) is not among the part's top k, nor the row's.  About 2.6 k of 16384 pass at
 // k = 50.  A logit of -inf has no mass and is left out; a part with a NaN, or one
-// with more than PART_CAP candidates (masses of equal logits), sends its row the whole way.  Greedy: the part's
+// with more than part_cap candidates (masses of equal logits), sends its row the whole way.  Greedy: the part's
 // argmax is its one candidate.
 //
 // Bound by latency: one round of loads, 22 ballots, three barriers, a few dozen appends.  64 rows of 128256
@@ -491,7 +492,7 @@ sample_parts_kernel(SampleParams p) {
     };
     const unsigned int tail_idx = (unsigned int)(begin + 4 * n4 + tid);
     const int64_t slot = (int64_t)row_idx * p.parts + part;
-    uint2* list = p.part_list + slot * PART_CAP;
+    uint2* list = p.part_list + slot * (GREEDY ? GREEDY_CAP : p.part_cap);
 
     if constexpr (GREEDY) {
         // ascending indices within a lane (the tail's lie above all others), the lowest one wins a tie
@@ -557,11 +558,11 @@ sample_parts_kernel(SampleParams p) {
         const uint32_t key = order_key(apply_temperature<T>(raw_x[i], p.temperature));
         if (key >= key_ls) {
             const unsigned int j = atomicAdd(&n_list, 1u);
-            if (j < PART_CAP) list[j] = make_uint2(key, raw_i[i]);
+            if (j < (unsigned int)p.part_cap) list[j] = make_uint2(key, raw_i[i]);
         }
     }
     __syncthreads();
-    if (tid == 0) p.part_count[slot] = whole || nr > RAW_CAP || n_list > PART_CAP ? PART_WHOLE : n_list;
+    if (tid == 0) p.part_count[slot] = whole || nr > RAW_CAP || n_list > (unsigned int)p.part_cap ? PART_WHOLE : n_list;
 }
 
 // Index of the row's maximum, the lowest one among equals (0: nothing above -inf).
@@ -1089,8 +1090,8 @@ sample_merge_kernel(SampleParams p) {
 #pragma unroll
     for (int q = 0; q < MAX_PARTS; ++q) {
         const unsigned int c = q < p.parts ? counts[q] : 0u;
-        fits = fits && c <= PART_CAP;
-        total += min(c, (unsigned int)PART_CAP);
+        fits = fits && c <= (unsigned int)p.part_cap;
+        total += min(c, (unsigned int)p.part_cap);
         end[q] = total;
     }
     if (fits && total == 0) {                // nothing above -inf
@@ -1099,7 +1100,7 @@ sample_merge_kernel(SampleParams p) {
     }
     if (fits && total <= (unsigned int)(NT * MERGE_SLOTS)) {
         // candidate j goes to wave j % 16, so that the waves' shares are alike; lanes without one: key 0
-        const uint2* lists = p.part_list + (int64_t)row_idx * p.parts * PART_CAP;
+        const uint2* lists = p.part_list + (int64_t)row_idx * p.parts * p.part_cap;
         uint2 e[MERGE_SLOTS];
         uint32_t top = 0;
 #pragma unroll
@@ -1112,7 +1113,7 @@ sample_merge_kernel(SampleParams p) {
 #pragma unroll
                 for (int c = 0; c < MAX_PARTS - 1; ++c)
                     if (j >= end[c]) { q = c + 1; start = end[c]; }
-                e[u] = lists[(int64_t)q * PART_CAP + (j - start)];
+                e[u] = lists[(int64_t)q * p.part_cap + (j - start)];
             }
             top = max(top, e[u].x);
         }
@@ -1159,9 +1160,9 @@ greedy_kernel(SampleParams p) {
     const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
     int best_i;
     if (p.parts) {
-        uint2 c = p.part_list[(int64_t)row_idx * p.parts * PART_CAP];
+        uint2 c = p.part_list[(int64_t)row_idx * p.parts * GREEDY_CAP];
         for (int q = 1; q < p.parts; ++q) {
-            const uint2 o = p.part_list[((int64_t)row_idx * p.parts + q) * PART_CAP];
+            const uint2 o = p.part_list[((int64_t)row_idx * p.parts + q) * GREEDY_CAP];
             if (o.x > c.x || (o.x == c.x && o.y < c.y)) c = o;
         }
         best_i = c.y == 0x7fffffffu ? 0 : (int)c.y;
@@ -1198,9 +1199,16 @@ static int sample_parts(int batch, int vocab, int64_t row_stride, float temperat
     return dtype == AICOMP_KV_F32 || all <= 512 ? parts : 1;
 }
 
+// Candidates a part has room for.  Of 16384 normally distributed logits about 2.7 k pass the bound of sixteen waves
+// (55 for k <= 16), the most seen in 12000 parts 335 at k = 50 and 825 at k = 256; a part with more (masses
+// of equal logits) sends its row the whole way.  At k = 50 a row of 128256 has 42 KB, 43 MB for 1024 rows.
+// Greedy, 64 rows of eight parts: 9.75 us with the parts 2 KB or 8 KB apart, 9.9 with 1 KB, 10.1 with 128 bytes
+// and the distance an argument.
+static int part_capacity(int top_k, int greedy) { return greedy ? GREEDY_CAP : 256 + 8 * top_k < 1024 ? 256 + 8 * top_k : 1024; }
+
 size_t sample_workspace_bytes(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy, int dtype) {
     const int parts = sample_parts(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
-    return parts < 2 ? 0 : (size_t)batch * parts * (PART_CAP * sizeof(uint2) + sizeof(unsigned int));
+    return parts < 2 ? 0 : (size_t)batch * parts * (part_capacity(top_k, greedy) * sizeof(uint2) + sizeof(unsigned int));
 }
 
 template <typename T>
@@ -1223,14 +1231,15 @@ int launch_sample(int64_t* out, const void* logits, int64_t row_stride, float* p
     p.out = out; p.logits = logits; p.row_stride = row_stride; p.probs_out = probs_out;
     p.uniforms = uniforms; p.vocab = vocab; p.temperature = temperature; p.top_k = top_k;
     p.top_p = top_p; p.greedy = greedy;
-    p.part_count = nullptr; p.part_list = nullptr; p.parts = 0; p.part_size = 0;
+    p.part_count = nullptr; p.part_list = nullptr; p.parts = 0; p.part_size = 0; p.part_cap = 0;
     const size_t need = sample_workspace_bytes(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
     if (need && workspace && workspace_bytes >= need) {
         const int parts = sample_parts(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
         p.part_size = ((vocab + parts - 1) / parts + 3) / 4 * 4;       // parts * part_size < vocab + 4 parts
         p.parts = (vocab + p.part_size - 1) / p.part_size;             // none is empty
+        p.part_cap = part_capacity(top_k, greedy);
         p.part_list = (uint2*)workspace;
-        p.part_count = (unsigned int*)(p.part_list + (size_t)batch * p.parts * PART_CAP);
+        p.part_count = (unsigned int*)(p.part_list + (size_t)batch * p.parts * p.part_cap);
     }
     if (dtype == AICOMP_KV_F32) launch_rows<float>(p, batch, stream);
     else if (dtype == AICOMP_KV_F16) launch_rows<f16_t>(p, batch, stream);

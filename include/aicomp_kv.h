@@ -347,7 +347,9 @@ int aicomp_sample_tokens(int64_t* out, const void* logits, int64_t row_stride,
  * large vocabulary are then cut into parts of a row, so that a small batch fills the chip (two launches).
  *   workspace       device scratch of aicomp_sample_workspace_bytes(...) bytes, 8-byte aligned, needing no
  *                   initialisation; calls that may overlap need separate ones.  NULL or less: one
- *                   launch, as aicomp_sample_tokens.
+ *                   launch, as aicomp_sample_tokens.  Per row and part of at most 16384 logits 2052 bytes
+ *                   (greedy) or 8 * min(1024, 256 + 8 * top_k) + 4; at most 1024 rows of 16 parts are
+ *                   cut.  64 rows of 128256, top_k 50: 2.7 MB.
  */
 int aicomp_sample_tokens_split(int64_t* out, const void* logits, int64_t row_stride,
                                float* probs_out, const float* uniforms,

@@ -106,3 +106,13 @@ def test_torch_operator_library_registers_the_named_ops():
                         "Tensor block_table, Tensor context_lens, float scale")
     assert "Tensor(a!) k_pool" in str(ns.kv_append.default._schema)
     assert str(ns.decode_step.default._schema).endswith("-> Tensor")
+
+
+def test_sampling_scratch_is_sized_by_what_the_call_keeps():
+    """A greedy call has 2 KB per part; the candidates of a top-k call follow k and stay a small part of the
+    logits they are taken from."""
+    lib = _lib.load()
+    need = lambda B, V, k, greedy=0: lib.aicomp_sample_workspace_bytes(B, V, V, 0.8, k, greedy, _lib.F32)
+    assert need(16, 128256, 0, 1) == 16 * 8 * 2052 and need(1024, 50257, 0, 1) == 1024 * 4 * 2052
+    assert need(1024, 128256, 50) == 1024 * 8 * (8 * 656 + 4) < 1024 * 128256 * 4 // 12
+    assert need(4, 128256, 20) < need(4, 128256, 50) < need(4, 128256, 200) == need(4, 128256, 256)

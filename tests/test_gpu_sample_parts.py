@@ -68,3 +68,18 @@ def test_parts_in_a_graph(device):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(tokens, _one_launch(x, 0.8, 50, 0.9, True, u)[0])
+
+
+@pytest.mark.parametrize("k,room", [(1, 264), (50, 656), (96, 1024), (256, 1024)])
+def test_a_part_with_as_many_candidates_as_it_has_room_for(device, k, room):
+    """Equal logits on top, as many as one part's list holds and one more (its row then goes the whole way)."""
+    V, lib = 131072, _lib.load()
+    assert lib.aicomp_sample_workspace_bytes(4, V, V, 1.0, k, 0, _lib.F32) == 4 * 8 * (8 * room + 4)
+    x = torch.randn(4, V, generator=torch.Generator().manual_seed(k)).to(device)
+    for row, n in enumerate((room - 1, room, room + 1)):
+        x[row, 3 * 16384 + 5:3 * 16384 + 5 + n] = 9.0
+    u = torch.tensor([0.999, 0.5, 0.25, 0.75], device=device)
+    want, dist = _one_launch(x, 1.0, k, 0.9, True, u)
+    got, probs = ops.sample_tokens(x, 1.0, k, 0.9, True, u, return_probs=True)
+    assert torch.equal(got, want) and torch.equal(probs > 0, dist > 0)
+    assert torch.allclose(probs, dist, rtol=2.0 ** -22, atol=0.0)

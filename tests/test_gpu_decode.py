@@ -516,10 +516,11 @@ def test_balanced_schedule_records_the_parts_the_host_model_predicts(hkv, group,
 @pytest.mark.routing("balanced")
 @pytest.mark.parametrize("name,batch,ctx_hi,kv", [("llama3_8b_decode", 1, 500, None), ("llama3_8b_decode", 3, 2000, None),
                                                  ("llama32_1b_decode", 2, 300, None), ("llama32_1b_decode", 4, 1500, None),
-                                                 ("llama3_70b_decode_fp8", 2, 1100, "fp8")])
+                                                 ("llama3_70b_decode_fp8", 2, 1100, "fp8"), ("llama3_8b_decode", 2, 750, None),
+                                                 ("llama32_1b_decode", 2, 1270, None)])
 def test_small_calls_take_the_grid_schedule(device, name, batch, ctx_hi, kv):
     """With partition_size = 0 a call over few short rows is routed to the grid schedule (whole rows
-    when no row can exceed 640 tokens, 256-token partitions otherwise).  Same numbers as the balanced
+    when no row can exceed 768 tokens at head_dim 128, 1280 at 64 or 640 of fp8, 256-token partitions otherwise).  Same numbers as the balanced
     schedule to the tolerance between split sizes, same pools after the fused append, oracle parity,
     and the sizing helpers agree with what the call does."""
     from aicomp_amd import _lib
@@ -535,7 +536,7 @@ def test_small_calls_take_the_grid_schedule(device, name, batch, ctx_hi, kv):
     assert batch * mb * 16 <= 32768, "the case is meant to be below the default limit"
     qd, kd = ops._DT[w.query.dtype], ops._DT[w.k_pool.dtype]
     ps = lib.aicomp_paged_decode_partition_size(batch, s.num_q_heads, s.num_kv_heads, s.head_dim, 16, mb, qd, kd)
-    assert ps == (-(-mb * 16 // 64) * 64 if mb * 16 <= 640 else 256)
+    assert ps == (-(-mb * 16 // 64) * 64 if mb * 16 <= (640 if kv else 1280 if s.head_dim == 64 else 768) else 256)
     parts = -(-mb * 16 // ps)
     need = lib.aicomp_paged_decode_workspace_bytes(batch, s.num_q_heads, s.num_kv_heads, s.head_dim, 16, mb, qd, kd, 0)
     assert need == (0 if parts == 1 else batch * s.num_q_heads * parts * (s.head_dim + 2) * 4)

@@ -1,7 +1,8 @@
 // Generic paged attention kernel (vector ALU): any supported storage type,
 // head_dim 64/128/256, any GQA group, any block size.  It is the path for
 // shapes the MFMA kernels do not cover (head_dim 256, block sizes other than 16, wide
-// groups, more than 1024 rows with a partition size that is not a whole number of tiles) and the split-K reduce shared by every decode kernel.
+// groups, float32 queries over fp8 pools, partitions that are not whole tiles) and the
+// split-K reduce shared by every decode kernel.
 //
 // Replaces  F.scaled_dot_product_attention(query, full_key, full_value,
 //           attn_mask=None, is_causal=False)       opt_prime/opt_prime/kv_cache.py:397-403

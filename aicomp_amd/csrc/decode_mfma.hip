@@ -6,9 +6,9 @@
 // K and V are read once, in place, through the block table.
 //
 // Shape covered: head_dim 128, block_size 16, bf16 or fp16 queries, pools of the query type or
-// fp8-e4m3 (the kernels are written over a 16-bit element format, see common.h), up to 16 query heads per KV head; and head_dim 64 (up to 8 heads per KV
-// head) by treating two consecutive tokens, which are contiguous in the pool, as
-// one 128-element row: every head takes two B-operand columns, one per token
+// fp8-e4m3 (the kernels are written over a 16-bit element format, see common.h), up to 16 query
+// heads per KV head; and head_dim 64 (up to 8 heads per KV head) by treating two consecutive
+// tokens, which are contiguous in the pool, as one 128-element row: every head takes two B-operand columns, one per token
 // parity, with the query in the matching half of the row and zeros in the other,
 // and the two columns' partial softmaxes are merged at the end.  Same instruction
 // stream per byte as head_dim 128.  Float32 queries over float32 pools, head_dim 128 and
@@ -19,8 +19,8 @@
 // used exactly once; 4 * G flop per byte (bf16), far below the MFMA roof, so
 // the design goal is bytes in flight, not flops.
 //
-// Work split   one workgroup (4 waves) per (partition, KV head, sequence).
-//              A wave owns whole 32-token tiles (two 16-token blocks) and its
+// Work split   one workgroup per (partition, KV head, sequence), of 4 waves, or of 8 where a CU has
+//              one workgroup at most and a partition more than 16 tiles.  A wave owns whole 32-token tiles (two 16-token blocks) and its
 //              own online-softmax state; no workgroup barrier in the loop.
 // Loads        a (block, KV head) tile is 16 rows * 256 B contiguous (bf16):
 //              each global_load_dwordx4 of a wave reads 1 KB = 4 whole rows,

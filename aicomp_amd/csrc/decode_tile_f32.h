@@ -1,8 +1,10 @@
 // TileF32: float32 queries and pools, head_dim 128 (tiles of 16 tokens) or 64 (32 tokens), on the
 // float32 matrix instruction v_mfma_f32_16x16x4_f32.  Included by decode_mfma.hip, inside its namespace.
 //
-// HBM-bound like the 16-bit tiles: 32 MFMAs of 32 cycles per 8 KB of K and V each and wave, a third of
-// what a wave waits for its bytes.  What it replaced is the vector-ALU kernel, bound by the lane
+// A tile (8 KB of K, 8 KB of V) costs a wave 64 MFMAs of 32 cycles, 2048 cycles: 19 TB/s with all 1024 SIMDs
+// at work, so a batch that fills the chip is bound by HBM like the 16-bit tiles.  The rows of a small call
+// are on few CUs, and a row is then a chain of such tiles on its CU's four SIMDs (640 tokens of D 128, one
+// workgroup: ten tiles each, 17.6 us).  What it replaced is the vector-ALU kernel, bound by the lane
 // reductions of its dot products, with the append as a launch of its own and always a merge launch:
 //   64 rows of 256..2048 tokens, 32 / 8 heads     D 128  170.5 -> 100.6 us per call (6.0 TB/s)
 //                                                 D 64    90.0 ->  56.8 us

@@ -1,4 +1,5 @@
-// Token sampling: temperature -> top-k -> top-p (nucleus) -> multinomial, one launch.
+// Token sampling: temperature -> top-k -> top-p (nucleus) -> multinomial, one launch, or two when the rows
+// are cut into parts.
 //
 // Replaces the step after the attention path,
 //   opt_prime/opt_prime/inference.py:786-843 (_sample_token):
@@ -8,7 +9,7 @@
 // which in PyTorch is a full-vocabulary sort plus about ten elementwise / scan launches
 // per token.  Greedy decoding (do_sample == False, :806-808) is the argmax.
 //
-// One workgroup of 1024 lanes per row; nothing is sorted.
+// One workgroup of 1024 lanes per row (or part of a row); nothing is sorted.
 //   1  row maximum and argmax on the raw logits (a positive temperature keeps the order)
 //   2  top-k (k <= 1024, the usual case): the k-th largest of the 1024 per-lane maxima bounds the
 //      row's k-th largest value from below, so a second pass over the row collects the

@@ -161,6 +161,9 @@ def pool_blocks_for_budget(budget_bytes: int, num_layers: int, num_kv_heads: int
     return int(budget_bytes // per_block)
 
 
+_UNSEEN = object()             # no entry yet in a plan's item lists (None is one: no list)
+
+
 @dataclass
 class StepPlan:
     """Index tensors of one step, in the row order of the kernels.
@@ -193,7 +196,7 @@ class StepPlan:
         """What an item list, and the choice whether there is one, depend on: the lengths and counts as they are
         now, the chunk bound and the geometry that give the kernel's tile, and the device."""
         return (kind, self.num_prefill_seqs, self.max_q_len, self.new_lens.tobytes(), self.host_context_lens.tobytes(),
-                query.shape[1], k_pool.shape[1:], query.dtype, k_pool.dtype, query.device)
+                query.shape[1], k_pool.shape, query.dtype, k_pool.dtype, query.device)
 
     def prefill_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:
         """The (sequence, query tile) pairs of this step's prompt chunks, most expensive first, as the
@@ -207,7 +210,8 @@ class StepPlan:
         key = self._list_key("chunks", query, k_pool)
         if self._prefill_items is None:
             self._prefill_items = {}
-        if key not in self._prefill_items:         # (3 us to look up, building a list is tens)
+        items = self._prefill_items.get(key, _UNSEEN)          # (2 us a layer; building a list is tens)
+        if items is _UNSEEN:
             hq, (_, hkv, bs, d) = query.shape[1], k_pool.shape
             tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
             items = None
@@ -218,7 +222,7 @@ class StepPlan:
                 items = ops.prefill_items(self.host_context_lens[:npre], self.new_lens[:npre], tile, hgroups, cus)
                 items = torch.from_numpy(items).to(query.device, non_blocking=True)
             self._prefill_items[key] = items
-        return self._prefill_items[key]
+        return items
 
     # Longest decode row and largest decode batch for which a mixed step goes through one launch
     # (measured on MI355X, 32 / 8 and 64 / 8 heads, head_dim 64 and 128, 1 to 16 chunks of 128 to
@@ -244,7 +248,8 @@ class StepPlan:
         key = self._list_key(("step", self.ONE_LAUNCH_MAX_CONTEXT), query, k_pool)
         if self._prefill_items is None:
             self._prefill_items = {}
-        if key not in self._prefill_items:
+        items = self._prefill_items.get(key, _UNSEEN)
+        if items is _UNSEEN:
             items = None
             if int(self.host_context_lens[npre:].max()) <= self.ONE_LAUNCH_MAX_CONTEXT:
                 hq, (_, hkv, bs, d) = query.shape[1], k_pool.shape
@@ -257,7 +262,7 @@ class StepPlan:
                     items = ops.step_items(self.host_context_lens, self.new_lens, npre, tile, hgroups, cus)
                     items = torch.from_numpy(items).to(query.device, non_blocking=True)
             self._prefill_items[key] = items
-        return self._prefill_items[key]
+        return items
 
     @property
     def num_seqs(self) -> int:

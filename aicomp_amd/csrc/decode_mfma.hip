@@ -556,7 +556,7 @@ paged_decode_mfma_kernel(MfmaParams p) {
         const int head = kvh * G + h;
         if (direct) {
             ((typename T::Fmt::raw*)p.out)[((int64_t)seq * p.hq + head) * DQ + dd] =
-                T::Fmt::from_f32(den > 0.f ? vs * num / den : 0.f);
+                T::Fmt::from_f32(den == 0.f ? 0.f : vs * num / den);     // (a NaN stays one, as in the merge kernels)
         } else {
             const int64_t slot = ((int64_t)seq * p.hq + head) * p.num_parts + part;
             p.ws_acc[slot * DQ + dd] = num;

@@ -38,3 +38,17 @@ def test_one_workgroup_per_cu_and_one_more_row(device, d, kv, dtype, longest, ro
     got = to_f64(ops.paged_decode_attn(torch.full_like(c["q"], float("nan")), c["q"], c["k_pool"], c["v_pool"], c["table"],
                                        c["ctx"], c["scale"], c["ks"], c["vs"], partition_size=ps))
     assert_close_attn(got, tp.oracle(c), *((1e-5, 1e-5) if dtype == torch.float32 else (1e-2, 2e-2)), f"{d} {dtype} {rows}")
+
+
+@pytest.mark.parametrize("partition", [0, 256, 448])
+@pytest.mark.parametrize("d,dtype", [(128, torch.float32), (64, torch.float32), (128, torch.bfloat16), (64, torch.float16)])
+def test_a_nan_score_is_a_nan_row_whatever_the_split(device, d, dtype, partition):
+    """Attention over a key that is not a number has no value, as in torch; a call of one workgroup per row
+    says so like one that is merged.  The other KV head's rows and the other sequence are untouched."""
+    ops.set_small_decode_tokens(1 << 40)
+    c = tp.build_case(device, [400, 399], [1, 1], 8, 2, d, dtype=dtype, seed=d)
+    c["k_pool"][c["table"][0, 12].item(), 1, 3, 5] = float("nan")                    # token 195 of sequence 0, KV head 1
+    out = ops.paged_decode_attn(torch.zeros_like(c["q"]), c["q"], c["k_pool"], c["v_pool"], c["table"], c["ctx"], c["scale"],
+                                partition_size=partition)
+    assert torch.isnan(out[0, 4:]).all()
+    assert torch.isfinite(out[0, :4]).all() and torch.isfinite(out[1]).all() and bool(out[1].any())

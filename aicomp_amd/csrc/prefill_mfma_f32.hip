@@ -4,29 +4,32 @@
 //           is_causal=True)                       opt_prime/opt_prime/kv_cache.py:404-415
 // when the engine runs in float32 (examples/single_gpu_inference_llama.py:98-110, --dtype
 // float32): queries, pools and output are float32, and every product and sum stays float32
-// (v_mfma_f32_16x16x4_f32: D[16x16] += A[16x4] B[4x16], 2048 flop in 32 cycles per SIMD, the
-// same 157 TFLOP/s roof as the vector ALUs but with a sixteenth of the instructions, beside which
-// another wave's softmax runs; 70 % of the roof on a 2048-token prompt).  Same mask rule as the 16-bit kernel: query i
-// of a chunk with prior context P sees keys j <= P + i.
+// (v_mfma_f32_16x16x4_f32: D[16x16] += A[16x4] B[4x16], 2048 flop in 32 cycles per SIMD).  Same mask rule as the
+// 16-bit kernel: query i of a chunk with prior context P sees keys j <= P + i.
+//
+// What bounds it: the float32 matrix instruction runs on the vector ALU's own multipliers, so every vector
+// instruction of any wave of the SIMD takes its time from it (SQ_VALU_MFMA_COEXEC_CYCLES is 0).  A tile step of a wave
+// is 128 products and had 185 other vector instructions: exp2f's range handling, a row max per tile, per-lane block ids
+// and addresses, selects for masks that mask nothing.  It has 36: the hardware exponential, a max that moves only when
+// a row's probabilities outgrow 2^8, block ids and tile addresses in scalar registers, masks behind branches.
+//   us, 32/8 heads, before -> now     D 128                     D 64
+//   2048 tokens                       309 -> 270 (127 TFLOP/s)  180 -> 153
+//   4096                              1184 -> 1118              680 -> 582
+//   512 after 1300                    118 -> 104                68 -> 58
+// Products are busy 84 % of the first one's cycles; of 64 chunks of 32 tokens over 4000, 1112 -> 1005 us, 89 %.
 //
 // Work split   one workgroup (8 waves) per (128 query rows, sequence); a row is a (position,
 //              head) pair, the G heads of one KV head packed per position when G divides 16, so a
-//              K/V tile staged in LDS serves the whole group.  A wave owns 16 rows: a workgroup that
-//              is alone on its CU, as the last ones of a causal prompt are, still has two waves per
-//              SIMD to run one's softmax beside the other's products.  Four waves of 32 rows read the
-//              LDS tiles half as often and were slower at every size (us, 4 -> 8 waves, 32/8 heads):
-//              one chunk of 24 rows D 128 39.6 -> 14.0, 512 after 2048 275.5 -> 256.5, 2048 389 -> 371,
-//              4096 1311 -> 1304; D 64: 512 after 2048 168.0 -> 135.2, 2048 240.4 -> 192.3, 4096 682 -> 672.
-// K/V tiles    32 tokens, global -> registers (one tile ahead) -> LDS rows of head_dim floats + 16
-//              bytes (the operand reads below are then free of bank conflicts), double-buffered,
-//              one barrier per tile.
+//              K/V tile staged in LDS serves the whole group.  A wave owns 16 rows.
+// K/V tiles    32 tokens, global -> registers (one tile ahead) -> LDS, double-buffered, one barrier per
+//              tile.  K rows of head_dim floats + 16 bytes, V rows unpadded: either operand read has every four lanes in
+//              one 64-byte segment of a bank line and a half-wave in all four.
 // S^T = K Q^T  A = K rows from LDS, B = the wave's query rows (registers, pre-multiplied by
 //              scale * log2 e).  The k index of MFMA m in lane group g is 16 (m / 4) + 4 g + m % 4:
-//              one 16-byte LDS read supplies the A operands of four MFMAs.
-// softmax      online, base 2, per lane one query; the row max crosses the four lanes of a row
-//              with two shuffles; the accumulators are rescaled only when a max moved.
-// O^T += V^T P^T  A = V^T: lane (dim r, g) reads V[token 4 g + m][16 j + r], one 4-byte LDS read per
-//              MFMA; B = P^T is exactly what the lane already holds.
+//              one 16-byte LDS read supplies the A operands of four MFMAs, read one group of products ahead.
+// softmax      online, base 2, per lane one query.
+// O^T += V^T P^T  A = V^T: lane (r, g) reads dims 64 half + 4 r .. + 3 of token 4 g + e, one 16-byte LDS read per four
+//              MFMAs (a 4-byte read per MFMA before: 3 % more); B = P^T is exactly what the lane already holds.
 #include "common.h"
 
 #include <atomic>
@@ -41,6 +44,7 @@ constexpr int WAVES = 8;
 constexpr int NT = 64 * WAVES;
 constexpr int WG_ROWS = 16 * WAVES;     // query rows per workgroup
 constexpr float NEG_BIG = -1.0e30f;
+constexpr float LAZY = 256.f;           // sum of a lane's probabilities up to which a row's reference max stays
 
 struct PrefillF32Params {
     float* out;
@@ -64,14 +68,16 @@ __global__ void __launch_bounds__(NT, 4)
 paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     constexpr int KROW = DH * 4 + 16;           // LDS row stride in bytes
     constexpr int KROWF = KROW / 4;             // ... in floats
-    constexpr int TILE_F = KT * KROWF;          // floats per K (or V) tile
+    constexpr int KTILE_F = KT * KROWF;         // floats per K tile
+    constexpr int TILES_F = KTILE_F + KT * DH;  // ... and of a K and a V tile
+    constexpr int HALVES = DH / 64;
     constexpr int NQ = DH / 16;                 // 16-element chunks of a row (QK: 4 MFMAs each; PV: output tiles)
     constexpr int CPR = DH / 4;                 // float4 chunks per row
     constexpr int RPL = NT / CPR;               // rows one load of the workgroup covers (16 or 32)
     constexpr int NL = KT / RPL;                // loads per tile and pool (2 or 1)
     const int hgroup = blockIdx.x;
     int seq = blockIdx.y;
-    int qtile = prefill_tile_of_slice(blockIdx.z, gridDim.z, p.num_cus, gridDim.x * gridDim.y);
+    int64_t qtile = prefill_tile_of_slice(blockIdx.z, gridDim.z, p.num_cus, gridDim.x * gridDim.y);
     if (p.items != nullptr) {           // the caller's own order: workgroup row y takes pair y
         seq = p.items[2 * blockIdx.y];
         qtile = p.items[2 * blockIdx.y + 1];
@@ -89,8 +95,8 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     const int n = p.cu_q_lens[seq + 1] - q_begin;
     const int ctx = min(p.context_lens[seq], p.max_blocks * BS);
     const int prior = ctx - n;
-    const int q0 = qtile * pos_per_wg;
-    if (q0 >= n || n <= 0) return;
+    if (qtile * pos_per_wg >= n || n <= 0) return;
+    const int q0 = (int)qtile * pos_per_wg;
     if (prior < 0) {
         // a context shorter than the chunk itself: the rows are defined as zero, as in the other kernels
         for (int i = tid; i < WG_ROWS * CPR; i += NT) {
@@ -116,13 +122,13 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     const int ntiles = (kv_end + KT - 1) / KT;
 
     // Q as the B operand: MFMA 4 q + e of chunk q takes element 16 q + 4 g4 + e of this lane's row
-    float4 qf[NQ];
+    f32x4_t qf[NQ];
     const float* qrow = p.query + ((int64_t)(q_begin + min(qpos, n - 1)) * p.hq + head) * DH + 4 * g4;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        float4 v = *(const float4*)(qrow + 16 * q);
-        v.x *= p.qk_mul; v.y *= p.qk_mul; v.z *= p.qk_mul; v.w *= p.qk_mul;
-        qf[q] = v;
+        qf[q] = *(const f32x4_t*)(qrow + 16 * q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qf[q][e] *= p.qk_mul;
     }
 
     float m = NEG_BIG, lsum = 0.f;
@@ -142,30 +148,32 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     f32x4_t sk[NL], sv[NL];
     int blk[NL];
     const int trow = tid / CPR, tchunk = 4 * (tid % CPR);
+    const int wrow = __builtin_amdgcn_readfirstlane(trow) & ~15;      // first row of the wave's block within a load
+    const uint32_t in_block = (uint32_t)((trow & 15) * DH + tchunk);  // elements
     auto fetch_ids = [&](int t) {
 #pragma unroll
-        for (int i = 0; i < NL; ++i) blk[i] = table[min((t * KT + RPL * i + trow) >> 4, last_blk)];
+        for (int i = 0; i < NL; ++i) blk[i] = table[min((t * KT + RPL * i + wrow) >> 4, last_blk)];
     };
     auto fetch = [&]() {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
-            const int64_t id = max(0, min(blk[i], p.num_blocks - 1));
-            const int64_t off = ((id * p.hkv + kvh) * BS + ((RPL * i + trow) & 15)) * DH + tchunk;
-            sk[i] = *(const f32x4_t*)(p.k_pool + off);
-            sv[i] = *(const f32x4_t*)(p.v_pool + off);
+            const int64_t base = ((int64_t)max(0, min(blk[i], p.num_blocks - 1)) * p.hkv + kvh) * (BS * DH);
+            sk[i] = *(const f32x4_t*)(p.k_pool + base + in_block);
+            sv[i] = *(const f32x4_t*)(p.v_pool + base + in_block);
         }
     };
     auto stash = [&](int t, int buf) {
-        float* kb = lds + buf * 2 * TILE_F + trow * KROWF + tchunk;
-        float* vb = kb + TILE_F;
+        float* kb = lds + buf * TILES_F + trow * KROWF + tchunk;
+        float* vb = lds + buf * TILES_F + KTILE_F + trow * DH + tchunk;
+        if ((t + 1) * KT > ctx) {                                       // the context's last tile
+#pragma unroll
+            for (int i = 0; i < NL; ++i)
+                if (t * KT + RPL * i + trow >= ctx) sv[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
-            const bool in = t * KT + RPL * i + trow < ctx;
-            f32x4_t vv = sv[i];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) vv[e] = in ? vv[e] : 0.f;
             *(f32x4_t*)(kb + RPL * i * KROWF) = sk[i];
-            *(f32x4_t*)(vb + RPL * i * KROWF) = vv;
+            *(f32x4_t*)(vb + RPL * i * DH) = sv[i];
         }
     };
 
@@ -181,104 +189,107 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
         }
         __syncthreads();          // tile t visible; everyone is done with the buffer tile t + 1 will use
         const int tile_start = t * KT;
-        if (tile_start >= wave_kv_end) continue;                       // wave-uniform: above the diagonal
-        const float* kb = lds + buf * 2 * TILE_F;
-        const float* vb = kb + TILE_F;
+        if (tile_start >= wave_kv_end) continue;                            // wave-uniform: above the diagonal
+        const float* kb = lds + buf * TILES_F;
+        const float* vb = kb + KTILE_F;
 
-        // ---- S^T = K Q^T for the two 16-token blocks of the tile (two accumulators in turn)
-        f32x4_t sa[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+        // ---- S^T = K Q^T for the two 16-token blocks of the tile
+        f32x4_t sa[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) sa[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        f32x4_t ka[2][2];
+        auto read_k = [&](int q, f32x4_t (&x)[2]) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) x[h] = *(const f32x4_t*)(kb + (16 * h + r16) * KROWF + 16 * q + 4 * g4);
+        };
+        read_k(0, ka[0]);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-            float4 a[2];
+            if (q + 1 < NQ) read_k(q + 1, ka[(q + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) a[h] = *(const float4*)(kb + (16 * h + r16) * KROWF + 16 * q + 4 * g4);
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].x, qf[q].x, sa[h], 0, 0, 0);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].y, qf[q].y, sa[h], 0, 0, 0);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].z, qf[q].z, sa[h], 0, 0, 0);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h].w, qf[q].w, sa[h], 0, 0, 0);
+                for (int h = 0; h < 2; ++h)
+                    sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[q & 1][h][e], qf[q][e], sa[h], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
 
-        // ---- online softmax: lane (query r16, g4) holds tokens tile_start + 16 h + 4 g4 + i
-        const bool need_mask = tile_start + KT - 1 > wave_kv_min;      // wave-uniform
-        float pr[8], sc[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) sc[k] = sa[k >> 2][k & 3];
-        if (need_mask) {
+        // ---- online softmax: lane (query r16, g4) holds tokens tile_start + 16 h + 4 g4 + i.  The reference max m moves only
+        // when a lane's probabilities of this tile add up to more than LAZY (always on a row's first tile), for all
+        // rows of the wave together: sums and products are the same floats scaled by a power of two at most 2^8.
+        if (tile_start + KT - 1 > wave_kv_min) {                       // wave-uniform
 #pragma unroll
             for (int k = 0; k < 8; ++k)
-                if (tile_start + 16 * (k >> 2) + 4 * g4 + (k & 3) > qabs) sc[k] = NEG_BIG;
+                if (tile_start + 16 * (k >> 2) + 4 * g4 + (k & 3) > qabs) sa[k >> 2][k & 3] = -INFINITY;
         }
-        float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m, mx);
-        const float alpha = exp2f(m - m_new);
-        float psum = 0.f;
+        float pr[8], psum = 0.f;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            float e = exp2f(sc[k] - m_new);
-            if (need_mask && sc[k] == NEG_BIG) e = 0.f;
-            pr[k] = e;
-            psum += e;
+            pr[k] = __builtin_amdgcn_exp2f(sa[k >> 2][k & 3] - m);
+            psum += pr[k];
         }
-        lsum = lsum * alpha + psum;
-        m = m_new;
-        if (__any(alpha != 1.f)) {
+        if (__any(!(psum <= LAZY))) {
+            float mx = sa[0][0];
+#pragma unroll
+            for (int k = 1; k < 8; ++k) mx = fmaxf(mx, sa[k >> 2][k & 3]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float m_new = fmaxf(m, mx);
+            const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+            psum = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                pr[k] = __builtin_amdgcn_exp2f(sa[k >> 2][k & 3] - m_new);
+                psum += pr[k];
+            }
+            lsum *= alpha;
+            m = m_new;
 #pragma unroll
             for (int j = 0; j < NQ; ++j) O[j] *= alpha;
         }
+        lsum += psum;
 
-        // ---- O^T += V^T P^T: A = V[token 16 h + 4 g4 + e][16 j + r16], B = this lane's own P values.
-        // In groups of EG tokens of two output blocks; a group's operands are read while the products of the
-        // one before it run (read when needed, every pair of products waited for its LDS read).  EG is what the
-        // registers hold: four tokens at D 128 spill three of 128 registers.  2048 tokens, 32/8 heads, D 128:
-        // 326 -> 313 us (310 with the spill, but 64/8 heads 608 against 596); D 64: 187 -> 176 (EG 2 180).
-        // The same for K, eight products ahead, spills ten: 340 us.
-        constexpr int EG = DH == 64 ? 4 : 2;
-        constexpr int PER_H = 4 / EG, NG = NQ * PER_H;
-        float a[2][EG][2];
-        auto read_v = [&](int g, float (&x)[EG][2]) {
-            const int j = g / (2 * PER_H) * 2, h = g / PER_H & 1, e0 = g % PER_H * EG;
+        // ---- O^T += V^T P^T: A = V[token 16 h + 4 g4 + e][dims 64 half + 4 r16 + x], B = this lane's own P values
+        f32x4_t va[2][HALVES];
+        auto read_v = [&](int t8, f32x4_t (&x)[HALVES]) {
 #pragma unroll
-            for (int e = 0; e < EG; ++e)
-#pragma unroll
-                for (int i = 0; i < 2; ++i) x[e][i] = vb[(16 * h + 4 * g4 + e0 + e) * KROWF + 16 * (j + i) + r16];
+            for (int f = 0; f < HALVES; ++f)
+                x[f] = *(const f32x4_t*)(vb + (16 * (t8 >> 2) + 4 * g4 + (t8 & 3)) * DH + 64 * f + 4 * r16);
         };
-        read_v(0, a[0]);
+        read_v(0, va[0]);
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const int j = g / (2 * PER_H) * 2, h = g / PER_H & 1, e0 = g % PER_H * EG;
-            if (g + 1 < NG) read_v(g + 1, a[(g + 1) & 1]);
+        for (int t8 = 0; t8 < 8; ++t8) {
+            if (t8 + 1 < 8) read_v(t8 + 1, va[(t8 + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int e = 0; e < EG; ++e)
+            for (int f = 0; f < HALVES; ++f)
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    O[j + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[g & 1][e][i], pr[4 * h + e0 + e], O[j + i], 0, 0, 0);
+                for (int x = 0; x < 4; ++x)
+                    O[4 * f + x] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[t8 & 1][f][x], pr[t8], O[4 * f + x], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 
-    // lane (query r16, g4) holds O^T[element 16 j + 4 g4 + i][query] in O[j][i]
+    // lane (query r16, g4) holds O^T[dim 64 half + 16 g4 + 4 i + x][query] in O[4 half + x][i]
     float l = lsum;
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
     if (row_valid) {
         const float inv = l > 0.f ? 1.f / l : 0.f;
-        float* o = p.out + ((int64_t)(q_begin + qpos) * p.hq + head) * DH + 4 * g4;
+        float* o = p.out + ((int64_t)(q_begin + qpos) * p.hq + head) * DH + 16 * g4;
 #pragma unroll
-        for (int j = 0; j < NQ; ++j)
-            *(float4*)(o + 16 * j) = make_float4(O[j][0] * inv, O[j][1] * inv, O[j][2] * inv, O[j][3] * inv);
+        for (int f = 0; f < HALVES; ++f)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *(float4*)(o + 64 * f + 4 * i) =
+                    make_float4(O[4 * f][i] * inv, O[4 * f + 1][i] * inv, O[4 * f + 2][i] * inv, O[4 * f + 3][i] * inv);
     }
 }
 
 template <int DH>
 hipError_t launch_f32_variant(const PrefillF32Params& p, dim3 grid, hipStream_t stream) {
-    constexpr size_t lds_bytes = (size_t)4 * KT * (DH * 4 + 16);       // two buffers of a K and a V tile
+    constexpr size_t lds_bytes = (size_t)2 * KT * (2 * DH * 4 + 16);   // two buffers of a K and a V tile
     if (lds_bytes > 64 * 1024) {
         // above the 64 KB a kernel may use without asking: a per-device function attribute, set once
         static std::atomic<unsigned long long> done{0};

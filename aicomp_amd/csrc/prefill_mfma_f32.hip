@@ -21,7 +21,11 @@
 // Work split   one workgroup (8 waves) per (128 query rows, sequence); a row is a (position,
 //              head) pair, the G heads of one KV head packed per position when G divides 16, so a
 //              K/V tile staged in LDS serves the whole group.  A wave owns 16 rows.
-// K/V tiles    32 tokens, global -> registers (one tile ahead) -> LDS, double-buffered, one barrier per
+// Small grids  a row of tiles is a chain of steps on one CU, 3.5 us each, and a small grid leaves the other CUs idle.
+//              There KW = 4 or 2 waves share the 16 rows and split the keys of a tile, a workgroup has 128 / KW rows, and
+//              the waves' partial rows are added up through LDS at the end: KW times the workgroups, steps KW
+//              times shorter (launch_prefill_mfma_f32 has the lines and both sides).
+// K/V tiles    32 tokens (KW = 4: 64), global -> registers (one tile ahead) -> LDS, double-buffered, one barrier per
 //              tile.  K rows of head_dim floats + 16 bytes, V rows unpadded: either operand read has every four lanes in
 //              one 64-byte segment of a bank line and a half-wave in all four.
 // S^T = K Q^T  A = K rows from LDS, B = the wave's query rows (registers, pre-multiplied by
@@ -32,6 +36,7 @@
 //              MFMAs (a 4-byte read per MFMA before: 3 % more); B = P^T is exactly what the lane already holds.
 #include "common.h"
 
+#include <algorithm>
 #include <atomic>
 
 namespace aicomp {
@@ -39,10 +44,9 @@ namespace aicomp {
 namespace {
 
 constexpr int BS = 16;
-constexpr int KT = 32;                  // tokens per LDS tile
 constexpr int WAVES = 8;
 constexpr int NT = 64 * WAVES;
-constexpr int WG_ROWS = 16 * WAVES;     // query rows per workgroup
+constexpr int WG_ROWS = 16 * WAVES;     // query rows per workgroup, where every wave has rows of its own
 constexpr float NEG_BIG = -1.0e30f;
 constexpr float LAZY = 256.f;           // sum of a lane's probabilities up to which a row's reference max stays
 
@@ -63,9 +67,14 @@ struct PrefillF32Params {
     int num_seqs;
 };
 
-template <int DH>
-__global__ void __launch_bounds__(NT, 4)
+// KW: waves that share 16 query rows and split the keys of a tile (1: none do).
+template <int DH, int KW>
+__global__ void __launch_bounds__(NT, KW <= 2 ? 4 : 2)
 paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
+    constexpr int HB = KW == 1 ? 2 : 1;         // 16-token blocks of a tile that a wave multiplies
+    constexpr int KT = 16 * HB * KW;            // tokens per LDS tile
+    constexpr int RW = WAVES / KW;              // waves with rows of their own
+    constexpr int ROWS = 16 * RW;               // query rows per workgroup
     constexpr int KROW = DH * 4 + 16;           // LDS row stride in bytes
     constexpr int KROWF = KROW / 4;             // ... in floats
     constexpr int KTILE_F = KT * KROWF;         // floats per K tile
@@ -82,12 +91,15 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
         seq = p.items[2 * blockIdx.y];
         qtile = p.items[2 * blockIdx.y + 1];
         if (seq < 0 || seq >= p.num_seqs || qtile < 0) return;
+        qtile = qtile * KW + (int)blockIdx.z;       // (a pair's tile is WG_ROWS rows)
     }
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g4 = lane >> 4;
-    const int pos_per_wg = WG_ROWS / p.gpack;
+    const int pos_per_wg = ROWS / p.gpack;
+    const int rw = KW == 1 ? w : w % RW;             // which rows
+    const int key0 = KW == 1 ? 0 : 16 * HB * (w / RW);  // which keys of a tile
 
     extern __shared__ __attribute__((aligned(16))) float lds[];     // [2][K tile | V tile]
 
@@ -99,7 +111,7 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     const int q0 = (int)qtile * pos_per_wg;
     if (prior < 0) {
         // a context shorter than the chunk itself: the rows are defined as zero, as in the other kernels
-        for (int i = tid; i < WG_ROWS * CPR; i += NT) {
+        for (int i = tid; i < ROWS * CPR; i += NT) {
             const int zrow = i / CPR, chunk = i % CPR;
             const int pos = q0 + zrow / p.gpack, hd = hgroup * p.gpack + zrow % p.gpack;
             if (pos < n)
@@ -109,15 +121,15 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     }
 
     const int kvh = (hgroup * p.gpack) / p.group;
-    const int row = 16 * w + r16;
+    const int row = 16 * rw + r16;
     const int qpos = q0 + row / p.gpack;
     const int head = hgroup * p.gpack + row % p.gpack;
     const bool row_valid = qpos < n;
     const int qabs = row_valid ? prior + qpos : ctx - 1;        // padded rows: computed, never stored
     // (a wave whose rows all lie beyond the chunk's end has nothing to compute: it only takes part in
     // the tile loads and barriers)
-    const int wave_kv_end = q0 + (16 * w) / p.gpack >= n ? 0 : min(ctx, prior + q0 + (16 * w + 15) / p.gpack + 1);
-    const int wave_kv_min = prior + q0 + (16 * w) / p.gpack;
+    const int wave_kv_end = q0 + (16 * rw) / p.gpack >= n ? 0 : min(ctx, prior + q0 + (16 * rw + 15) / p.gpack + 1);
+    const int wave_kv_min = prior + q0 + (16 * rw) / p.gpack;
     const int kv_end = min(ctx, prior + q0 + pos_per_wg);
     const int ntiles = (kv_end + KT - 1) / KT;
 
@@ -189,18 +201,19 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
         }
         __syncthreads();          // tile t visible; everyone is done with the buffer tile t + 1 will use
         const int tile_start = t * KT;
-        if (tile_start >= wave_kv_end) continue;                            // wave-uniform: above the diagonal
-        const float* kb = lds + buf * TILES_F;
-        const float* vb = kb + KTILE_F;
+        const int first = tile_start + key0;
+        if (first >= wave_kv_end) continue;                            // wave-uniform: above the diagonal
+        const float* kb = lds + buf * TILES_F + key0 * KROWF;
+        const float* vb = lds + buf * TILES_F + KTILE_F + key0 * DH;
 
-        // ---- S^T = K Q^T for the two 16-token blocks of the tile
-        f32x4_t sa[2];
+        // ---- S^T = K Q^T for the wave's 16-token blocks of the tile
+        f32x4_t sa[HB];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) sa[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        f32x4_t ka[2][2];
-        auto read_k = [&](int q, f32x4_t (&x)[2]) {
+        for (int h = 0; h < HB; ++h) sa[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        f32x4_t ka[2][HB];
+        auto read_k = [&](int q, f32x4_t (&x)[HB]) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) x[h] = *(const f32x4_t*)(kb + (16 * h + r16) * KROWF + 16 * q + 4 * g4);
+            for (int h = 0; h < HB; ++h) x[h] = *(const f32x4_t*)(kb + (16 * h + r16) * KROWF + 16 * q + 4 * g4);
         };
         read_k(0, ka[0]);
 #pragma unroll
@@ -210,36 +223,36 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
+                for (int h = 0; h < HB; ++h)
                     sa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[q & 1][h][e], qf[q][e], sa[h], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
 
-        // ---- online softmax: lane (query r16, g4) holds tokens tile_start + 16 h + 4 g4 + i.  The reference max m moves only
+        // ---- online softmax: lane (query r16, g4) holds tokens first + 16 h + 4 g4 + i.  The reference max m moves only
         // when a lane's probabilities of this tile add up to more than LAZY (always on a row's first tile), for all
         // rows of the wave together: sums and products are the same floats scaled by a power of two at most 2^8.
-        if (tile_start + KT - 1 > wave_kv_min) {                       // wave-uniform
+        if (first + 16 * HB - 1 > wave_kv_min) {                       // wave-uniform
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (tile_start + 16 * (k >> 2) + 4 * g4 + (k & 3) > qabs) sa[k >> 2][k & 3] = -INFINITY;
+            for (int k = 0; k < 4 * HB; ++k)
+                if (first + 16 * (k >> 2) + 4 * g4 + (k & 3) > qabs) sa[k >> 2][k & 3] = -INFINITY;
         }
-        float pr[8], psum = 0.f;
+        float pr[4 * HB], psum = 0.f;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
+        for (int k = 0; k < 4 * HB; ++k) {
             pr[k] = __builtin_amdgcn_exp2f(sa[k >> 2][k & 3] - m);
             psum += pr[k];
         }
         if (__any(!(psum <= LAZY))) {
             float mx = sa[0][0];
 #pragma unroll
-            for (int k = 1; k < 8; ++k) mx = fmaxf(mx, sa[k >> 2][k & 3]);
+            for (int k = 1; k < 4 * HB; ++k) mx = fmaxf(mx, sa[k >> 2][k & 3]);
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const float m_new = fmaxf(m, mx);
             const float alpha = __builtin_amdgcn_exp2f(m - m_new);
             psum = 0.f;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
+            for (int k = 0; k < 4 * HB; ++k) {
                 pr[k] = __builtin_amdgcn_exp2f(sa[k >> 2][k & 3] - m_new);
                 psum += pr[k];
             }
@@ -259,8 +272,8 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
         };
         read_v(0, va[0]);
 #pragma unroll
-        for (int t8 = 0; t8 < 8; ++t8) {
-            if (t8 + 1 < 8) read_v(t8 + 1, va[(t8 + 1) & 1]);
+        for (int t8 = 0; t8 < 4 * HB; ++t8) {
+            if (t8 + 1 < 4 * HB) read_v(t8 + 1, va[(t8 + 1) & 1]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int f = 0; f < HALVES; ++f)
@@ -275,6 +288,40 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     float l = lsum;
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
+    if constexpr (KW > 1) {
+        // the waves of a row add up through LDS: row r of wave w at part + (16 w + r) * OROW, its (max, sum) behind the rows
+        constexpr int OROW = DH + 4;
+        float* part = lds;
+        float* ml = lds + WAVES * 16 * OROW;
+        __syncthreads();                                               // everyone is done with the tiles
+#pragma unroll
+        for (int f = 0; f < HALVES; ++f)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *(float4*)(part + (16 * w + r16) * OROW + 64 * f + 16 * g4 + 4 * i) =
+                    make_float4(O[4 * f][i], O[4 * f + 1][i], O[4 * f + 2][i], O[4 * f + 3][i]);
+        if (g4 == 0) { ml[2 * (16 * w + r16)] = m; ml[2 * (16 * w + r16) + 1] = l; }
+        __syncthreads();
+        for (int i = tid; i < ROWS * CPR; i += NT) {
+            const int orow = i / CPR, chunk = 4 * (i % CPR);
+            const int pos = q0 + orow / p.gpack, hd = hgroup * p.gpack + orow % p.gpack;
+            if (pos >= n) continue;
+            float mx = NEG_BIG, den = 0.f;
+#pragma unroll
+            for (int k = 0; k < KW; ++k) mx = fmaxf(mx, ml[2 * (k * ROWS + orow)]);
+            f32x4_t num = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < KW; ++k) {
+                const int r = k * ROWS + orow;                         // 16 w + row within the wave, w = k RW + its row wave
+                const float f = __builtin_amdgcn_exp2f(ml[2 * r] - mx);
+                den = fmaf(f, ml[2 * r + 1], den);
+                num += f * *(const f32x4_t*)(part + r * OROW + chunk);
+            }
+            const float inv = den > 0.f ? 1.f / den : 0.f;
+            *(f32x4_t*)(p.out + ((int64_t)(q_begin + pos) * p.hq + hd) * DH + chunk) = num * inv;
+        }
+        return;
+    }
     if (row_valid) {
         const float inv = l > 0.f ? 1.f / l : 0.f;
         float* o = p.out + ((int64_t)(q_begin + qpos) * p.hq + head) * DH + 16 * g4;
@@ -287,9 +334,12 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
     }
 }
 
-template <int DH>
+template <int DH, int KW>
 hipError_t launch_f32_variant(const PrefillF32Params& p, dim3 grid, hipStream_t stream) {
-    constexpr size_t lds_bytes = (size_t)2 * KT * (2 * DH * 4 + 16);   // two buffers of a K and a V tile
+    // two buffers of a K and a V tile, where the waves of a row then leave their partial rows and (max, sum)
+    constexpr size_t tiles = (size_t)2 * (KW <= 2 ? 32 : 16 * KW) * (2 * DH * 4 + 16);
+    constexpr size_t rows = KW == 1 ? 0 : (size_t)WAVES * 16 * (DH + 4 + 2) * 4;
+    constexpr size_t lds_bytes = tiles > rows ? tiles : rows;
     if (lds_bytes > 64 * 1024) {
         // above the 64 KB a kernel may use without asking: a per-device function attribute, set once
         static std::atomic<unsigned long long> done{0};
@@ -297,13 +347,13 @@ hipError_t launch_f32_variant(const PrefillF32Params& p, dim3 grid, hipStream_t 
         hipError_t e = hipGetDevice(&dev);
         if (e != hipSuccess) return e;
         if (!(dev < 64 && ((done.load(std::memory_order_acquire) >> dev) & 1ull))) {
-            e = hipFuncSetAttribute((const void*)paged_prefill_mfma_f32_kernel<DH>,
+            e = hipFuncSetAttribute((const void*)paged_prefill_mfma_f32_kernel<DH, KW>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
             if (e != hipSuccess) return e;
             if (dev < 64) done.fetch_or(1ull << dev, std::memory_order_release);
         }
     }
-    hipLaunchKernelGGL((paged_prefill_mfma_f32_kernel<DH>), grid, dim3(NT), lds_bytes, stream, p);
+    hipLaunchKernelGGL((paged_prefill_mfma_f32_kernel<DH, KW>), grid, dim3(NT), lds_bytes, stream, p);
     return hipSuccess;
 }
 
@@ -344,12 +394,27 @@ int launch_prefill_mfma_f32(const DecodeArgs& a, int max_q_len) {
     }
     p.num_cus = num_cus;
     p.items = a.items; p.num_seqs = a.num_seqs;
-    const int pos_per_wg = WG_ROWS / p.gpack;
-    const int qtiles = (max_q_len + pos_per_wg - 1) / pos_per_wg;
+    const int groups = a.hq / p.gpack, pos_per_wg = WG_ROWS / p.gpack;
+    const int64_t tiles = (max_q_len + pos_per_wg - 1) / pos_per_wg;
+    const int64_t wgs = groups * std::min(tiles * a.num_seqs, a.rows / pos_per_wg + a.num_seqs);
+    // Waves that share rows (us, 32/8 heads, D 128, with 1 / 2 / 4 of them; in brackets the workgroups of 128 rows):
+    //   8 chunks of 32 over 2000 (64)    262 /     /  94    16 of 32 over 2000 (128)    270 /     / 188
+    //   one prompt of 512 (128)           73 /     /  31    one of 1024 (256)           143 /  88 / 110
+    //   48 of 32 over 1000 (384)         269 / 232 /        one of 1600 (400)           223 / 201 /
+    //   32 of 32 over 1000 (256)         152 / 154 / 188    one of 2048 (512)           280 / 318 /
+    // Two of them also even out what CUs get in a causal prompt; beyond 400 the larger K/V traffic and a second round
+    // cost more.  The count is from what the host knows (all rows, the longest chunk), the same with and
+    // without a list of items, whose pairs name tiles of 128 rows.
+    const int kw = wgs <= 128 ? 4 : wgs <= 400 ? 2 : 1;
+    const int pos = pos_per_wg / kw;
+    const int qtiles = (max_q_len + pos - 1) / pos;
     AICOMP_REQUIRE(qtiles <= 65535, AICOMP_KV_EINVAL, "paged_prefill_attn: grid too large");
-    dim3 grid((unsigned)(a.hq / p.gpack), (unsigned)a.num_seqs, (unsigned)qtiles);
-    if (a.items != nullptr) grid = dim3((unsigned)(a.hq / p.gpack), (unsigned)a.num_items, 1);
-    const hipError_t e = a.d == 64 ? launch_f32_variant<64>(p, grid, a.stream) : launch_f32_variant<128>(p, grid, a.stream);
+    dim3 grid((unsigned)groups, (unsigned)a.num_seqs, (unsigned)qtiles);
+    if (a.items != nullptr) grid = dim3((unsigned)groups, (unsigned)a.num_items, (unsigned)kw);
+    const bool d64 = a.d == 64;
+    const hipError_t e = kw == 4   ? (d64 ? launch_f32_variant<64, 4>(p, grid, a.stream) : launch_f32_variant<128, 4>(p, grid, a.stream))
+                         : kw == 2 ? (d64 ? launch_f32_variant<64, 2>(p, grid, a.stream) : launch_f32_variant<128, 2>(p, grid, a.stream))
+                                   : (d64 ? launch_f32_variant<64, 1>(p, grid, a.stream) : launch_f32_variant<128, 1>(p, grid, a.stream));
     AICOMP_REQUIRE(e == hipSuccess, AICOMP_KV_EHIP, "paged_prefill_attn: %s", hipGetErrorString(e));
     AICOMP_HIP_LAUNCH_CHECK();
     return AICOMP_KV_OK;

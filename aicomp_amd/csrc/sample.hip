@@ -454,7 +454,7 @@ __device__ __forceinline__ Nucleus nucleus_threshold(Shared& s, Src src, uint32_
 // argmax is its one candidate.
 //
 // Bound by latency: one round of loads, 22 ballots, three barriers, a few dozen appends.  64 rows of 128256
-// float32, k = 50: 8.8 us here and 11.9 us in sample_merge_kernel as traced, where one launch took 25.5 us.
+// float32, k = 50: 8.8 us here and 5.2 us in sample_merge_kernel as traced, where one launch took 25.5 us.
 template <typename T, bool GREEDY>
 __global__ void __launch_bounds__(NT)
 sample_parts_kernel(SampleParams p) {
@@ -1074,6 +1074,155 @@ __device__ __forceinline__ void sample_row(const SampleParams& p, Shared& s, int
     }
 }
 
+// Sum over the lanes up to and including this one, in the vector ALU (every lane active): four shifts within a
+// row of sixteen lanes, then the rows' last lanes broadcast onwards.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_add64(unsigned long long v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xf, false);
+    return v + ((unsigned long long)hi << 32 | lo);
+}
+__device__ __forceinline__ unsigned long long wave_scan_dpp64(unsigned long long v) {
+    v = dpp_add64<0x111, 0xf>(v);            // row_shr 1, 2, 4, 8
+    v = dpp_add64<0x112, 0xf>(v);
+    v = dpp_add64<0x114, 0xf>(v);
+    v = dpp_add64<0x118, 0xf>(v);
+    v = dpp_add64<0x142, 0xa>(v);            // row_bcast 15: into rows 1 and 3
+    return dpp_add64<0x143, 0xc>(v);         // row_bcast 31: into rows 2 and 3
+}
+__device__ __forceinline__ unsigned long long readlane64(unsigned long long v, int lane) {
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+    return (unsigned long long)hi << 32 | lo;
+}
+
+// The usual draw from the candidates of a row's parts, top_k <= 64: false (for the whole workgroup, nothing written)
+// where a list is longer than its lanes' FEW_SLOTS or more than FEW candidates pass the bound.
+//
+// Latency bound, one workgroup per row: what it takes is a chain of memory and LDS latencies and barriers, so it has
+// three of the latter.  The lists are read while their lengths are still on the way; a candidate's rank is counted with
+// one 64-bit compare and a ballot per 64 others, a wave for the candidates of four lanes; and once they are in order
+// at most 64 are left, which the first wave finishes in registers.  64 rows of eight parts, k = 50: 11.5 -> 5.2 us as traced (about ten barriers before, the mass
+// before an entry by two scans over all waves).
+constexpr int FEW = 256, FEW_K = 64;
+constexpr int FEW_SLOTS = 4;               // 512 entries of a list of eight parts; at k = 50 one in 60 rows has a longer one than 256
+template <typename T>
+__device__ __forceinline__ bool merge_few(const SampleParams& p, Shared& s, int row_idx) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // lane -> part lane >> lp of 2^(6 - lp) >= parts; a list goes round the waves in pieces of at most eight entries
+    // (64 bytes), so that their shares of it are alike
+    const int lp = __clz(p.parts - 1) - 26, piece = min(lp, 3);
+    const int q = lane >> lp, l = lane & ((1 << lp) - 1), stride = NW << lp;
+    const int at = ((((l >> piece) * NW) + wave) << piece) + (l & ((1 << piece) - 1));
+    const bool in = q < p.parts;
+    const unsigned int* counts = p.part_count + (int64_t)row_idx * p.parts;
+    const uint2* list = p.part_list + ((int64_t)row_idx * p.parts + (in ? q : 0)) * p.part_cap;
+    uint2 e[FEW_SLOTS];
+#pragma unroll
+    for (int u = 0; u < FEW_SLOTS; ++u) e[u] = list[min(at + u * stride, p.part_cap - 1)];
+    const unsigned int c = in ? counts[q] : 0u;
+    if (tid < FEW) s.list_w[tid] = 0;
+    if (tid < NW) s.cnt[tid] = 0;
+    if (tid == 0) s.n_list = 0;
+    if (__any(c > (unsigned int)min(p.part_cap, FEW_SLOTS * stride)) || !__any(c != 0u)) return false;
+    uint32_t top = 0;
+#pragma unroll
+    for (int u = 0; u < FEW_SLOTS; ++u) {
+        if ((unsigned int)(at + u * stride) >= c) e[u].x = 0u;             // (no candidate has key 0)
+        top = max(top, e[u].x);
+    }
+    const uint32_t bound = wave_rth_bound(top, (p.top_k + NW - 1) / NW);
+    if (lane == 0) s.seg_tied[wave] = bound;
+    __syncthreads();
+    // Each wave's bound, and how many lanes of all waves reach it: the largest one that top_k lanes reach is the
+    // row's (the smallest of the sixteen always is such a one, but lets several times as many pass).
+    const uint32_t t = s.seg_tied[lane & 15];
+    unsigned int reach = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const unsigned int r = (unsigned int)__popcll(__ballot(top >= (uint32_t)__builtin_amdgcn_readlane((int)t, w)));
+        reach = lane == w ? r : reach;
+    }
+    if (lane < NW) atomicAdd(&s.cnt[lane], reach);
+    __syncthreads();
+    uint32_t key_l = s.cnt[lane & 15] >= (unsigned int)p.top_k ? t : 0u;
+    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x128, 0xf, 0xf, false));   // row_ror 8, 4, 2, 1
+    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x124, 0xf, 0xf, false));
+    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x122, 0xf, 0xf, false));
+    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x121, 0xf, 0xf, false));
+    key_l = max(key_l, 1u);
+    unsigned long long pass[FEW_SLOTS];
+    unsigned int mine_n = 0;
+#pragma unroll
+    for (int u = 0; u < FEW_SLOTS; ++u) {
+        pass[u] = __ballot(e[u].x >= key_l);
+        mine_n += (unsigned int)__popcll(pass[u]);
+    }
+    unsigned int j = 0;
+    if (lane == 0 && mine_n) j = atomicAdd(&s.n_list, mine_n);
+    j = __builtin_amdgcn_readfirstlane(j);
+#pragma unroll
+    for (int u = 0; u < FEW_SLOTS; ++u) {
+        const unsigned int at_u = j + __popcll(pass[u] & ((1ull << lane) - 1ull));
+        if (e[u].x >= key_l && at_u < FEW) s.list_w[at_u] = (unsigned long long)e[u].x << 32 | ~e[u].y;
+        j += (unsigned int)__popcll(pass[u]);
+    }
+    __syncthreads();
+    const int n = (int)s.n_list;
+    if (n > FEW) return false;
+    // ranks by (key, then index): entry 64 g + l in lane l, this wave counts for the entries of lanes 4 wave ..
+    unsigned long long x[FEW / 64];
+#pragma unroll
+    for (int g = 0; g < FEW / 64; ++g) x[g] = s.list_w[64 * g + lane];
+    unsigned long long* sorted = s.mass;
+#pragma unroll
+    for (int g = 0; g < FEW / 64; ++g) {
+        if (64 * g >= n) break;
+        int rank = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned long long me = readlane64(x[g], 4 * wave + i);
+            int r = 0;
+#pragma unroll
+            for (int h = 0; h < FEW / 64; ++h) r += __popcll(__ballot(x[h] > me));       // (zeros are above nothing)
+            rank = lane == 4 * wave + i ? r : rank;
+        }
+        if (lane >> 2 == wave && x[g] != 0) sorted[rank] = x[g];
+    }
+    __syncthreads();
+    const uint32_t kth = n >= p.top_k ? (uint32_t)(sorted[p.top_k - 1] >> 32) : 1u;        // fewer than k: all of them stay
+    const uint32_t key_m = (uint32_t)(sorted[0] >> 32);
+    const bool ties = n > FEW_K && (uint32_t)(sorted[FEW_K] >> 32) >= kth;           // more than a lane each
+    if (ties || !(key_value(key_m) < INFINITY)) return false;
+    if (wave != 0) return true;
+    // lane t: the t-th largest.  Nucleus: an entry stays while the mass before it is at most top_p of the total.
+    const unsigned long long mine = lane < n ? sorted[lane] : 0;
+    const uint32_t key = (uint32_t)(mine >> 32);
+    const bool stays = key >= kth;
+    unsigned int idx = ~(uint32_t)mine;
+    unsigned long long w = stays ? weight_of(key_value(key), key_value(key_m)) : 0;
+    int left = __popcll(__ballot(stays));                                     // lanes 0 .. left - 1
+    if (p.top_p < 1.f) {
+        const unsigned long long incl = wave_scan_dpp64(w), z = readlane64(incl, 63);
+        const unsigned long long limit = (unsigned long long)((double)fmaxf(p.top_p, 0.f) * (double)z);
+        if (incl - w > limit) w = 0;
+        left = __popcll(__ballot(stays && incl - w <= limit));
+    }
+    // into index order: a lane's place is the number of lower indices
+    int place = 0;
+    for (int u = 0; u < left; ++u) place += (unsigned int)__builtin_amdgcn_readlane((int)idx, u) < idx ? 1 : 0;
+    if (lane >= left) { place = lane; w = 0; }
+    idx = (unsigned int)__builtin_amdgcn_ds_permute(4 * place, (int)idx);
+    const uint32_t w_lo = (uint32_t)__builtin_amdgcn_ds_permute(4 * place, (int)(uint32_t)w);
+    const uint32_t w_hi = (uint32_t)__builtin_amdgcn_ds_permute(4 * place, (int)(uint32_t)(w >> 32));
+    w = (unsigned long long)w_hi << 32 | w_lo;
+    const unsigned long long incl = wave_scan_dpp64(w), z = readlane64(incl, 63);
+    unsigned long long target = (unsigned long long)((double)p.uniforms[row_idx] * (double)z);
+    if (target >= z) target = z - 1;
+    if (incl - w <= target && target < incl) p.out[row_idx] = idx;
+    return true;
+}
+
 // The draw from the candidates of a row's parts: those of all parts hold the row's top k, with ties (all finite
 // logits if there are fewer).  The same bound once more, over one maximum per lane, leaves a list a few times k
 // long.  A row that its parts gave up, or whose list is longer than the lanes, is done whole.
@@ -1085,6 +1234,10 @@ sample_merge_kernel(SampleParams p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
     const bool vec_ok = ((uintptr_t)row % 16) == 0;
+    if (p.top_k <= FEW_K && p.probs_out == nullptr) {
+        if (merge_few<T>(p, s, row_idx)) return;
+        __syncthreads();
+    }
     const unsigned int* counts = p.part_count + (int64_t)row_idx * p.parts;
     unsigned int end[MAX_PARTS], total = 0;
     bool fits = true;
@@ -1177,16 +1330,19 @@ greedy_kernel(SampleParams p) {
 
 }  // namespace
 
-// How many parts the rows of a call are cut into (1: none).  A second launch and the merge cost about 7 us, so it has to save more.
-// Device time in a graph, one launch -> parts, us:
+// How many parts the rows of a call are cut into (1: none).  A second launch and the merge cost about 5 us for top_k <= 64
+// (merge_few) and 9 us beyond, so it has to save more.  us per call, one launch -> parts:
+//   top_k <= 64 (k 50)  float32  20000, 2 parts: 1 row 14.4 -> 10.0, 64 15.8 -> 11.3, 1024 61.3 -> 44.3
+//                                50256, 4 parts: 1 row 16.0 -> 10.9, 64 16.7 -> 11.7, 128 17.2 -> 13.9, 1024 86.7 -> 66.5
+//                                128256, 8 parts: 1 row 20 -> 10.7, 64 23 -> 14.4, 512 88 -> 61;  262144: 16 rows 29 -> 11.3
+//                       16-bit   32000: 64 rows 16.6 -> 11.6, 1024 63.4 -> 45.6;  81920: 64 20.7 -> 13.9, 1024 90.4 -> 78.8
+//                                128256: 64 rows 22.3 -> 13.9, 128 22.5 -> 20.3, 1024 109 -> 115;  262144: 64 31.7 -> 25.8,
+//                                128 34.2 -> 37.9 (half the bytes to save on): six parts and more up to 1024 parts
 //   rows whose loads cannot be vectors (a stride that is no multiple of 16 bytes): at once
-//     float32, k 50     50257: 64 rows 23.5 -> 16.9, 512 79.6 -> 47.9;  128255: 64 rows 64.4 -> 22.1, 1024 455 -> 167
-//     bf16              50257: 64 rows 24.4 -> 17.3;  greedy float32 50257: 64 rows 11.4 -> 7.6
-//   other rows from six parts on (65536, four parts: 64 rows 17.4 -> 16.7, 128 rows 18.0 -> 19.3), with k <= 64
-//     float32           128256: 1 row 19.9 -> 15.5, 64 22.9 -> 20.1, 512 88.2 -> 70.8;  262144: 16 rows 29.2 -> 17.6
-//     16-bit            128256: 64 rows 22.3 -> 20.1, but 128 rows 23.3 -> 26.6 (half the bytes to save on): up to 512 parts
-//   k to 256            128256: 1 row 24.3 -> 21.1, 16 25.5 -> 24.6, 64 27.0 -> 30.3: up to 128 parts
-//   greedy              128256: 16 rows 9.1 -> 7.2, 64 10.8 -> 9.8, 128 14.1 -> 17.2: up to 512 parts
+//     bf16, k 50        50257: 64 rows 24.4 -> 17.3;  greedy float32 50257: 64 rows 11.4 -> 7.6
+//   other calls from six parts on
+//     k to 256          128256: 1 row 24.3 -> 21.1, 16 25.5 -> 24.6, 64 27.0 -> 30.3: up to 128 parts
+//     greedy            128256: 16 rows 9.1 -> 7.2, 64 10.8 -> 9.8, 128 14.1 -> 17.2: up to 512 parts
 static int sample_parts(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy, int dtype) {
     const int parts = (int)(((int64_t)vocab + PART_MAX - 1) / PART_MAX);
     if (parts < 2 || parts > MAX_PARTS || batch > PART_MAX_BATCH) return 1;
@@ -1194,10 +1350,9 @@ static int sample_parts(int batch, int vocab, int64_t row_stride, float temperat
     const int per_16 = dtype == AICOMP_KV_F32 ? 4 : 8;
     if (batch > 1 && row_stride % per_16 != 0) return parts;
     const int all = batch * parts;
+    if (!greedy && top_k <= FEW_K) return dtype == AICOMP_KV_F32 || parts < 6 || all <= 1024 ? parts : 1;
     if (parts < 6) return 1;
-    if (greedy) return all <= 512 ? parts : 1;
-    if (top_k > 64) return all <= 128 ? parts : 1;
-    return dtype == AICOMP_KV_F32 || all <= 512 ? parts : 1;
+    return all <= (greedy ? 512 : 128) ? parts : 1;
 }
 
 // Candidates a part has room for.  Of 16384 normally distributed logits about 2.7 k pass the bound of sixteen waves

@@ -83,3 +83,21 @@ def test_a_part_with_as_many_candidates_as_it_has_room_for(device, k, room):
     got, probs = ops.sample_tokens(x, 1.0, k, 0.9, True, u, return_probs=True)
     assert torch.equal(got, want) and torch.equal(probs > 0, dist > 0)
     assert torch.allclose(probs, dist, rtol=2.0 ** -22, atol=0.0)
+
+
+@pytest.mark.parametrize("k", [1, 15, 16, 17, 63, 64, 65])
+@pytest.mark.parametrize("V", [16385, 20000, 50257, 81920, 128256, 262144])
+def test_the_short_merge_draws_what_one_launch_draws(device, V, k):
+    """Up to 64 kept candidates are drawn from by one wave: k on either side, as many equal logits at the top as its
+    lanes and one more, all candidates in one part, fewer finite logits than k, several draws each."""
+    x = torch.cat([_rows(V, torch.float32, device), torch.randn(4, V, generator=torch.Generator().manual_seed(k)).to(device)])
+    x[10, torch.arange(64, device=device) * (V // 64)] = 9.0
+    x[11, torch.arange(65, device=device) * (V // 65)] = 9.0
+    x[12, 7:7 + 300] += 20.0
+    x[13, 5:] = float("-inf")
+    for i in range(6):
+        u = torch.rand(x.shape[0], generator=torch.Generator().manual_seed(i)).to(device)
+        u[:2] = torch.tensor([0.0, 1.0 - 2.0 ** -24])
+        top_p = (1.0, 0.9, 0.5, 0.05, 0.0, 0.999)[i]
+        got = ops.sample_tokens(x, 0.7, k, top_p, uniforms=u)
+        assert torch.equal(got, _one_launch(x, 0.7, k, top_p, True, u)[0]), (top_p, i)

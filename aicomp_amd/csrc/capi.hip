@@ -94,11 +94,10 @@ static int auto_partition(int64_t rows, int hkv, int d, int bs, int max_blocks, 
         // device and 3 us of host time) costs what the longer chain of one workgroup does: 1000 and
         // 1200 tokens at D 64 whole 7.2 and 7.4 us, split 8.0 us, 2000 tokens 9.7 and 7.9; D 128: 760
         // tokens 7.7 and 8.8, 1000 tokens 9.2 and 8.2 us.  Other pools: 640.  Float32 at D 64: 640 tokens of
-        // one row whole 10.4 us, split 10.5, 768 tokens 12.0 and 10.6.  A float32 row at D 128 is four times the
-        // matrix instructions of a bf16 one on its CU: whole up to 448 tokens where the split has a CU for
-        // each of its workgroups (one row of 448 13.0 whole, 13.2 split; 512 tokens 15.0 and 13.9, 640 17.6
-        // and 13.7; 16 rows of 8 KV heads, 512 tokens 18.0 and 16.9), otherwise up to 640 (those 16 rows,
-        // 576 tokens 19.2 and 22.1, 768 tokens 24.2 and 23.9).
+        // one row whole 10.1 us, split 9.4 (and 3 us of host time), 768 tokens 11.3 and 9.9.  A float32 row at D 128
+        // is as many bytes as two bf16 rows on its CU: whole up to 448 tokens where the split has a CU for each of its
+        // workgroups (one row of 448 12.2 whole, 11.5 split; 512 tokens 13.1 and 12.1, 640 15.3
+        // and 11.9), otherwise up to 640 (16 rows of 8 KV heads, 640 tokens 19.1 and 21.5, 768 tokens 21.8 and 23.2).
         const bool f32_few = kv_dtype == AICOMP_KV_F32 && d == 128 && rows * hkv * ((max_ctx + 255) / 256) <= 256;
         const int64_t whole = f32_few ? 448 : !is_16bit_float(kv_dtype) ? 640 : d == 64 ? 1280 : 768;
         ps = max_ctx <= whole ? (int)((max_ctx + 63) / 64 * 64) : 256;

@@ -13,7 +13,7 @@
 // and the two columns' partial softmaxes are merged at the end.  Same instruction
 // stream per byte as head_dim 128.  Float32 queries over float32 pools, head_dim 128 and
 // 64, up to 16 heads per KV head, run the same two schedules on the float32 matrix
-// instruction (decode_tile_f32.h).  Everything else goes to the vector-ALU kernel.
+// instruction (decode_tile_f32_quad.h up to four heads per KV head, decode_tile_f32.h beyond).  Everything else goes to the vector-ALU kernel.
 //
 // HBM-bound: per sequence 2 * L * Hkv * D * e_kv bytes of K/V are streamed and
 // used exactly once; 4 * G flop per byte (bf16), far below the MFMA roof, so
@@ -358,7 +358,7 @@ __device__ __forceinline__ void inject_new_row(TileRegs<FP8>& kr, TileRegs<FP8>&
 template <typename E, bool FP8_, bool PAIR_>
 struct Tile16 {
     typedef E Fmt;
-    static constexpr bool FP8 = FP8_, PAIR = PAIR_;
+    static constexpr bool FP8 = FP8_, PAIR = PAIR_, QUAD = false;
     static constexpr int DQ = PAIR ? 64 : D;             // head_dim of the tensors
     static constexpr int TT = PAIR ? 2 * TILE : TILE;    // tokens per tile
     static constexpr int BPT = TT / BS;                  // blocks per tile
@@ -424,6 +424,7 @@ struct Tile16 {
 };
 
 #include "decode_tile_f32.h"
+#include "decode_tile_f32_quad.h"
 
 template <typename T, int NW>
 __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1)
@@ -474,7 +475,7 @@ paged_decode_mfma_kernel(MfmaParams p) {
     const float cmul = p.qk_mul * (T::FP8 ? p.k_scale[kvh] : 1.f);
 
     typename T::State st;
-    clear_state(st);
+    if constexpr (!T::QUAD) clear_state(st);
 
     // physical blocks of tile tt (wave-uniform); the held table slice is refilled every 64 blocks
     int64_t bb[4] = {0, 0, 0, 0};
@@ -518,16 +519,19 @@ paged_decode_mfma_kernel(MfmaParams p) {
         else
             T::template process<false, false>(st, kv, qf, kt, ko, p, bb, kvh, lane, tile_start, end, cmul);
     }
-    const float m = st.m;
-    float lsum = st.lsum;
-
     // ---- wave result: the accumulators of column r16 into its row of the wave's own K tile region
-    lsum += __shfl_xor(lsum, 16);
-    lsum += __shfl_xor(lsum, 32);
     float* osm = (float*)kt;        // 16 columns of at most 128 floats: 8192 bytes, the whole tile
-    if (r16 < ncol) {
-        T::store_acc(osm + r16 * T::OROW, st, g4);
-        if (g4 == 0) { sm_m[w][r16] = m; sm_l[w][r16] = lsum; }
+    if constexpr (T::QUAD) {
+        T::finish(st, osm, sm_m[w], sm_l[w], 1, lane, G);
+    } else {
+        const float m = st.m;
+        float lsum = st.lsum;
+        lsum += __shfl_xor(lsum, 16);
+        lsum += __shfl_xor(lsum, 32);
+        if (r16 < ncol) {
+            T::store_acc(osm + r16 * T::OROW, st, g4);
+            if (g4 == 0) { sm_m[w][r16] = m; sm_l[w][r16] = lsum; }
+        }
     }
     __syncthreads();
 
@@ -763,7 +767,7 @@ streamk_decode_kernel(StreamKParams p) {
         }
 
         typename T::State st;
-        clear_state(st);
+        if constexpr (!T::QUAD) clear_state(st);
 
         int64_t bb[4] = {0, 0, 0, 0};
         int k = 0;
@@ -796,11 +800,17 @@ streamk_decode_kernel(StreamKParams p) {
         }
 
         // ---- flush
-        float lsum = st.lsum;
-        lsum += __shfl_xor(lsum, 16);
-        lsum += __shfl_xor(lsum, 32);
         const int64_t slot = (int64_t)kvh * (p.waves_per_head + B) + part + seq;
-        if constexpr (T::PAIR) {
+        float lsum = 0.f;
+        if constexpr (!T::QUAD) {
+            lsum = st.lsum;
+            lsum += __shfl_xor(lsum, 16);
+            lsum += __shfl_xor(lsum, 32);
+        }
+        if constexpr (T::QUAD) {
+            float* ml = p.ws_ml + slot * G * 2;
+            T::finish(st, p.ws_acc + slot * G * DQ, ml, ml + 1, 2, lane, G);
+        } else if constexpr (T::PAIR) {
             // Column (head, parity) holds its own token's half of the pair rows: parity 0 elements 0..63 of
             // its accumulator (lanes g4 = 0, 1), parity 1 elements 64..127 (lanes g4 = 2, 3).  The two are
             // partial softmaxes over the even and the odd tokens of the same segment: merged here, inside the
@@ -1034,8 +1044,13 @@ int launch_decode_streamk(const DecodeArgs& a, void* workspace) {
         else hipLaunchKernelGGL((streamk_decode_kernel<Tile16<E, false, PAIR>>), dim3(wgs), dim3(256), 0, a.stream, p);    \
     } while (0)
     if (f32) {
-        if (a.d == 64) hipLaunchKernelGGL((streamk_decode_kernel<TileF32<64>>), dim3(wgs), dim3(256), 0, a.stream, p);
-        else hipLaunchKernelGGL((streamk_decode_kernel<TileF32<128>>), dim3(wgs), dim3(256), 0, a.stream, p);
+#define AICOMP_LAUNCH_SK32(DQ)                                                                                                 \
+    do {                                                                                                                       \
+        if (group <= 4) hipLaunchKernelGGL((streamk_decode_kernel<TileF32Quad<DQ>>), dim3(wgs), dim3(256), 0, a.stream, p);    \
+        else hipLaunchKernelGGL((streamk_decode_kernel<TileF32<DQ>>), dim3(wgs), dim3(256), 0, a.stream, p);                   \
+    } while (0)
+        if (a.d == 64) AICOMP_LAUNCH_SK32(64); else AICOMP_LAUNCH_SK32(128);
+#undef AICOMP_LAUNCH_SK32
     } else if (pair) { if (f16) AICOMP_LAUNCH_SK(F16Fmt, true); else AICOMP_LAUNCH_SK(Bf16Fmt, true); }
     else { if (f16) AICOMP_LAUNCH_SK(F16Fmt, false); else AICOMP_LAUNCH_SK(Bf16Fmt, false); }
 #undef AICOMP_LAUNCH_SK
@@ -1089,10 +1104,13 @@ int launch_decode_mfma(const DecodeArgs& a) {
         if (d64) { if (fp8) AICOMP_LAUNCH_GRID(Tile16<E, true, true>); else AICOMP_LAUNCH_GRID(Tile16<E, false, true>); } \
         else { if (fp8) AICOMP_LAUNCH_GRID(Tile16<E, true, false>); else AICOMP_LAUNCH_GRID(Tile16<E, false, false>); }   \
     } while (0)
-    if (a.q_dtype == AICOMP_KV_F32) { if (d64) AICOMP_LAUNCH_GRID(TileF32<64>); else AICOMP_LAUNCH_GRID(TileF32<128>); }
+#define AICOMP_LAUNCH_GRID32(DQ)                                                                              \
+    do { if (p.group <= 4) AICOMP_LAUNCH_GRID(TileF32Quad<DQ>); else AICOMP_LAUNCH_GRID(TileF32<DQ>); } while (0)
+    if (a.q_dtype == AICOMP_KV_F32) { if (d64) AICOMP_LAUNCH_GRID32(64); else AICOMP_LAUNCH_GRID32(128); }
     else if (a.q_dtype == AICOMP_KV_F16) AICOMP_LAUNCH_GRID16(F16Fmt);
     else AICOMP_LAUNCH_GRID16(Bf16Fmt);
 #undef AICOMP_LAUNCH_GRID16
+#undef AICOMP_LAUNCH_GRID32
 #undef AICOMP_LAUNCH_GRID
     AICOMP_HIP_LAUNCH_CHECK();
     if (a.num_parts > 1) return launch_split_reduce(a);

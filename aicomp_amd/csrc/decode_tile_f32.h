@@ -1,5 +1,6 @@
 // TileF32: float32 queries and pools, head_dim 128 (tiles of 16 tokens) or 64 (32 tokens), on the
-// float32 matrix instruction v_mfma_f32_16x16x4_f32.  Included by decode_mfma.hip, inside its namespace.
+// float32 matrix instruction v_mfma_f32_16x16x4_f32, for groups of more than four query heads per KV head (smaller
+// ones: decode_tile_f32_quad.h).  Included by decode_mfma.hip, inside its namespace.
 //
 // A tile (8 KB of K, 8 KB of V) costs a wave 64 MFMAs of 32 cycles, 2048 cycles: 19 TB/s with all 1024 SIMDs
 // at work, so a batch that fills the chip is bound by HBM like the 16-bit tiles.  The rows of a small call
@@ -24,7 +25,7 @@
 template <int DQ_>
 struct TileF32 {
     typedef F32Fmt Fmt;
-    static constexpr bool FP8 = false, PAIR = false;
+    static constexpr bool FP8 = false, PAIR = false, QUAD = false;
     static constexpr int DQ = DQ_;
     static constexpr int TT = DQ == 128 ? 16 : 32;       // tokens per tile
     static constexpr int BPT = TT / BS;

@@ -26,13 +26,14 @@ SYMBOLS = (
     "aicomp_paged_prefill_attn_items",
     "aicomp_paged_prefill_tile_positions",
     "aicomp_rope_kv_append",
+    "aicomp_rope_paged_decode_attn",
     "aicomp_sample_tokens",
     "aicomp_sample_tokens_split",
     "aicomp_sample_workspace_bytes",
 )
 
 F32, BF16, FP8_E4M3, F16 = 0, 1, 2, 3
-MIN_VERSION = 300            # 0.3.0: the entry points of SYMBOLS above
+MIN_VERSION = 301            # 0.3.1: the entry points of SYMBOLS above
 
 _lock = threading.RLock()       # torch_ops() loads the HIP library while holding it
 _lib = None
@@ -64,6 +65,10 @@ def _declare(lib: C.CDLL) -> None:
     lib.aicomp_paged_decode_attn_append_static.argtypes = [vp, vp, vp, vp, i64, i64, vp, vp, vp, i64, vp, i32,
                                                            i32, i32, i32, i32, i32, i64, f32, i32, i32, vp,
                                                            vp, i32, vp]
+    lib.aicomp_rope_paged_decode_attn.restype = i32
+    lib.aicomp_rope_paged_decode_attn.argtypes = [vp, vp, i64, i64, vp, vp, i64, i64, vp, vp, i64, i64, vp, vp, vp, vp, vp,
+                                                  i64, vp, i32, i32, i32, i32, i32, i32, i64, f32, i32, i32, vp, vp, vp,
+                                                  sz, vp]
     lib.aicomp_paged_decode_workspace_bytes.restype = sz
     lib.aicomp_paged_decode_workspace_bytes.argtypes = [i32] * 9
     lib.aicomp_paged_decode_partition_size.restype = i32

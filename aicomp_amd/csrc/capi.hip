@@ -117,7 +117,7 @@ using namespace aicomp;
 
 extern "C" {
 
-int aicomp_kv_version(void) { return 300; }
+int aicomp_kv_version(void) { return 301; }
 
 const char* aicomp_kv_last_error(void) { return g_err; }
 
@@ -386,6 +386,62 @@ int aicomp_paged_decode_attn_append(void* out, const void* query, const void* ne
                        head_dim, block_size, max_blocks_per_seq, num_blocks, scale, q_dtype, kv_dtype,
                        k_scale, v_scale, partition_size, workspace, workspace_bytes, stream,
                        "paged_decode_attn_append");
+}
+
+int aicomp_rope_paged_decode_attn(void* out, const void* query, int64_t q_token_stride, int64_t q_head_stride,
+                                  const void* new_key, const void* new_value, int64_t kv_token_stride,
+                                  int64_t kv_head_stride, const void* cos, const void* sin, int64_t table_stride,
+                                  int64_t table_rows, const int64_t* positions, const int64_t* slot_mapping, void* k_pool,
+                                  void* v_pool, const int32_t* block_table, int64_t block_table_stride,
+                                  const int32_t* context_lens, int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                  int block_size, int max_blocks_per_seq, int64_t num_blocks, float scale, int q_dtype,
+                                  int kv_dtype, const float* k_scale, const float* v_scale, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+    const char* who = "rope_paged_decode_attn";
+    AICOMP_REQUIRE(batch >= 0, AICOMP_KV_EINVAL, "%s: negative batch", who);
+    if (batch == 0) return AICOMP_KV_OK;
+    AICOMP_REQUIRE(out && query && new_key && new_value && cos && sin && positions && slot_mapping && k_pool && v_pool &&
+                   block_table && context_lens, AICOMP_KV_EINVAL, "%s: null pointer", who);
+    int rc = check_common(num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, num_blocks, q_dtype,
+                          kv_dtype, k_scale, v_scale, who);
+    if (rc) return rc;
+    AICOMP_REQUIRE(max_blocks_per_seq > 0 && block_table_stride >= max_blocks_per_seq, AICOMP_KV_EINVAL,
+                   "%s: block table stride %lld < width %d", who, (long long)block_table_stride, max_blocks_per_seq);
+    AICOMP_REQUIRE(q_head_stride >= head_dim && kv_head_stride >= head_dim && table_stride >= head_dim && table_rows > 0 &&
+                   q_token_stride >= 0 && kv_token_stride >= 0, AICOMP_KV_EINVAL,
+                   "%s: strides overlap rows of %d elements", who, head_dim);
+    const int64_t v = 16 / dtype_size(q_dtype);
+    const bool vectors = (q_token_stride | q_head_stride | kv_token_stride | kv_head_stride | table_stride) % v == 0 &&
+                         ((uintptr_t)new_key | (uintptr_t)new_value | (uintptr_t)cos | (uintptr_t)sin | (uintptr_t)query) % 16 == 0;
+    const bool shape = streamk_shape(batch, num_q_heads, num_kv_heads, head_dim, block_size, q_dtype, kv_dtype);
+    DecodeArgs a;
+    memset(&a, 0, sizeof(a));
+    a.out = out; a.query = query; a.k_pool = k_pool; a.v_pool = v_pool;
+    a.block_table = block_table; a.block_table_stride = block_table_stride; a.context_lens = context_lens;
+    a.num_seqs = batch; a.rows = batch;
+    a.hq = num_q_heads; a.hkv = num_kv_heads; a.d = head_dim; a.bs = block_size;
+    a.max_blocks = max_blocks_per_seq; a.num_blocks = num_blocks;
+    a.scale = scale; a.q_dtype = q_dtype; a.kv_dtype = kv_dtype;
+    a.k_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? k_scale : nullptr;
+    a.v_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? v_scale : nullptr;
+    a.num_parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, shape, a.partition_size);
+    a.stream = (hipStream_t)stream;
+    // (a batch for the balanced schedule streams for tens of microseconds: the launch saved is lost in it)
+    AICOMP_REQUIRE(vectors && shape && small_call(batch, block_size, max_blocks_per_seq) && decode_mfma_supported(a),
+                   AICOMP_KV_EUNSUPPORTED, "%s: not a call of the matrix-core grid schedule", who);
+    a.new_key = new_key; a.new_value = new_value;
+    a.new_token_stride = kv_token_stride; a.new_head_stride = kv_head_stride;
+    a.cos_tab = cos; a.sin_tab = sin; a.tab_stride = table_stride; a.tab_rows = table_rows;
+    a.positions = positions; a.slots = slot_mapping;
+    a.q_token_stride = q_token_stride; a.q_head_stride = q_head_stride;
+    if (a.num_parts > 1) {
+        const size_t need = split_workspace_bytes(a.rows, a.hq, a.hkv, a.d, a.num_parts);
+        AICOMP_REQUIRE(workspace && workspace_bytes >= need, AICOMP_KV_EWORKSPACE,
+                       "%s: workspace of %zu bytes needed, %zu given", who, need, workspace ? workspace_bytes : (size_t)0);
+        AICOMP_REQUIRE((uintptr_t)workspace % 16 == 0, AICOMP_KV_EINVAL, "%s: workspace must be 16-byte aligned", who);
+        a.ws = split_workspace_view(workspace, a.rows, a.hq, a.hkv, a.d, a.num_parts);
+    }
+    return launch_decode_mfma(a);
 }
 
 // Device address of `scratch` on the current device, looked up once per device.

@@ -205,6 +205,7 @@ struct F16Fmt {
 
 // float32 tensors: outputs are stored as they are
 struct F32Fmt {
+    typedef float elem;
     typedef float raw;
     __device__ __forceinline__ static float from_f32(float f) { return f; }
 };
@@ -277,6 +278,14 @@ struct DecodeArgs {
     const void* new_key;
     const void* new_value;
     int64_t new_token_stride, new_head_stride;
+    // rotary embedding of the query rows and the new K row inside the decode launch (decode only; NULL = none): the
+    // query then has the strides below, new rows go to slots[row]
+    const void* cos_tab;
+    const void* sin_tab;
+    int64_t tab_stride, tab_rows;
+    const int64_t* positions;
+    const int64_t* slots;
+    int64_t q_token_stride, q_head_stride;
     // prefill only (NULL = none): (sequence, query tile) pairs, one workgroup row each, in the order
     // the workgroups are to take them
     const int32_t* items;

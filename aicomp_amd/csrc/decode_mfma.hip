@@ -43,6 +43,7 @@
 // Split-K      partitions write (max, sum, unnormalised output) to the
 //              workspace; a second, small kernel merges them.
 #include "common.h"
+#include "rope_math.h"
 
 #include <atomic>
 
@@ -79,6 +80,13 @@ struct MfmaParams {
     const void* new_key;
     const void* new_value;
     int64_t new_token_stride, new_head_stride;     // elements
+    // rotary embedding of the query rows and the new K row (kernels with ROPE; see rope_append.hip)
+    const void* cos_tab;
+    const void* sin_tab;
+    int64_t tab_stride, tab_rows;
+    const int64_t* positions;
+    const int64_t* slots;                          // where the new row goes
+    int64_t q_token_stride, q_head_stride;
 };
 
 template <bool FP8> struct TileRegs;
@@ -320,8 +328,8 @@ __device__ __forceinline__ uint2 quant8_fp8(const uint4& x, float scale) {
 // needed.  A tile row is one token (16 lanes of 8 elements), or with PAIR half a row (8 lanes).
 template <typename E, bool FP8, bool PAIR, typename Params>
 __device__ __forceinline__ void inject_new_row(TileRegs<FP8>& kr, TileRegs<FP8>& vr, const Params& p,
-                                                    int seq, int kvh, int lane, int tile_start, int len,
-                                                    const int64_t (&bb)[4]) {
+                                               const uint16_t* key, const uint16_t* value, int kvh, int lane,
+                                               int tile_start, int len, const int64_t (&bb)[4]) {
     constexpr int DQ = PAIR ? 64 : D;
     const int tau = len - 1 - tile_start;              // token within the tile, wave-uniform
     const int blk_i = tau >> 4, tb = tau & 15;         // block of the tile, token within the block
@@ -330,9 +338,8 @@ __device__ __forceinline__ void inject_new_row(TileRegs<FP8>& kr, TileRegs<FP8>&
     const int row = PAIR ? (tau >> 1) : tau;
     const bool mine = (lane >> 4) == (row & 3) && (!PAIR || ((lane >> 3) & 1) == (tau & 1));
     const int slot = row >> 2;
-    const int64_t src = (int64_t)seq * p.new_token_stride + (int64_t)kvh * p.new_head_stride + 8 * c;
-    const uint4 nk = *(const uint4*)((const uint16_t*)p.new_key + src);
-    const uint4 nv = *(const uint4*)((const uint16_t*)p.new_value + src);
+    const uint4 nk = *(const uint4*)(key + 8 * c);
+    const uint4 nv = *(const uint4*)(value + 8 * c);
     const int64_t blk = bb[blk_i];
     const int64_t dst = ((blk * p.hkv + kvh) * BS + tb) * (DQ / 8) + c;        // 8-element chunks
     if constexpr (FP8) {
@@ -370,14 +377,13 @@ struct Tile16 {
     struct Regs { TileRegs<FP8> k, v; };
     __device__ __forceinline__ static Offsets offsets(int lane) { return k_tile_offsets(lane); }
 
-    // raw query rows of (sequence, KV head); columns beyond the group are zeroed by q_operand only
+    // raw query rows of a (sequence, KV head), one after the other; columns beyond the group are zeroed by q_operand only
     // when the rows are used, so that issuing the loads never waits for them.
     // PAIR: column c = (head c / 2, parity c % 2): k-slot s covers row elements 32s + 8 g4 .., which are
     // the query's elements (32s + 8 g4) % 64 when the slot lies in the column's own half of the row.
-    template <typename Params>
-    __device__ __forceinline__ static void load_q(Q& q, const Params& p, int seq, int kvh, int lane) {
+    __device__ __forceinline__ static void load_q(Q& q, const uint16_t* rows, int group, int lane) {
         const int r16 = lane & 15, g4 = lane >> 4, h = PAIR ? (r16 >> 1) : r16;
-        const uint16_t* row = (const uint16_t*)p.query + ((int64_t)seq * p.hq + kvh * p.group + min(h, p.group - 1)) * DQ;
+        const uint16_t* row = rows + min(h, group - 1) * DQ;
 #pragma unroll
         for (int s = 0; s < 4; ++s) q.r[s] = *(const uint4*)(row + (PAIR ? ((32 * s + 8 * g4) & 63) : 32 * s + 8 * g4));
     }
@@ -408,9 +414,9 @@ struct Tile16 {
                                                kvh_next, lane, lane >> 4, tile_start, end, cmul, nb[2], nb[3]);
     }
     template <typename Params>
-    __device__ __forceinline__ static void inject(Regs& t, const Params& p, int seq, int kvh, int lane, int tile_start,
-                                                  int len, const int64_t (&bb)[4]) {
-        inject_new_row<E, FP8, PAIR>(t.k, t.v, p, seq, kvh, lane, tile_start, len, bb);
+    __device__ __forceinline__ static void inject(Regs& t, const Params& p, const uint16_t* key, const uint16_t* value,
+                                                  int kvh, int lane, int tile_start, int len, const int64_t (&bb)[4]) {
+        inject_new_row<E, FP8, PAIR>(t.k, t.v, p, key, value, kvh, lane, tile_start, len, bb);
     }
     // this lane's accumulators into the row of its column: elements 32 g4 + 8 i + j from O[j][i]
     __device__ __forceinline__ static void store_acc(float* row, const State& st, int g4) {
@@ -426,7 +432,72 @@ struct Tile16 {
 #include "decode_tile_f32.h"
 #include "decode_tile_f32_quad.h"
 
-template <typename T, int NW>
+// query rows of (sequence, KV head) in the tensor, and its new rows
+template <typename T, typename Params>
+__device__ __forceinline__ const typename T::Fmt::raw* q_rows(const Params& p, int seq, int kvh) {
+    return (const typename T::Fmt::raw*)p.query + ((int64_t)seq * p.hq + kvh * p.group) * T::DQ;
+}
+template <typename T, typename Params>
+__device__ __forceinline__ const typename T::Fmt::raw* new_row(const void* rows, const Params& p, int seq, int kvh) {
+    return (const typename T::Fmt::raw*)rows + (int64_t)seq * p.new_token_stride + (int64_t)kvh * p.new_head_stride;
+}
+
+// The rotary embedding of a workgroup's rows, every wave for itself: the group's query rows to q_lds, one after the
+// other, and the new K row to k_lds.  Bit for bit what rope_append.hip leaves (same roundings, same order).
+template <typename T>
+__device__ __forceinline__ void rope_rows(const MfmaParams& p, int seq, int kvh, int64_t pos, typename T::Fmt::raw* q_lds,
+                                          typename T::Fmt::raw* k_lds, int lane) {
+    typedef typename T::Fmt::elem Elem;
+    constexpr int CH = T::DQ / 16, HALF = T::DQ / 2, PER = 64 / CH;          // lanes per row, rows per pass
+    const int c8 = 8 * (lane & (CH - 1)), G = p.group;
+    const Elem* cr = (const Elem*)p.cos_tab + pos * p.tab_stride + c8;
+    const Elem* sr = (const Elem*)p.sin_tab + pos * p.tab_stride + c8;
+    Raw8<Elem> raw[4];
+    raw[0].load(cr); raw[1].load(cr + HALF); raw[2].load(sr); raw[3].load(sr + HALF);
+    for (int row = lane / CH; row <= G; row += PER) {
+        const Elem* src = (row < G ? (const Elem*)p.query + seq * p.q_token_stride + (int64_t)(kvh * G + row) * p.q_head_stride
+                                   : (const Elem*)new_row<T>(p.new_key, p, seq, kvh)) + c8;
+        Raw8<Elem> lo, hi;
+        lo.load(src);
+        hi.load(src + HALF);
+        float xl[8], xh[8], cl[8], ch[8], sl[8], sh[8];
+        lo.unpack(xl); hi.unpack(xh);
+        raw[0].unpack(cl); raw[1].unpack(ch); raw[2].unpack(sl); raw[3].unpack(sh);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float ol = rot1<Elem, true>(xl[j], xh[j], cl[j], sl[j]);
+            xh[j] = rot1<Elem>(xh[j], xl[j], ch[j], sh[j]);
+            xl[j] = ol;
+        }
+        Elem* dst = (Elem*)(row < G ? q_lds + row * T::DQ : k_lds) + c8;
+        Row8<Elem>::store(dst, xl);
+        Row8<Elem>::store(dst + HALF, xh);
+    }
+}
+
+// A new row into its slot alone (a slot that is not where the table has the row's last token).
+template <typename T>
+__device__ __forceinline__ void store_new_row(const MfmaParams& p, const typename T::Fmt::raw* key,
+                                              const typename T::Fmt::raw* value, int kvh, int64_t slot, int lane) {
+    typedef typename T::Fmt::raw Raw;
+    const int64_t row = (slot / BS * p.hkv + kvh) * BS + slot % BS;
+    if constexpr (T::FP8) {
+        if (lane < T::DQ / 8) {
+            ((uint2*)p.k_pool)[row * (T::DQ / 8) + lane] = quant8_fp8<typename T::Fmt>(*(const uint4*)(key + 8 * lane), p.k_scale[kvh]);
+            ((uint2*)p.v_pool)[row * (T::DQ / 8) + lane] = quant8_fp8<typename T::Fmt>(*(const uint4*)(value + 8 * lane), p.v_scale[kvh]);
+        }
+    } else {
+        for (int d = lane; d < T::DQ; d += 64) {
+            ((Raw*)p.k_pool)[row * T::DQ + d] = key[d];
+            ((Raw*)p.v_pool)[row * T::DQ + d] = value[d];
+        }
+    }
+}
+
+// ROPE: the query rows come as projected, with strides of their own, and are rotated here, like the new K row: a decode
+// step of a layer is then this launch alone, where the rotary + append launch before it and the rotated query's way
+// through memory cost 3.3 us of device and 6 us of host time (8 rows of 900 tokens, 32 / 8 heads, D 64).
+template <typename T, int NW, bool ROPE>
 __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1)
 paged_decode_mfma_kernel(MfmaParams p) {
     // KV head fastest: the workgroups launched together read the Hkv slices of the same
@@ -454,20 +525,31 @@ paged_decode_mfma_kernel(MfmaParams p) {
     int tab = (blk_base + lane < p.max_blocks) ? table[blk_base + lane] : 0;
 
     typename T::Q qf;
-    T::load_q(qf, p, seq, kvh, lane);
+    if constexpr (!ROPE) T::load_q(qf, q_rows<T>(p, seq, kvh), G, lane);
 
     const int len = min(p.context_lens[seq], p.max_blocks * BS);   // never read past the table row
+    // (a position without a row in the tables rotates by row 0 and is not stored, a slot outside the pool is a padding row's)
+    const int64_t pos_in = ROPE ? p.positions[seq] : 0, slot = ROPE ? p.slots[seq] : -1;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[NW * KTILE_BYTES];
+    const bool pos_ok = pos_in >= 0 && pos_in < p.tab_rows;
+    const bool stored = ROPE && pos_ok && slot >= 0 && slot < p.num_blocks * BS;
+    __shared__ __attribute__((aligned(16))) typename T::Fmt::raw k_new[ROPE ? NW : 1][ROPE ? DQ : 1];
     if (start >= len) {
         if (len <= 0 && part == 0) {   // nothing to attend to: the output row is defined as zero
             auto* o = (typename T::Fmt::raw*)p.out + ((int64_t)seq * p.hq + kvh * G) * DQ;
             for (int i = tid; i < G * DQ; i += blockDim.x) o[i] = 0;
+            if constexpr (ROPE) {
+                if (stored && w == 0) {
+                    rope_rows<T>(p, seq, kvh, pos_in, (typename T::Fmt::raw*)lds, k_new[0], lane);
+                    store_new_row<T>(p, k_new[0], new_row<T>(p.new_value, p, seq, kvh), kvh, slot, lane);
+                }
+            }
         }
         return;
     }
     const int end = min(len, start + p.partition_size);
     const int ntiles = (end - start + TT - 1) / TT;
 
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NW * KTILE_BYTES];
     __shared__ float sm_m[NW][16];
     __shared__ float sm_l[NW][16];
     unsigned char* kt = lds + w * KTILE_BYTES;
@@ -497,6 +579,11 @@ paged_decode_mfma_kernel(MfmaParams p) {
         typename T::Regs kv;
         tile_blocks(w);
         T::load(kv, p, bb, kvh, lane);
+        if constexpr (ROPE) {                     // through the wave's K tile, before any K is there
+            rope_rows<T>(p, seq, kvh, pos_ok ? pos_in : 0, (typename T::Fmt::raw*)kt, k_new[w], lane);
+            __builtin_amdgcn_wave_barrier();
+            T::load_q(qf, (const typename T::Fmt::raw*)kt, G, lane);
+        }
         T::q_operand(qf, qf, G, lane);
         int tt = w;
         for (; tt + NW < ntiles; tt += NW) {      // steady state: never the partition's last tile
@@ -511,8 +598,16 @@ paged_decode_mfma_kernel(MfmaParams p) {
             // block of the pool and the length fits the table; otherwise the call leaves the pools alone
             // (and attends over what the clamped table entry holds, like the unfused sequence of calls).
             const int raw_blk = __builtin_amdgcn_readlane(tab, BPT * tt + ((len - 1 - tile_start) >> 4) - tab_first);
-            if (p.context_lens[seq] == len && raw_blk >= 0 && raw_blk < p.num_blocks)
-                T::inject(kv, p, seq, kvh, lane, tile_start, len, bb);
+            const bool at_table = p.context_lens[seq] == len && raw_blk >= 0 && raw_blk < p.num_blocks;
+            const typename T::Fmt::raw* nv = new_row<T>(p.new_value, p, seq, kvh);
+            if constexpr (ROPE) {
+                if (stored && at_table && (int64_t)raw_blk * BS + ((len - 1) & (BS - 1)) == slot)
+                    T::inject(kv, p, k_new[w], nv, kvh, lane, tile_start, len, bb);
+                else if (stored)
+                    store_new_row<T>(p, k_new[w], nv, kvh, slot, lane);
+            } else if (at_table) {
+                T::inject(kv, p, new_row<T>(p.new_key, p, seq, kvh), nv, kvh, lane, tile_start, len, bb);
+            }
         }
         if (tile_start + TT > end)
             T::template process<false, true>(st, kv, qf, kt, ko, p, bb, kvh, lane, tile_start, end, cmul);
@@ -719,7 +814,7 @@ streamk_decode_kernel(StreamKParams p) {
 
     int nt = (int)min((int64_t)(row_tiles - t), g1 - g0);          // tiles of the current segment (>= 1)
     typename T::Q qf, qraw;
-    T::load_q(qraw, p, seq, kvh, lane);
+    T::load_q(qraw, q_rows<T>(p, seq, kvh), G, lane);
     int tab = load_tab(seq, BPT * t);
     typename T::Regs kv;
     // the blocks of a tile out of a table slice held one entry per lane
@@ -762,7 +857,7 @@ streamk_decode_kernel(StreamKParams p) {
         int tabn = 0;
         typename T::Q qn;
         if (has_next) {
-            T::load_q(qraw, p, nseq, nkvh, lane);
+            T::load_q(qraw, q_rows<T>(p, nseq, nkvh), G, lane);
             tabn = load_tab(nseq, 0);
         }
 
@@ -783,7 +878,8 @@ streamk_decode_kernel(StreamKParams p) {
             // (and attends over what the clamped table entry holds, like the unfused sequence of calls).
             const int raw_blk = __builtin_amdgcn_readlane(tab, BPT * k + ((len - 1 - tile_start) >> 4) - tab_first);
             if (p.context_lens[seq] == len && raw_blk >= 0 && raw_blk < p.num_blocks)
-                T::inject(kv, p, seq, kvh, lane, tile_start, len, bb);
+                T::inject(kv, p, new_row<T>(p.new_key, p, seq, kvh), new_row<T>(p.new_value, p, seq, kvh), kvh, lane,
+                          tile_start, len, bb);
         }
         // The segment's last tile always runs the masked body (a full tile simply masks nothing):
         // one prefetching call site, so the prefetched registers need no merging afterwards.
@@ -1083,6 +1179,10 @@ int launch_decode_mfma(const DecodeArgs& a) {
     p.ws_acc = a.ws.acc; p.ws_ml = a.ws.ml;
     p.new_key = a.new_key; p.new_value = a.new_value;
     p.new_token_stride = a.new_token_stride; p.new_head_stride = a.new_head_stride;
+    p.cos_tab = a.cos_tab; p.sin_tab = a.sin_tab; p.tab_stride = a.tab_stride; p.tab_rows = a.tab_rows;
+    p.positions = a.positions; p.slots = a.slots;
+    p.q_token_stride = a.q_token_stride; p.q_head_stride = a.q_head_stride;
+    const bool rope = a.cos_tab != nullptr;
     dim3 grid((unsigned)a.hkv, (unsigned)a.num_parts, (unsigned)a.rows);
     const bool fp8 = a.kv_dtype == AICOMP_KV_FP8_E4M3, d64 = a.d == 64;
     // Eight waves instead of four per workgroup for partitions of more than sixteen tiles in at most one
@@ -1096,8 +1196,10 @@ int launch_decode_mfma(const DecodeArgs& a) {
     const bool wide = a.partition_size > 16 * tile && a.rows * a.hkv * a.num_parts <= 256;
 #define AICOMP_LAUNCH_GRID(...)                                                                                        \
     do {                                                                                                               \
-        if (wide) hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 8>), grid, dim3(512), 0, a.stream, p);     \
-        else hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 4>), grid, dim3(256), 0, a.stream, p);          \
+        if (rope && wide) hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 8, true>), grid, dim3(512), 0, a.stream, p); \
+        else if (rope) hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 4, true>), grid, dim3(256), 0, a.stream, p);    \
+        else if (wide) hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 8, false>), grid, dim3(512), 0, a.stream, p);   \
+        else hipLaunchKernelGGL((paged_decode_mfma_kernel<__VA_ARGS__, 4, false>), grid, dim3(256), 0, a.stream, p);             \
     } while (0)
 #define AICOMP_LAUNCH_GRID16(E)                                                                     \
     do {                                                                                            \

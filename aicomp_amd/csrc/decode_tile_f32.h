@@ -55,10 +55,9 @@ struct TileF32 {
         return i * 1024 + o.wr + (o.cb ^ (((RPL * i) & 15) << 4));
     }
 
-    template <typename Params>
-    __device__ __forceinline__ static void load_q(Q& q, const Params& p, int seq, int kvh, int lane) {
+    __device__ __forceinline__ static void load_q(Q& q, const float* rows, int group, int lane) {
         const int r16 = lane & 15, g4 = lane >> 4;
-        const float* row = (const float*)p.query + ((int64_t)seq * p.hq + kvh * p.group + min(r16, p.group - 1)) * DQ + 4 * g4;
+        const float* row = rows + min(r16, group - 1) * DQ + 4 * g4;
 #pragma unroll
         for (int s = 0; s < DQ / 16; ++s) q.r[s] = *(const float4*)(row + 16 * s);
     }
@@ -172,12 +171,10 @@ struct TileF32 {
     // fused append (see inject_new_row): the lanes that loaded the newest token's chunks take the new
     // row's instead and write them to the pools
     template <typename Params>
-    __device__ __forceinline__ static void inject(Regs& t, const Params& p, int seq, int kvh, int lane, int tile_start,
-                                                  int len, const int64_t (&bb)[4]) {
+    __device__ __forceinline__ static void inject(Regs& t, const Params& p, const float* key, const float* value, int kvh,
+                                                  int lane, int tile_start, int len, const int64_t (&bb)[4]) {
         const int tau = len - 1 - tile_start;                            // wave-uniform
-        const int64_t src = (int64_t)seq * p.new_token_stride + (int64_t)kvh * p.new_head_stride;
-        const uint4* nk = (const uint4*)((const float*)p.new_key + src);
-        const uint4* nv = (const uint4*)((const float*)p.new_value + src);
+        const uint4 *nk = (const uint4*)key, *nv = (const uint4*)value;
         const int64_t dst = ((bb[tau >> 4] * p.hkv + kvh) * BS + (tau & 15)) * (DQ / 4);
         constexpr int RPL = 1024 / ROWB;                                 // tile rows per load
         const int row0 = DQ == 128 ? lane >> 5 : lane >> 4, chunk = DQ == 128 ? lane & 31 : lane & 15;

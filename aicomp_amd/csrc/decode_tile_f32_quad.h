@@ -66,10 +66,9 @@ struct TileF32Quad {
         return i * 1024 + o.wr + (o.cb ^ (swz << 4));
     }
 
-    template <typename Params>
-    __device__ __forceinline__ static void load_q(Q& q, const Params& p, int seq, int kvh, int lane) {
-        const int part = DQ == 64 ? lane >> 5 : lane >> 4, h = min(lane & 3, p.group - 1);
-        const float* row = (const float*)p.query + ((int64_t)seq * p.hq + kvh * p.group + h) * DQ + 32 * part;
+    __device__ __forceinline__ static void load_q(Q& q, const float* rows, int group, int lane) {
+        const int part = DQ == 64 ? lane >> 5 : lane >> 4;
+        const float* row = rows + min(lane & 3, group - 1) * DQ + 32 * part;
 #pragma unroll
         for (int c = 0; c < 8; ++c) q.r[c] = *(const f32x4_t*)(row + 4 * c);
     }
@@ -190,15 +189,13 @@ struct TileF32Quad {
     // fused append (see inject_new_row): the lanes that loaded the newest token's chunks take the new
     // row's instead and write them to the pools
     template <typename Params>
-    __device__ __forceinline__ static void inject(Regs& t, const Params& p, int seq, int kvh, int lane, int tile_start,
-                                                  int len, const int64_t (&bb)[4]) {
+    __device__ __forceinline__ static void inject(Regs& t, const Params& p, const float* key, const float* value, int kvh,
+                                                  int lane, int tile_start, int len, const int64_t (&bb)[4]) {
         const int tau = len - 1 - tile_start;                            // wave-uniform
-        const int64_t src = (int64_t)seq * p.new_token_stride + (int64_t)kvh * p.new_head_stride;
         const int64_t dst = ((bb[tau >> 4] * p.hkv + kvh) * BS + (tau & 15)) * (DQ / 4);
         const int chunk = lane & (DQ / 4 - 1);
         const bool mine = lane / (DQ / 4) == tau % RPL;
-        const uint4 k4 = ((const uint4*)((const float*)p.new_key + src))[chunk];
-        const uint4 v4 = ((const uint4*)((const float*)p.new_value + src))[chunk];
+        const uint4 k4 = ((const uint4*)key)[chunk], v4 = ((const uint4*)value)[chunk];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (mine && i == tau / RPL) { t.k[i] = k4; t.v[i] = v4; }

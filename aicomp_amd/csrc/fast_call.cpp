@@ -24,6 +24,8 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <hip/hip_runtime_api.h>
+
 #include <algorithm>
 #include <climits>
 #include <map>
@@ -392,6 +394,80 @@ PyObject* paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     }
 }
 
+// The table columns that `lens` tokens (a contiguous int32 buffer of n lengths) take, at most `columns`; all of
+// them without such a buffer, and for a launch that is being recorded.
+int columns_in_use(PyObject* lens, int64_t n, int bs, int64_t columns, void* stream) {
+    if (lens == Py_None) return (int)columns;
+    Py_buffer b;
+    if (PyObject_GetBuffer(lens, &b, PyBUF_FORMAT | PyBUF_ND) != 0) { PyErr_Clear(); return (int)columns; }
+    int64_t longest = columns * bs;
+    if (b.itemsize == 4 && b.ndim == 1 && b.shape[0] == n && b.format && b.format[0] == 'i' && b.format[1] == 0) {
+        longest = 1;
+        for (int64_t i = 0; i < n; ++i) longest = std::max<int64_t>(longest, ((const int32_t*)b.buf)[i]);
+    }
+    PyBuffer_Release(&b);
+    const int64_t used = std::min<int64_t>(columns, (longest + bs - 1) / bs);
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (used < columns && (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone))
+        return (int)columns;
+    return (int)used;
+}
+
+// (the output comes back as a new tensor; None: not a plain call of the one launch, nothing done)
+PyObject* rope_paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        Pools p;
+        double scale;
+        if (nargs != 15)
+            FAIL("rope_paged_decode_attn(query, key, value, cos, sin, positions, k_pool, v_pool, slot_mapping, block_table, "
+                 "context_lens, host_lens, scale, k_scale, v_scale)");
+        const at::Tensor *q = plain(args[0]), *key = plain(args[1]), *value = plain(args[2]), *cos = plain(args[3]),
+                         *sin = plain(args[4]), *pos = plain(args[5]), *slots = plain(args[8]), *table = plain(args[9]),
+                         *ctx = plain(args[10]);
+        if (!q || !key || !value || !cos || !sin || !pos || !slots || !table || !ctx || !p.get(args[6], args[7]) ||
+            !as_double(args[12], scale) || q->dim() != 3 || key->dim() != 3 ||
+            value->sizes() != key->sizes())
+            Py_RETURN_NONE;
+        const int64_t B = q->size(0);
+        const at::ScalarType st = q->scalar_type();
+        const int dt = dtype_code(st);
+        if (B == 0 || B > INT_MAX || dt < 0 || key->size(0) != B || key->size(1) != p.hkv || key->size(2) != p.d ||
+            q->size(2) != p.d || key->scalar_type() != st || value->scalar_type() != st || q->stride(2) != 1 ||
+            key->stride(2) != 1 || key->strides() != value->strides() || cos->dim() != 2 || cos->size(1) != p.d ||
+            sin->sizes() != cos->sizes() || cos->scalar_type() != st || sin->scalar_type() != st || cos->stride(1) != 1 ||
+            cos->strides() != sin->strides() || table->scalar_type() != at::kInt || table->dim() != 2 ||
+            p.bs <= 0 || table->size(0) != B || table->stride(1) != 1 || table->size(1) <= 0 || table->size(1) > INT_MAX ||
+            !vector_of(pos, at::kLong, B, *q) || !vector_of(slots, at::kLong, B, *q) || !vector_of(ctx, at::kInt, B, *q) ||
+            !on(*table, *q) || !on(*key, *q) || !on(*value, *q) || !on(*cos, *q) || !on(*sin, *q) || !on(*p.k, *q) ||
+            (p.dt != dt && p.dt != AICOMP_KV_FP8_E4M3) || !p.scales(args[13], args[14]))
+            Py_RETURN_NONE;
+        const int hq = (int)q->size(1);
+        const c10::DeviceGuard guard(q->device());
+        void* stream = stream_of(*q);
+        const int width = columns_in_use(args[11], B, p.bs, table->size(1), stream);
+        at::Tensor scratch;
+        const size_t need = aicomp_paged_decode_workspace_bytes((int)B, hq, p.hkv, p.d, p.bs, width, dt, p.dt, 0);
+        if (need) scratch = cached_scratch(q->device(), stream, need);
+        at::Tensor out(at::detail::empty_cuda(q->sizes(), st, q->device(), c10::MemoryFormat::Contiguous));
+        const int rc = unlocked([&] {
+            std::unique_lock<std::mutex> one_at_a_time(scratch_launches(), std::defer_lock);
+            if (need) one_at_a_time.lock();
+            return aicomp_rope_paged_decode_attn(
+                out.data_ptr(), q->data_ptr(), q->stride(0), q->stride(1), key->data_ptr(), value->data_ptr(), key->stride(0),
+                key->stride(1), cos->data_ptr(), sin->data_ptr(), cos->stride(0), cos->size(0),
+                (const int64_t*)pos->data_ptr(), (const int64_t*)slots->data_ptr(), p.k->data_ptr(), p.v->data_ptr(),
+                (const int32_t*)table->data_ptr(), table->stride(0), (const int32_t*)ctx->data_ptr(), (int)B, hq, p.hkv, p.d,
+                p.bs, width, p.nb, (float)scale, dt, p.dt, p.ks, p.vs, need ? scratch.data_ptr() : nullptr,
+                need ? (size_t)scratch.numel() : 0, stream);
+        });
+        if (rc == AICOMP_KV_EUNSUPPORTED) Py_RETURN_NONE;
+        if (rc != AICOMP_KV_OK) FAIL("aicomp_kv error %d: %s", rc, aicomp_kv_last_error());
+        return THPVariable_Wrap(std::move(out));
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
 PyObject* paged_prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     try {
         Pools p;
@@ -473,6 +549,7 @@ PyMethodDef methods[] = {
     {"kv_append", FAST(kv_append), "ops.kv_append of a plain call: True once launched, False if it is not one"},
     {"rope_kv_append", FAST(rope_kv_append), "ops.rope_kv_append of a plain call, out given"},
     {"paged_decode_attn", FAST(paged_decode_attn), "ops.paged_decode_attn of a plain call"},
+    {"rope_paged_decode_attn", FAST(rope_paged_decode_attn), "a layer's decode step in one launch: the output, or None if it is not one"},
     {"paged_prefill_attn", FAST(paged_prefill_attn), "ops.paged_prefill_attn of a plain call, max_q_len given"},
     {"sample_tokens", FAST(sample_tokens), "ops.sample_tokens of a plain call: the tokens, or None if it is not one"},
     {nullptr, nullptr, 0, nullptr}};

@@ -71,6 +71,12 @@ class PagedAttentionBackend:
             raise RuntimeError("PagedAttentionBackend.attend called outside a step (begin_step first)")
         kp, vp = self.k_pools[layer_idx], self.v_pools[layer_idx]
         ks, vs = self.k_scales[layer_idx], self.v_scales[layer_idx]
+        if self.cos is not None and plan.num_prefill_seqs == 0:          # one token per sequence: one launch, if it can be
+            out = ops.rope_paged_decode_attn(query, key, value, self.cos, self.sin, plan.positions, kp, vp,
+                                             plan.slot_mapping, plan.block_table, plan.context_lens,
+                                             plan.host_context_lens, self.scale, ks, vs)
+            if out is not None:
+                return out
         out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
         if self.cos is None:
             from .block_manager import paged_attention_step

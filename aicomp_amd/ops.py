@@ -427,6 +427,26 @@ def step_items(context_lens, new_lens, num_prefill_seqs: int, tile_positions: in
     return np.concatenate([dec[:per_round], pre[:per_round], rest, a[k:], b[k:]]).astype(np.int32)
 
 
+def rope_paged_decode_attn(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                           positions: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, slot_mapping: torch.Tensor,
+                           block_table: torch.Tensor, context_lens: torch.Tensor, host_lens, scale: float,
+                           k_scale: Optional[torch.Tensor] = None,
+                           v_scale: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``rope_kv_append`` of one new token per sequence and ``paged_decode_attn`` with its rotated query, in one launch:
+    the attention output ``[B, Hq, D]``, bit for bit that of the two calls, or ``None`` (nothing done) where the two are to be
+    made: a batch for the balanced schedule, and whatever is not a plain call.
+
+    ``host_lens``: the same lengths on the host (a contiguous int32 numpy array), or ``None``.  With them the call is sized
+    for the table columns in use and not for the longest sequence the table could hold, so that rows that are short
+    now are whole in one launch; a launch recorded into a graph, whose lengths may grow, is sized for the whole table.
+    """
+    if not (_native("aicomp_rope_paged_decode_attn") and _lib.untouched("aicomp_rope_kv_append")
+            and _lib.untouched("aicomp_paged_decode_attn")):
+        return None
+    return _FAST.rope_paged_decode_attn(query, key, value, cos, sin, positions, k_pool, v_pool, slot_mapping, block_table,
+                                        context_lens, host_lens, scale, k_scale, v_scale)
+
+
 def paged_prefill_attn(out: torch.Tensor, query: torch.Tensor, k_pool: torch.Tensor,
                        v_pool: torch.Tensor, block_table: torch.Tensor,
                        context_lens: torch.Tensor, cu_q_lens: torch.Tensor, scale: float,

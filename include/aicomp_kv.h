@@ -182,6 +182,39 @@ int aicomp_paged_decode_attn_append(void* out, const void* query,
                                     void* stream);
 
 /*
+ * A layer's whole decode step in one main kernel: rotary embedding of the query rows and of
+ * the new K row, append of the new rows, attention.
+ *
+ *   query               [B, Hq, D] of q_dtype as projected, element (b,h,d) at
+ *                       b*q_token_stride + h*q_head_stride + d; new_key, new_value as in
+ *                       aicomp_paged_decode_attn_append
+ *   cos, sin, table_stride, table_rows, positions, slot_mapping
+ *                       as in aicomp_rope_kv_append, one entry per row b
+ * The result equals aicomp_rope_kv_append of the rows followed by aicomp_paged_decode_attn on
+ * the rotated query, bit for bit; a row whose position has no table row is not stored and its
+ * output row is unspecified.  Covers small calls of the matrix-core kernels (what
+ * aicomp_kv_set_small_decode_tokens says of batch * max_blocks_per_seq * block_size), rows that can be
+ * read 16 bytes at a time; any other call is AICOMP_KV_EUNSUPPORTED with nothing done.  Scratch:
+ * aicomp_paged_decode_workspace_bytes with partition_size 0.
+ */
+int aicomp_rope_paged_decode_attn(void* out, const void* query,
+                                  int64_t q_token_stride, int64_t q_head_stride,
+                                  const void* new_key, const void* new_value,
+                                  int64_t kv_token_stride, int64_t kv_head_stride,
+                                  const void* cos, const void* sin,
+                                  int64_t table_stride, int64_t table_rows,
+                                  const int64_t* positions, const int64_t* slot_mapping,
+                                  void* k_pool, void* v_pool,
+                                  const int32_t* block_table, int64_t block_table_stride,
+                                  const int32_t* context_lens,
+                                  int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                  int block_size, int max_blocks_per_seq, int64_t num_blocks,
+                                  float scale, int q_dtype, int kv_dtype,
+                                  const float* k_scale, const float* v_scale,
+                                  void* workspace, size_t workspace_bytes,
+                                  void* stream);
+
+/*
  * aicomp_paged_decode_attn_append for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  It has no
  * counterpart in the reference.  Same arguments, results and bit patterns as

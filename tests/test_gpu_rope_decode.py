@@ -1,0 +1,107 @@
+"""A layer's decode step in one launch (rotary embedding, append, attention) against the two calls it stands for: the
+same bits in the output and in the pools."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from aicomp_amd import _lib, ops
+
+pytestmark = [pytest.mark.gpu, pytest.mark.routing("library")]
+CTX = [1, 2, 16, 17, 31, 32, 33, 63, 64, 65, 128, 129, 300, 7]
+
+
+def _case(device, dtype, kv, hq, hkv, d, ctx, seed):
+    g = torch.Generator().manual_seed(seed)
+    B, need = len(ctx), [-(-n // 16) for n in ctx]
+    nb = sum(need) + 3
+    table, perm, at = torch.zeros(B, max(need) + 2, dtype=torch.int32), torch.randperm(nb, generator=g), 0
+    for s, n in enumerate(need):
+        table[s, :n] = perm[at:at + n].to(torch.int32)
+        at += n
+    pools, scales = [], [None, None]
+    for i in range(2):
+        x = torch.randn(nb, hkv, 16, d, generator=g) * 0.5
+        if kv == torch.float8_e4m3fn:
+            scales[i] = torch.full((hkv,), 2.75 / 448).to(device)
+            x = (x / (2.75 / 448)).clamp(-448, 448)
+        pools.append(x.to(kv).to(device))
+    qkv = (torch.randn(B, hq + 2 * hkv, d, generator=g) * 0.7).to(dtype).to(device)
+    cos, sin = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, d, 2) / d).to(device), 512, dtype)
+    lens = np.asarray(ctx, dtype=np.int32)
+    slots = torch.tensor([int(table[s, (n - 1) // 16]) * 16 + (n - 1) % 16 for s, n in enumerate(ctx)])
+    return dict(q=qkv[:, :hq], k=qkv[:, hq:hq + hkv], v=qkv[:, hq + hkv:], cos=cos, sin=sin,
+                pos=torch.tensor([n - 1 for n in ctx]).to(device), slots=slots.to(device), table=table.to(device),
+                ctx=torch.from_numpy(lens).to(device), lens=lens, pools=pools, scales=scales, scale=1 / math.sqrt(d))
+
+
+def _bits(t):
+    return t.view({1: torch.uint8, 2: torch.int16, 4: torch.int32}[t.element_size()])
+
+
+def _one(c, lens):
+    kp, vp = (p.clone() for p in c["pools"])
+    out = ops.rope_paged_decode_attn(c["q"], c["k"], c["v"], c["cos"], c["sin"], c["pos"], kp, vp, c["slots"], c["table"],
+                                     c["ctx"], lens, c["scale"], *c["scales"])
+    return out, kp, vp
+
+
+def _two(c, width):
+    kp, vp = (p.clone() for p in c["pools"])
+    q, out = torch.empty_like(c["q"].contiguous()), torch.empty_like(c["q"].contiguous())
+    ops.rope_kv_append(c["q"], c["k"], c["v"], c["cos"], c["sin"], c["pos"], kp, vp, c["slots"], *c["scales"], query_out=q)
+    ops.paged_decode_attn(out, q, kp, vp, c["table"][:, :width], c["ctx"], c["scale"], *c["scales"])
+    return out, kp, vp
+
+
+KINDS = [(torch.bfloat16, None), (torch.float16, None), (torch.float32, None), (torch.bfloat16, torch.float8_e4m3fn),
+         (torch.float16, torch.float8_e4m3fn)]
+
+
+@pytest.mark.parametrize("dtype,kv", KINDS)
+@pytest.mark.parametrize("hq,hkv,d", [(4, 4, 64), (8, 2, 64), (16, 2, 64), (8, 2, 128), (10, 2, 128), (32, 2, 128)])
+def test_one_launch_equals_two(device, decode_routing, dtype, kv, hq, hkv, d):
+    c = _case(device, dtype, kv or dtype, hq, hkv, d, CTX, hq + d)
+    for lens, width in ((c["lens"], 19), (None, c["table"].shape[1])):
+        for got, want in zip(_one(c, lens), _two(c, width)):
+            assert torch.equal(_bits(got), _bits(want)), (width,)
+
+
+@pytest.mark.parametrize("dtype,kv,d", [(torch.bfloat16, None, 64), (torch.float32, None, 128), (torch.float16, torch.float8_e4m3fn, 128)])
+def test_split_rows_and_odd_slots(device, decode_routing, dtype, kv, d):
+    """Rows of several partitions; a padding row, a row stored elsewhere, one without a table row, an empty one."""
+    c = _case(device, dtype, kv or dtype, 8, 2, d, [1500, 1, 800, 257, 40, 33], 3)
+    c["cos"], c["sin"] = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, d, 2) / d).to(device), 1600, dtype)
+    for got, want in zip(_one(c, c["lens"]), _two(c, 94)):
+        assert torch.equal(_bits(got), _bits(want))
+    used = set(c["table"][:, :94].flatten().tolist())
+    spare = next(b for b in range(c["pools"][0].shape[0]) if b not in used)
+    c["slots"][1], c["slots"][2], c["pos"][3] = -1, spare * 16 + 5, 5000
+    c["ctx"][4] = 0
+    got, want = _one(c, c["lens"]), _two(c, 94)
+    rows = [0, 1, 2, 4, 5]
+    assert torch.equal(_bits(got[0][rows]), _bits(want[0][rows]))
+    assert torch.equal(_bits(got[1]), _bits(want[1])) and torch.equal(_bits(got[2]), _bits(want[2]))
+
+
+def test_what_it_declines(device, decode_routing):
+    """Batches for the balanced schedule, other head dims, rows that cannot be read in vectors: None, and nothing written."""
+    c = _case(device, torch.bfloat16, torch.bfloat16, 8, 2, 64, CTX, 1)
+    prev = ops.set_small_decode_tokens(0)
+    try:
+        assert _one(c, c["lens"])[0] is None
+    finally:
+        ops.set_small_decode_tokens(prev)
+    odd = torch.empty(c["q"].numel() + 1, dtype=torch.bfloat16, device=device)[1:].view(c["q"].shape)
+    odd.copy_(c["q"])
+    c["q"] = odd
+    out, kp, vp = _one(c, c["lens"])
+    assert out is None and torch.equal(_bits(kp), _bits(c["pools"][0])) and torch.equal(_bits(vp), _bits(c["pools"][1]))
+    w = _case(device, torch.bfloat16, torch.bfloat16, 4, 2, 256, [5, 20], 2)
+    assert _one(w, w["lens"])[0] is None
+    w["table"] = w["table"].long()
+    assert _one(w, w["lens"])[0] is None
+    lib = _lib.load()
+    assert lib.aicomp_rope_paged_decode_attn(*([None] * 2), 0, 0, None, None, 0, 0, None, None, 0, 0, *([None] * 5), 0, None, 1,
+                                             4, 2, 64, 16, 1, 4, 1.0, 1, 1, None, None, None, 0, None) == 1

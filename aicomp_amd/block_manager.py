@@ -37,6 +37,11 @@ from typing import Deque, Dict, Iterable, List, Optional
 import numpy as np
 import torch
 
+try:
+    from . import _aicomp_fast as _FAST
+except ImportError:
+    _FAST = None
+
 
 class OutOfBlocks(ValueError):
     """The pool has fewer free blocks than the request needs (the reference's cache
@@ -297,6 +302,7 @@ class _Staging:
         # typed views of the device buffers, made once: a plan's tensors are then one slice each
         self.dev32 = [d[:nbytes // 8 * 8].view(torch.int32) for d in self.dev]
         self.dev64 = [d[:nbytes // 8 * 8].view(torch.int64) for d in self.dev]
+        self.host_np = [h.numpy() for h in self.host]
         self.done = [torch.cuda.Event() if self.cuda else None for _ in range(depth)]
         self.used = [False] * depth
         self.i = 0
@@ -311,9 +317,12 @@ class _Staging:
     def upload(self, i: int, nbytes: int) -> int:
         if self.cuda:
             self.dev[i][:nbytes].copy_(self.host[i][:nbytes], non_blocking=True)
-            self.done[i].record()
-            self.used[i] = True
+            self.uploaded(i)
         return i
+
+    def uploaded(self, i: int) -> None:
+        self.done[i].record()
+        self.used[i] = True
 
 
 class StepPlanner:
@@ -376,6 +385,7 @@ class StepPlanner:
         self._maxnew = np.zeros(max_seqs, dtype=np.int64)     # -1: unbounded
         self._arr = np.zeros(max_seqs, dtype=np.int64)
         self._live = np.zeros(max_seqs, dtype=bool)
+        self._row_state = (self._live, self._len, self._prompt, self._orig, self._nblk, self._maxnew, self._arr)
         # packed layout (bytes): slot_mapping int64 [T] | positions int64 [T] | block_table int32 [S*MB] |
         # context_lens [S] | cu_q_lens [S+1]
         cap = 16 * max_num_batched_tokens + 4 * (max_seqs * MB + 2 * max_seqs + 1) + 64
@@ -433,6 +443,9 @@ class StepPlanner:
 
     def completed(self) -> List[object]:
         """Running sequences that have produced their ``max_new_tokens``; the caller finishes them."""
+        rows = None if _FAST is None else _FAST.rows_done(*self._row_state)
+        if rows is not None:
+            return [self._id_of[r] for r in rows]
         rows = np.flatnonzero(self._live & (self._maxnew >= 0) & (self._len >= self._prompt) &
                               (self._len - self._orig + 1 >= self._maxnew))
         return [self._id_of[r] for r in rows]
@@ -474,6 +487,11 @@ class StepPlanner:
         """Plan one step.  ``decode`` restricts which running sequences may take their one
         token this step (default: all of them); a driver that ingests a whole batch of prompts
         before its first decode step passes ``()`` until the last prompt is in."""
+        if (_FAST is not None and decode is None and not self.waiting and not self.check_plans
+                and type(self.alloc) is BlockAllocator):
+            plan = self._plan_decode()
+            if plan is not None:
+                return plan
         budget = self.max_num_batched_tokens
         BS = self.block_size
         preempted: List[object] = []
@@ -567,6 +585,32 @@ class StepPlanner:
         lens = np.concatenate([np.asarray([n for _, n in multi], dtype=np.int32),
                                np.ones(dec.size + ones.size, dtype=np.int32)])
         return self._pack(rows, lens, len(multi), preempted)
+
+    def _plan_decode(self) -> Optional[StepPlan]:
+        """A step of one token per running sequence (no prompt to ingest, blocks for all), selected and packed natively;
+        ``None``, nothing changed, for any other step."""
+        st, alloc, MB = self._staging, self.alloc, self.max_blocks_per_seq
+        i = st.next()
+        got = _FAST.plan_decode(*self._row_state, self._tab, alloc._free, alloc._owned, alloc._top, self.block_size,
+                                self.max_seq_len, self.max_num_batched_tokens, st.host_np[i])
+        if got is None:
+            st.i = i
+            return None
+        rows, taken = got
+        alloc._top -= taken
+        S = len(rows)
+        table, lens, cu, slots, positions = _FAST.plan_upload(st.host[i], st.dev[i], st.dev32[i], st.dev64[i], S, MB)
+        if st.cuda:
+            st.uploaded(i)
+        c = 16 * S + 4 * S * MB                          # (the layout of _pack)
+        host = st.host_np[i][:c + 4 * (2 * S + 1)].copy()
+        ids = self._id_of
+        return StepPlan(
+            seq_ids=[ids[r] for r in rows], num_prefill_seqs=0, new_lens=np.ones(S, dtype=np.int32), max_q_len=0,
+            total_new_tokens=S, block_table=table, context_lens=lens, cu_q_lens=cu, slot_mapping=slots, positions=positions,
+            preempted=[], host_block_table=host[16 * S:c].view(np.int32).reshape(S, MB),
+            host_context_lens=host[c:c + 4 * S].view(np.int32), host_cu_q_lens=host[c + 4 * S:].view(np.int32),
+            host_slot_mapping=host[:8 * S].view(np.int64), host_positions=host[8 * S:16 * S].view(np.int64))
 
     def _pack(self, rows: np.ndarray, new_lens: np.ndarray, npre: int, preempted: List[object]) -> StepPlan:
         S, MB, BS = int(rows.size), self.max_blocks_per_seq, self.block_size

@@ -29,6 +29,7 @@
 #include <algorithm>
 #include <climits>
 #include <map>
+#include <vector>
 #include <mutex>
 #include <utility>
 
@@ -539,6 +540,149 @@ PyObject* sample_tokens(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
 }
 
+// ---------------------------------------------------------------- the step planner's decode step
+// What StepPlanner.schedule and _pack do with about forty numpy operations of a microsecond each, for a step that is one
+// token per running sequence and nothing else: 52 us of host time at 8 sequences, of which these functions leave 20
+// (most of that the copy's own call, its event and the plan's tensors).
+
+// A contiguous buffer of at least n elements of `size` bytes, released with the object; null data where it is not one.
+struct Buf {
+    Py_buffer b{};
+    bool held = false;
+    void* data(PyObject* o, Py_ssize_t size, int64_t n, bool writable = false) {
+        held = PyObject_GetBuffer(o, &b, PyBUF_ND | (writable ? PyBUF_WRITABLE : 0)) == 0;
+        if (!held) { PyErr_Clear(); return nullptr; }
+        return b.itemsize == size && b.len >= size * n ? b.buf : nullptr;
+    }
+    int64_t items() const { return held && b.itemsize ? (int64_t)(b.len / b.itemsize) : 0; }
+    ~Buf() { if (held) PyBuffer_Release(&b); }
+};
+
+// per row of the planner: live (bool), len, prompt, orig, nblk (int32), maxnew, arrival (int64)
+struct Rows {
+    Buf b[7];
+    int64_t n = 0;
+    const uint8_t* live;
+    int32_t *len, *nblk;
+    const int32_t *prompt, *orig;
+    const int64_t *maxnew, *arrival;
+    bool get(PyObject* const* a, bool writable) {
+        live = (const uint8_t*)b[0].data(a[0], 1, 0);
+        n = b[0].items();
+        len = (int32_t*)b[1].data(a[1], 4, n, writable);
+        prompt = (const int32_t*)b[2].data(a[2], 4, n);
+        orig = (const int32_t*)b[3].data(a[3], 4, n);
+        nblk = (int32_t*)b[4].data(a[4], 4, n, writable);
+        maxnew = (const int64_t*)b[5].data(a[5], 8, n);
+        arrival = (const int64_t*)b[6].data(a[6], 8, n);
+        return live && len && prompt && orig && nblk && maxnew && arrival;
+    }
+    int64_t generated(int64_t r) const { return (int64_t)len[r] - orig[r] + 1; }
+};
+
+PyObject* rows_done(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    Rows R;
+    if (nargs != 7) FAIL("rows_done(live, len, prompt, orig, nblk, maxnew, arrival)");
+    if (!R.get(args, false)) Py_RETURN_NONE;
+    PyObject* out = PyList_New(0);
+    for (int64_t r = 0; out && r < R.n; ++r) {
+        if (!R.live[r] || R.maxnew[r] < 0 || R.len[r] < R.prompt[r] || R.generated(r) < R.maxnew[r]) continue;
+        PyObject* i = PyLong_FromLongLong(r);
+        if (!i || PyList_Append(out, i) != 0) Py_CLEAR(out);
+        Py_XDECREF(i);
+    }
+    return out;
+}
+
+// -> (rows in plan order, blocks taken), the plan packed into `raw` and the rows' state moved on; None with nothing
+// changed where the step is another one (a prompt to ingest, no free block, a sequence too long, nothing to do).
+PyObject* plan_decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 15)
+        FAIL("plan_decode(live, len, prompt, orig, nblk, maxnew, arrival, table, free, owned, top, block_size, max_seq_len, "
+             "budget, raw)");
+    Rows R;
+    int top, bs, longest, budget;
+    if (!R.get(args, true) || !as_int(args[10], top) || !as_int(args[11], bs) || !as_int(args[12], longest) ||
+        !as_int(args[13], budget) || bs <= 0 || R.n == 0)
+        Py_RETURN_NONE;
+    Buf bt, bf, bo, br;
+    int32_t* table = (int32_t*)bt.data(args[7], 4, R.n, true);
+    const int32_t* free_ids = (const int32_t*)bf.data(args[8], 4, 0);
+    uint8_t* owned = (uint8_t*)bo.data(args[9], 1, 0, true);
+    uint8_t* raw = (uint8_t*)br.data(args[14], 1, 0, true);
+    if (!table || !free_ids || !owned || !raw || top < 0 || top > bf.items() || (uintptr_t)raw % 8) Py_RETURN_NONE;
+    const int64_t MB = bt.items() / R.n;
+    try {
+        std::vector<int> rows;
+        for (int64_t r = 0; r < R.n; ++r) {
+            if (!R.live[r]) continue;
+            if (R.len[r] < R.prompt[r]) Py_RETURN_NONE;
+            if (R.maxnew[r] < 0 || R.generated(r) < R.maxnew[r]) rows.push_back((int)r);
+        }
+        std::stable_sort(rows.begin(), rows.end(), [&](int a, int b) { return R.arrival[a] < R.arrival[b]; });
+        if ((int64_t)rows.size() > budget) rows.resize(std::max(budget, 0));
+        const int64_t S = (int64_t)rows.size(), end = 16 * S + 4 * (S * MB + 2 * S + 1);
+        int taken = 0;
+        for (int r : rows) {
+            if (R.len[r] + 1 > longest || R.len[r] < 0 || R.len[r] / bs >= MB || R.nblk[r] < 0 || R.nblk[r] > MB) Py_RETURN_NONE;
+            const bool opens = (int64_t)R.nblk[r] * bs == R.len[r];
+            if (!opens && R.len[r] / bs >= R.nblk[r]) Py_RETURN_NONE;
+            taken += opens;
+        }
+        if (S == 0 || taken > top || end > br.items()) Py_RETURN_NONE;
+        for (int i = 0; i < taken; ++i)
+            if (free_ids[top - 1 - i] < 0 || free_ids[top - 1 - i] >= bo.items()) Py_RETURN_NONE;
+        PyObject* ids = PyList_New(S);
+        if (!ids) return nullptr;
+        int64_t* slot = (int64_t*)raw;
+        int64_t* pos = slot + S;
+        int32_t* tab = (int32_t*)(pos + S);
+        int32_t *ctx = tab + S * MB, *cu = ctx + S;
+        cu[0] = 0;
+        int next = top;
+        for (int64_t i = 0; i < S; ++i) {
+            const int r = rows[i];
+            int32_t* mine = table + (int64_t)r * MB;
+            const int32_t p = R.len[r];
+            if ((int64_t)R.nblk[r] * bs == p) {
+                const int32_t blk = free_ids[--next];
+                owned[blk] = 1;
+                mine[R.nblk[r]++] = blk;
+            }
+            std::copy(mine, mine + MB, tab + i * MB);
+            slot[i] = (int64_t)mine[p / bs] * bs + p % bs;
+            pos[i] = p;
+            ctx[i] = R.len[r] = p + 1;
+            cu[i + 1] = (int32_t)(i + 1);
+            PyList_SET_ITEM(ids, i, PyLong_FromLong(r));
+        }
+        return Py_BuildValue("(Ni)", ids, taken);
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
+// The packed plan's copy to the device, and its five tensors there: block_table, context_lens, cu_q_lens, slot_mapping,
+// positions of a step of one token per sequence.
+PyObject* plan_upload(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        int S, MB;
+        if (nargs != 6) FAIL("plan_upload(host, device, device as int32, device as int64, sequences, table width)");
+        for (int i = 0; i < 4; ++i)
+            if (!THPVariable_Check(args[i])) FAIL("plan_upload: argument %d is not a tensor", i);
+        if (!as_int(args[4], S) || !as_int(args[5], MB) || S <= 0 || MB < 0) FAIL("plan_upload: bad sizes");
+        const at::Tensor &host = THPVariable_Unpack(args[0]), &dev = THPVariable_Unpack(args[1]);
+        const at::Tensor &d32 = THPVariable_Unpack(args[2]), &d64 = THPVariable_Unpack(args[3]);
+        const int64_t t = 4 * (int64_t)S, c = t + (int64_t)S * MB, end = 4 * (c + 2 * (int64_t)S + 1);
+        if (!dev.is_same(host)) dev.narrow(0, 0, end).copy_(host.narrow(0, 0, end), /*non_blocking=*/true);
+        return Py_BuildValue("(NNNNN)", THPVariable_Wrap(d32.narrow(0, t, c - t).view({S, MB})),
+                             THPVariable_Wrap(d32.narrow(0, c, S)), THPVariable_Wrap(d32.narrow(0, c + S, S + 1)),
+                             THPVariable_Wrap(d64.narrow(0, 0, S)), THPVariable_Wrap(d64.narrow(0, S, S)));
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
 #define FAST(f) (PyCFunction)(void (*)(void))f, METH_FASTCALL
 
 PyMethodDef methods[] = {
@@ -550,6 +694,9 @@ PyMethodDef methods[] = {
     {"rope_kv_append", FAST(rope_kv_append), "ops.rope_kv_append of a plain call, out given"},
     {"paged_decode_attn", FAST(paged_decode_attn), "ops.paged_decode_attn of a plain call"},
     {"rope_paged_decode_attn", FAST(rope_paged_decode_attn), "a layer's decode step in one launch: the output, or None if it is not one"},
+    {"rows_done", FAST(rows_done), "planner rows that have produced their tokens"},
+    {"plan_decode", FAST(plan_decode), "a step of one token per running sequence, packed: (rows, blocks taken), or None"},
+    {"plan_upload", FAST(plan_upload), "the packed plan on its way to the device: its five tensors there"},
     {"paged_prefill_attn", FAST(paged_prefill_attn), "ops.paged_prefill_attn of a plain call, max_q_len given"},
     {"sample_tokens", FAST(sample_tokens), "ops.sample_tokens of a plain call: the tokens, or None if it is not one"},
     {nullptr, nullptr, 0, nullptr}};

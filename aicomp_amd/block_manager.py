@@ -690,10 +690,9 @@ def paged_attention_step(plan: StepPlan, out: torch.Tensor, query: torch.Tensor,
                                       v_scale=v_scale, items=items)
     if plan.only_chunks and t_pre == query.shape[0] == out.shape[0] == key.shape[0] == value.shape[0]:
         # chunks alone: the tensors as they are (a slice costs a microsecond)
-        ops.kv_append(key, value, k_pool, v_pool, plan.slot_mapping, k_scale, v_scale)
-        return ops.paged_prefill_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens, plan.cu_q_lens,
-                                      scale, max_q_len=plan.max_q_len, k_scale=k_scale, v_scale=v_scale,
-                                      items=plan.prefill_items(query, k_pool))
+        return ops.append_prefill_attn(out, query, key, value, k_pool, v_pool, plan.slot_mapping, plan.block_table,
+                                       plan.context_lens, plan.cu_q_lens, scale, plan.max_q_len, k_scale, v_scale,
+                                       plan.prefill_items(query, k_pool))
     if S and npre == 0:
         return ops.paged_decode_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens, scale, k_scale,
                                      v_scale, new_key=key, new_value=value)

@@ -290,6 +290,7 @@ struct DecodeArgs {
     // the workgroups are to take them
     const int32_t* items;
     int num_items;
+    bool chunks;                // prefill only: the call is a step's prompt chunks and nothing else
 };
 
 int launch_decode_generic(const DecodeArgs& a);
@@ -298,6 +299,7 @@ int launch_decode_mfma(const DecodeArgs& a);
 bool decode_streamk_supported(const DecodeArgs& a);
 size_t decode_streamk_workspace_bytes(int64_t rows, int hq, int hkv, int d);
 int launch_decode_streamk(const DecodeArgs& a, void* workspace);
+int launch_prefill_rows(const DecodeArgs& a, int max_q_len, int tile_pos, int64_t wgs);
 int launch_kv_append_last(const void* key, const void* value, int64_t token_stride, int64_t head_stride,
                           void* k_pool, void* v_pool, const int32_t* block_table,
                           int64_t block_table_stride, const int32_t* context_lens, int batch, int hkv,

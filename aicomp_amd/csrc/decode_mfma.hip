@@ -113,16 +113,21 @@ template <> struct TileRegs<true> { uint2 r[8]; };
 // everything else in L2 (measured: 114 -> 101 us on the Llama-3-8B decode shape).
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+// (ONCE; prefill's workgroups share their rows and keep them in L2)
+template <bool ONCE = true>
 __device__ __forceinline__ uint4 tile_ld(const uint4* p) {
-    u32x4_t v = __builtin_nontemporal_load((const u32x4_t*)p);
+    u32x4_t v;
+    if constexpr (ONCE) v = __builtin_nontemporal_load((const u32x4_t*)p); else v = *(const u32x4_t*)p;
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
+template <bool ONCE = true>
 __device__ __forceinline__ uint2 tile_ld(const uint2* p) {
-    u32x2_t v = __builtin_nontemporal_load((const u32x2_t*)p);
+    u32x2_t v;
+    if constexpr (ONCE) v = __builtin_nontemporal_load((const u32x2_t*)p); else v = *(const u32x2_t*)p;
     return make_uint2(v[0], v[1]);
 }
-#define TILE_LD(ptr) tile_ld(ptr)
-template <bool FP8>
+#define TILE_LD(ptr) tile_ld<ONCE>(ptr)
+template <bool FP8, bool ONCE>
 __device__ __forceinline__ void load_tile(TileRegs<FP8>& t, const void* pool, int64_t blk0,
                                           int64_t blk1, int hkv, int kvh, int lane) {
     if constexpr (FP8) {
@@ -147,7 +152,7 @@ __device__ __forceinline__ void load_tile(TileRegs<FP8>& t, const void* pool, in
 // head_dim 64: a 32-row tile of 128-element rows is 64 tokens, each row a PAIR of consecutive
 // tokens (token 2r in elements 0..63, token 2r+1 in 64..127; contiguous in the pool).  Four
 // blocks of 8 such rows.
-template <bool FP8>
+template <bool FP8, bool ONCE>
 __device__ __forceinline__ void load_tile_pair(TileRegs<FP8>& t, const void* pool, int64_t blk0, int64_t blk1,
                                                int64_t blk2, int64_t blk3, int hkv, int kvh, int lane) {
     const int64_t blk[4] = {blk0, blk1, blk2, blk3};
@@ -220,15 +225,16 @@ __device__ __forceinline__ void clear_state(WaveStateT<NO>& st) {
 
 // One 32-token tile: K registers -> LDS -> S^T = K Q^T -> online softmax -> O^T += V^T P^T.
 // NEXT: prefetch the wave's next tile (blocks nb0/nb1) into the same registers.
-// MASK: the tile crosses `end`; scores beyond it are dropped and their V rows zeroed.
+// MASK: the tile crosses `end` (of this lane's column) or `v_end` (of all); scores beyond the one are dropped, V rows
+// beyond the other zeroed.
 // PAIR: rows are token pairs (head_dim 64): row r of the tile holds tokens tile_start + 2r and
 // + 2r + 1, the B-operand columns are (head, parity) pairs, column c scoring token 2r + (c & 1).
-template <typename E, bool FP8, bool NEXT, bool MASK, bool PAIR = false>
+template <typename E, bool FP8, bool NEXT, bool MASK, bool PAIR, bool ONCE>
 __device__ __forceinline__ void process_tile(WaveState& st, TileRegs<FP8>& kr, TileRegs<FP8>& vr,
                                              const uint4 (&qf)[4], unsigned char* kt, const KTileOffsets& ko,
                                              const void* k_pool, const void* v_pool,
                                              int64_t nb0, int64_t nb1, int hkv, int kvh_next, int lane,
-                                             int g4, int tile_start, int end, float cmul,
+                                             int g4, int tile_start, int end, int v_end, float cmul,
                                              int64_t nb2 = 0, int64_t nb3 = 0) {
     // ---- K tile -> LDS, then prefetch the next K tile into the same registers
 #pragma unroll
@@ -236,12 +242,12 @@ __device__ __forceinline__ void process_tile(WaveState& st, TileRegs<FP8>& kr, T
         uint4 kk = tile_elems<E, FP8>(kr, i);
         // PAIR: a row's two tokens share every dot product (the query column is zero over the other
         // token's half), so a token beyond the context must not leave non-finite values in the row
-        if (PAIR && MASK && tile_start + 2 * (4 * i + g4) + ((lane & 15) >> 3) >= end) kk = make_uint4(0, 0, 0, 0);
+        if (PAIR && MASK && tile_start + 2 * (4 * i + g4) + ((lane & 15) >> 3) >= v_end) kk = make_uint4(0, 0, 0, 0);
         *(uint4*)(kt + ko.wr[i & 3] + i * 4 * KROW) = kk;
     }
     if (NEXT) {
-        if constexpr (PAIR) load_tile_pair<FP8>(kr, k_pool, nb0, nb1, nb2, nb3, hkv, kvh_next, lane);
-        else load_tile<FP8>(kr, k_pool, nb0, nb1, hkv, kvh_next, lane);
+        if constexpr (PAIR) load_tile_pair<FP8, ONCE>(kr, k_pool, nb0, nb1, nb2, nb3, hkv, kvh_next, lane);
+        else load_tile<FP8, ONCE>(kr, k_pool, nb0, nb1, hkv, kvh_next, lane);
     }
 
     // ---- S^T = K Q^T for the two 16-token sub-tiles
@@ -295,7 +301,7 @@ __device__ __forceinline__ void process_tile(WaveState& st, TileRegs<FP8>& kr, T
         vv[i] = tile_elems<E, FP8>(vr, i);
         // PAIR: chunks 8..15 of a row belong to the pair's second token
         const int vtok = PAIR ? tile_start + 2 * (4 * i + g4) + ((lane & 15) >> 3) : tile_start + 4 * i + g4;
-        if (MASK && vtok >= end) vv[i] = make_uint4(0, 0, 0, 0);
+        if (MASK && vtok >= v_end) vv[i] = make_uint4(0, 0, 0, 0);
     }
     uint4 af[8];
 #pragma unroll
@@ -308,8 +314,8 @@ __device__ __forceinline__ void process_tile(WaveState& st, TileRegs<FP8>& kr, T
         af[j].w = __builtin_amdgcn_perm(v0[4 * 7 + (j >> 1)], v0[4 * 6 + (j >> 1)], sel);
     }
     if (NEXT) {
-        if constexpr (PAIR) load_tile_pair<FP8>(vr, v_pool, nb0, nb1, nb2, nb3, hkv, kvh_next, lane);
-        else load_tile<FP8>(vr, v_pool, nb0, nb1, hkv, kvh_next, lane);
+        if constexpr (PAIR) load_tile_pair<FP8, ONCE>(vr, v_pool, nb0, nb1, nb2, nb3, hkv, kvh_next, lane);
+        else load_tile<FP8, ONCE>(vr, v_pool, nb0, nb1, hkv, kvh_next, lane);
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -374,7 +380,7 @@ __device__ __forceinline__ void inject_new_row(TileRegs<FP8>& kr, TileRegs<FP8>&
 // one of these.  A tile is TT tokens of one KV head, BPT blocks, 8 KB of K and 8 KB of V per wave
 // (half of that for fp8), loaded with eight loads of each.
 // Tile16: 16-bit queries E over pools of E or fp8, head_dim 128, or 64 as rows of token pairs.
-template <typename E, bool FP8_, bool PAIR_>
+template <typename E, bool FP8_, bool PAIR_, bool ONCE = true>
 struct Tile16 {
     typedef E Fmt;
     static constexpr bool FP8 = FP8_, PAIR = PAIR_, QUAD = false;
@@ -394,8 +400,11 @@ struct Tile16 {
     // PAIR: column c = (head c / 2, parity c % 2): k-slot s covers row elements 32s + 8 g4 .., which are
     // the query's elements (32s + 8 g4) % 64 when the slot lies in the column's own half of the row.
     __device__ __forceinline__ static void load_q(Q& q, const uint16_t* rows, int group, int lane) {
-        const int r16 = lane & 15, g4 = lane >> 4, h = PAIR ? (r16 >> 1) : r16;
-        const uint16_t* row = rows + min(h, group - 1) * DQ;
+        const int r16 = lane & 15, h = PAIR ? (r16 >> 1) : r16;
+        load_q_row(q, rows + min(h, group - 1) * DQ, lane);
+    }
+    __device__ __forceinline__ static void load_q_row(Q& q, const uint16_t* row, int lane) {      // the row of the lane's column
+        const int g4 = lane >> 4;
 #pragma unroll
         for (int s = 0; s < 4; ++s) q.r[s] = *(const uint4*)(row + (PAIR ? ((32 * s + 8 * g4) & 63) : 32 * s + 8 * g4));
     }
@@ -411,19 +420,26 @@ struct Tile16 {
     template <typename Params>
     __device__ __forceinline__ static void load(Regs& t, const Params& p, const int64_t (&bb)[4], int kvh, int lane) {
         if constexpr (PAIR) {
-            load_tile_pair<FP8>(t.k, p.k_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kvh, lane);
-            load_tile_pair<FP8>(t.v, p.v_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kvh, lane);
+            load_tile_pair<FP8, ONCE>(t.k, p.k_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kvh, lane);
+            load_tile_pair<FP8, ONCE>(t.v, p.v_pool, bb[0], bb[1], bb[2], bb[3], p.hkv, kvh, lane);
         } else {
-            load_tile<FP8>(t.k, p.k_pool, bb[0], bb[1], p.hkv, kvh, lane);
-            load_tile<FP8>(t.v, p.v_pool, bb[0], bb[1], p.hkv, kvh, lane);
+            load_tile<FP8, ONCE>(t.k, p.k_pool, bb[0], bb[1], p.hkv, kvh, lane);
+            load_tile<FP8, ONCE>(t.v, p.v_pool, bb[0], bb[1], p.hkv, kvh, lane);
         }
     }
     template <bool NEXT, bool MASK, typename Params>
     __device__ __forceinline__ static void process(State& st, Regs& t, const Q& q, unsigned char* kt, const Offsets& ko,
                                                    const Params& p, const int64_t (&nb)[4], int kvh_next, int lane,
                                                    int tile_start, int end, float cmul) {
-        process_tile<E, FP8, NEXT, MASK, PAIR>(st, t.k, t.v, q.r, kt, ko, p.k_pool, p.v_pool, nb[0], nb[1], p.hkv,
-                                               kvh_next, lane, lane >> 4, tile_start, end, cmul, nb[2], nb[3]);
+        process_rows<NEXT, MASK>(st, t, q, kt, ko, p, nb, kvh_next, lane, tile_start, end, end, cmul);
+    }
+    // columns with ends of their own (rows of a chunk)
+    template <bool NEXT, bool MASK, typename Params>
+    __device__ __forceinline__ static void process_rows(State& st, Regs& t, const Q& q, unsigned char* kt, const Offsets& ko,
+                                                        const Params& p, const int64_t (&nb)[4], int kvh_next, int lane,
+                                                        int tile_start, int end, int v_end, float cmul) {
+        process_tile<E, FP8, NEXT, MASK, PAIR, ONCE>(st, t.k, t.v, q.r, kt, ko, p.k_pool, p.v_pool, nb[0], nb[1], p.hkv,
+                                               kvh_next, lane, lane >> 4, tile_start, end, v_end, cmul, nb[2], nb[3]);
     }
     template <typename Params>
     __device__ __forceinline__ static void inject(Regs& t, const Params& p, const uint16_t* key, const uint16_t* value,
@@ -676,6 +692,145 @@ paged_decode_mfma_kernel(MfmaParams p) {
     }
 }
 
+
+// ---------------------------------------------------------------------------------------
+// Prompt chunks of a small grid (see launch_prefill_rows).  A workgroup of the prefill kernel proper walks all keys of
+// its 128 query rows tile by tile, 1.3 us a step when it has a CU to itself, and a call of few chunks leaves most CUs
+// without one.  Here the columns of the decode tiles are 16 query rows of a chunk (D 64: 8, two columns each), the waves
+// of a workgroup split the keys like those of a decode row, and the rows' partial softmaxes are merged
+// through LDS: eight (sixteen) times the workgroups, a chain of keys / (tile x waves) rounds.  Every workgroup reads its
+// keys through its CU's 64 bytes per clock, which is what bounds it, and why large grids, whose CUs are busy
+// anyway, share a tile between 128 rows instead.
+struct PrefillRowsParams {
+    void* out;
+    const void* query;
+    void* k_pool;
+    void* v_pool;
+    const int32_t* block_table;
+    int64_t block_table_stride;
+    const int32_t* context_lens;
+    const int32_t* cu_q_lens;
+    int hq, hkv, group, gpack, max_blocks;
+    int64_t num_blocks;
+    float qk_mul;
+    const float* k_scale;
+    const float* v_scale;
+    const int32_t* items;       // (sequence, tile of `sub` workgroups) pairs, grid.y of them (NULL: grid.y numbers sequences)
+    int num_seqs, sub;
+};
+
+template <typename T, int NW>
+__global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1)
+paged_prefill_rows_kernel(PrefillRowsParams p) {
+    constexpr int DQ = T::DQ, TT = T::TT, BPT = T::BPT, NPAR = T::NPAR;
+    constexpr int ROWS = 16 / NPAR;                                  // query rows per workgroup
+    typedef typename T::Fmt::raw Raw;
+    const int hgroup = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g4 = lane >> 4;
+    const int pos_per_wg = ROWS / p.gpack;
+    int seq = blockIdx.y;
+    int64_t qtile = (int)(gridDim.z - 1 - blockIdx.z);              // expensive first
+    if (p.items != nullptr) {
+        seq = p.items[2 * blockIdx.y];
+        const int q = p.items[2 * blockIdx.y + 1];
+        if (seq < 0 || seq >= p.num_seqs || q < 0) return;
+        qtile = (int64_t)q * p.sub + blockIdx.z;
+    }
+    const int q_begin = p.cu_q_lens[seq];
+    const int n = p.cu_q_lens[seq + 1] - q_begin;
+    const int ctx = min(p.context_lens[seq], p.max_blocks * BS);
+    const int prior = ctx - n;
+    if (n <= 0 || qtile * pos_per_wg >= n) return;
+    const int q0 = (int)qtile * pos_per_wg;
+    auto out_row = [&](int row) -> Raw* {                            // NULL: beyond the chunk
+        const int pos = q0 + row / p.gpack;
+        return pos < n ? (Raw*)p.out + ((int64_t)(q_begin + pos) * p.hq + hgroup * p.gpack + row % p.gpack) * DQ : nullptr;
+    };
+    if (prior < 0) {                   // a context shorter than the chunk itself: zero rows, as in the other kernels
+        for (int i = tid; i < ROWS * DQ; i += 64 * NW)
+            if (Raw* o = out_row(i / DQ)) o[i % DQ] = 0;
+        return;
+    }
+    __shared__ __attribute__((aligned(16))) unsigned char lds[NW * KTILE_BYTES];
+    __shared__ float sm_m[NW][16];
+    __shared__ float sm_l[NW][16];
+    unsigned char* kt = lds + w * KTILE_BYTES;
+
+    const int kvh = (hgroup * p.gpack) / p.group;                    // workgroup-uniform
+    const int32_t* table = p.block_table + (int64_t)seq * p.block_table_stride;
+    int tab_first = 0;
+    int tab = lane < p.max_blocks ? table[lane] : 0;
+
+    // this lane's column: its row, and the first key the row does not see (rows beyond the chunk: computed, not stored)
+    const int row = r16 / NPAR, qpos = q0 + row / p.gpack;
+    const int kv_end = min(ctx, prior + q0 + pos_per_wg), kv_min = prior + q0 + 1;
+    const int end = qpos < n ? prior + qpos + 1 : kv_end;
+    typename T::Q qf;
+    T::load_q_row(qf, (const Raw*)p.query + ((int64_t)(q_begin + min(qpos, n - 1)) * p.hq + hgroup * p.gpack + row % p.gpack) * DQ, lane);
+    const float cmul = p.qk_mul * (T::FP8 ? p.k_scale[kvh] : 1.f);
+    const int ntiles = (kv_end + TT - 1) / TT;
+    typename T::State st;
+    clear_state(st);
+
+    int64_t bb[4] = {0, 0, 0, 0};
+    auto tile_blocks = [&](int tt) {
+        const int i0 = BPT * tt;
+        if (i0 - tab_first >= 64) {
+            tab_first = i0;
+            tab = i0 + lane < p.max_blocks ? table[i0 + lane] : 0;
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0) here, so the common path never waits on `tab`
+        }
+#pragma unroll
+        for (int j = 0; j < BPT; ++j) bb[j] = clamp_block(__builtin_amdgcn_readlane(tab, i0 + j - tab_first), p.num_blocks);
+    };
+    const typename T::Offsets ko = T::offsets(lane);
+    if (w < ntiles) {
+        typename T::Regs kv;
+        tile_blocks(w);
+        T::load(kv, p, bb, kvh, lane);
+        T::q_operand(qf, qf, ROWS, lane);
+        int tt = w;
+        // (the rows of a workgroup end within 16 tokens of each other: only the last NW tiles, each its wave's last, can
+        // need a mask)
+        for (; tt + NW < ntiles; tt += NW) {
+            tile_blocks(tt + NW);
+            T::template process_rows<true, false>(st, kv, qf, kt, ko, p, bb, kvh, lane, tt * TT, end, kv_end, cmul);
+        }
+        if (tt * TT + TT > kv_min)
+            T::template process_rows<false, true>(st, kv, qf, kt, ko, p, bb, kvh, lane, tt * TT, end, kv_end, cmul);
+        else
+            T::template process_rows<false, false>(st, kv, qf, kt, ko, p, bb, kvh, lane, tt * TT, end, kv_end, cmul);
+    }
+    float lsum = st.lsum;
+    lsum += __shfl_xor(lsum, 16);
+    lsum += __shfl_xor(lsum, 32);
+    T::store_acc((float*)kt + r16 * T::OROW, st, g4);
+    if (g4 == 0) { sm_m[w][r16] = st.m; sm_l[w][r16] = lsum; }
+    __syncthreads();
+    const float vs = T::FP8 ? p.v_scale[kvh] : 1.f;
+    for (int idx = tid; idx < ROWS * DQ; idx += 64 * NW) {
+        const int h = idx / DQ, dd = idx % DQ;
+        Raw* o = out_row(h);
+        if (o == nullptr) continue;
+        float mx = NEG_BIG, num = 0.f, den = 0.f;
+#pragma unroll
+        for (int ww = 0; ww < NW; ++ww)
+#pragma unroll
+            for (int par = 0; par < NPAR; ++par) mx = fmaxf(mx, sm_m[ww][NPAR * h + par]);
+#pragma unroll
+        for (int ww = 0; ww < NW; ++ww)
+#pragma unroll
+            for (int par = 0; par < NPAR; ++par) {
+                const int c = NPAR * h + par;
+                const float f = exp2f(sm_m[ww][c] - mx);
+                num = fmaf(f, ((const float*)(lds + ww * KTILE_BYTES))[c * T::OROW + dd + 64 * par], num);
+                den = fmaf(f, sm_l[ww][c], den);
+            }
+        o[dd] = T::Fmt::from_f32(den == 0.f ? 0.f : vs * num / den);
+    }
+}
 
 // ---------------------------------------------------------------------------------------
 // Balanced schedule.  The grid above gives the hardware dispatcher workgroups of unequal
@@ -1228,6 +1383,44 @@ int launch_decode_mfma(const DecodeArgs& a) {
 #undef AICOMP_LAUNCH_GRID
     AICOMP_HIP_LAUNCH_CHECK();
     if (a.num_parts > 1) return launch_split_reduce(a);
+    return AICOMP_KV_OK;
+}
+
+// Prefill of 16-bit queries on the decode tiles: `wgs` workgroups of the prefill kernel proper, of tile_pos positions each
+// (what a pair of the item list names), would be too few.
+int launch_prefill_rows(const DecodeArgs& a, int max_q_len, int tile_pos, int64_t wgs) {
+    PrefillRowsParams p;
+    p.out = a.out; p.query = a.query; p.k_pool = (void*)a.k_pool; p.v_pool = (void*)a.v_pool;
+    p.block_table = a.block_table; p.block_table_stride = a.block_table_stride;
+    p.context_lens = a.context_lens; p.cu_q_lens = a.cu_q_lens;
+    const bool d64 = a.d == 64, fp8 = a.kv_dtype == AICOMP_KV_FP8_E4M3;
+    const int rows = d64 ? 8 : 16;
+    p.hq = a.hq; p.hkv = a.hkv; p.group = a.hq / a.hkv; p.max_blocks = a.max_blocks; p.num_blocks = a.num_blocks;
+    p.gpack = rows % p.group == 0 ? p.group : 1;
+    p.qk_mul = a.scale * LOG2E;
+    p.k_scale = a.k_scale; p.v_scale = a.v_scale;
+    p.items = a.items; p.num_seqs = a.num_seqs;
+    const int pos = rows / p.gpack, groups = a.hq / p.gpack;
+    p.sub = (tile_pos + pos - 1) / pos;
+    const int tiles = (max_q_len + pos - 1) / pos;
+    AICOMP_REQUIRE(tiles <= 65535 && tile_pos % pos == 0, AICOMP_KV_EINVAL, "paged_prefill_attn: grid too large");
+    dim3 grid((unsigned)groups, (unsigned)a.num_seqs, (unsigned)tiles);
+    if (a.items != nullptr) grid = dim3((unsigned)groups, (unsigned)a.num_items, (unsigned)p.sub);
+    const bool wide = wgs <= 32;
+#define AICOMP_LAUNCH_ROWS(...)                                                                                              \
+    do {                                                                                                                     \
+        if (wide) hipLaunchKernelGGL((paged_prefill_rows_kernel<__VA_ARGS__, 8>), grid, dim3(512), 0, a.stream, p);          \
+        else hipLaunchKernelGGL((paged_prefill_rows_kernel<__VA_ARGS__, 4>), grid, dim3(256), 0, a.stream, p);               \
+    } while (0)
+#define AICOMP_LAUNCH_ROWS16(E)                                                                                       \
+    do {                                                                                                              \
+        if (d64) { if (fp8) AICOMP_LAUNCH_ROWS(Tile16<E, true, true, false>); else AICOMP_LAUNCH_ROWS(Tile16<E, false, true, false>); }   \
+        else { if (fp8) AICOMP_LAUNCH_ROWS(Tile16<E, true, false, false>); else AICOMP_LAUNCH_ROWS(Tile16<E, false, false, false>); }     \
+    } while (0)
+    if (a.q_dtype == AICOMP_KV_F16) AICOMP_LAUNCH_ROWS16(F16Fmt); else AICOMP_LAUNCH_ROWS16(Bf16Fmt);
+#undef AICOMP_LAUNCH_ROWS16
+#undef AICOMP_LAUNCH_ROWS
+    AICOMP_HIP_LAUNCH_CHECK();
     return AICOMP_KV_OK;
 }
 

@@ -506,6 +506,55 @@ PyObject* paged_prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs)
     }
 }
 
+// key, value and slot_mapping None: the rows are in the pools already
+PyObject* append_prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        Pools p;
+        const at::Tensor *out, *q, *table, *ctx;
+        int dt, max_q_len;
+        int64_t S;
+        double scale;
+        if (nargs != 15)
+            FAIL("append_prefill_attn(out, query, k_pool, v_pool, block_table, context_lens, cu_q_lens, scale, max_q_len, "
+                 "k_scale, v_scale, items, key, value, slot_mapping)");
+        if (!attention_args(args, out, q, p, table, ctx, dt, S) || !as_double(args[7], scale) ||
+            !as_int(args[8], max_q_len) || !p.scales(args[9], args[10]))
+            Py_RETURN_FALSE;
+        const at::Tensor* cu = plain(args[6]);
+        if (!vector_of(cu, at::kInt, S + 1, *q)) Py_RETURN_FALSE;
+        const at::Tensor *items = nullptr, *key = nullptr, *value = nullptr, *slots = nullptr;
+        if (args[11] != Py_None) {
+            items = plain(args[11]);
+            if (!items || items->numel() == 0 || items->scalar_type() != at::kInt || items->dim() != 2 ||
+                items->size(1) != 2 || items->size(0) > INT_MAX || !items->is_contiguous() || !on(*items, *q))
+                Py_RETURN_FALSE;
+        }
+        if (args[12] != Py_None) {
+            key = plain(args[12]); value = plain(args[13]); slots = plain(args[14]);
+            if (!key || !value || !slots || key->dim() != 3 || value->sizes() != key->sizes() ||
+                key->scalar_type() != q->scalar_type() || value->scalar_type() != q->scalar_type() ||
+                key->size(0) != q->size(0) || key->size(1) != p.hkv || key->size(2) != p.d || slots->dim() != 1 ||
+                !vector_of(slots, at::kLong, key->size(0), *q) || !on(*key, *q) || !on(*value, *q) ||
+                key->stride(2) != 1 || key->strides() != value->strides())
+                Py_RETURN_FALSE;
+        }
+        const c10::DeviceGuard guard(q->device());
+        void* stream = stream_of(*q);
+        const int rc = unlocked([&] {
+            return aicomp_kv_append_prefill_attn(
+                out->data_ptr(), q->data_ptr(), key ? key->data_ptr() : nullptr, key ? value->data_ptr() : nullptr,
+                key ? key->stride(0) : 0, key ? key->stride(1) : 0, p.k->data_ptr(), p.v->data_ptr(),
+                key ? (const int64_t*)slots->data_ptr() : nullptr, (const int32_t*)table->data_ptr(), table->stride(0),
+                (const int32_t*)ctx->data_ptr(), (const int32_t*)cu->data_ptr(), (int)S, q->size(0), max_q_len,
+                (int)q->size(1), p.hkv, p.d, p.bs, (int)table->size(1), p.nb, (float)scale, dt, p.dt, p.ks, p.vs,
+                items ? (const int32_t*)items->data_ptr() : nullptr, items ? (int)items->size(0) : 0, stream);
+        });
+        DONE(rc);
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
 // (tokens come back as a new tensor; None: take the Python way)
 PyObject* sample_tokens(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     try {
@@ -698,6 +747,7 @@ PyMethodDef methods[] = {
     {"plan_decode", FAST(plan_decode), "a step of one token per running sequence, packed: (rows, blocks taken), or None"},
     {"plan_upload", FAST(plan_upload), "the packed plan on its way to the device: its five tensors there"},
     {"paged_prefill_attn", FAST(paged_prefill_attn), "ops.paged_prefill_attn of a plain call, max_q_len given"},
+    {"append_prefill_attn", FAST(append_prefill_attn), "ops.append_prefill_attn of a plain call"},
     {"sample_tokens", FAST(sample_tokens), "ops.sample_tokens of a plain call: the tokens, or None if it is not one"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -40,6 +40,7 @@
 //              read feeds two MFMAs.
 #include "common.h"
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -709,6 +710,22 @@ int prefill_mfma_tile_positions(int hq, int hkv, int max_q_len) {
 }
 
 int launch_prefill_mfma(const DecodeArgs& a, int max_q_len) {
+    if (a.chunks) {
+        // Small grids (see paged_prefill_rows_kernel); in brackets the workgroups this kernel would have.  us of a step, its
+        // append included, here / there (12 to 14 us are the host's):
+        //   D 128  8/8 heads  200 after 1500 (16) 40 / 18;  2 of 162 after 1700 (32) 43 / 19;  4 of 164 after 1000 (64) 31 / 22
+        //          32/8       200 after 1500 (56) 41 / 25;  4 of 64 after 1000 (64) 30 / 21;   2 of 162 after 1700 (96) 44 / 42;
+        //                     500 (128) 19.3 / 22.9;  64/8  200 after 1500 (104) 41 / 44
+        //   D 64   16/2       200 after 1500 (26) 30 / 20;  4 of 64 after 1000 (32) 22 / 18;   8 of 40 after 500 (48) 15 / 17;
+        //                     2 of 162 after 1700 (44) 32 / 27;  32/8  4 of 64 after 1000 (64) 22 / 24
+        // What is counted is known to the host (all rows, the longest chunk) and the same with and without a list.
+        const int tile_pos = prefill_mfma_tile_positions(a.hq, a.hkv, max_q_len);
+        const int group = a.hq / a.hkv, groups = a.hq / (16 % group == 0 ? group : 1);
+        const int64_t tiles = (max_q_len + tile_pos - 1) / tile_pos;
+        const int64_t wgs = groups * std::min(tiles * a.num_seqs, a.rows / tile_pos + a.num_seqs);
+        // (sixteen heads of 64 are more rows per position than its workgroups have)
+        if (wgs <= (a.d == 64 ? 32 : 64) && !(a.d == 64 && group == 16)) return launch_prefill_rows(a, max_q_len, tile_pos, wgs);
+    }
     PrefillParams p;
     p.out = a.out; p.query = a.query; p.k_pool = a.k_pool; p.v_pool = a.v_pool;
     p.block_table = a.block_table; p.block_table_stride = a.block_table_stride;

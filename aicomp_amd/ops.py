@@ -511,6 +511,24 @@ def paged_prefill_attn(out: torch.Tensor, query: torch.Tensor, k_pool: torch.Ten
     return out
 
 
+def append_prefill_attn(out: torch.Tensor, query: torch.Tensor, key: Optional[torch.Tensor],
+                        value: Optional[torch.Tensor], k_pool: torch.Tensor, v_pool: torch.Tensor,
+                        slot_mapping: Optional[torch.Tensor], block_table: torch.Tensor, context_lens: torch.Tensor,
+                        cu_q_lens: torch.Tensor, scale: float, max_q_len: int, k_scale: Optional[torch.Tensor] = None,
+                        v_scale: Optional[torch.Tensor] = None, items: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """A layer's step of prompt chunks and nothing else: ``kv_append`` of the new rows (``key`` None: they are in the pools
+    already) and ``paged_prefill_attn``, in one call, which may take the kernel for few chunks."""
+    if _native("aicomp_kv_append_prefill_attn") and _lib.untouched("aicomp_kv_append") \
+            and _lib.untouched("aicomp_paged_prefill_attn") and _lib.untouched("aicomp_paged_prefill_attn_items") \
+            and _FAST.append_prefill_attn(out, query, k_pool, v_pool, block_table, context_lens, cu_q_lens, scale, max_q_len,
+                                          k_scale, v_scale, items, key, value, slot_mapping):
+        return out
+    if key is not None:
+        kv_append(key, value, k_pool, v_pool, slot_mapping, k_scale, v_scale)
+    return paged_prefill_attn(out, query, k_pool, v_pool, block_table, context_lens, cu_q_lens, scale, max_q_len=max_q_len,
+                              k_scale=k_scale, v_scale=v_scale, items=items)
+
+
 def rotary_tables(inv_freq: torch.Tensor, num_positions: int, dtype: torch.dtype,
                   attention_scaling: float = 1.0, device=None):
     """cos / sin tables ``[num_positions, D]`` the way the reference's rotary module builds them

@@ -309,6 +309,27 @@ int aicomp_paged_prefill_attn_items(void* out, const void* query,
                                     const float* k_scale, const float* v_scale,
                                     const int32_t* items, int num_items, void* stream);
 
+/*
+ * A layer's step of prompt chunks and nothing else: aicomp_kv_append of the T = total_q new rows
+ * (key, value, strides and slot_mapping as there; NULL key: they are in the pools already), then the
+ * attention of aicomp_paged_prefill_attn_items.  That all sequences are chunks lets a call of few of
+ * them take a kernel that splits their keys between waves; results agree with the other entry
+ * points to the rounding of the 16-bit formats, not bit for bit.
+ */
+int aicomp_kv_append_prefill_attn(void* out, const void* query,
+                                  const void* key, const void* value,
+                                  int64_t kv_token_stride, int64_t kv_head_stride,
+                                  void* k_pool, void* v_pool, const int64_t* slot_mapping,
+                                  const int32_t* block_table, int64_t block_table_stride,
+                                  const int32_t* context_lens, const int32_t* cu_q_lens,
+                                  int num_seqs, int64_t total_q, int max_q_len,
+                                  int num_q_heads, int num_kv_heads, int head_dim,
+                                  int block_size, int max_blocks_per_seq, int64_t num_blocks,
+                                  float scale, int q_dtype, int kv_dtype,
+                                  const float* k_scale, const float* v_scale,
+                                  const int32_t* items, int num_items,
+                                  void* stream);
+
 /* Positions per query tile of the kernel a prefill call with these shapes runs on (0: none that takes an item list). */
 int aicomp_paged_prefill_tile_positions(int num_q_heads, int num_kv_heads, int head_dim, int block_size,
                                         int q_dtype, int kv_dtype, int max_q_len);

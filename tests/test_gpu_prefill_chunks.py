@@ -1,0 +1,72 @@
+"""A step of prompt chunks alone (append and attention in one call) on either side of the line below which a chunk's keys
+are split between waves: every row against the float64 oracle, the pools bit for bit, the same bits with an item list."""
+import numpy as np
+import pytest
+import torch
+
+import test_gpu_prefill as tp
+from aicomp_amd import ops
+from helpers import assert_close_attn, to_f64
+
+pytestmark = pytest.mark.gpu
+
+# chunk lengths and priors at the edges of 16-row workgroups, 32- and 64-token tiles and the waves' rounds
+CHUNKS = [([0], [1]), ([0], [17]), ([31], [33]), ([0, 63, 64, 65], [64, 1, 2, 15]), ([127, 128, 129], [16, 17, 31]),
+          ([500, 0, 255, 257], [40, 129, 3, 65]), ([1000], [48]), ([2049, 7], [5, 20])]
+
+
+@pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, None), (torch.float16, None), (torch.bfloat16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("hq,hkv,d", [(4, 4, 128), (8, 2, 128), (16, 2, 64), (6, 2, 64), (16, 1, 64), (16, 1, 128)])
+def test_chunks_alone(device, dtype, kv, hq, hkv, d):
+    for i, (priors, news) in enumerate(CHUNKS):
+        c = tp.build_case(device, priors, news, hq, hkv, d, dtype=dtype, kv_dtype=kv, seed=i + d)
+        want = tp.oracle(c)
+        outs = []
+        for listed in (False, True):
+            items = None
+            tile = ops.prefill_tile_positions(hq, hkv, d, 16, dtype, kv or dtype, max(news))
+            if listed and tile:
+                lens = np.asarray(c["ctx_list"], dtype=np.int32)
+                group = hq // hkv
+                items = torch.from_numpy(ops.prefill_items(lens, np.asarray(news, dtype=np.int32), tile,
+                                                           hq // (group if 16 % group == 0 else 1), 256)).to(device)
+            out = torch.full_like(c["q"], float("nan"))
+            ops.append_prefill_attn(out, c["q"], None, None, c["k_pool"], c["v_pool"], None, c["table"], c["ctx"], c["cu"],
+                                    c["scale"], max(news), c["ks"], c["vs"], items)
+            outs.append(out)
+            assert_close_attn(to_f64(out), want, 1e-2, 2e-2, f"{hq}/{hkv} {d} {priors} {news}")
+        assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, None), (torch.float16, torch.float8_e4m3fn), (torch.float32, None)])
+@pytest.mark.parametrize("hq", [4, 48])
+def test_append_and_attention_in_one_call(device, dtype, kv, hq):
+    """The new rows come as arguments, strided; 48 heads are beyond the line."""
+    priors, news, hkv, d = [5, 200], [70, 33], hq // 2, 64
+    c = tp.build_case(device, priors, news, hq, hkv, d, dtype=dtype, kv_dtype=kv, seed=hq)
+    want_k, want_v, T = c["k_pool"].clone(), c["v_pool"].clone(), sum(news)
+    rows = (torch.randn(T, 2 * hkv, d, generator=torch.Generator().manual_seed(1)) * 0.5).to(dtype).to(device)
+    key, value = rows[:, :hkv], rows[:, hkv:]
+    slots = torch.cat([c["table"][s, t // 16].long() * 16 + t % 16 for s, (p, n) in enumerate(zip(priors, news))
+                       for t in [torch.arange(p, p + n, device=device)]])
+    ops.kv_append(key, value, want_k, want_v, slots, c["ks"], c["vs"])
+    out = torch.full_like(c["q"], float("nan"))
+    ops.append_prefill_attn(out, c["q"], key, value, c["k_pool"], c["v_pool"], slots, c["table"], c["ctx"], c["cu"],
+                            c["scale"], max(news), c["ks"], c["vs"])
+    assert torch.equal(c["k_pool"].view(torch.uint8), want_k.view(torch.uint8))
+    assert torch.equal(c["v_pool"].view(torch.uint8), want_v.view(torch.uint8))
+    tol = (1e-5, 1e-5) if dtype == torch.float32 else (1e-2, 2e-2)
+    assert_close_attn(to_f64(out), tp.oracle(c), *tol, f"{dtype} {hq}")
+
+
+def test_chunks_alone_zero_rows_and_junk_pairs(device):
+    """A context shorter than its chunk gives zero rows; pairs of the list that name nothing are skipped."""
+    c = tp.build_case(device, [0, 10], [40, 20], 4, 4, 128, seed=3)
+    c["ctx"][0] = 39
+    for items in (None, torch.tensor([[0, 0], [-1, 0], [1, 0], [7, 0], [1, 90], [0, -2], [1, 2 ** 30]], dtype=torch.int32, device=device)):
+        out = torch.full_like(c["q"], float("nan"))
+        ops.append_prefill_attn(out, c["q"], None, None, c["k_pool"], c["v_pool"], None, c["table"], c["ctx"], c["cu"],
+                                c["scale"], 40, None, None, items)
+        assert (out[:40] == 0).all() and torch.isfinite(out.float()).all()
+        want = tp.oracle(dict(c, ctx_list=[40, 30]))[40:]
+        assert_close_attn(to_f64(out[40:]), want, 1e-2, 2e-2, "second chunk")

@@ -1,5 +1,5 @@
-// Token sampling: temperature -> top-k -> top-p (nucleus) -> multinomial, one launch, or two when the rows
-// are cut into parts.
+// Token sampling: temperature -> top-k -> top-p (nucleus) -> multinomial, one launch, or two to four when the
+// rows are cut into parts.
 //
 // Replaces the step after the attention path,
 //   opt_prime/opt_prime/inference.py:786-843 (_sample_token):
@@ -27,7 +27,8 @@
 // A row (128 K logits = 512 KB in fp32) on one CU is bound by what that CU can load and compare, two
 // passes of it, with three quarters of the chip idle at 64 rows; the full-row histogram passes are
 // LDS-atomic bound when many logits share the leading key bits.  A caller with scratch memory therefore
-// has greedy and top-k calls cut into parts of a row first (sample_parts_kernel).
+// has greedy and top-k calls cut into parts of a row first (sample_parts_kernel), and draws from the whole row or
+// a nucleus of it too (sample_max_kernel and what follows it).
 #include "common.h"
 
 #include <type_traits>
@@ -60,6 +61,13 @@ struct SampleParams {
     uint2* part_list;                    // [B, parts, part_cap] (order key of the scaled logit, index)
     int parts, part_size;                // part_size: a multiple of 4 and at most PART_MAX
     int part_cap;                        // candidates of a part: part_capacity()
+    // a draw from the whole row, cut into parts: what sample_max_kernel and sample_mass_kernel leave
+    unsigned long long* seg_mass;        // [B, parts, NW] mass of each segment
+    float* part_max;                     // [B, parts] raw maximum
+    // ... and for a nucleus of it (NULL: top_p >= 1), with part_list and part_count
+    unsigned long long* part_hist;       // [B, parts, NBINS] mass of each slice of logits
+    unsigned long long* kept_mass;       // [B, parts, NW] of the segments' logits above the slice that holds the threshold
+    unsigned long long* cut;             // [B, 2] that slice (NBINS: not found), what is left of the mass limit at it
 };
 
 constexpr int PART_SLOTS = 16;                      // logits a lane of a part holds in registers
@@ -567,8 +575,8 @@ sample_parts_kernel(SampleParams p) {
 }
 
 // Index of the row's maximum, the lowest one among equals (0: nothing above -inf).
-template <typename T, int U>
-__device__ __forceinline__ int block_argmax(Shared& s, const T* row, int V, bool vec_ok) {
+template <typename T, int U, typename S>
+__device__ __forceinline__ int block_argmax(S& s, const T* row, int V, bool vec_ok) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float best = -INFINITY;
     int best_i = 0x7fffffff;
@@ -594,8 +602,8 @@ __device__ __forceinline__ int block_argmax(Shared& s, const T* row, int V, bool
 }
 
 // A row without finite mass (all -inf, NaN): the argmax, and an all-zero distribution.
-template <typename T, int U>
-__device__ __forceinline__ void no_mass(Shared& s, const SampleParams& p, int row_idx, const T* row, bool vec_ok) {
+template <typename T, int U, typename S>
+__device__ __forceinline__ void no_mass(S& s, const SampleParams& p, int row_idx, const T* row, bool vec_ok) {
     const int best_i = block_argmax<T, U>(s, row, p.vocab, vec_ok);
     if (threadIdx.x == 0) p.out[row_idx] = best_i;
     if (p.probs_out)
@@ -1298,6 +1306,340 @@ sample_merge_kernel(SampleParams p) {
     sample_row<T, 4>(p, s, row_idx);
 }
 
+// A draw from the whole row (neither top-k nor top-p), the row cut into parts of sixteen segments: the parts' maxima, the
+// segments' masses under the row's maximum (whole numbers, so any order of the sum gives the same one), and the
+// element within the segment that holds the target.
+//
+// One CU reads a row of 128256 float32 twice in 40 us, at its 64 bytes per clock and with an exponential per logit; three
+// launches of a few latencies each have the whole chip for it.  64 rows of 128256 float32: 54.9 -> 16.0 us.
+//
+// A nucleus (top_p alone) goes the same way with one launch more: the masses of 2048 slices of logits below the
+// maximum give the slice that holds the threshold (a few dozen logits of a usual row), and what lies above it is summed by
+// segment.  64 rows: 45.7 -> 38.4 us; 8 rows 42.2 -> 23.6, of which 3.4, 7.0, 8.2 and 6.8 in the four kernels.
+// Rows of unit variance at temperature 1, whose nucleus is half the row: 64 rows 154 -> 62 us (of equal logits only, which are
+// done whole all the same: 715 -> 768).
+constexpr int SEG = PART_MAX / NW;                  // logits of a segment, one wave's: 16 per lane
+// The lane's sixteen logits of the segment [begin, begin + n), -inf beyond it: four groups of four, 256 apart (IN_ORDER:
+// next to each other).
+template <typename T, bool IN_ORDER>
+__device__ __forceinline__ void load_segment(const T* row, int begin, int n, bool vec_ok, int lane, float (&x)[PART_SLOTS]) {
+    if (vec_ok && n == SEG) {
+#pragma unroll
+        for (int u = 0; u < PART_SLOTS / 4; ++u)
+            Load4<T>::get(row + begin + (IN_ORDER ? PART_SLOTS * lane + 4 * u : 4 * (lane + 64 * u)), x + 4 * u);
+    } else {
+#pragma unroll
+        for (int i = 0; i < PART_SLOTS; ++i)
+            x[i] = scaled_logit<T>(row, begin + max(0, min(IN_ORDER ? PART_SLOTS * lane + i : lane + 64 * i, n - 1)), 1.f);
+#pragma unroll
+        for (int i = 0; i < PART_SLOTS; ++i)
+            if ((IN_ORDER ? PART_SLOTS * lane + i : lane + 64 * i) >= n) x[i] = -INFINITY;
+    }
+}
+// Segment `seg` (part NW + wave) of a row: where it begins, how many logits it has (0 or less: none).
+__device__ __forceinline__ int segment_begin(const SampleParams& p, int seg, int& n) {
+    const int part = seg / NW, begin = part * p.part_size + seg % NW * SEG;
+    n = min(SEG, min(p.vocab, (part + 1) * p.part_size) - begin);
+    return n > 0 ? begin : 0;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(NT)
+sample_max_kernel(SampleParams p) {
+    __shared__ float red[NW];
+    const int row_idx = blockIdx.x, part = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
+    int n;
+    const int begin = segment_begin(p, part * NW + wave, n);
+    float x[PART_SLOTS];
+    load_segment<T, false>(row, begin, n, ((uintptr_t)row % 16) == 0, lane, x);
+    float best = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < PART_SLOTS; ++i) best = fmaxf(best, x[i]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) best = fmaxf(best, __shfl_xor(best, o));
+    if (lane == 0) red[wave] = best;
+    __syncthreads();
+    if (tid == 0) {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) best = fmaxf(best, red[w]);
+        p.part_max[(int64_t)row_idx * p.parts + part] = best;
+    }
+}
+
+// (the loads of a loop over the parts would be waited for one by one)
+__device__ __forceinline__ float row_max_of_parts(const SampleParams& p, int row_idx, int lane) {
+    float best = p.part_max[(int64_t)row_idx * p.parts + min(lane, p.parts - 1)];
+#pragma unroll
+    for (int o = MAX_PARTS / 2; o > 0; o >>= 1) best = fmaxf(best, __shfl_xor(best, o));
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(best)));
+}
+
+// Slices of the logits below the row's maximum, for the nucleus threshold: 160 to a unit, 12.8 units in all.
+constexpr int NBINS = 2048;
+constexpr float BINS_PER_UNIT = 160.f;
+constexpr int NUCLEUS_CAP = 512;                    // logits of a part in one slice
+__device__ __forceinline__ int slice_of(float x, float m) {          // never falls as x does; NBINS: below all of them, or NaN
+    const float d = (m - x) * BINS_PER_UNIT;
+    return d < (float)NBINS ? (int)d : NBINS;
+}
+
+// NUCLEUS: the masses of the slices too, by LDS atomics.
+template <typename T, bool NUCLEUS>
+__global__ void __launch_bounds__(NT)
+sample_mass_kernel(SampleParams p) {
+    __shared__ unsigned long long hist[NUCLEUS ? NBINS : 1];
+    const int row_idx = blockIdx.x, part = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
+    const int64_t slot = (int64_t)row_idx * p.parts + part;
+    int n;
+    const int begin = segment_begin(p, part * NW + wave, n);
+    float x[PART_SLOTS];
+    load_segment<T, false>(row, begin, n, ((uintptr_t)row % 16) == 0, lane, x);
+    const float m = apply_temperature<T>(row_max_of_parts(p, row_idx, lane), p.temperature);
+    if constexpr (NUCLEUS) {
+        for (int b = tid; b < NBINS; b += NT) hist[b] = 0;
+        __syncthreads();
+    }
+    unsigned long long mass = 0;
+#pragma unroll
+    for (int i = 0; i < PART_SLOTS; ++i) {
+        const float v = apply_temperature<T>(x[i], p.temperature);
+        const unsigned long long w = weight_of(v, m);
+        mass += w;
+        if constexpr (NUCLEUS) {
+            const int b = slice_of(v, m);
+            if (b < NBINS) atomicAdd(&hist[b], w);
+        }
+    }
+    mass = readlane64(wave_scan_dpp64(mass), 63);
+    if (lane == 0) p.seg_mass[slot * NW + wave] = mass;
+    if constexpr (NUCLEUS) {
+        __syncthreads();
+        for (int b = tid; b < NBINS; b += NT) p.part_hist[slot * NBINS + b] = hist[b];
+    }
+}
+
+// A lane's segments of a row, in index order, and their masses
+constexpr int SEGS = MAX_PARTS * NW, SEGS_PER_LANE = SEGS / 64;
+__device__ __forceinline__ unsigned long long lane_segments(const unsigned long long* segs, int nsegs, int lane,
+                                                            unsigned long long (&w)[SEGS_PER_LANE]) {
+    unsigned long long mine = 0;
+#pragma unroll
+    for (int j = 0; j < SEGS_PER_LANE; ++j) {
+        const unsigned long long v = segs[min(SEGS_PER_LANE * lane + j, nsegs - 1)];
+        w[j] = SEGS_PER_LANE * lane + j < nsegs ? v : 0;
+        mine += w[j];
+    }
+    return mine;
+}
+// The segment that holds `target` and the mass before it (the whole wave; `incl`: of the segments up to this lane's).
+__device__ __forceinline__ int find_segment(const unsigned long long (&w)[SEGS_PER_LANE], unsigned long long mine,
+                                            unsigned long long incl, unsigned long long target, int lane,
+                                            unsigned long long& base) {
+    int seg = 0;
+    unsigned long long before = incl - mine;
+    bool found = false;
+    base = 0;
+#pragma unroll
+    for (int j = 0; j < SEGS_PER_LANE; ++j) {
+        if (w[j] && before <= target && target < before + w[j]) { seg = SEGS_PER_LANE * lane + j; base = before; found = true; }
+        before += w[j];
+    }
+    const unsigned long long hit = __ballot(found);                 // one lane: the target is below the sum
+    const int owner = hit ? __ffsll((long long)hit) - 1 : 0;
+    base = readlane64(base, owner);
+    return __builtin_amdgcn_readlane(seg, owner);
+}
+// The draw within a segment: the element whose share of the mass, after `at` before this lane's first, holds `target`.
+__device__ __forceinline__ void draw_in_lane(const SampleParams& p, int row_idx, int first, const unsigned long long (&w)[PART_SLOTS],
+                                             unsigned long long at, unsigned long long target) {
+#pragma unroll
+    for (int i = 0; i < PART_SLOTS; ++i) {
+        if (w[i] && at <= target && target < at + w[i]) p.out[row_idx] = first + i;
+        at += w[i];
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(NT)
+sample_locate_kernel(SampleParams p) {
+    __shared__ struct { float red_f[NW]; int red_i[NW]; } s;
+    const int row_idx = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
+    const bool vec_ok = ((uintptr_t)row % 16) == 0;
+    unsigned long long w[SEGS_PER_LANE];
+    const unsigned long long mine = lane_segments(p.seg_mass + (int64_t)row_idx * p.parts * NW, p.parts * NW, lane, w);
+    const unsigned long long incl = wave_scan_dpp64(mine), z = readlane64(incl, 63);
+    if (z == 0) {                                   // the same in every wave
+        no_mass<T, 4>(s, p, row_idx, row, vec_ok);
+        return;
+    }
+    if (wave != 0) return;
+    unsigned long long target = (unsigned long long)((double)p.uniforms[row_idx] * (double)z), base;
+    if (target >= z) target = z - 1;
+    int n;
+    const int begin = segment_begin(p, find_segment(w, mine, incl, target, lane, base), n);
+    float x[PART_SLOTS];
+    load_segment<T, true>(row, begin, n, vec_ok, lane, x);
+    const float m = apply_temperature<T>(row_max_of_parts(p, row_idx, lane), p.temperature);
+    unsigned long long we[PART_SLOTS], sum = 0;
+#pragma unroll
+    for (int i = 0; i < PART_SLOTS; ++i) {
+        we[i] = weight_of(apply_temperature<T>(x[i], p.temperature), m);
+        sum += we[i];
+    }
+    draw_in_lane(p, row_idx, begin + PART_SLOTS * lane, we, base + wave_scan_dpp64(sum) - sum, target);
+}
+
+// The slice that holds the nucleus threshold, from the parts' slices: what lies above it is summed by segment, its own
+// logits leave the part as a list.
+template <typename T>
+__global__ void __launch_bounds__(NT)
+sample_slice_kernel(SampleParams p) {
+    __shared__ unsigned long long wave_mass[NW];
+    __shared__ unsigned int n_list, found;
+    __shared__ unsigned long long left;
+    const int row_idx = blockIdx.x, part = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
+    const int64_t slot = (int64_t)row_idx * p.parts + part;
+    int n;
+    const int begin = segment_begin(p, part * NW + wave, n);
+    const bool vec = ((uintptr_t)row % 16) == 0 && n == SEG;
+    float x[PART_SLOTS];
+    load_segment<T, false>(row, begin, n, ((uintptr_t)row % 16) == 0, lane, x);
+    // this lane's two slices over all parts
+    static_assert(NBINS == 2 * NT, "two slices per lane");
+    unsigned long long h0 = 0, h1 = 0;
+    const unsigned long long* hist = p.part_hist + (int64_t)row_idx * p.parts * NBINS + 2 * tid;
+    for (int q0 = 0; q0 < p.parts; q0 += 8) {
+        ulonglong2 h[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) h[q] = *(const ulonglong2*)(hist + (int64_t)min(q0 + q, p.parts - 1) * NBINS);
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (q0 + q < p.parts) { h0 += h[q].x; h1 += h[q].y; }
+    }
+    unsigned long long w[SEGS_PER_LANE];
+    const unsigned long long z = readlane64(
+        wave_scan_dpp64(lane_segments(p.seg_mass + (int64_t)row_idx * p.parts * NW, p.parts * NW, lane, w)), 63);
+    const unsigned long long limit = (unsigned long long)((double)fmaxf(p.top_p, 0.f) * (double)z);
+    if (tid == 0) { n_list = 0; found = NBINS; left = 0; }
+    const unsigned long long incl = wave_scan_dpp64(h0 + h1);
+    if (lane == 63) wave_mass[wave] = incl;
+    __syncthreads();
+    unsigned long long above = incl - h0 - h1;
+    for (int v = 0; v < wave; ++v) above += wave_mass[v];
+    // the slice at which the sum passes the limit: one, or none if the slices do not reach it
+    if (above <= limit && limit < above + h0) { found = 2 * tid; left = limit - above; }
+    if (above + h0 <= limit && limit < above + h0 + h1) { found = 2 * tid + 1; left = limit - above - h0; }
+    __syncthreads();
+    const int slice = (int)found;
+    if (part == 0 && tid == 0) { p.cut[2 * row_idx] = slice; p.cut[2 * row_idx + 1] = left; }
+    if (slice == NBINS) return;
+    const float m = apply_temperature<T>(row_max_of_parts(p, row_idx, lane), p.temperature);
+    uint2* list = p.part_list + slot * NUCLEUS_CAP;
+    unsigned long long mass = 0;
+#pragma unroll
+    for (int i = 0; i < PART_SLOTS; ++i) {
+        const float v = apply_temperature<T>(x[i], p.temperature);
+        const int b = slice_of(v, m);
+        if (b < slice) mass += weight_of(v, m);
+        if (b == slice) {
+            const unsigned int j = atomicAdd(&n_list, 1u);
+            const int at = vec ? 4 * (lane + 64 * (i / 4)) + (i & 3) : lane + 64 * i;
+            if (j < NUCLEUS_CAP) list[j] = make_uint2(order_key(v), (unsigned int)(begin + at));
+        }
+    }
+    mass = readlane64(wave_scan_dpp64(mass), 63);
+    if (lane == 0) p.kept_mass[slot * NW + wave] = mass;
+    __syncthreads();
+    if (tid == 0) p.part_count[slot] = n_list;
+}
+
+// The draw from the nucleus.  Of the slice's logits those stay whose mass before them, by falling value and then by
+// index, is at most what is left of the limit; with them added to their segments the draw goes as from the whole row.
+// A row whose slice was not found, or holds more logits than the lanes, is done whole.
+template <typename T>
+__global__ void __launch_bounds__(NT)
+sample_nucleus_kernel(SampleParams p) {
+    __shared__ Shared s;
+    __shared__ unsigned int stays[SEG / 32];
+    const int row_idx = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
+    const int nsegs = p.parts * NW, slice = (int)p.cut[2 * row_idx];
+    const unsigned long long left = p.cut[2 * row_idx + 1];
+    int total = 0, mine_at = -1;                    // this lane's entry of the parts' lists
+    if (slice < NBINS) {
+        const int counts = lane < p.parts ? (int)p.part_count[(int64_t)row_idx * p.parts + lane] : 0;
+        const bool fits = !__any(counts > NUCLEUS_CAP);
+        for (int q = 0; q < p.parts; ++q) {
+            const int c = __builtin_amdgcn_readlane(counts, q);
+            if (tid >= total && tid < total + c) mine_at = q * NUCLEUS_CAP + tid - total;
+            total += c;
+        }
+        if (!fits) total = NT + 1;
+    }
+    if (slice == NBINS || total > NT) {             // the same in every lane
+        sample_row<T, 4>(p, s, row_idx);
+        return;
+    }
+    const float m = apply_temperature<T>(row_max_of_parts(p, row_idx, lane), p.temperature);
+    unsigned long long* segs = s.mass;              // [SEGS]
+    if (tid < SEGS) segs[tid] = tid < nsegs ? p.kept_mass[(int64_t)row_idx * nsegs + tid] : 0;
+    if (tid < SEG / 32) stays[tid] = 0;
+    // entries with a larger order come first; zeros are no entries
+    unsigned long long me = 0, w = 0;
+    if (mine_at >= 0) {
+        const uint2 e = p.part_list[(int64_t)row_idx * p.parts * NUCLEUS_CAP + mine_at];
+        me = (unsigned long long)e.x << 32 | ~e.y;
+        w = weight_of(key_value(e.x), m);
+    }
+    unsigned long long* order = s.list_w;
+    unsigned long long* weight = s.list_w + NT;
+    order[tid] = me;
+    weight[tid] = w;
+    __syncthreads();
+    unsigned long long before = 0;
+    for (int j0 = 0; j0 < total; j0 += 8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) before += order[j0 + j] > me ? weight[j0 + j] : 0ull;       // (NT is a multiple of 8)
+    }
+    const bool stay = me != 0 && before <= left;
+    const int idx = (int)~(unsigned int)me, part = stay ? idx / p.part_size : 0, in_part = idx - part * p.part_size;
+    const int seg = part * NW + in_part / SEG;
+    if (stay) atomicAdd(&segs[seg], w);
+    __syncthreads();
+    unsigned long long ws[SEGS_PER_LANE];
+    const unsigned long long mine = lane_segments(segs, SEGS, lane, ws);
+    const unsigned long long incl = wave_scan_dpp64(mine), z = readlane64(incl, 63);
+    unsigned long long target = (unsigned long long)((double)p.uniforms[row_idx] * (double)z), base;
+    if (target >= z) target = z - 1;
+    const int at_seg = find_segment(ws, mine, incl, target, lane, base);     // in every wave alike
+    if (stay && seg == at_seg) atomicOr(&stays[in_part % SEG / 32], 1u << (in_part & 31));
+    __syncthreads();
+    if (wave != 0) return;
+    int n;
+    const int begin = segment_begin(p, at_seg, n);
+    float x[PART_SLOTS];
+    load_segment<T, true>(row, begin, n, ((uintptr_t)row % 16) == 0, lane, x);
+    const unsigned int mask = stays[lane / 2] >> PART_SLOTS * (lane & 1);
+    unsigned long long we[PART_SLOTS], sum = 0;
+#pragma unroll
+    for (int i = 0; i < PART_SLOTS; ++i) {
+        const float v = apply_temperature<T>(x[i], p.temperature);
+        const int b = slice_of(v, m);
+        we[i] = b < slice || (b == slice && (mask >> i & 1u)) ? weight_of(v, m) : 0ull;
+        sum += we[i];
+    }
+    draw_in_lane(p, row_idx, begin + PART_SLOTS * lane, we, base + wave_scan_dpp64(sum) - sum, target);
+}
+
 template <typename T>
 __global__ void __launch_bounds__(NT)
 sample_kernel(SampleParams p) {
@@ -1340,13 +1682,26 @@ greedy_kernel(SampleParams p) {
 //                                128 34.2 -> 37.9 (half the bytes to save on): six parts and more up to 1024 parts
 //   rows whose loads cannot be vectors (a stride that is no multiple of 16 bytes): at once
 //     bf16, k 50        50257: 64 rows 24.4 -> 17.3;  greedy float32 50257: 64 rows 11.4 -> 7.6
+//   the whole row       float32  20000, 2 parts: 1 row 14.8 -> 10.9, 1024 62.9 -> 49.3;  50256: 64 rows 26.3 -> 11.7
+//   (top_p off)         128256: 1 row 50.9 -> 11.3, 64 54.9 -> 16.0, 1024 281 -> 203;  262144: 64 rows 106 -> 31.5
+//                       bf16     20000: 64 rows 17.5 -> 12.1, 1024 66.2 -> 42.7;  128256: 64 61.0 -> 16.0, 1024 258 -> 146
 //   other calls from six parts on
 //     k to 256          128256: 1 row 24.3 -> 21.1, 16 25.5 -> 24.6, 64 27.0 -> 30.3: up to 128 parts
 //     greedy            128256: 16 rows 9.1 -> 7.2, 64 10.8 -> 9.8, 128 14.1 -> 17.2: up to 512 parts
+// A nucleus of the whole row takes four launches, the third of which reads 16 KB of slices for every part of its row from each
+// part's workgroup, so it pays from four parts on and as long as the workgroups are resident at once.  us per call,
+// temperature 0.8, top_p 0.9, one launch -> parts:
+//   float32  32000, 2 parts: 1 row 21.0 -> 22.1;  50256, 4: 1 row 24.3 -> 22.7, 64 25.7 -> 24.4, 128 26.1 -> 36.6;  50257: 64 35.3 -> 25.5
+//            81920, 5: 64 rows 35.9 -> 32.9, 128 38.4 -> 53.3;  128256, 8: 1 row 41.5 -> 23.3, 32 45.5 -> 24.9, 64 45.7 -> 38.4,
+//            128 55.1 -> 79.1;  262144, 16: 1 row 74.4 -> 24.4, 32 86.9 -> 42.6
+//   bf16     128256: 1 row 44.7 -> 24.2, 64 48.1 -> 36.2, 128 49.1 -> 64.9
+constexpr int NUCLEUS_MIN_PARTS = 4, NUCLEUS_MAX_BATCH = 64, NUCLEUS_MAX_ALL = 512;
+static bool whole_row(int vocab, int top_k, int greedy) { return !greedy && (top_k <= 0 || top_k >= vocab); }
 static int sample_parts(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy, int dtype) {
     const int parts = (int)(((int64_t)vocab + PART_MAX - 1) / PART_MAX);
     if (parts < 2 || parts > MAX_PARTS || batch > PART_MAX_BATCH) return 1;
-    if (!greedy && (top_k <= 0 || top_k >= vocab || top_k > PART_MAX_K || !(temperature <= LIST_MAX_TEMPERATURE))) return 1;
+    if (whole_row(vocab, top_k, greedy)) return parts;
+    if (!greedy && (top_k > PART_MAX_K || !(temperature <= LIST_MAX_TEMPERATURE))) return 1;
     const int per_16 = dtype == AICOMP_KV_F32 ? 4 : 8;
     if (batch > 1 && row_stride % per_16 != 0) return parts;
     const int all = batch * parts;
@@ -1362,9 +1717,35 @@ static int sample_parts(int batch, int vocab, int64_t row_stride, float temperat
 // and the distance an argument.
 static int part_capacity(int top_k, int greedy) { return greedy ? GREEDY_CAP : 256 + 8 * top_k < 1024 ? 256 + 8 * top_k : 1024; }
 
+// Scratch of a draw from the whole row: the nucleus' share only where such a call is cut
+struct WholeRowSpace {
+    unsigned long long *seg_mass, *kept_mass, *part_hist, *cut;
+    uint2* list;
+    unsigned int* count;
+    float* part_max;
+    size_t bytes;
+    WholeRowSpace(int batch, int parts, void* at) {
+        char* p = (char*)at;
+        auto take = [&](size_t bytes_each, size_t n) { char* q = p; p += bytes_each * n; return q; };
+        const size_t all = (size_t)batch * parts;
+        const bool nucleus = parts >= NUCLEUS_MIN_PARTS && batch <= NUCLEUS_MAX_BATCH && all <= NUCLEUS_MAX_ALL;
+        part_hist = (unsigned long long*)take(8 * NBINS, nucleus ? all : 0);         // first: 16-byte loads
+        seg_mass = (unsigned long long*)take(8 * NW, all);
+        kept_mass = (unsigned long long*)take(8 * NW, nucleus ? all : 0);
+        list = (uint2*)take(8 * NUCLEUS_CAP, nucleus ? all : 0);
+        cut = (unsigned long long*)take(16, nucleus ? batch : 0);
+        count = (unsigned int*)take(4, nucleus ? all : 0);
+        part_max = (float*)take(4, all);
+        bytes = p - (char*)at;
+        if (!nucleus) part_hist = nullptr;
+    }
+};
+
 size_t sample_workspace_bytes(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy, int dtype) {
     const int parts = sample_parts(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
-    return parts < 2 ? 0 : (size_t)batch * parts * (part_capacity(top_k, greedy) * sizeof(uint2) + sizeof(unsigned int));
+    if (parts < 2) return 0;
+    if (whole_row(vocab, top_k, greedy)) return WholeRowSpace(batch, parts, nullptr).bytes;
+    return (size_t)batch * parts * (part_capacity(top_k, greedy) * sizeof(uint2) + sizeof(unsigned int));
 }
 
 template <typename T>
@@ -1372,6 +1753,16 @@ static void launch_rows(const SampleParams& p, int batch, hipStream_t stream) {
     if (p.greedy) {
         if (p.parts) hipLaunchKernelGGL((sample_parts_kernel<T, true>), dim3(batch, p.parts), dim3(NT), 0, stream, p);
         hipLaunchKernelGGL((greedy_kernel<T>), dim3(batch), dim3(NT), 0, stream, p);
+    } else if (p.parts && p.seg_mass) {
+        hipLaunchKernelGGL((sample_max_kernel<T>), dim3(batch, p.parts), dim3(NT), 0, stream, p);
+        if (p.part_hist) {
+            hipLaunchKernelGGL((sample_mass_kernel<T, true>), dim3(batch, p.parts), dim3(NT), 0, stream, p);
+            hipLaunchKernelGGL((sample_slice_kernel<T>), dim3(batch, p.parts), dim3(NT), 0, stream, p);
+            hipLaunchKernelGGL((sample_nucleus_kernel<T>), dim3(batch), dim3(NT), 0, stream, p);
+        } else {
+            hipLaunchKernelGGL((sample_mass_kernel<T, false>), dim3(batch, p.parts), dim3(NT), 0, stream, p);
+            hipLaunchKernelGGL((sample_locate_kernel<T>), dim3(batch), dim3(NT), 0, stream, p);
+        }
     } else if (p.parts) {
         hipLaunchKernelGGL((sample_parts_kernel<T, false>), dim3(batch, p.parts), dim3(NT), 0, stream, p);
         hipLaunchKernelGGL((sample_merge_kernel<T>), dim3(batch), dim3(NT), 0, stream, p);
@@ -1388,14 +1779,30 @@ int launch_sample(int64_t* out, const void* logits, int64_t row_stride, float* p
     p.uniforms = uniforms; p.vocab = vocab; p.temperature = temperature; p.top_k = top_k;
     p.top_p = top_p; p.greedy = greedy;
     p.part_count = nullptr; p.part_list = nullptr; p.parts = 0; p.part_size = 0; p.part_cap = 0;
+    p.seg_mass = nullptr; p.part_max = nullptr;
+    p.part_hist = nullptr; p.kept_mass = nullptr; p.cut = nullptr;
     const size_t need = sample_workspace_bytes(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
     if (need && workspace && workspace_bytes >= need) {
         const int parts = sample_parts(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
         p.part_size = ((vocab + parts - 1) / parts + 3) / 4 * 4;       // parts * part_size < vocab + 4 parts
         p.parts = (vocab + p.part_size - 1) / p.part_size;             // none is empty
-        p.part_cap = part_capacity(top_k, greedy);
-        p.part_list = (uint2*)workspace;
-        p.part_count = (unsigned int*)(p.part_list + (size_t)batch * p.parts * p.part_cap);
+        if (whole_row(vocab, top_k, greedy)) {
+            const WholeRowSpace at(batch, parts, workspace);
+            const bool nucleus = top_p < 1.f;
+            // the distribution itself is written by one workgroup per row
+            if (probs_out || (nucleus && (!at.part_hist || (uintptr_t)workspace % 16))) p.parts = 0;
+            else {
+                p.seg_mass = at.seg_mass; p.part_max = at.part_max;
+                if (nucleus) {
+                    p.part_hist = at.part_hist; p.kept_mass = at.kept_mass; p.cut = at.cut;
+                    p.part_list = at.list; p.part_count = at.count;
+                }
+            }
+        } else {
+            p.part_cap = part_capacity(top_k, greedy);
+            p.part_list = (uint2*)workspace;
+            p.part_count = (unsigned int*)(p.part_list + (size_t)batch * p.parts * p.part_cap);
+        }
     }
     if (dtype == AICOMP_KV_F32) launch_rows<float>(p, batch, stream);
     else if (dtype == AICOMP_KV_F16) launch_rows<f16_t>(p, batch, stream);

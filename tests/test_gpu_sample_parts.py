@@ -101,3 +101,38 @@ def test_the_short_merge_draws_what_one_launch_draws(device, V, k):
         top_p = (1.0, 0.9, 0.5, 0.05, 0.0, 0.999)[i]
         got = ops.sample_tokens(x, 0.7, k, top_p, uniforms=u)
         assert torch.equal(got, _one_launch(x, 0.7, k, top_p, True, u)[0]), (top_p, i)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,stride,B", [(16385, 16385, 10), (32769, 32776, 10), (50257, 50257, 10), (50256, 50256, 70),
+                                        (81921, 81928, 10), (128255, 128255, 10), (128256, 128256, 10),
+                                        (262144, 262144, 10), (262145, 262152, 10)])
+def test_whole_rows_in_parts(device, V, stride, B, dtype):
+    """Draws without top-k: the whole row, and a nucleus of it whose threshold falls among ties, into the largest value, below
+    the slices of logits that are looked at (a flat row), or nowhere (no mass).  Masses are whole numbers, so the tokens
+    are the same ones."""
+    x = torch.zeros(B, stride, dtype=dtype, device=device)[:, :V]
+    x.copy_(_rows(V, dtype, device).repeat(B // 10, 1))
+    u = torch.rand(B, generator=torch.Generator().manual_seed(V)).to(device)
+    u[0], u[1] = 0.0, 1.0 - 2.0 ** -24
+    for temperature, top_k, top_p in [(1.0, 0, 1.0), (0.8, V, 1.0), (40.0, 0, 1.0), (0.8, 0, 0.9), (1.0, -1, 0.5), (0.6, 0, 0.95),
+                                      (1.3, V, 0.999), (40.0, 0, 0.9), (1.0, 0, 0.0), (0.05, 0, 0.7)]:
+        want, _ = _one_launch(x, temperature, top_k, top_p, True, u)
+        got = ops.sample_tokens(x, temperature, top_k, top_p, True, u)
+        assert torch.equal(got, want), (temperature, top_k, top_p, got, want)
+
+
+@pytest.mark.parametrize("top_p", [1.0, 0.9])
+def test_whole_rows_in_parts_in_a_graph(device, top_p):
+    x, u = _rows(81920, torch.float32, device), torch.rand(10, device=device)
+    ops.sample_tokens(x, 0.8, 0, top_p, uniforms=u)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = ops.sample_tokens(x, 0.8, 0, top_p, uniforms=u)
+    for i in range(3):
+        u.copy_(torch.rand(10, device=device))
+        x.copy_(x.roll(1, 0))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, _one_launch(x, 0.8, 0, top_p, True, u)[0]), i

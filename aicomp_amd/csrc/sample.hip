@@ -66,6 +66,7 @@ struct SampleParams {
     float* part_max;                     // [B, parts] raw maximum
     // ... and for a nucleus of it (NULL: top_p >= 1), with part_list and part_count
     unsigned long long* part_hist;       // [B, parts, NBINS] mass of each slice of logits
+    unsigned long long* part_group;      // [B, parts, GROUPS] and of each 32 of them
     unsigned long long* kept_mass;       // [B, parts, NW] of the segments' logits above the slice that holds the threshold
     unsigned long long* cut;             // [B, 2] that slice (NBINS: not found), what is left of the mass limit at it
 };
@@ -1315,9 +1316,10 @@ sample_merge_kernel(SampleParams p) {
 //
 // A nucleus (top_p alone) goes the same way with one launch more: the masses of 2048 slices of logits below the
 // maximum give the slice that holds the threshold (a few dozen logits of a usual row), and what lies above it is summed by
-// segment.  64 rows: 45.7 -> 38.4 us; 8 rows 42.2 -> 23.6, of which 3.4, 7.0, 8.2 and 6.8 in the four kernels.
-// Rows of unit variance at temperature 1, whose nucleus is half the row: 64 rows 154 -> 62 us (of equal logits only, which are
-// done whole all the same: 715 -> 768).
+// segment.  64 rows: 45.7 -> 34.5 us (38.4 while every part read its row's 2048 slices of all parts, 128 KB, where it now reads
+// the sums of 64 groups of them and one group); 8 rows 42.2 -> 23.8.
+// Rows of unit variance at temperature 1, whose nucleus is half the row: 64 rows 154 -> 60 us (of equal logits only, which are
+// done whole all the same: 715 -> 766).
 constexpr int SEG = PART_MAX / NW;                  // logits of a segment, one wave's: 16 per lane
 // The lane's sixteen logits of the segment [begin, begin + n), -inf beyond it: four groups of four, 256 apart (IN_ORDER:
 // next to each other).
@@ -1379,6 +1381,7 @@ __device__ __forceinline__ float row_max_of_parts(const SampleParams& p, int row
 // Slices of the logits below the row's maximum, for the nucleus threshold: 160 to a unit, 12.8 units in all.
 constexpr int NBINS = 2048;
 constexpr float BINS_PER_UNIT = 160.f;
+constexpr int GROUPS = 64, GROUP = NBINS / GROUPS;
 constexpr int NUCLEUS_CAP = 512;                    // logits of a part in one slice
 __device__ __forceinline__ int slice_of(float x, float m) {          // never falls as x does; NBINS: below all of them, or NaN
     const float d = (m - x) * BINS_PER_UNIT;
@@ -1389,7 +1392,7 @@ __device__ __forceinline__ int slice_of(float x, float m) {          // never fa
 template <typename T, bool NUCLEUS>
 __global__ void __launch_bounds__(NT)
 sample_mass_kernel(SampleParams p) {
-    __shared__ unsigned long long hist[NUCLEUS ? NBINS : 1];
+    __shared__ alignas(16) unsigned long long hist[NUCLEUS ? NBINS : 2];
     const int row_idx = blockIdx.x, part = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
@@ -1418,7 +1421,15 @@ sample_mass_kernel(SampleParams p) {
     if (lane == 0) p.seg_mass[slot * NW + wave] = mass;
     if constexpr (NUCLEUS) {
         __syncthreads();
-        for (int b = tid; b < NBINS; b += NT) p.part_hist[slot * NBINS + b] = hist[b];
+        static_assert(NBINS == 2 * NT && GROUP == 32, "two slices per lane, a group per sixteen lanes");
+        const ulonglong2 h = *(const ulonglong2*)(hist + 2 * tid);
+        *(ulonglong2*)(p.part_hist + slot * NBINS + 2 * tid) = h;
+        unsigned long long g = h.x + h.y;
+        g = dpp_add64<0x111, 0xf>(g);            // row_shr 1, 2, 4, 8: the last of sixteen lanes has their sum
+        g = dpp_add64<0x112, 0xf>(g);
+        g = dpp_add64<0x114, 0xf>(g);
+        g = dpp_add64<0x118, 0xf>(g);
+        if ((lane & 15) == 15) p.part_group[slot * GROUPS + tid / 16] = g;
     }
 }
 
@@ -1495,14 +1506,34 @@ sample_locate_kernel(SampleParams p) {
     draw_in_lane(p, row_idx, begin + PART_SLOTS * lane, we, base + wave_scan_dpp64(sum) - sum, target);
 }
 
+// Sum over the parts of a row of the lane's element of `at` (n of them per part)
+__device__ __forceinline__ unsigned long long sum_of_parts(const unsigned long long* at, int n, int parts, int i) {
+    unsigned long long sum = 0;
+    for (int q0 = 0; q0 < parts; q0 += 8) {
+        unsigned long long h[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) h[q] = at[(int64_t)min(q0 + q, parts - 1) * n + i];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) sum += q0 + q < parts ? h[q] : 0ull;
+    }
+    return sum;
+}
+// The first of the wave's entries at which the running sum passes `left` (64: none); `left` less what lies before it.
+__device__ __forceinline__ int pass_point(unsigned long long mine, unsigned long long& left) {
+    const unsigned long long incl = wave_scan_dpp64(mine);
+    const unsigned long long over = __ballot(incl > left);
+    if (!over) return 64;
+    const int at = __ffsll((long long)over) - 1;
+    left -= readlane64(incl - mine, at);
+    return at;
+}
+
 // The slice that holds the nucleus threshold, from the parts' slices: what lies above it is summed by segment, its own
 // logits leave the part as a list.
 template <typename T>
 __global__ void __launch_bounds__(NT)
 sample_slice_kernel(SampleParams p) {
-    __shared__ unsigned long long wave_mass[NW];
-    __shared__ unsigned int n_list, found;
-    __shared__ unsigned long long left;
+    __shared__ unsigned int n_list;
     const int row_idx = blockIdx.x, part = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
@@ -1512,33 +1543,21 @@ sample_slice_kernel(SampleParams p) {
     const bool vec = ((uintptr_t)row % 16) == 0 && n == SEG;
     float x[PART_SLOTS];
     load_segment<T, false>(row, begin, n, ((uintptr_t)row % 16) == 0, lane, x);
-    // this lane's two slices over all parts
-    static_assert(NBINS == 2 * NT, "two slices per lane");
-    unsigned long long h0 = 0, h1 = 0;
-    const unsigned long long* hist = p.part_hist + (int64_t)row_idx * p.parts * NBINS + 2 * tid;
-    for (int q0 = 0; q0 < p.parts; q0 += 8) {
-        ulonglong2 h[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) h[q] = *(const ulonglong2*)(hist + (int64_t)min(q0 + q, p.parts - 1) * NBINS);
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-            if (q0 + q < p.parts) { h0 += h[q].x; h1 += h[q].y; }
-    }
+    if (tid == 0) n_list = 0;
     unsigned long long w[SEGS_PER_LANE];
-    const unsigned long long z = readlane64(
-        wave_scan_dpp64(lane_segments(p.seg_mass + (int64_t)row_idx * p.parts * NW, p.parts * NW, lane, w)), 63);
-    const unsigned long long limit = (unsigned long long)((double)fmaxf(p.top_p, 0.f) * (double)z);
-    if (tid == 0) { n_list = 0; found = NBINS; left = 0; }
-    const unsigned long long incl = wave_scan_dpp64(h0 + h1);
-    if (lane == 63) wave_mass[wave] = incl;
+    const unsigned long long mine = lane_segments(p.seg_mass + (int64_t)row_idx * p.parts * NW, p.parts * NW, lane, w);
+    // every wave for itself: the group of slices, then the slice, at which the sum passes the limit
+    const unsigned long long groups = sum_of_parts(p.part_group + (int64_t)row_idx * p.parts * GROUPS, GROUPS, p.parts, lane);
+    const unsigned long long z = readlane64(wave_scan_dpp64(mine), 63);
+    unsigned long long left = (unsigned long long)((double)fmaxf(p.top_p, 0.f) * (double)z);
+    const int group = pass_point(groups, left);
+    int slice = NBINS;                               // the slices do not reach it (or there is no mass)
+    if (group < GROUPS) {
+        const int64_t at = (int64_t)row_idx * p.parts * NBINS + group * GROUP;
+        const unsigned long long h = sum_of_parts(p.part_hist + at, NBINS, p.parts, lane % GROUP);
+        slice = group * GROUP + pass_point(lane < GROUP ? h : 0, left);
+    }
     __syncthreads();
-    unsigned long long above = incl - h0 - h1;
-    for (int v = 0; v < wave; ++v) above += wave_mass[v];
-    // the slice at which the sum passes the limit: one, or none if the slices do not reach it
-    if (above <= limit && limit < above + h0) { found = 2 * tid; left = limit - above; }
-    if (above + h0 <= limit && limit < above + h0 + h1) { found = 2 * tid + 1; left = limit - above - h0; }
-    __syncthreads();
-    const int slice = (int)found;
     if (part == 0 && tid == 0) { p.cut[2 * row_idx] = slice; p.cut[2 * row_idx + 1] = left; }
     if (slice == NBINS) return;
     const float m = apply_temperature<T>(row_max_of_parts(p, row_idx, lane), p.temperature);
@@ -1688,14 +1707,13 @@ greedy_kernel(SampleParams p) {
 //   other calls from six parts on
 //     k to 256          128256: 1 row 24.3 -> 21.1, 16 25.5 -> 24.6, 64 27.0 -> 30.3: up to 128 parts
 //     greedy            128256: 16 rows 9.1 -> 7.2, 64 10.8 -> 9.8, 128 14.1 -> 17.2: up to 512 parts
-// A nucleus of the whole row takes four launches, the third of which reads 16 KB of slices for every part of its row from each
-// part's workgroup, so it pays from four parts on and as long as the workgroups are resident at once.  us per call,
-// temperature 0.8, top_p 0.9, one launch -> parts:
-//   float32  32000, 2 parts: 1 row 21.0 -> 22.1;  50256, 4: 1 row 24.3 -> 22.7, 64 25.7 -> 24.4, 128 26.1 -> 36.6;  50257: 64 35.3 -> 25.5
-//            81920, 5: 64 rows 35.9 -> 32.9, 128 38.4 -> 53.3;  128256, 8: 1 row 41.5 -> 23.3, 32 45.5 -> 24.9, 64 45.7 -> 38.4,
-//            128 55.1 -> 79.1;  262144, 16: 1 row 74.4 -> 24.4, 32 86.9 -> 42.6
-//   bf16     128256: 1 row 44.7 -> 24.2, 64 48.1 -> 36.2, 128 49.1 -> 64.9
-constexpr int NUCLEUS_MIN_PARTS = 4, NUCLEUS_MAX_BATCH = 64, NUCLEUS_MAX_ALL = 512;
+// A nucleus of the whole row takes four launches, about 22 us of them where a row is short, so it pays from four parts on and
+// while the rows leave CUs idle.  us per call, temperature 0.8, top_p 0.9, one launch -> parts:
+//   float32  32000, 2 parts: 1 row 21.0 -> 22.4;  50256, 4: 1 row 24.3 -> 22.4, 64 25.7 -> 24.8, 128 26.1 -> 34.2;  50257: 64 35.3 -> 25.7
+//            81920, 5: 64 rows 35.9 -> 31.7, 128 38.4 -> 48.1;  128256, 8: 1 row 41.5 -> 23.3, 32 45.5 -> 25.1, 64 45.7 -> 34.5,
+//            128 55.1 -> 65.5;  262144, 16: 1 row 74.4 -> 25.0, 64 92.5 -> 67.7, 128 101 -> 114
+//   bf16     128256: 1 row 44.7 -> 23.8, 64 48.1 -> 34.1, 128 49.1 -> 53.8
+constexpr int NUCLEUS_MIN_PARTS = 4, NUCLEUS_MAX_BATCH = 64;
 static bool whole_row(int vocab, int top_k, int greedy) { return !greedy && (top_k <= 0 || top_k >= vocab); }
 static int sample_parts(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy, int dtype) {
     const int parts = (int)(((int64_t)vocab + PART_MAX - 1) / PART_MAX);
@@ -1719,7 +1737,7 @@ static int part_capacity(int top_k, int greedy) { return greedy ? GREEDY_CAP : 2
 
 // Scratch of a draw from the whole row: the nucleus' share only where such a call is cut
 struct WholeRowSpace {
-    unsigned long long *seg_mass, *kept_mass, *part_hist, *cut;
+    unsigned long long *seg_mass, *kept_mass, *part_hist, *part_group, *cut;
     uint2* list;
     unsigned int* count;
     float* part_max;
@@ -1728,9 +1746,10 @@ struct WholeRowSpace {
         char* p = (char*)at;
         auto take = [&](size_t bytes_each, size_t n) { char* q = p; p += bytes_each * n; return q; };
         const size_t all = (size_t)batch * parts;
-        const bool nucleus = parts >= NUCLEUS_MIN_PARTS && batch <= NUCLEUS_MAX_BATCH && all <= NUCLEUS_MAX_ALL;
+        const bool nucleus = parts >= NUCLEUS_MIN_PARTS && batch <= NUCLEUS_MAX_BATCH;
         part_hist = (unsigned long long*)take(8 * NBINS, nucleus ? all : 0);         // first: 16-byte loads
         seg_mass = (unsigned long long*)take(8 * NW, all);
+        part_group = (unsigned long long*)take(8 * GROUPS, nucleus ? all : 0);
         kept_mass = (unsigned long long*)take(8 * NW, nucleus ? all : 0);
         list = (uint2*)take(8 * NUCLEUS_CAP, nucleus ? all : 0);
         cut = (unsigned long long*)take(16, nucleus ? batch : 0);
@@ -1780,7 +1799,7 @@ int launch_sample(int64_t* out, const void* logits, int64_t row_stride, float* p
     p.top_p = top_p; p.greedy = greedy;
     p.part_count = nullptr; p.part_list = nullptr; p.parts = 0; p.part_size = 0; p.part_cap = 0;
     p.seg_mass = nullptr; p.part_max = nullptr;
-    p.part_hist = nullptr; p.kept_mass = nullptr; p.cut = nullptr;
+    p.part_hist = nullptr; p.part_group = nullptr; p.kept_mass = nullptr; p.cut = nullptr;
     const size_t need = sample_workspace_bytes(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
     if (need && workspace && workspace_bytes >= need) {
         const int parts = sample_parts(batch, vocab, row_stride, temperature, top_k, greedy, dtype);
@@ -1794,7 +1813,7 @@ int launch_sample(int64_t* out, const void* logits, int64_t row_stride, float* p
             else {
                 p.seg_mass = at.seg_mass; p.part_max = at.part_max;
                 if (nucleus) {
-                    p.part_hist = at.part_hist; p.kept_mass = at.kept_mass; p.cut = at.cut;
+                    p.part_hist = at.part_hist; p.part_group = at.part_group; p.kept_mass = at.kept_mass; p.cut = at.cut;
                     p.part_list = at.list; p.part_count = at.count;
                 }
             }

@@ -403,10 +403,10 @@ int aicomp_sample_tokens(int64_t* out, const void* logits, int64_t row_stride,
  *   workspace       device scratch of aicomp_sample_workspace_bytes(...) bytes, 8-byte aligned, needing no
  *                   initialisation; calls that may overlap need separate ones.  NULL or less: one
  *                   launch, as aicomp_sample_tokens.  Per row and part of at most 16384 logits 2052 bytes
- *                   (greedy), 8 * min(1024, 256 + 8 * top_k) + 4, or with top_k off 132 (20.8 KB where a
- *                   nucleus is cut: up to 64 rows and 512 parts; the block then 16-byte aligned, or that
- *                   call is one launch); at most 1024 rows of 16 parts are cut.  64 rows of 128256:
- *                   2.7 MB at top_k 50, 10.6 MB with top_k off.
+ *                   (greedy), 8 * min(1024, 256 + 8 * top_k) + 4, or with top_k off 132 (21.3 KB where a
+ *                   nucleus is cut: up to 64 rows of at least four parts; the block then 16-byte
+ *                   aligned, or that call is one launch); at most 1024 rows of 16 parts are cut.  64
+ *                   rows of 128256: 2.7 MB at top_k 50, 10.9 MB with top_k off.
  */
 int aicomp_sample_tokens_split(int64_t* out, const void* logits, int64_t row_stride,
                                float* probs_out, const float* uniforms,

@@ -17,7 +17,9 @@ kernels read (``block_table``, ``context_lens``, ``slot_mapping``,
                     finish.  ``schedule()`` returns a ``StepPlan`` whose
                     tensors are already on the device: the whole plan is
                     packed into one pinned staging buffer and moved with a
-                    single asynchronous copy.
+                    single asynchronous copy.  A step of one token per
+                    running sequence is selected, packed and uploaded by
+                    ``csrc/fast_call.cpp`` where that is built.
 
 Row order inside a plan: sequences that ingest more than one token (prompt
 chunks) first, then the one-token sequences; ``paged_attention_step`` below

@@ -12,8 +12,8 @@
 //
 // Same checks, same errors (RuntimeError), same results as the registered operator.
 //
-// Beside it, the plain calls of aicomp_amd.ops (kv_append, rope_kv_append, paged_decode_attn,
-// paged_prefill_attn, sample_tokens): the same checks made here instead of in Python.  A call that
+// Beside it, the plain calls of aicomp_amd.ops (kv_append, rope_kv_append, paged_decode_attn, rope_paged_decode_attn,
+// paged_prefill_attn, append_prefill_attn, sample_tokens): the same checks made here instead of in Python.  A call that
 // passes them all is launched and returns true; any other returns false without having touched
 // anything, and the Python function goes on to convert what may be converted or to name what is wrong.
 #include <Python.h>

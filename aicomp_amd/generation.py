@@ -17,7 +17,8 @@ sequence, ``clear_cache`` resets.  Differences, all on purpose:
 
 ``PagedAttentionBackend`` owns one K and one V pool per layer and runs, per layer and
 step, the rotary embedding fused with the append followed by the chunked-prefill
-kernel on the prompt-chunk rows and the decode kernel on the one-token rows.
+kernel on the prompt-chunk rows and the decode kernel on the one-token rows; a small
+step of one-token rows alone is one launch (``ops.rope_paged_decode_attn``).
 """
 from __future__ import annotations
 

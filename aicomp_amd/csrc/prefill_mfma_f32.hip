@@ -402,8 +402,10 @@ int launch_prefill_mfma_f32(const DecodeArgs& a, int max_q_len) {
     //   one prompt of 512 (128)           73 /     /  31    one of 1024 (256)           143 /  88 / 110
     //   48 of 32 over 1000 (384)         269 / 232 /        one of 1600 (400)           223 / 201 /
     //   32 of 32 over 1000 (256)         152 / 154 / 188    one of 2048 (512)           280 / 318 /
+    //   11 of 9 to 38 over up to 431 (176) 72 / 40 /        13 of 46 over nothing (208) 16.8 / 19.3 /
     // Two of them also even out what CUs get in a causal prompt; beyond 400 the larger K/V traffic and a second round
-    // cost more.  The count is from what the host knows (all rows, the longest chunk), the same with and
+    // cost more.  Many short chunks without a prior context are where the split does not pay (two tiles of keys at most); the
+    // host does not know the priors, and with them it pays up to twice.  The count is from what the host knows (all rows, the longest chunk), the same with and
     // without a list of items, whose pairs name tiles of 128 rows.
     const int kw = wgs <= 128 ? 4 : wgs <= 400 ? 2 : 1;
     const int pos = pos_per_wg / kw;

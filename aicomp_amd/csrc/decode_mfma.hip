@@ -229,6 +229,9 @@ __device__ __forceinline__ void clear_state(WaveStateT<NO>& st) {
 // beyond the other zeroed.
 // PAIR: rows are token pairs (head_dim 64): row r of the tile holds tokens tile_start + 2r and
 // + 2r + 1, the B-operand columns are (head, parity) pairs, column c scoring token 2r + (c & 1).
+// ONCE (a decode row, which sees both tokens of a pair): the two share every dot product, the query column being zero
+// over the other token's half.  Rows of a chunk need not see the second token, and 0 times its key is NaN where that is
+// not finite: there each half of a row is summed by itself and a column takes its own (as many products).
 template <typename E, bool FP8, bool NEXT, bool MASK, bool PAIR, bool ONCE>
 __device__ __forceinline__ void process_tile(WaveState& st, TileRegs<FP8>& kr, TileRegs<FP8>& vr,
                                              const uint4 (&qf)[4], unsigned char* kt, const KTileOffsets& ko,
@@ -240,9 +243,9 @@ __device__ __forceinline__ void process_tile(WaveState& st, TileRegs<FP8>& kr, T
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         uint4 kk = tile_elems<E, FP8>(kr, i);
-        // PAIR: a row's two tokens share every dot product (the query column is zero over the other
-        // token's half), so a token beyond the context must not leave non-finite values in the row
-        if (PAIR && MASK && tile_start + 2 * (4 * i + g4) + ((lane & 15) >> 3) >= v_end) kk = make_uint4(0, 0, 0, 0);
+        // PAIR, one dot product for a row's two tokens: a token beyond the context must not leave non-finite
+        // values in the row
+        if (PAIR && ONCE && MASK && tile_start + 2 * (4 * i + g4) + ((lane & 15) >> 3) >= v_end) kk = make_uint4(0, 0, 0, 0);
         *(uint4*)(kt + ko.wr[i & 3] + i * 4 * KROW) = kk;
     }
     if (NEXT) {
@@ -251,13 +254,22 @@ __device__ __forceinline__ void process_tile(WaveState& st, TileRegs<FP8>& kr, T
     }
 
     // ---- S^T = K Q^T for the two 16-token sub-tiles
-    f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+    constexpr int NH = PAIR && !ONCE ? 2 : 1;            // sums of a row's score: its halves, or one
+    f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f}, t0 = s0, t1 = s1;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         const uint4 a0 = *(const uint4*)(kt + ko.rd[s]);
         const uint4 a1 = *(const uint4*)(kt + ko.rd[s] + 16 * KROW);
-        s0 = E::mfma(a0, qf[s], s0);
-        s1 = E::mfma(a1, qf[s], s1);
+        f32x4_t &x0 = NH == 2 && s >= 2 ? t0 : s0, &x1 = NH == 2 && s >= 2 ? t1 : s1;
+        x0 = E::mfma(a0, qf[s], x0);
+        x1 = E::mfma(a1, qf[s], x1);
+    }
+    if constexpr (NH == 2) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            s0[i] = lane & 1 ? t0[i] : s0[i];
+            s1[i] = lane & 1 ? t1[i] : s1[i];
+        }
     }
     // lane (head r16, g4) now holds tokens tile_start + 16a + 4i + g4 in s_a[i]
     float sc[8];

@@ -70,3 +70,32 @@ def test_chunks_alone_zero_rows_and_junk_pairs(device):
         assert (out[:40] == 0).all() and torch.isfinite(out.float()).all()
         want = tp.oracle(dict(c, ctx_list=[40, 30]))[40:]
         assert_close_attn(to_f64(out[40:]), want, 1e-2, 2e-2, "second chunk")
+
+
+@pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, None), (torch.float16, None), (torch.float16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("hq,hkv,d", [(4, 4, 64), (8, 2, 64), (6, 2, 64), (16, 2, 64), (8, 2, 128)])
+def test_keys_a_row_does_not_see(device, dtype, kv, hq, hkv, d):
+    """A later token's key that is not finite leaves the rows before it as they are, bit for bit; a visible key whose score
+    is -inf has weight 0, like one whose exponential underflows."""
+    c = tp.build_case(device, [2], [41], hq, hkv, d, dtype=dtype, kv_dtype=kv, seed=d + hq)
+    c["q"][..., 7] = c["q"][..., 7].abs() + 0.5
+
+    def run(t=None, key=None):
+        k = c["k_pool"].clone()
+        if t is not None:
+            rows = k[int(c["table"][0, (2 + t) // 16]), :, (2 + t) % 16]
+            rows[:, 7] = torch.tensor(key).to(k.dtype)
+            if kv is not None:
+                rows[:, 7] = torch.tensor(float("nan")).to(k.dtype)      # (e4m3 has no infinities)
+        out = torch.full_like(c["q"], float("nan"))
+        ops.append_prefill_attn(out, c["q"], None, None, k, c["v_pool"], None, c["table"], c["ctx"], c["cu"], c["scale"], 41,
+                                c["ks"], c["vs"])
+        return out.view(torch.int16)
+
+    clean = run()
+    assert torch.isfinite(clean.view(dtype)).all()
+    for t in (1, 2, 13, 14, 29, 30, 31, 40):
+        for key in (float("inf"), float("nan"), float("-inf")):
+            assert torch.equal(run(t, key)[:t], clean[:t]), (t, key)
+        if kv is None:
+            assert torch.equal(run(t, float("-inf")), run(t, -30000.0)), t

@@ -322,14 +322,26 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
         }
         return;
     }
+    // As they lie, the four lanes of a row would each write 16 bytes of four 64-byte segments.  Transposed over them (lane
+    // group and i change places: swaps of the halves of the wave, then of its odd and even rows) they write one segment.
+    // Of short fresh chunks the output is most of the bytes: 13 of 46, D 128 18.2 -> 17.0 us, D 64 11.2 -> 10.3;
+    // 32 of 24, 64/8 heads, D 128 25.8 -> 24.1.
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+        const auto u = __builtin_amdgcn_permlane32_swap(__float_as_uint(O[j][0]), __float_as_uint(O[j][2]), false, false);
+        const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(O[j][1]), __float_as_uint(O[j][3]), false, false);
+        const auto a = __builtin_amdgcn_permlane16_swap(u[0], v[0], false, false);
+        const auto b = __builtin_amdgcn_permlane16_swap(u[1], v[1], false, false);
+        O[j] = f32x4_t{__uint_as_float(a[0]), __uint_as_float(a[1]), __uint_as_float(b[0]), __uint_as_float(b[1])};
+    }
     if (row_valid) {
         const float inv = l > 0.f ? 1.f / l : 0.f;
-        float* o = p.out + ((int64_t)(q_begin + qpos) * p.hq + head) * DH + 16 * g4;
+        float* o = p.out + ((int64_t)(q_begin + qpos) * p.hq + head) * DH + 4 * g4;
 #pragma unroll
         for (int f = 0; f < HALVES; ++f)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                *(float4*)(o + 64 * f + 4 * i) =
+                *(float4*)(o + 64 * f + 16 * i) =
                     make_float4(O[4 * f][i] * inv, O[4 * f + 1][i] * inv, O[4 * f + 2][i] * inv, O[4 * f + 3][i] * inv);
     }
 }

@@ -407,19 +407,31 @@ int launch_prefill_mfma_f32(const DecodeArgs& a, int max_q_len) {
     p.num_cus = num_cus;
     p.items = a.items; p.num_seqs = a.num_seqs;
     const int groups = a.hq / p.gpack, pos_per_wg = WG_ROWS / p.gpack;
-    const int64_t tiles = (max_q_len + pos_per_wg - 1) / pos_per_wg;
-    const int64_t wgs = groups * std::min(tiles * a.num_seqs, a.rows / pos_per_wg + a.num_seqs);
+    // workgroups of `share` waves per row, from what the host knows (all rows, the longest chunk): the same with and
+    // without a list of items, whose pairs name tiles of 128 rows
+    const auto workgroups = [&](int share) {
+        const int64_t pos = pos_per_wg / share, tiles = (max_q_len + pos - 1) / pos;
+        return groups * std::min(tiles * a.num_seqs, a.rows / pos + a.num_seqs);
+    };
     // Waves that share rows (us, 32/8 heads, D 128, with 1 / 2 / 4 of them; in brackets the workgroups of 128 rows):
-    //   8 chunks of 32 over 2000 (64)    262 /     /  94    16 of 32 over 2000 (128)    270 /     / 188
+    //   8 chunks of 32 over 2000 (64)    262 /     /  94    one of 400 over 1024 (104)   188 / 110 / 113
     //   one prompt of 512 (128)           73 /     /  31    one of 1024 (256)           143 /  88 / 110
     //   48 of 32 over 1000 (384)         269 / 232 /        one of 1600 (400)           223 / 201 /
     //   32 of 32 over 1000 (256)         152 / 154 / 188    one of 2048 (512)           280 / 318 /
-    //   11 of 9 to 38 over up to 431 (176) 72 / 40 /        13 of 46 over nothing (208) 16.8 / 19.3 /
+    //   11 of 9 to 38 over up to 431 (176) 72 / 40 /
     // Two of them also even out what CUs get in a causal prompt; beyond 400 the larger K/V traffic and a second round
-    // cost more.  Many short chunks without a prior context are where the split does not pay (two tiles of keys at most); the
-    // host does not know the priors, and with them it pays up to twice.  The count is from what the host knows (all rows, the longest chunk), the same with and
-    // without a list of items, whose pairs name tiles of 128 rows.
-    const int kw = wgs <= 128 ? 4 : wgs <= 400 ? 2 : 1;
+    // cost more.  Many chunks have tiles alike, with nothing to even out: there workgroups beyond one per CU only wait
+    // for each other, whatever the prior contexts (in brackets the workgroups with 1 / 2 / 4):
+    //   8 of 46   (128 / 192 / 384)  14.6 / 13.7 / 18.4   over 1024  145 / 87 / 100
+    //   16 of 24  (128 / 256 / 384)  13.9 / 12.2 / 17.5   over 1024  143 / 85 / 102
+    //   13 of 46  (208 / 312 / 624)  17.0 / 19.1 / 25.6   over 256    51 / 53 / 58
+    //   8 of 70   (192 / 320 / 576)  20.1 / 22.6 / 23.9   over 64     29 / 31 / 33
+    const int64_t wgs = workgroups(1);
+    int kw = wgs <= 128 ? 4 : wgs <= 400 ? 2 : 1;
+    if (a.num_seqs >= 8) {
+        if (kw == 4 && workgroups(4) > 256) kw = 2;
+        else if (kw == 2 && wgs <= 256 && workgroups(2) > 256) kw = 1;
+    }
     const int pos = pos_per_wg / kw;
     const int qtiles = (max_q_len + pos - 1) / pos;
     AICOMP_REQUIRE(qtiles <= 65535, AICOMP_KV_EINVAL, "paged_prefill_attn: grid too large");

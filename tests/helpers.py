@@ -32,3 +32,12 @@ def assert_close_attn(got: np.ndarray, want: np.ndarray, atol: float, rtol: floa
         raise AssertionError(f"{what}: {(~ok).sum()} of {ok.size} elements out of tolerance; "
                              f"worst at {i}: got {got[i]}, want {want[i]}, max abs err {err.max():.3e}")
     assert np.isfinite(got).all(), f"{what}: non-finite output"
+
+
+def kernels_of(call) -> list:
+    """Names of the GPU kernels that `call()` launches, as the device ran them."""
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CUDA], acc_events=True) as prof:
+        call()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]

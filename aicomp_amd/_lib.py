@@ -28,13 +28,14 @@ SYMBOLS = (
     "aicomp_paged_prefill_tile_positions",
     "aicomp_rope_kv_append",
     "aicomp_rope_paged_decode_attn",
+    "aicomp_rope_paged_decode_attn_sized",
     "aicomp_sample_tokens",
     "aicomp_sample_tokens_split",
     "aicomp_sample_workspace_bytes",
 )
 
 F32, BF16, FP8_E4M3, F16 = 0, 1, 2, 3
-MIN_VERSION = 301            # 0.3.1: the entry points of SYMBOLS above
+MIN_VERSION = 302            # 0.3.2: the entry points of SYMBOLS above
 
 _lock = threading.RLock()       # torch_ops() loads the HIP library while holding it
 _lib = None
@@ -70,6 +71,9 @@ def _declare(lib: C.CDLL) -> None:
     lib.aicomp_rope_paged_decode_attn.argtypes = [vp, vp, i64, i64, vp, vp, i64, i64, vp, vp, i64, i64, vp, vp, vp, vp, vp,
                                                   i64, vp, i32, i32, i32, i32, i32, i32, i64, f32, i32, i32, vp, vp, vp,
                                                   sz, vp]
+    lib.aicomp_rope_paged_decode_attn_sized.restype = i32
+    lib.aicomp_rope_paged_decode_attn_sized.argtypes = (lib.aicomp_rope_paged_decode_attn.argtypes[:-3]
+                                                        + [i32] + lib.aicomp_rope_paged_decode_attn.argtypes[-3:])
     lib.aicomp_paged_decode_workspace_bytes.restype = sz
     lib.aicomp_paged_decode_workspace_bytes.argtypes = [i32] * 9
     lib.aicomp_paged_decode_partition_size.restype = i32

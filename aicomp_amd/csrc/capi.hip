@@ -3,6 +3,7 @@
 // include/aicomp_kv.h.
 #include "common.h"
 
+#include <algorithm>
 #include <stdlib.h>
 #include <string.h>
 
@@ -117,7 +118,7 @@ using namespace aicomp;
 
 extern "C" {
 
-int aicomp_kv_version(void) { return 301; }
+int aicomp_kv_version(void) { return 302; }
 
 const char* aicomp_kv_last_error(void) { return g_err; }
 
@@ -388,15 +389,15 @@ int aicomp_paged_decode_attn_append(void* out, const void* query, const void* ne
                        "paged_decode_attn_append");
 }
 
-int aicomp_rope_paged_decode_attn(void* out, const void* query, int64_t q_token_stride, int64_t q_head_stride,
-                                  const void* new_key, const void* new_value, int64_t kv_token_stride,
-                                  int64_t kv_head_stride, const void* cos, const void* sin, int64_t table_stride,
-                                  int64_t table_rows, const int64_t* positions, const int64_t* slot_mapping, void* k_pool,
-                                  void* v_pool, const int32_t* block_table, int64_t block_table_stride,
-                                  const int32_t* context_lens, int batch, int num_q_heads, int num_kv_heads, int head_dim,
-                                  int block_size, int max_blocks_per_seq, int64_t num_blocks, float scale, int q_dtype,
-                                  int kv_dtype, const float* k_scale, const float* v_scale, void* workspace,
-                                  size_t workspace_bytes, void* stream) {
+static int rope_decode_impl(void* out, const void* query, int64_t q_token_stride, int64_t q_head_stride,
+                            const void* new_key, const void* new_value, int64_t kv_token_stride,
+                            int64_t kv_head_stride, const void* cos, const void* sin, int64_t table_stride,
+                            int64_t table_rows, const int64_t* positions, const int64_t* slot_mapping, void* k_pool,
+                            void* v_pool, const int32_t* block_table, int64_t block_table_stride,
+                            const int32_t* context_lens, int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                            int block_size, int max_blocks_per_seq, int64_t num_blocks, float scale, int q_dtype,
+                            int kv_dtype, const float* k_scale, const float* v_scale, int longest_context, void* workspace,
+                            size_t workspace_bytes, void* stream) {
     const char* who = "rope_paged_decode_attn";
     AICOMP_REQUIRE(batch >= 0, AICOMP_KV_EINVAL, "%s: negative batch", who);
     if (batch == 0) return AICOMP_KV_OK;
@@ -410,6 +411,10 @@ int aicomp_rope_paged_decode_attn(void* out, const void* query, int64_t q_token_
     AICOMP_REQUIRE(q_head_stride >= head_dim && kv_head_stride >= head_dim && table_stride >= head_dim && table_rows > 0 &&
                    q_token_stride >= 0 && kv_token_stride >= 0, AICOMP_KV_EINVAL,
                    "%s: strides overlap rows of %d elements", who, head_dim);
+    AICOMP_REQUIRE(longest_context >= 0, AICOMP_KV_EINVAL, "%s: negative longest context", who);
+    // table columns to size the call for; the kernel's last partition takes a row that is longer after all
+    const int columns = longest_context == 0 ? max_blocks_per_seq
+                                             : std::min(max_blocks_per_seq, (int)(((int64_t)longest_context + block_size - 1) / block_size));
     const int64_t v = 16 / dtype_size(q_dtype);
     const bool vectors = (q_token_stride | q_head_stride | kv_token_stride | kv_head_stride | table_stride) % v == 0 &&
                          ((uintptr_t)new_key | (uintptr_t)new_value | (uintptr_t)cos | (uintptr_t)sin | (uintptr_t)query) % 16 == 0;
@@ -424,10 +429,10 @@ int aicomp_rope_paged_decode_attn(void* out, const void* query, int64_t q_token_
     a.scale = scale; a.q_dtype = q_dtype; a.kv_dtype = kv_dtype;
     a.k_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? k_scale : nullptr;
     a.v_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? v_scale : nullptr;
-    a.num_parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, shape, a.partition_size);
+    a.num_parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, columns, kv_dtype, shape, a.partition_size);
     a.stream = (hipStream_t)stream;
     // (a batch for the balanced schedule streams for tens of microseconds: the launch saved is lost in it)
-    AICOMP_REQUIRE(vectors && shape && small_call(batch, block_size, max_blocks_per_seq) && decode_mfma_supported(a),
+    AICOMP_REQUIRE(vectors && shape && small_call(batch, block_size, columns) && decode_mfma_supported(a),
                    AICOMP_KV_EUNSUPPORTED, "%s: not a call of the matrix-core grid schedule", who);
     a.new_key = new_key; a.new_value = new_value;
     a.new_token_stride = kv_token_stride; a.new_head_stride = kv_head_stride;
@@ -442,6 +447,38 @@ int aicomp_rope_paged_decode_attn(void* out, const void* query, int64_t q_token_
         a.ws = split_workspace_view(workspace, a.rows, a.hq, a.hkv, a.d, a.num_parts);
     }
     return launch_decode_mfma(a);
+}
+
+int aicomp_rope_paged_decode_attn(void* out, const void* query, int64_t q_token_stride, int64_t q_head_stride,
+                                  const void* new_key, const void* new_value, int64_t kv_token_stride,
+                                  int64_t kv_head_stride, const void* cos, const void* sin, int64_t table_stride,
+                                  int64_t table_rows, const int64_t* positions, const int64_t* slot_mapping, void* k_pool,
+                                  void* v_pool, const int32_t* block_table, int64_t block_table_stride,
+                                  const int32_t* context_lens, int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                  int block_size, int max_blocks_per_seq, int64_t num_blocks, float scale, int q_dtype,
+                                  int kv_dtype, const float* k_scale, const float* v_scale, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
+    return rope_decode_impl(out, query, q_token_stride, q_head_stride, new_key, new_value, kv_token_stride,
+                            kv_head_stride, cos, sin, table_stride, table_rows, positions, slot_mapping, k_pool, v_pool,
+                            block_table, block_table_stride, context_lens, batch, num_q_heads, num_kv_heads, head_dim,
+                            block_size, max_blocks_per_seq, num_blocks, scale, q_dtype, kv_dtype, k_scale, v_scale, 0,
+                            workspace, workspace_bytes, stream);
+}
+
+int aicomp_rope_paged_decode_attn_sized(void* out, const void* query, int64_t q_token_stride, int64_t q_head_stride,
+                                        const void* new_key, const void* new_value, int64_t kv_token_stride,
+                                        int64_t kv_head_stride, const void* cos, const void* sin, int64_t table_stride,
+                                        int64_t table_rows, const int64_t* positions, const int64_t* slot_mapping, void* k_pool,
+                                        void* v_pool, const int32_t* block_table, int64_t block_table_stride,
+                                        const int32_t* context_lens, int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                        int block_size, int max_blocks_per_seq, int64_t num_blocks, float scale, int q_dtype,
+                                        int kv_dtype, const float* k_scale, const float* v_scale, int longest_context, void* workspace,
+                                        size_t workspace_bytes, void* stream) {
+    return rope_decode_impl(out, query, q_token_stride, q_head_stride, new_key, new_value, kv_token_stride,
+                            kv_head_stride, cos, sin, table_stride, table_rows, positions, slot_mapping, k_pool, v_pool,
+                            block_table, block_table_stride, context_lens, batch, num_q_heads, num_kv_heads, head_dim,
+                            block_size, max_blocks_per_seq, num_blocks, scale, q_dtype, kv_dtype, k_scale, v_scale,
+                            longest_context, workspace, workspace_bytes, stream);
 }
 
 // Device address of `scratch` on the current device, looked up once per device.

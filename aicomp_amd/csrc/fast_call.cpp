@@ -395,23 +395,22 @@ PyObject* paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     }
 }
 
-// The table columns that `lens` tokens (a contiguous int32 buffer of n lengths) take, at most `columns`; all of
-// them without such a buffer, and for a launch that is being recorded.
-int columns_in_use(PyObject* lens, int64_t n, int bs, int64_t columns, void* stream) {
-    if (lens == Py_None) return (int)columns;
+// The longest of `lens` (a contiguous int32 buffer of n lengths), which sizes a call and bounds nothing; 0, for the whole
+// table, without such a buffer and for a launch that is being recorded, whose lengths may grow.
+int longest_of(PyObject* lens, int64_t n, void* stream) {
+    if (lens == Py_None) return 0;
     Py_buffer b;
-    if (PyObject_GetBuffer(lens, &b, PyBUF_FORMAT | PyBUF_ND) != 0) { PyErr_Clear(); return (int)columns; }
-    int64_t longest = columns * bs;
+    if (PyObject_GetBuffer(lens, &b, PyBUF_FORMAT | PyBUF_ND) != 0) { PyErr_Clear(); return 0; }
+    int longest = 0;
     if (b.itemsize == 4 && b.ndim == 1 && b.shape[0] == n && b.format && b.format[0] == 'i' && b.format[1] == 0) {
         longest = 1;
-        for (int64_t i = 0; i < n; ++i) longest = std::max<int64_t>(longest, ((const int32_t*)b.buf)[i]);
+        for (int64_t i = 0; i < n; ++i) longest = std::max(longest, ((const int32_t*)b.buf)[i]);
     }
     PyBuffer_Release(&b);
-    const int64_t used = std::min<int64_t>(columns, (longest + bs - 1) / bs);
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (used < columns && (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone))
-        return (int)columns;
-    return (int)used;
+    if (longest && (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone))
+        return 0;
+    return longest;
 }
 
 // (the output comes back as a new tensor; None: not a plain call of the one launch, nothing done)
@@ -445,20 +444,21 @@ PyObject* rope_paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t na
         const int hq = (int)q->size(1);
         const c10::DeviceGuard guard(q->device());
         void* stream = stream_of(*q);
-        const int width = columns_in_use(args[11], B, p.bs, table->size(1), stream);
+        const int width = (int)table->size(1), longest = longest_of(args[11], B, stream);
+        const int sized = longest == 0 ? width : (int)std::min<int64_t>(width, ((int64_t)longest + p.bs - 1) / p.bs);
         at::Tensor scratch;
-        const size_t need = aicomp_paged_decode_workspace_bytes((int)B, hq, p.hkv, p.d, p.bs, width, dt, p.dt, 0);
+        const size_t need = aicomp_paged_decode_workspace_bytes((int)B, hq, p.hkv, p.d, p.bs, sized, dt, p.dt, 0);
         if (need) scratch = cached_scratch(q->device(), stream, need);
         at::Tensor out(at::detail::empty_cuda(q->sizes(), st, q->device(), c10::MemoryFormat::Contiguous));
         const int rc = unlocked([&] {
             std::unique_lock<std::mutex> one_at_a_time(scratch_launches(), std::defer_lock);
             if (need) one_at_a_time.lock();
-            return aicomp_rope_paged_decode_attn(
+            return aicomp_rope_paged_decode_attn_sized(
                 out.data_ptr(), q->data_ptr(), q->stride(0), q->stride(1), key->data_ptr(), value->data_ptr(), key->stride(0),
                 key->stride(1), cos->data_ptr(), sin->data_ptr(), cos->stride(0), cos->size(0),
                 (const int64_t*)pos->data_ptr(), (const int64_t*)slots->data_ptr(), p.k->data_ptr(), p.v->data_ptr(),
                 (const int32_t*)table->data_ptr(), table->stride(0), (const int32_t*)ctx->data_ptr(), (int)B, hq, p.hkv, p.d,
-                p.bs, width, p.nb, (float)scale, dt, p.dt, p.ks, p.vs, need ? scratch.data_ptr() : nullptr,
+                p.bs, width, p.nb, (float)scale, dt, p.dt, p.ks, p.vs, longest, need ? scratch.data_ptr() : nullptr,
                 need ? (size_t)scratch.numel() : 0, stream);
         });
         if (rc == AICOMP_KV_EUNSUPPORTED) Py_RETURN_NONE;

@@ -437,10 +437,11 @@ def rope_paged_decode_attn(query: torch.Tensor, key: torch.Tensor, value: torch.
     made: a batch for the balanced schedule, and whatever is not a plain call.
 
     ``host_lens``: the same lengths on the host (a contiguous int32 numpy array), or ``None``.  With them the call is sized
-    for the table columns in use and not for the longest sequence the table could hold, so that rows that are short
-    now are whole in one launch; a launch recorded into a graph, whose lengths may grow, is sized for the whole table.
+    for the longest of them and not for the longest sequence the table could hold, so that rows that are short
+    now are whole in one launch; what is attended to follows from ``context_lens`` alone.  A launch recorded into a graph,
+    whose lengths may grow, is sized for the whole table.
     """
-    if not (_native("aicomp_rope_paged_decode_attn") and _lib.untouched("aicomp_rope_kv_append")
+    if not (_native("aicomp_rope_paged_decode_attn_sized") and _lib.untouched("aicomp_rope_kv_append")
             and _lib.untouched("aicomp_paged_decode_attn")):
         return None
     return _FAST.rope_paged_decode_attn(query, key, value, cos, sin, positions, k_pool, v_pool, slot_mapping, block_table,

@@ -46,7 +46,8 @@ extern "C" {
 #define AICOMP_KV_FP8_E4M3  2       /* OCP e4m3 ("e4m3fn"), max finite 448       */
 #define AICOMP_KV_F16       3       /* IEEE binary16                             */
 
-/* Library version (major*10000 + minor*100 + patch).  301 = 0.3.1: added
+/* Library version (major*10000 + minor*100 + patch).  302 = 0.3.2: added
+ * aicomp_rope_paged_decode_attn_sized.  301 = 0.3.1: added
  * aicomp_rope_paged_decode_attn and aicomp_kv_append_prefill_attn.  300 = 0.3.0: added
  * aicomp_sample_tokens_split and aicomp_sample_workspace_bytes.  200 = 0.2.0: added
  * aicomp_kv_set_small_decode_tokens, aicomp_paged_prefill_attn_items and
@@ -214,6 +215,30 @@ int aicomp_rope_paged_decode_attn(void* out, const void* query,
                                   const float* k_scale, const float* v_scale,
                                   void* workspace, size_t workspace_bytes,
                                   void* stream);
+
+/*
+ * The same, sized for rows of at most longest_context tokens (0: for the whole table, as above): the rows
+ * that are short now are then whole in one launch, or in the partitions they fill.  It says how the work is cut
+ * and nothing else: a row that is longer is attended to in full (in more time), and what counts as a small call
+ * and the scratch follow from the table columns that longest_context tokens take.
+ */
+int aicomp_rope_paged_decode_attn_sized(void* out, const void* query,
+                                        int64_t q_token_stride, int64_t q_head_stride,
+                                        const void* new_key, const void* new_value,
+                                        int64_t kv_token_stride, int64_t kv_head_stride,
+                                        const void* cos, const void* sin,
+                                        int64_t table_stride, int64_t table_rows,
+                                        const int64_t* positions, const int64_t* slot_mapping,
+                                        void* k_pool, void* v_pool,
+                                        const int32_t* block_table, int64_t block_table_stride,
+                                        const int32_t* context_lens,
+                                        int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                        int block_size, int max_blocks_per_seq, int64_t num_blocks,
+                                        float scale, int q_dtype, int kv_dtype,
+                                        const float* k_scale, const float* v_scale,
+                                        int longest_context,
+                                        void* workspace, size_t workspace_bytes,
+                                        void* stream);
 
 /*
  * aicomp_paged_decode_attn_append for callers that cannot allocate device memory (code under

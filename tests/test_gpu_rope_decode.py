@@ -105,3 +105,17 @@ def test_what_it_declines(device, decode_routing):
     lib = _lib.load()
     assert lib.aicomp_rope_paged_decode_attn(*([None] * 2), 0, 0, None, None, 0, 0, None, None, 0, 0, *([None] * 5), 0, None, 1,
                                              4, 2, 64, 16, 1, 4, 1.0, 1, 1, None, None, None, 0, None) == 1
+
+
+@pytest.mark.parametrize("dtype,kv,d", [(torch.bfloat16, None, 64), (torch.float32, None, 128), (torch.float16, torch.float8_e4m3fn, 128)])
+@pytest.mark.parametrize("known", [1, 40, 300, 900])
+def test_lengths_on_the_host_only_size_the_call(device, decode_routing, dtype, kv, d, known):
+    """Rows that have grown past what the host knows of them: in full, whether the call is sized for whole rows (40, 300
+    tokens) or for partitions (900)."""
+    c = _case(device, dtype, kv or dtype, 8, 2, d, [1500, 1, 800, 257, 40, 33], 4)
+    c["cos"], c["sin"] = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, d, 2) / d).to(device), 1600, dtype)
+    got, want = _one(c, np.minimum(c["lens"], known)), _two(c, c["table"].shape[1])
+    # float32 sums and weights in another order, then the output's own rounding
+    tol = 2e-6 if dtype == torch.float32 else 2e-3
+    assert (got[0].float() - want[0].float()).abs().max().item() <= tol
+    assert torch.equal(_bits(got[1]), _bits(want[1])) and torch.equal(_bits(got[2]), _bits(want[2]))

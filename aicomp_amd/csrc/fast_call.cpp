@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cstring>
 #include <map>
 #include <vector>
 #include <mutex>
@@ -413,14 +414,42 @@ int longest_of(PyObject* lens, int64_t n, void* stream) {
     return longest;
 }
 
+// Whether every row's slot is where its table has the row's last token, or none (a padding row): host copies of the
+// lengths, slots and table (contiguous int32 [n], int64 [n], int32 [n, columns]).
+bool slots_at_table(PyObject* lens, PyObject* slots, PyObject* table, int64_t n, int bs) {
+    struct View {
+        Py_buffer b{};
+        bool held;
+        View(PyObject* o, const char* kind, Py_ssize_t size) {
+            held = PyObject_GetBuffer(o, &b, PyBUF_FORMAT | PyBUF_ND) == 0;
+            if (!held) PyErr_Clear();
+            ok = held && b.itemsize == size && b.format && strchr(kind, b.format[0]) && b.format[1] == 0;
+        }
+        ~View() { if (held) PyBuffer_Release(&b); }
+        bool ok;
+    };
+    const View l(lens, "i", 4), s(slots, "lq", 8), t(table, "i", 4);
+    if (!l.ok || !s.ok || !t.ok || l.b.ndim != 1 || s.b.ndim != 1 || t.b.ndim != 2 || l.b.shape[0] != n || s.b.shape[0] != n ||
+        t.b.shape[0] != n)
+        return false;
+    const int64_t columns = t.b.shape[1];
+    for (int64_t r = 0; r < n; ++r) {
+        const int64_t slot = ((const int64_t*)s.b.buf)[r], last = (int64_t)((const int32_t*)l.b.buf)[r] - 1;
+        if (slot < 0) continue;
+        if (last < 0 || last / bs >= columns || slot != (int64_t)((const int32_t*)t.b.buf)[r * columns + last / bs] * bs + last % bs)
+            return false;
+    }
+    return true;
+}
+
 // (the output comes back as a new tensor; None: not a plain call of the one launch, nothing done)
 PyObject* rope_paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     try {
         Pools p;
         double scale;
-        if (nargs != 15)
+        if (nargs != 17)
             FAIL("rope_paged_decode_attn(query, key, value, cos, sin, positions, k_pool, v_pool, slot_mapping, block_table, "
-                 "context_lens, host_lens, scale, k_scale, v_scale)");
+                 "context_lens, host_lens, scale, k_scale, v_scale, host_slots, host_table)");
         const at::Tensor *q = plain(args[0]), *key = plain(args[1]), *value = plain(args[2]), *cos = plain(args[3]),
                          *sin = plain(args[4]), *pos = plain(args[5]), *slots = plain(args[8]), *table = plain(args[9]),
                          *ctx = plain(args[10]);
@@ -439,7 +468,8 @@ PyObject* rope_paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t na
             p.bs <= 0 || table->size(0) != B || table->stride(1) != 1 || table->size(1) <= 0 || table->size(1) > INT_MAX ||
             !vector_of(pos, at::kLong, B, *q) || !vector_of(slots, at::kLong, B, *q) || !vector_of(ctx, at::kInt, B, *q) ||
             !on(*table, *q) || !on(*key, *q) || !on(*value, *q) || !on(*cos, *q) || !on(*sin, *q) || !on(*p.k, *q) ||
-            (p.dt != dt && p.dt != AICOMP_KV_FP8_E4M3) || !p.scales(args[13], args[14]))
+            (p.dt != dt && p.dt != AICOMP_KV_FP8_E4M3) || !p.scales(args[13], args[14]) ||
+            (args[15] != Py_None && !slots_at_table(args[11], args[15], args[16], B, p.bs)))
             Py_RETURN_NONE;
         const int hq = (int)q->size(1);
         const c10::DeviceGuard guard(q->device());

@@ -75,7 +75,8 @@ class PagedAttentionBackend:
         if self.cos is not None and plan.num_prefill_seqs == 0:          # one token per sequence: one launch, if it can be
             out = ops.rope_paged_decode_attn(query, key, value, self.cos, self.sin, plan.positions, kp, vp,
                                              plan.slot_mapping, plan.block_table, plan.context_lens,
-                                             plan.host_context_lens, self.scale, ks, vs)
+                                             plan.host_context_lens, self.scale, ks, vs, plan.host_slot_mapping,
+                                             plan.host_block_table)
             if out is not None:
                 return out
         out = torch.empty(query.shape, dtype=query.dtype, device=query.device)

@@ -430,11 +430,18 @@ def step_items(context_lens, new_lens, num_prefill_seqs: int, tile_positions: in
 def rope_paged_decode_attn(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                            positions: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, slot_mapping: torch.Tensor,
                            block_table: torch.Tensor, context_lens: torch.Tensor, host_lens, scale: float,
-                           k_scale: Optional[torch.Tensor] = None,
-                           v_scale: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                           k_scale: Optional[torch.Tensor] = None, v_scale: Optional[torch.Tensor] = None,
+                           host_slots=None, host_table=None) -> Optional[torch.Tensor]:
     """``rope_kv_append`` of one new token per sequence and ``paged_decode_attn`` with its rotated query, in one launch:
-    the attention output ``[B, Hq, D]``, bit for bit that of the two calls, or ``None`` (nothing done) where the two are to be
-    made: a batch for the balanced schedule, and whatever is not a plain call.
+    the attention output ``[B, Hq, D]``, or ``None`` (nothing done) where the two are to be made: a batch for the balanced
+    schedule, and whatever is not a plain call.  The pools are those of the two calls bit for bit; so is the output where
+    both cut the rows alike (a table as wide as ``host_lens`` makes it here), and otherwise it agrees as results of
+    different splits do.
+
+    A row's slot has to be where its table has the row's last token, and in no other row's context: rows are stored while
+    others are read.  (A slot in no context of the call, or none, is fine.)  ``host_slots`` / ``host_table``: host copies
+    of ``slot_mapping`` (int64) and ``block_table`` (int32), by which, with ``host_lens``, the first is checked and
+    ``None`` returned where it does not hold.
 
     ``host_lens``: the same lengths on the host (a contiguous int32 numpy array), or ``None``.  With them the call is sized
     for the longest of them and not for the longest sequence the table could hold, so that rows that are short
@@ -445,7 +452,7 @@ def rope_paged_decode_attn(query: torch.Tensor, key: torch.Tensor, value: torch.
             and _lib.untouched("aicomp_paged_decode_attn")):
         return None
     return _FAST.rope_paged_decode_attn(query, key, value, cos, sin, positions, k_pool, v_pool, slot_mapping, block_table,
-                                        context_lens, host_lens, scale, k_scale, v_scale)
+                                        context_lens, host_lens, scale, k_scale, v_scale, host_slots, host_table)
 
 
 def paged_prefill_attn(out: torch.Tensor, query: torch.Tensor, k_pool: torch.Tensor,

@@ -193,8 +193,11 @@ int aicomp_paged_decode_attn_append(void* out, const void* query,
  *   cos, sin, table_stride, table_rows, positions, slot_mapping
  *                       as in aicomp_rope_kv_append, one entry per row b
  * The result equals aicomp_rope_kv_append of the rows followed by aicomp_paged_decode_attn on
- * the rotated query, bit for bit; a row whose position has no table row is not stored and its
- * output row is unspecified.  Covers small calls of the matrix-core kernels (what
+ * the rotated query, bit for bit, provided that no slot is read by the call except as the last
+ * token of its own row: a slot is block_table[b][n / block_size] * block_size + n % block_size of
+ * row b, n = context_lens[b] - 1, and in no other row's context, or it is in no context of the call
+ * (rows are stored while others are read; an append before the call has no such restriction).  A
+ * row whose position has no table row is not stored and its output row is unspecified.  Covers small calls of the matrix-core kernels (what
  * aicomp_kv_set_small_decode_tokens says of batch * max_blocks_per_seq * block_size), rows that can be
  * read 16 bytes at a time; any other call is AICOMP_KV_EUNSUPPORTED with nothing done.  Scratch:
  * aicomp_paged_decode_workspace_bytes with partition_size 0.

@@ -69,49 +69,10 @@ def test_one_launch_equals_two(device, decode_routing, dtype, kv, hq, hkv, d):
 
 
 @pytest.mark.parametrize("dtype,kv,d", [(torch.bfloat16, None, 64), (torch.float32, None, 128), (torch.float16, torch.float8_e4m3fn, 128)])
-def test_split_rows_and_odd_slots(device, decode_routing, dtype, kv, d):
-    """Rows of several partitions; a padding row, a row stored elsewhere, one without a table row, an empty one."""
-    c = _case(device, dtype, kv or dtype, 8, 2, d, [1500, 1, 800, 257, 40, 33], 3)
-    c["cos"], c["sin"] = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, d, 2) / d).to(device), 1600, dtype)
-    for got, want in zip(_one(c, c["lens"]), _two(c, 94)):
-        assert torch.equal(_bits(got), _bits(want))
-    used = set(c["table"][:, :94].flatten().tolist())
-    spare = next(b for b in range(c["pools"][0].shape[0]) if b not in used)
-    c["slots"][1], c["slots"][2], c["pos"][3] = -1, spare * 16 + 5, 5000
-    c["ctx"][4] = 0
-    got, want = _one(c, c["lens"]), _two(c, 94)
-    rows = [0, 1, 2, 4, 5]
-    assert torch.equal(_bits(got[0][rows]), _bits(want[0][rows]))
-    assert torch.equal(_bits(got[1]), _bits(want[1])) and torch.equal(_bits(got[2]), _bits(want[2]))
-
-
-def test_what_it_declines(device, decode_routing):
-    """Batches for the balanced schedule, other head dims, rows that cannot be read in vectors: None, and nothing written."""
-    c = _case(device, torch.bfloat16, torch.bfloat16, 8, 2, 64, CTX, 1)
-    prev = ops.set_small_decode_tokens(0)
-    try:
-        assert _one(c, c["lens"])[0] is None
-    finally:
-        ops.set_small_decode_tokens(prev)
-    odd = torch.empty(c["q"].numel() + 1, dtype=torch.bfloat16, device=device)[1:].view(c["q"].shape)
-    odd.copy_(c["q"])
-    c["q"] = odd
-    out, kp, vp = _one(c, c["lens"])
-    assert out is None and torch.equal(_bits(kp), _bits(c["pools"][0])) and torch.equal(_bits(vp), _bits(c["pools"][1]))
-    w = _case(device, torch.bfloat16, torch.bfloat16, 4, 2, 256, [5, 20], 2)
-    assert _one(w, w["lens"])[0] is None
-    w["table"] = w["table"].long()
-    assert _one(w, w["lens"])[0] is None
-    lib = _lib.load()
-    assert lib.aicomp_rope_paged_decode_attn(*([None] * 2), 0, 0, None, None, 0, 0, None, None, 0, 0, *([None] * 5), 0, None, 1,
-                                             4, 2, 64, 16, 1, 4, 1.0, 1, 1, None, None, None, 0, None) == 1
-
-
-@pytest.mark.parametrize("dtype,kv,d", [(torch.bfloat16, None, 64), (torch.float32, None, 128), (torch.float16, torch.float8_e4m3fn, 128)])
-@pytest.mark.parametrize("known", [1, 40, 300, 900])
+@pytest.mark.parametrize("known", [1, 40, 300, 900, 1500])
 def test_lengths_on_the_host_only_size_the_call(device, decode_routing, dtype, kv, d, known):
-    """Rows that have grown past what the host knows of them: in full, whether the call is sized for whole rows (40, 300
-    tokens) or for partitions (900)."""
+    """Rows that have grown past what the host knows of them: in full, whether the call is sized for whole rows (1 to 300
+    tokens) or for partitions; against a call that is sized for the table."""
     c = _case(device, dtype, kv or dtype, 8, 2, d, [1500, 1, 800, 257, 40, 33], 4)
     c["cos"], c["sin"] = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, d, 2) / d).to(device), 1600, dtype)
     got, want = _one(c, np.minimum(c["lens"], known)), _two(c, c["table"].shape[1])
@@ -119,3 +80,38 @@ def test_lengths_on_the_host_only_size_the_call(device, decode_routing, dtype, k
     tol = 2e-6 if dtype == torch.float32 else 2e-3
     assert (got[0].float() - want[0].float()).abs().max().item() <= tol
     assert torch.equal(_bits(got[1]), _bits(want[1])) and torch.equal(_bits(got[2]), _bits(want[2]))
+
+
+@pytest.mark.parametrize("dtype,kv", KINDS)
+def test_a_slot_that_is_read_takes_two_calls(device, decode_routing, dtype, kv):
+    """Rows whose slot is an earlier place of their own sequence, or the last one of another's: the append comes first, as in
+    the two calls; a padding row does not stand in the way of the one launch."""
+    import aicomp_amd.block_manager as bm
+    from aicomp_amd.generation import PagedAttentionBackend
+    c = _case(device, dtype, kv or dtype, 8, 2, 64, [70, 33, 18, 129], 5)
+    B, host_table, slots = 4, c["table"].cpu().numpy(), c["slots"].cpu().numpy()
+    backend = PagedAttentionBackend(1, c["pools"][0].shape[0], 2, 64, dtype=dtype, device=device, kv_dtype=kv,
+                                    inv_freq=1.0 / 10000 ** (torch.arange(0, 64, 2) / 64).to(device), max_positions=512)
+    if kv is not None:
+        backend.set_scales(0, *c["scales"])
+    for slot, one in ((None, True), (-1, True), (host_table[0, 1] * 16 + 3, False), (slots[3], False)):
+        s = slots.copy()
+        if slot is not None:
+            s[0] = slot
+        if slot == slots[3]:
+            s[3] = -1
+        c["slots"] = torch.from_numpy(s).to(device)
+        backend.k_pools[0], backend.v_pools[0] = (p.clone() for p in c["pools"])
+        assert one == (ops.rope_paged_decode_attn(
+            c["q"], c["k"], c["v"], c["cos"], c["sin"], c["pos"], c["pools"][0].clone(), c["pools"][1].clone(), c["slots"],
+            c["table"], c["ctx"], c["lens"], c["scale"], *c["scales"], s, host_table) is not None)
+        cu = np.arange(B + 1, dtype=np.int32)
+        backend.begin_step(bm.StepPlan(
+            seq_ids=list(range(B)), num_prefill_seqs=0, new_lens=np.ones(B, dtype=np.int32), max_q_len=0, total_new_tokens=B,
+            block_table=c["table"], context_lens=c["ctx"], cu_q_lens=torch.from_numpy(cu).to(device), slot_mapping=c["slots"],
+            positions=c["pos"], preempted=[], host_block_table=host_table, host_context_lens=c["lens"], host_cu_q_lens=cu,
+            host_slot_mapping=s, host_positions=c["lens"].astype(np.int64) - 1))
+        out = backend.attend(0, c["q"], c["k"], c["v"])
+        want = _two(c, c["table"].shape[1] if not one else 9)
+        assert torch.equal(_bits(out), _bits(want[0])), slot
+        assert torch.equal(_bits(backend.k_pools[0]), _bits(want[1])) and torch.equal(_bits(backend.v_pools[0]), _bits(want[2]))

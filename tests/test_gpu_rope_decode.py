@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from aicomp_amd import _lib, ops
+from helpers import kernels_of
 
 pytestmark = [pytest.mark.gpu, pytest.mark.routing("library")]
 CTX = [1, 2, 16, 17, 31, 32, 33, 63, 64, 65, 128, 129, 300, 7]
@@ -66,6 +67,61 @@ def test_one_launch_equals_two(device, decode_routing, dtype, kv, hq, hkv, d):
     for lens, width in ((c["lens"], 19), (None, c["table"].shape[1])):
         for got, want in zip(_one(c, lens), _two(c, width)):
             assert torch.equal(_bits(got), _bits(want)), (width,)
+
+
+@pytest.mark.parametrize("dtype,kv,hq,hkv,d,longest", [
+    (torch.bfloat16, None, 8, 2, 128, 600), (torch.float16, None, 4, 4, 128, 513), (torch.bfloat16, torch.float8_e4m3fn, 8, 2, 128, 600),
+    (torch.float16, torch.float8_e4m3fn, 16, 2, 128, 640), (torch.bfloat16, None, 8, 2, 64, 1100), (torch.float16, None, 16, 2, 64, 1280),
+    (torch.float32, None, 8, 2, 64, 640), (torch.float32, None, 16, 2, 64, 600), (torch.float32, None, 8, 2, 128, 400),
+    (torch.float32, None, 16, 2, 128, 448)])
+def test_rows_of_eight_waves(device, decode_routing, dtype, kv, hq, hkv, d, longest):
+    """Rows that are whole and long in few workgroups."""
+    c = _case(device, dtype, kv or dtype, hq, hkv, d, [longest, 1, longest - 17, 65, 255, 256, 257], hq + d)
+    c["cos"], c["sin"] = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, d, 2) / d).to(device), 1300, dtype)
+    got = []
+    names = [n for n in kernels_of(lambda: got.extend(_one(c, c["lens"]))) if "paged_decode" in n]
+    assert len(names) == 1 and "8, true>" in names[0], names
+    for a, b in zip(got, _two(c, -(-longest // 16))):
+        assert torch.equal(_bits(a), _bits(b))
+
+
+@pytest.mark.parametrize("dtype,kv,d", [(torch.bfloat16, None, 64), (torch.float32, None, 128), (torch.float16, torch.float8_e4m3fn, 128)])
+def test_split_rows_and_odd_slots(device, decode_routing, dtype, kv, d):
+    """Rows of several partitions; a padding row, a row stored elsewhere, one without a table row, an empty one."""
+    c = _case(device, dtype, kv or dtype, 8, 2, d, [1500, 1, 800, 257, 40, 33], 3)
+    c["cos"], c["sin"] = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, d, 2) / d).to(device), 1600, dtype)
+    for got, want in zip(_one(c, c["lens"]), _two(c, 94)):
+        assert torch.equal(_bits(got), _bits(want))
+    used = set(c["table"][:, :94].flatten().tolist())
+    spare = next(b for b in range(c["pools"][0].shape[0]) if b not in used)
+    c["slots"][1], c["slots"][2], c["pos"][3] = -1, spare * 16 + 5, 5000
+    c["ctx"][4] = 0
+    got, want = _one(c, c["lens"]), _two(c, 94)
+    rows = [0, 1, 2, 4, 5]
+    assert torch.equal(_bits(got[0][rows]), _bits(want[0][rows]))
+    assert torch.equal(_bits(got[1]), _bits(want[1])) and torch.equal(_bits(got[2]), _bits(want[2]))
+
+
+def test_what_it_declines(device, decode_routing):
+    """Batches for the balanced schedule, other head dims, rows that cannot be read in vectors: None, and nothing written."""
+    c = _case(device, torch.bfloat16, torch.bfloat16, 8, 2, 64, CTX, 1)
+    prev = ops.set_small_decode_tokens(0)
+    try:
+        assert _one(c, c["lens"])[0] is None
+    finally:
+        ops.set_small_decode_tokens(prev)
+    odd = torch.empty(c["q"].numel() + 1, dtype=torch.bfloat16, device=device)[1:].view(c["q"].shape)
+    odd.copy_(c["q"])
+    c["q"] = odd
+    out, kp, vp = _one(c, c["lens"])
+    assert out is None and torch.equal(_bits(kp), _bits(c["pools"][0])) and torch.equal(_bits(vp), _bits(c["pools"][1]))
+    w = _case(device, torch.bfloat16, torch.bfloat16, 4, 2, 256, [5, 20], 2)
+    assert _one(w, w["lens"])[0] is None
+    w["table"] = w["table"].long()
+    assert _one(w, w["lens"])[0] is None
+    lib = _lib.load()
+    assert lib.aicomp_rope_paged_decode_attn(*([None] * 2), 0, 0, None, None, 0, 0, None, None, 0, 0, *([None] * 5), 0, None, 1,
+                                             4, 2, 64, 16, 1, 4, 1.0, 1, 1, None, None, None, 0, None) == 1
 
 
 @pytest.mark.parametrize("dtype,kv,d", [(torch.bfloat16, None, 64), (torch.float32, None, 128), (torch.float16, torch.float8_e4m3fn, 128)])

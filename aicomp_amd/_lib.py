@@ -18,6 +18,7 @@ SYMBOLS = (
     "aicomp_kv_set_small_decode_tokens",
     "aicomp_kv_append",
     "aicomp_kv_append_prefill_attn",
+    "aicomp_kv_append_prefill_attn_sized",
     "aicomp_paged_decode_attn",
     "aicomp_paged_decode_attn_append",
     "aicomp_paged_decode_attn_append_static",
@@ -89,6 +90,8 @@ def _declare(lib: C.CDLL) -> None:
     lib.aicomp_kv_append_prefill_attn.restype = i32
     lib.aicomp_kv_append_prefill_attn.argtypes = [vp, vp, vp, vp, i64, i64, vp, vp, vp, vp, i64, vp, vp, i32, i64, i32, i32,
                                                   i32, i32, i32, i32, i64, f32, i32, i32, vp, vp, vp, i32, vp]
+    lib.aicomp_kv_append_prefill_attn_sized.restype = i32
+    lib.aicomp_kv_append_prefill_attn_sized.argtypes = lib.aicomp_kv_append_prefill_attn.argtypes[:-1] + [i32, vp]
     lib.aicomp_paged_prefill_tile_positions.restype = i32
     lib.aicomp_paged_prefill_tile_positions.argtypes = [i32] * 7
     lib.aicomp_rope_kv_append.restype = i32

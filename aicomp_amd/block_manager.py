@@ -694,7 +694,7 @@ def paged_attention_step(plan: StepPlan, out: torch.Tensor, query: torch.Tensor,
         # chunks alone: the tensors as they are (a slice costs a microsecond)
         return ops.append_prefill_attn(out, query, key, value, k_pool, v_pool, plan.slot_mapping, plan.block_table,
                                        plan.context_lens, plan.cu_q_lens, scale, plan.max_q_len, k_scale, v_scale,
-                                       plan.prefill_items(query, k_pool))
+                                       plan.prefill_items(query, k_pool), plan.host_context_lens)
     if S and npre == 0:
         return ops.paged_decode_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens, scale, k_scale,
                                      v_scale, new_key=key, new_value=value)

@@ -550,7 +550,7 @@ static int prefill_impl(void* out, const void* query, const void* k_pool, const 
                         int head_dim, int block_size, int max_blocks_per_seq,
                         int64_t num_blocks, float scale, int q_dtype, int kv_dtype,
                         const float* k_scale, const float* v_scale, const int32_t* items, int num_items,
-                        bool chunks, void* stream) {
+                        bool chunks, int longest_context, void* stream) {
     AICOMP_REQUIRE(num_seqs >= 0 && total_q >= 0, AICOMP_KV_EINVAL,
                    "paged_prefill_attn: negative sizes");
     if (num_seqs == 0 || total_q == 0) return AICOMP_KV_OK;
@@ -582,7 +582,7 @@ static int prefill_impl(void* out, const void* query, const void* k_pool, const 
     // an item list is taken by the two matrix-instruction kernels (and only while its length fits a
     // grid dimension); the other kernels walk the whole grid, which covers the same tiles
     if (items != nullptr && num_items <= 65535) { a.items = items; a.num_items = num_items; }
-    a.chunks = chunks;
+    a.chunks = chunks; a.longest_context = longest_context;
     if (prefill_mfma_supported(a, max_q_len)) return launch_prefill_mfma(a, max_q_len);
     // float32 models at head_dim 64 / 128: the float32 matrix instruction
     if (prefill_mfma_f32_supported(a, max_q_len)) return launch_prefill_mfma_f32(a, max_q_len);
@@ -607,7 +607,7 @@ int aicomp_paged_prefill_attn(void* out, const void* query, const void* k_pool, 
     return prefill_impl(out, query, k_pool, v_pool, block_table, block_table_stride, context_lens, cu_q_lens,
                         num_seqs, total_q, max_q_len, num_q_heads, num_kv_heads, head_dim, block_size,
                         max_blocks_per_seq, num_blocks, scale, q_dtype, kv_dtype, k_scale, v_scale, nullptr, 0,
-                        false, stream);
+                        false, 0, stream);
 }
 
 int aicomp_paged_prefill_attn_items(void* out, const void* query, const void* k_pool, const void* v_pool,
@@ -623,16 +623,17 @@ int aicomp_paged_prefill_attn_items(void* out, const void* query, const void* k_
     return prefill_impl(out, query, k_pool, v_pool, block_table, block_table_stride, context_lens, cu_q_lens,
                         num_seqs, total_q, max_q_len, num_q_heads, num_kv_heads, head_dim, block_size,
                         max_blocks_per_seq, num_blocks, scale, q_dtype, kv_dtype, k_scale, v_scale,
-                        num_items > 0 ? items : nullptr, num_items, false, stream);
+                        num_items > 0 ? items : nullptr, num_items, false, 0, stream);
 }
 
-int aicomp_kv_append_prefill_attn(void* out, const void* query, const void* key, const void* value, int64_t kv_token_stride,
-                                  int64_t kv_head_stride, void* k_pool, void* v_pool, const int64_t* slot_mapping,
-                                  const int32_t* block_table, int64_t block_table_stride, const int32_t* context_lens,
-                                  const int32_t* cu_q_lens, int num_seqs, int64_t total_q, int max_q_len, int num_q_heads,
-                                  int num_kv_heads, int head_dim, int block_size, int max_blocks_per_seq, int64_t num_blocks,
-                                  float scale, int q_dtype, int kv_dtype, const float* k_scale, const float* v_scale,
-                                  const int32_t* items, int num_items, void* stream) {
+static int append_prefill_impl(void* out, const void* query, const void* key, const void* value, int64_t kv_token_stride,
+                               int64_t kv_head_stride, void* k_pool, void* v_pool, const int64_t* slot_mapping,
+                               const int32_t* block_table, int64_t block_table_stride, const int32_t* context_lens,
+                               const int32_t* cu_q_lens, int num_seqs, int64_t total_q, int max_q_len, int num_q_heads,
+                               int num_kv_heads, int head_dim, int block_size, int max_blocks_per_seq, int64_t num_blocks,
+                               float scale, int q_dtype, int kv_dtype, const float* k_scale, const float* v_scale,
+                               const int32_t* items, int num_items, int longest_context, void* stream) {
+    AICOMP_REQUIRE(longest_context >= 0, AICOMP_KV_EINVAL, "kv_append_prefill_attn: negative longest context");
     AICOMP_REQUIRE(num_items >= 0 && (items != nullptr || num_items == 0), AICOMP_KV_EINVAL,
                    "kv_append_prefill_attn: %d items without a list", num_items);
     if (key != nullptr) {
@@ -644,7 +645,33 @@ int aicomp_kv_append_prefill_attn(void* out, const void* query, const void* key,
     return prefill_impl(out, query, k_pool, v_pool, block_table, block_table_stride, context_lens, cu_q_lens,
                         num_seqs, total_q, max_q_len, num_q_heads, num_kv_heads, head_dim, block_size,
                         max_blocks_per_seq, num_blocks, scale, q_dtype, kv_dtype, k_scale, v_scale,
-                        num_items > 0 ? items : nullptr, num_items, true, stream);
+                        num_items > 0 ? items : nullptr, num_items, true, longest_context, stream);
+}
+
+int aicomp_kv_append_prefill_attn(void* out, const void* query, const void* key, const void* value, int64_t kv_token_stride,
+                                  int64_t kv_head_stride, void* k_pool, void* v_pool, const int64_t* slot_mapping,
+                                  const int32_t* block_table, int64_t block_table_stride, const int32_t* context_lens,
+                                  const int32_t* cu_q_lens, int num_seqs, int64_t total_q, int max_q_len, int num_q_heads,
+                                  int num_kv_heads, int head_dim, int block_size, int max_blocks_per_seq, int64_t num_blocks,
+                                  float scale, int q_dtype, int kv_dtype, const float* k_scale, const float* v_scale,
+                                  const int32_t* items, int num_items, void* stream) {
+    return append_prefill_impl(out, query, key, value, kv_token_stride, kv_head_stride, k_pool, v_pool, slot_mapping,
+                               block_table, block_table_stride, context_lens, cu_q_lens, num_seqs, total_q, max_q_len,
+                               num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, num_blocks, scale,
+                               q_dtype, kv_dtype, k_scale, v_scale, items, num_items, 0, stream);
+}
+
+int aicomp_kv_append_prefill_attn_sized(void* out, const void* query, const void* key, const void* value, int64_t kv_token_stride,
+                                        int64_t kv_head_stride, void* k_pool, void* v_pool, const int64_t* slot_mapping,
+                                        const int32_t* block_table, int64_t block_table_stride, const int32_t* context_lens,
+                                        const int32_t* cu_q_lens, int num_seqs, int64_t total_q, int max_q_len, int num_q_heads,
+                                        int num_kv_heads, int head_dim, int block_size, int max_blocks_per_seq, int64_t num_blocks,
+                                        float scale, int q_dtype, int kv_dtype, const float* k_scale, const float* v_scale,
+                                        const int32_t* items, int num_items, int longest_context, void* stream) {
+    return append_prefill_impl(out, query, key, value, kv_token_stride, kv_head_stride, k_pool, v_pool, slot_mapping,
+                               block_table, block_table_stride, context_lens, cu_q_lens, num_seqs, total_q, max_q_len,
+                               num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, num_blocks, scale,
+                               q_dtype, kv_dtype, k_scale, v_scale, items, num_items, longest_context, stream);
 }
 
 int aicomp_paged_prefill_tile_positions(int num_q_heads, int num_kv_heads, int head_dim, int block_size,

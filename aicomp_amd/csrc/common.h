@@ -291,6 +291,7 @@ struct DecodeArgs {
     const int32_t* items;
     int num_items;
     bool chunks;                // prefill only: the call is a step's prompt chunks and nothing else
+    int longest_context;        // prefill only: what the caller knows of context_lens (0: nothing); chooses a kernel, bounds nothing
 };
 
 int launch_decode_generic(const DecodeArgs& a);

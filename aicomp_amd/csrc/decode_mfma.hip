@@ -1419,16 +1419,14 @@ int launch_prefill_rows(const DecodeArgs& a, int max_q_len, int tile_pos, int64_
     AICOMP_REQUIRE(tiles <= 65535 && tile_pos % pos == 0, AICOMP_KV_EINVAL, "paged_prefill_attn: grid too large");
     dim3 grid((unsigned)groups, (unsigned)a.num_seqs, (unsigned)tiles);
     if (a.items != nullptr) grid = dim3((unsigned)groups, (unsigned)a.num_items, (unsigned)p.sub);
-    const bool wide = wgs <= 32;
-#define AICOMP_LAUNCH_ROWS(...)                                                                                              \
-    do {                                                                                                                     \
-        if (wide) hipLaunchKernelGGL((paged_prefill_rows_kernel<__VA_ARGS__, 8>), grid, dim3(512), 0, a.stream, p);          \
-        else hipLaunchKernelGGL((paged_prefill_rows_kernel<__VA_ARGS__, 4>), grid, dim3(256), 0, a.stream, p);               \
-    } while (0)
-#define AICOMP_LAUNCH_ROWS16(E)                                                                                       \
-    do {                                                                                                              \
-        if (d64) { if (fp8) AICOMP_LAUNCH_ROWS(Tile16<E, true, true, false>); else AICOMP_LAUNCH_ROWS(Tile16<E, false, true, false>); }   \
-        else { if (fp8) AICOMP_LAUNCH_ROWS(Tile16<E, true, false, false>); else AICOMP_LAUNCH_ROWS(Tile16<E, false, false, false>); }     \
+    const bool wide = wgs <= 32;                     // (at D 64 always)
+#define AICOMP_LAUNCH_ROWS(NW, ...)                                                                                          \
+    hipLaunchKernelGGL((paged_prefill_rows_kernel<__VA_ARGS__, NW>), grid, dim3(64 * NW), 0, a.stream, p)
+#define AICOMP_LAUNCH_ROWS16(E)                                                                                               \
+    do {                                                                                                                      \
+        if (d64) { if (fp8) AICOMP_LAUNCH_ROWS(8, Tile16<E, true, true, false>); else AICOMP_LAUNCH_ROWS(8, Tile16<E, false, true, false>); }        \
+        else if (wide) { if (fp8) AICOMP_LAUNCH_ROWS(8, Tile16<E, true, false, false>); else AICOMP_LAUNCH_ROWS(8, Tile16<E, false, false, false>); } \
+        else { if (fp8) AICOMP_LAUNCH_ROWS(4, Tile16<E, true, false, false>); else AICOMP_LAUNCH_ROWS(4, Tile16<E, false, false, false>); }          \
     } while (0)
     if (a.q_dtype == AICOMP_KV_F16) AICOMP_LAUNCH_ROWS16(F16Fmt); else AICOMP_LAUNCH_ROWS16(Bf16Fmt);
 #undef AICOMP_LAUNCH_ROWS16

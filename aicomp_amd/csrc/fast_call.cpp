@@ -397,8 +397,8 @@ PyObject* paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
 }
 
 // The longest of `lens` (a contiguous int32 buffer of n lengths), which sizes a call and bounds nothing; 0, for the whole
-// table, without such a buffer and for a launch that is being recorded, whose lengths may grow.
-int longest_of(PyObject* lens, int64_t n, void* stream) {
+// table, without such a buffer.
+int longest_of(PyObject* lens, int64_t n) {
     if (lens == Py_None) return 0;
     Py_buffer b;
     if (PyObject_GetBuffer(lens, &b, PyBUF_FORMAT | PyBUF_ND) != 0) { PyErr_Clear(); return 0; }
@@ -408,10 +408,13 @@ int longest_of(PyObject* lens, int64_t n, void* stream) {
         for (int64_t i = 0; i < n; ++i) longest = std::max(longest, ((const int32_t*)b.buf)[i]);
     }
     PyBuffer_Release(&b);
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (longest && (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone))
-        return 0;
     return longest;
+}
+
+// (a status that cannot be had counts as recording)
+bool recording(void* stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
 }
 
 // Whether every row's slot is where its table has the row's last token, or none (a padding row): host copies of the
@@ -474,7 +477,10 @@ PyObject* rope_paged_decode_attn(PyObject*, PyObject* const* args, Py_ssize_t na
         const int hq = (int)q->size(1);
         const c10::DeviceGuard guard(q->device());
         void* stream = stream_of(*q);
-        const int width = (int)table->size(1), longest = longest_of(args[11], B, stream);
+        // a recorded launch is sized for the whole table: the lengths of its replays may grow by any amount
+        const int width = (int)table->size(1);
+        int longest = longest_of(args[11], B);
+        if (longest != 0 && ((int64_t)longest + p.bs - 1) / p.bs < width && recording(stream)) longest = 0;
         const int sized = longest == 0 ? width : (int)std::min<int64_t>(width, ((int64_t)longest + p.bs - 1) / p.bs);
         at::Tensor scratch;
         const size_t need = aicomp_paged_decode_workspace_bytes((int)B, hq, p.hkv, p.d, p.bs, sized, dt, p.dt, 0);
@@ -544,9 +550,9 @@ PyObject* append_prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs
         int dt, max_q_len;
         int64_t S;
         double scale;
-        if (nargs != 15)
+        if (nargs != 16)
             FAIL("append_prefill_attn(out, query, k_pool, v_pool, block_table, context_lens, cu_q_lens, scale, max_q_len, "
-                 "k_scale, v_scale, items, key, value, slot_mapping)");
+                 "k_scale, v_scale, items, key, value, slot_mapping, host_lens)");
         if (!attention_args(args, out, q, p, table, ctx, dt, S) || !as_double(args[7], scale) ||
             !as_int(args[8], max_q_len) || !p.scales(args[9], args[10]))
             Py_RETURN_FALSE;
@@ -570,14 +576,15 @@ PyObject* append_prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs
         }
         const c10::DeviceGuard guard(q->device());
         void* stream = stream_of(*q);
+        const int longest = longest_of(args[15], S);
         const int rc = unlocked([&] {
-            return aicomp_kv_append_prefill_attn(
+            return aicomp_kv_append_prefill_attn_sized(
                 out->data_ptr(), q->data_ptr(), key ? key->data_ptr() : nullptr, key ? value->data_ptr() : nullptr,
                 key ? key->stride(0) : 0, key ? key->stride(1) : 0, p.k->data_ptr(), p.v->data_ptr(),
                 key ? (const int64_t*)slots->data_ptr() : nullptr, (const int32_t*)table->data_ptr(), table->stride(0),
                 (const int32_t*)ctx->data_ptr(), (const int32_t*)cu->data_ptr(), (int)S, q->size(0), max_q_len,
                 (int)q->size(1), p.hkv, p.d, p.bs, (int)table->size(1), p.nb, (float)scale, dt, p.dt, p.ks, p.vs,
-                items ? (const int32_t*)items->data_ptr() : nullptr, items ? (int)items->size(0) : 0, stream);
+                items ? (const int32_t*)items->data_ptr() : nullptr, items ? (int)items->size(0) : 0, longest, stream);
         });
         DONE(rc);
     } catch (const std::exception& e) {

@@ -711,20 +711,32 @@ int prefill_mfma_tile_positions(int hq, int hkv, int max_q_len) {
 
 int launch_prefill_mfma(const DecodeArgs& a, int max_q_len) {
     if (a.chunks) {
-        // Small grids (see paged_prefill_rows_kernel); in brackets the workgroups this kernel would have.  us of a step, its
-        // append included, here / there (12 to 14 us are the host's):
-        //   D 128  8/8 heads  200 after 1500 (16) 40 / 18;  2 of 162 after 1700 (32) 43 / 19;  4 of 164 after 1000 (64) 31 / 22
-        //          32/8       200 after 1500 (56) 41 / 25;  4 of 64 after 1000 (64) 30 / 21;   2 of 162 after 1700 (96) 44 / 42;
-        //                     500 (128) 19.3 / 22.9;  64/8  200 after 1500 (104) 41 / 44
-        //   D 64   16/2       200 after 1500 (26) 30 / 20;  4 of 64 after 1000 (32) 22 / 18;   8 of 40 after 500 (48) 15 / 17;
-        //                     2 of 162 after 1700 (44) 32 / 27;  32/8  4 of 64 after 1000 (64) 22 / 24
-        // What is counted is known to the host (all rows, the longest chunk) and the same with and without a list.
+        // Small grids (see paged_prefill_rows_kernel), where the keys that a workgroup of this kernel walks take longer than
+        // what its waves' merge costs.  In brackets the workgroups this kernel would have, of one or two column groups, then
+        // the longest context; device us of a step, its append included, here / there:
+        //   D 128, one group    8/8 heads  4 of 24 (32) 24: 6.7 / 9.4, 152: 8.8 / 9.6, 280: 10.9 / 11.1, 536: 15.2 / 12.3
+        //                       8/8        8 of 46 (64) 110: 8.6 / 10.0, 302: 12.1 / 11.7, 558: 16.8 / 13.4
+        //          two          32/8       2 of 46 (32) 46: 10.0 / 9.7, 302: 14.7 / 11.5;  8/8  200 (16) 200: 11.9 / 9.9
+        //                       32/8       4 of 46 (64) 46: 10.1 / 10.6, 174: 12.6 / 13.0, 302: 15.0 / 14.2, 1070: 29.3 / 21.9
+        //                       32/8       one of 200 (56) 200: 12.4 / 11.9, 456: 18.0 / 14.9;  400 (104) 1424: 35.5 / 38.3
+        //   D 64, one           8/8        100 (16) 100: 6.9 / 7.9, 164: 7.6 / 7.8, 228: 8.3 / 8.0, 612: 13.0 / 9.4
+        //         two           16/2       4 of 24 (16) 24: 8.4 / 8.0, 280: 11.8 / 8.5
+        //                       32/8       100 (32) 100: 9.3 / 11.9, 356: 12.4 / 12.9, 612: 15.9 / 15.2, 1124: 22.5 / 17.7
+        //                       16/2       8 of 46 (48) 302: 11.8 / 14.9, 1070: 21.7 / 20.9
+        // (The tiles of one chunk are unlike, which more workgroups even out; those of several are not.)
+        // At D 64 a workgroup there has eight rows and a CU to itself: 32 column groups here are 256 of them, and beyond that
+        // they take turns.  Four waves instead of eight, two workgroups to a CU: D 128 beyond 32.
+        // What is counted is known to the host (all rows, the longest chunk and context) and the same with and without a list.
         const int tile_pos = prefill_mfma_tile_positions(a.hq, a.hkv, max_q_len);
-        const int group = a.hq / a.hkv, groups = a.hq / (16 % group == 0 ? group : 1);
+        const int group = a.hq / a.hkv, gpack = 16 % group == 0 ? group : 1, groups = a.hq / gpack;
         const int64_t tiles = (max_q_len + tile_pos - 1) / tile_pos;
         const int64_t wgs = groups * std::min(tiles * a.num_seqs, a.rows / tile_pos + a.num_seqs);
+        const int64_t keys = a.longest_context > 0 ? a.longest_context : (int64_t)a.max_blocks * a.bs;
+        const int cols = tile_pos * gpack / ROWS;
         // (sixteen heads of 64 are more rows per position than its workgroups have)
-        if (wgs <= (a.d == 64 ? 32 : 64) && !(a.d == 64 && group == 16)) return launch_prefill_rows(a, max_q_len, tile_pos, wgs);
+        const bool rows = a.d == 128 ? wgs <= 64 && (keys >= 256 || (cols == 2 && (wgs <= 32 || a.num_seqs == 1)))
+                                     : wgs <= 32 && group != 16 && (wgs * cols <= 32 ? cols == 2 || keys >= 192 : keys >= 600);
+        if (rows) return launch_prefill_rows(a, max_q_len, tile_pos, wgs);
     }
     PrefillParams p;
     p.out = a.out; p.query = a.query; p.k_pool = a.k_pool; p.v_pool = a.v_pool;

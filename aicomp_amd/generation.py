@@ -93,7 +93,8 @@ class PagedAttentionBackend:
                                           self.scale, max_q_len=plan.max_q_len, k_scale=ks, v_scale=vs, items=items)
         if plan.only_chunks and t_pre == query.shape[0]:     # chunks alone, rows alone: the plan's tensors as they are
             return ops.append_prefill_attn(out, q, None, None, kp, vp, None, plan.block_table, plan.context_lens,
-                                           plan.cu_q_lens, self.scale, plan.max_q_len, ks, vs, plan.prefill_items(q, kp))
+                                           plan.cu_q_lens, self.scale, plan.max_q_len, ks, vs, plan.prefill_items(q, kp),
+                                           plan.host_context_lens)
         if S and npre == 0:
             return ops.paged_decode_attn(out, q, kp, vp, plan.block_table, plan.context_lens, self.scale, ks, vs)
         if npre:

@@ -523,13 +523,16 @@ def append_prefill_attn(out: torch.Tensor, query: torch.Tensor, key: Optional[to
                         value: Optional[torch.Tensor], k_pool: torch.Tensor, v_pool: torch.Tensor,
                         slot_mapping: Optional[torch.Tensor], block_table: torch.Tensor, context_lens: torch.Tensor,
                         cu_q_lens: torch.Tensor, scale: float, max_q_len: int, k_scale: Optional[torch.Tensor] = None,
-                        v_scale: Optional[torch.Tensor] = None, items: Optional[torch.Tensor] = None) -> torch.Tensor:
+                        v_scale: Optional[torch.Tensor] = None, items: Optional[torch.Tensor] = None,
+                        host_lens=None) -> torch.Tensor:
     """A layer's step of prompt chunks and nothing else: ``kv_append`` of the new rows (``key`` None: they are in the pools
-    already) and ``paged_prefill_attn``, in one call, which may take the kernel for few chunks."""
-    if _native("aicomp_kv_append_prefill_attn") and _lib.untouched("aicomp_kv_append") \
+    already) and ``paged_prefill_attn``, in one call, which may take the kernel for few chunks.  ``host_lens``: the same
+    context lengths on the host (a contiguous int32 numpy array), or ``None``; the longest decides which kernel is the
+    faster one and nothing else (without them: what the table holds)."""
+    if _native("aicomp_kv_append_prefill_attn_sized") and _lib.untouched("aicomp_kv_append") \
             and _lib.untouched("aicomp_paged_prefill_attn") and _lib.untouched("aicomp_paged_prefill_attn_items") \
             and _FAST.append_prefill_attn(out, query, k_pool, v_pool, block_table, context_lens, cu_q_lens, scale, max_q_len,
-                                          k_scale, v_scale, items, key, value, slot_mapping):
+                                          k_scale, v_scale, items, key, value, slot_mapping, host_lens):
         return out
     if key is not None:
         kv_append(key, value, k_pool, v_pool, slot_mapping, k_scale, v_scale)

@@ -47,7 +47,7 @@ extern "C" {
 #define AICOMP_KV_F16       3       /* IEEE binary16                             */
 
 /* Library version (major*10000 + minor*100 + patch).  302 = 0.3.2: added
- * aicomp_rope_paged_decode_attn_sized.  301 = 0.3.1: added
+ * aicomp_rope_paged_decode_attn_sized and aicomp_kv_append_prefill_attn_sized.  301 = 0.3.1: added
  * aicomp_rope_paged_decode_attn and aicomp_kv_append_prefill_attn.  300 = 0.3.0: added
  * aicomp_sample_tokens_split and aicomp_sample_workspace_bytes.  200 = 0.2.0: added
  * aicomp_kv_set_small_decode_tokens, aicomp_paged_prefill_attn_items and
@@ -358,6 +358,26 @@ int aicomp_kv_append_prefill_attn(void* out, const void* query,
                                   const float* k_scale, const float* v_scale,
                                   const int32_t* items, int num_items,
                                   void* stream);
+
+/*
+ * The same for a caller that knows the longest context of the call (0: nothing known, as above, where the table's
+ * width stands for it): few short contexts are faster in one kernel, few long ones in the other.  It chooses
+ * between the two and nothing else.
+ */
+int aicomp_kv_append_prefill_attn_sized(void* out, const void* query,
+                                        const void* key, const void* value,
+                                        int64_t kv_token_stride, int64_t kv_head_stride,
+                                        void* k_pool, void* v_pool, const int64_t* slot_mapping,
+                                        const int32_t* block_table, int64_t block_table_stride,
+                                        const int32_t* context_lens, const int32_t* cu_q_lens,
+                                        int num_seqs, int64_t total_q, int max_q_len,
+                                        int num_q_heads, int num_kv_heads, int head_dim,
+                                        int block_size, int max_blocks_per_seq, int64_t num_blocks,
+                                        float scale, int q_dtype, int kv_dtype,
+                                        const float* k_scale, const float* v_scale,
+                                        const int32_t* items, int num_items,
+                                        int longest_context,
+                                        void* stream);
 
 /* Positions per query tile of the kernel a prefill call with these shapes runs on (0: none that takes an item list). */
 int aicomp_paged_prefill_tile_positions(int num_q_heads, int num_kv_heads, int head_dim, int block_size,

@@ -270,7 +270,7 @@ struct DecodeArgs {
     int q_dtype, kv_dtype;
     const float* k_scale;
     const float* v_scale;
-    int partition_size;         // tokens, multiple of bs; the decode grid's last partition takes what is left of a row
+    int partition_size;         // tokens, multiple of bs; the last one of a decode with rotary embedding takes what is left of a row
     int num_parts;              // ceil(max_blocks*bs / partition_size)
     SplitWorkspace ws;
     hipStream_t stream;

@@ -587,8 +587,8 @@ paged_decode_mfma_kernel(MfmaParams p) {
         }
         return;
     }
-    // (the last partition takes what is left of a row, where the caller's idea of the lengths sized the grid)
-    const int end = part + 1 == (int)gridDim.y ? len : min(len, start + p.partition_size);
+    // (ROPE: the caller's idea of the lengths sized the grid, and the last partition takes what is left of a row)
+    const int end = ROPE && part + 1 == p.num_parts ? len : min(len, start + p.partition_size);
     const int ntiles = (end - start + TT - 1) / TT;
 
     __shared__ float sm_m[NW][16];

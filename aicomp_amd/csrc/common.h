@@ -203,6 +203,18 @@ struct F16Fmt {
     static constexpr uint32_t SIGN_PAIR = 0x80008000u;
 };
 
+// max over lanes l and l^16 (l^32) by gfx950's lane swaps: v_permlane16_swap exchanges the odd 16-lane rows of its first
+// operand with the even rows of its second; with x in both, a lane has its own value in one result and its partner's in
+// the other.
+__device__ __forceinline__ float xor16_max(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float xor32_max(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // float32 tensors: outputs are stored as they are
 struct F32Fmt {
     typedef float elem;

@@ -89,19 +89,6 @@ struct MfmaParams {
     int64_t q_token_stride, q_head_stride;
 };
 
-// max over lanes l and l^16 (l^32) by gfx950's lane swaps (v_permlane16_swap exchanges the odd 16-lane rows of its first
-// operand with the even rows of its second).  A tile of a short row is a chain of latencies, of which two shuffles through
-// LDS and the range handling of exp2f were a tenth: one row of 500 tokens, D 64 5.82 -> 5.62 us, D 128 6.86 -> 6.40,
-// 16 rows of 700, 16 / 2 heads 11.4 -> 10.9; rows that stream as before.
-__device__ __forceinline__ float xor16_max(float x) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float xor32_max(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 template <bool FP8> struct TileRegs;
 template <> struct TileRegs<false> { uint4 r[8]; };
 template <> struct TileRegs<true> { uint2 r[8]; };
@@ -285,6 +272,9 @@ __device__ __forceinline__ void process_tile(WaveState& st, TileRegs<FP8>& kr, T
     }
     float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])),
                      fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
+    // A tile of a short row is a chain of latencies, of which two shuffles through LDS and the range handling of exp2f were a
+    // tenth: one row of 500 tokens, D 64 5.82 -> 5.62 us, D 128 6.86 -> 6.40, 16 rows of 700, 16 / 2 heads 11.4 -> 10.9;
+    // rows that stream as before.  (exp2f and the bare instruction differ below 2^-126 alone, which leaves it as 0.)
     mx = xor32_max(xor16_max(mx));
     const float m_new = fmaxf(st.m, mx);
     const float alpha = __builtin_amdgcn_exp2f(st.m - m_new);
@@ -534,6 +524,29 @@ __device__ __forceinline__ void store_new_row(const MfmaParams& p, const typenam
     }
 }
 
+// Dim dd of row h over a workgroup's waves: its max, weighted sum and weight (PAIR: over the two parity columns of the
+// row too, whose useful halves are elements 0..63 and 64..127 of their accumulators).
+template <typename T, int NW>
+__device__ __forceinline__ void merge_waves(const unsigned char* lds, const float (&sm_m)[NW][16], const float (&sm_l)[NW][16],
+                                            int h, int dd, float& mx, float& num, float& den) {
+    constexpr int NPAR = T::NPAR;
+    mx = NEG_BIG;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+        for (int par = 0; par < NPAR; ++par) mx = fmaxf(mx, sm_m[w][NPAR * h + par]);
+    num = den = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+        for (int par = 0; par < NPAR; ++par) {
+            const int c = NPAR * h + par;
+            const float f = exp2f(sm_m[w][c] - mx);
+            num = fmaf(f, ((const float*)(lds + w * KTILE_BYTES))[c * T::OROW + dd + 64 * par], num);
+            den = fmaf(f, sm_l[w][c], den);
+        }
+}
+
 // ROPE: the query rows come as projected, with strides of their own, and are rotated here, like the new K row: a decode
 // step of a layer is then this launch alone, where the rotary + append launch before it and the rotated query's way
 // through memory cost 3.3 us of device and 6 us of host time (8 rows of 900 tokens, 32 / 8 heads, D 64).
@@ -671,28 +684,12 @@ paged_decode_mfma_kernel(MfmaParams p) {
     }
     __syncthreads();
 
-    // merge of the waves (PAIR: and of the two parity columns of a head, whose useful halves are
-    // elements 0..63 and 64..127 of their accumulators)
     const float vs = T::FP8 ? p.v_scale[kvh] : 1.f;
     const bool direct = p.num_parts == 1;     // unsplit call: no merge needed
     for (int idx = tid; idx < G * DQ; idx += 64 * NW) {
         const int h = idx / DQ, dd = idx % DQ;
-        float mxw = NEG_BIG;
-#pragma unroll
-        for (int ww = 0; ww < NW; ++ww)
-#pragma unroll
-            for (int par = 0; par < NPAR; ++par) mxw = fmaxf(mxw, sm_m[ww][NPAR * h + par]);
-        float num = 0.f, den = 0.f;
-#pragma unroll
-        for (int ww = 0; ww < NW; ++ww) {
-#pragma unroll
-            for (int par = 0; par < NPAR; ++par) {
-                const int c = NPAR * h + par;
-                const float f = exp2f(sm_m[ww][c] - mxw);
-                num = fmaf(f, ((const float*)(lds + ww * KTILE_BYTES))[c * T::OROW + dd + 64 * par], num);
-                den = fmaf(f, sm_l[ww][c], den);
-            }
-        }
+        float mxw, num, den;
+        merge_waves<T, NW>(lds, sm_m, sm_l, h, dd, mxw, num, den);
         const int head = kvh * G + h;
         if (direct) {
             ((typename T::Fmt::raw*)p.out)[((int64_t)seq * p.hq + head) * DQ + dd] =
@@ -827,20 +824,8 @@ paged_prefill_rows_kernel(PrefillRowsParams p) {
         const int h = idx / DQ, dd = idx % DQ;
         Raw* o = out_row(h);
         if (o == nullptr) continue;
-        float mx = NEG_BIG, num = 0.f, den = 0.f;
-#pragma unroll
-        for (int ww = 0; ww < NW; ++ww)
-#pragma unroll
-            for (int par = 0; par < NPAR; ++par) mx = fmaxf(mx, sm_m[ww][NPAR * h + par]);
-#pragma unroll
-        for (int ww = 0; ww < NW; ++ww)
-#pragma unroll
-            for (int par = 0; par < NPAR; ++par) {
-                const int c = NPAR * h + par;
-                const float f = exp2f(sm_m[ww][c] - mx);
-                num = fmaf(f, ((const float*)(lds + ww * KTILE_BYTES))[c * T::OROW + dd + 64 * par], num);
-                den = fmaf(f, sm_l[ww][c], den);
-            }
+        float mx, num, den;
+        merge_waves<T, NW>(lds, sm_m, sm_l, h, dd, mx, num, den);
         o[dd] = T::Fmt::from_f32(den == 0.f ? 0.f : vs * num / den);
     }
 }

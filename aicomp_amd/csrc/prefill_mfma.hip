@@ -71,20 +71,6 @@ struct PrefillParams {
     int num_seqs;
 };
 
-// max over lanes l and l^16 (l^32): gfx950's lane-swap instructions, no LDS round trip.
-// v_permlane16_swap exchanges the odd 16-lane rows of its first operand with the even rows of
-// its second; with both operands holding x, every lane ends up with its own value in one
-// result and its partner's in the other.
-typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float xor16_max(float x) {
-    const u32x2_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float xor32_max(float x) {
-    const u32x2_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
 // register stage of one K and one V tile: NL loads of the workgroup each
 template <bool FP8, int NL> struct Stage;
 template <int NL> struct Stage<false, NL> { uint4 k[NL], v[NL]; };

@@ -171,3 +171,33 @@ def test_a_slot_that_is_read_takes_two_calls(device, decode_routing, dtype, kv):
         want = _two(c, c["table"].shape[1] if not one else 9)
         assert torch.equal(_bits(out), _bits(want[0])), slot
         assert torch.equal(_bits(backend.k_pools[0]), _bits(want[1])) and torch.equal(_bits(backend.v_pools[0]), _bits(want[2]))
+
+
+@pytest.mark.parametrize("dtype,kv,d", [(torch.bfloat16, None, 64), (torch.float32, None, 128), (torch.float16, torch.float8_e4m3fn, 128)])
+def test_a_recorded_launch_is_sized_for_the_table(device, decode_routing, dtype, kv, d):
+    """Recorded while the rows are short, replayed as they grow: the bits of the two calls over the whole table each time."""
+    c = _case(device, dtype, kv or dtype, 8, 2, d, [1500, 40, 800, 257], 6)
+    c["cos"], c["sin"] = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, d, 2) / d).to(device), 1600, dtype)
+    full, table = c["lens"].copy(), c["table"].cpu().numpy()
+
+    def at(lens):                                            # the rows as they are at these lengths
+        c["ctx"].copy_(torch.from_numpy(lens))
+        c["pos"].copy_(torch.from_numpy(lens.astype(np.int64) - 1))
+        c["slots"].copy_(torch.from_numpy(table[range(4), (lens - 1) // 16].astype(np.int64) * 16 + (lens - 1) % 16))
+
+    short = np.minimum(full, [30, 20, 10, 33]).astype(np.int32)
+    at(short)
+    _one(c, short)
+    kp, vp = (p.clone() for p in c["pools"])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.rope_paged_decode_attn(c["q"], c["k"], c["v"], c["cos"], c["sin"], c["pos"], kp, vp, c["slots"], c["table"],
+                                         c["ctx"], short, c["scale"], *c["scales"])
+    for lens in (short, np.minimum(full, 300), np.minimum(full, 1000), full):
+        at(lens)
+        for pool, first in zip((kp, vp), c["pools"]):
+            pool.copy_(first)
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, want in zip((out, kp, vp), _two(c, c["table"].shape[1])):
+            assert torch.equal(_bits(got), _bits(want)), lens

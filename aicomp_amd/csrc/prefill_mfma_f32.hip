@@ -230,7 +230,8 @@ paged_prefill_mfma_f32_kernel(PrefillF32Params p) {
 
         // ---- online softmax: lane (query r16, g4) holds tokens first + 16 h + 4 g4 + i.  The reference max m moves only
         // when a lane's probabilities of this tile add up to more than LAZY (always on a row's first tile), for all
-        // rows of the wave together: sums and products are the same floats scaled by a power of two at most 2^8.
+        // rows of the wave together: a lane's sum over a tile stays at most 2^8.  (Not the same floats as under the true
+        // max, which is further from m by some real number, but of the same relative error.)
         if (first + 16 * HB - 1 > wave_kv_min) {                       // wave-uniform
 #pragma unroll
             for (int k = 0; k < 4 * HB; ++k)

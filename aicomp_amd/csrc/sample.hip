@@ -1105,8 +1105,9 @@ __device__ __forceinline__ unsigned long long readlane64(unsigned long long v, i
     return (unsigned long long)hi << 32 | lo;
 }
 
-// The usual draw from the candidates of a row's parts, top_k <= 64: false (for the whole workgroup, nothing written)
-// where a list is longer than its lanes' FEW_SLOTS or more than FEW candidates pass the bound.
+// The usual draw from the candidates of a row's parts, top_k <= FewK: false (for the whole workgroup, nothing written)
+// where a list is longer than its lanes' FEW_SLOTS, more than FEW candidates pass the bound or, with the ties of the k-th,
+// more than 64 stay.
 //
 // Latency bound, one workgroup per row: what it takes is a chain of memory and LDS latencies and barriers, so it has
 // three of the latter.  The lists are read while their lengths are still on the way; a candidate's rank is counted with
@@ -1114,6 +1115,12 @@ __device__ __forceinline__ unsigned long long readlane64(unsigned long long v, i
 // at most 64 are left, which the first wave finishes in registers.  64 rows of eight parts, k = 50: 11.5 -> 5.2 us as traced (about ten barriers before, the mass
 // before an entry by two scans over all waves).
 constexpr int FEW = 256, FEW_K = 64;
+// 16-bit logits lie close enough for ties (bf16 a sixteenth apart between 8 and 16), so with k near 64 those of the k-th are
+// often a lane too many, and one such row holds up the launch.  64 rows of 32000, one launch, then parts: bf16 k 56 15.1 and
+// 13.2 us, k 60 15.2 and 16.8, k 64 15.4 and 17.6; fp16 k 60 15.3 and 13.4, k 64 15.4 and 17.5; 256 rows, k 64 15.5 and 20.2.
+template <typename T> struct FewK { static constexpr int value = FEW_K; };
+template <> struct FewK<bf16_t> { static constexpr int value = 56; };
+template <> struct FewK<f16_t> { static constexpr int value = 60; };
 constexpr int FEW_SLOTS = 4;               // 512 entries of a list of eight parts; at k = 50 one in 60 rows has a longer one than 256
 template <typename T>
 __device__ __forceinline__ bool merge_few(const SampleParams& p, Shared& s, int row_idx) {
@@ -1243,7 +1250,7 @@ sample_merge_kernel(SampleParams p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
     const bool vec_ok = ((uintptr_t)row % 16) == 0;
-    if (p.top_k <= FEW_K && p.probs_out == nullptr) {
+    if (p.top_k <= FewK<T>::value && p.probs_out == nullptr) {
         if (merge_few<T>(p, s, row_idx)) return;
         __syncthreads();
     }
@@ -1318,8 +1325,8 @@ sample_merge_kernel(SampleParams p) {
 // maximum give the slice that holds the threshold (a few dozen logits of a usual row), and what lies above it is summed by
 // segment.  64 rows: 45.7 -> 34.5 us (38.4 while every part read its row's 2048 slices of all parts, 128 KB, where it now reads
 // the sums of 64 groups of them and one group); 8 rows 42.2 -> 23.8.
-// Rows of unit variance at temperature 1, whose nucleus is half the row: 64 rows 154 -> 60 us (of equal logits only, which are
-// done whole all the same: 715 -> 766).
+// Rows of unit variance at temperature 1, whose nucleus is half the row: 64 rows 154 -> 60 us.  Nearly flat rows, whose
+// threshold slice holds more logits than the lists, are done whole after the three launches, see sample_parts().
 constexpr int SEG = PART_MAX / NW;                  // logits of a segment, one wave's: 16 per lane
 // The lane's sixteen logits of the segment [begin, begin + n), -inf beyond it: four groups of four, 256 apart (IN_ORDER:
 // next to each other).
@@ -1691,14 +1698,20 @@ greedy_kernel(SampleParams p) {
 
 }  // namespace
 
-// How many parts the rows of a call are cut into (1: none).  A second launch and the merge cost about 5 us for top_k <= 64
+// How many parts the rows of a call are cut into (1: none).  A second launch and the merge cost about 5 us for top_k <= FewK
 // (merge_few) and 9 us beyond, so it has to save more.  us per call, one launch -> parts:
-//   top_k <= 64 (k 50)  float32  20000, 2 parts: 1 row 14.4 -> 10.0, 64 15.8 -> 11.3, 1024 61.3 -> 44.3
+//   few (k 50)          float32  20000, 2 parts: 1 row 14.4 -> 10.0, 64 15.8 -> 11.3, 1024 61.3 -> 44.3
 //                                50256, 4 parts: 1 row 16.0 -> 10.9, 64 16.7 -> 11.7, 128 17.2 -> 13.9, 1024 86.7 -> 66.5
 //                                128256, 8 parts: 1 row 20 -> 10.7, 64 23 -> 14.4, 512 88 -> 61;  262144: 16 rows 29 -> 11.3
 //                       16-bit   32000: 64 rows 16.6 -> 11.6, 1024 63.4 -> 45.6;  81920: 64 20.7 -> 13.9, 1024 90.4 -> 78.8
 //                                128256: 64 rows 22.3 -> 13.9, 128 22.5 -> 20.3, 1024 109 -> 115;  262144: 64 31.7 -> 25.8,
 //                                128 34.2 -> 37.9 (half the bytes to save on): six parts and more up to 1024 parts
+//                                up to 256 rows of one launch are under way together, parts 512 at a time (k 20, of 40000, 65536
+//                                and 81920): 160 rows 14.4 -> 13.7, 128 15.3 -> 13.9, 128 18.1 -> 16.3;  256 rows 14.6 -> 16.7,
+//                                15.5 -> 19.6, 224 18.8 -> 21.9;  288 rows 26.8 -> 22.9, 28.9 -> 26.5, 39.2 -> 29.2.  512 of
+//                                65536: k 50 35.7 -> 39.1, with top_p 0.9 39.4 -> 36.8 (which the line does not know)
+//                       float32, k 64  32768, 2 parts: 128 rows 14.7 -> 13.8, 256 14.9 -> 17.2, 288 27.9 -> 26.3;  65536, 4: 128
+//                                15.8 -> 17.3, 192 26.1 -> 21.9
 //   rows whose loads cannot be vectors (a stride that is no multiple of 16 bytes): at once
 //     bf16, k 50        50257: 64 rows 24.4 -> 17.3;  greedy float32 50257: 64 rows 11.4 -> 7.6
 //   the whole row       float32  20000, 2 parts: 1 row 14.8 -> 10.9, 1024 62.9 -> 49.3;  50256: 64 rows 26.3 -> 11.7
@@ -1713,6 +1726,10 @@ greedy_kernel(SampleParams p) {
 //            81920, 5: 64 rows 35.9 -> 31.7, 128 38.4 -> 48.1;  128256, 8: 1 row 41.5 -> 23.3, 32 45.5 -> 25.1, 64 45.7 -> 34.5,
 //            128 55.1 -> 65.5;  262144, 16: 1 row 74.4 -> 25.0, 64 92.5 -> 67.7, 128 101 -> 114
 //   bf16     128256: 1 row 44.7 -> 23.8, 64 48.1 -> 34.1, 128 49.1 -> 53.8
+// Rows so flat that a slice of 1/160 holds more than 512 logits of a part or 1024 in all lose the three launches: top_p 0.9,
+// temperature 1, 128256 float32, standard deviation 0.1: 1 row 151 -> 170, 64 157 -> 190;  0.001: 64 158 -> 211;  equal
+// logits: 64 714 -> 766.  50257, standard deviation 0.1: 64 92 -> 69, 0.001: 94 -> 123.  What a row is like is not known
+// before its slices are, and a language model's rows are none of these (unit variance: 155 -> 60 and 93 -> 36).
 constexpr int NUCLEUS_MIN_PARTS = 4, NUCLEUS_MAX_BATCH = 64;
 static bool whole_row(int vocab, int top_k, int greedy) { return !greedy && (top_k <= 0 || top_k >= vocab); }
 static int sample_parts(int batch, int vocab, int64_t row_stride, float temperature, int top_k, int greedy, int dtype) {
@@ -1723,9 +1740,15 @@ static int sample_parts(int batch, int vocab, int64_t row_stride, float temperat
     const int per_16 = dtype == AICOMP_KV_F32 ? 4 : 8;
     if (batch > 1 && row_stride % per_16 != 0) return parts;
     const int all = batch * parts;
-    if (!greedy && top_k <= FEW_K) return dtype == AICOMP_KV_F32 || parts < 6 || all <= 1024 ? parts : 1;
+    const bool f32 = dtype == AICOMP_KV_F32, together = batch <= 256;
+    const int few = f32 ? FewK<float>::value : dtype == AICOMP_KV_F16 ? FewK<f16_t>::value : FewK<bf16_t>::value;
+    if (!greedy && top_k <= few) {
+        if (f32) return top_k <= 50 || parts >= 4 || batch <= 128 || !together ? parts : 1;
+        if (parts >= 6) return all <= 1024 ? parts : 1;
+        return !together || all <= (parts == 5 ? 640 : 512) ? parts : 1;
+    }
     if (parts < 6) return 1;
-    return all <= (greedy ? 512 : 128) ? parts : 1;
+    return all <= (greedy || top_k <= FEW_K ? 512 : 128) ? parts : 1;
 }
 
 // Candidates a part has room for.  Of 16384 normally distributed logits about 2.7 k pass the bound of sixteen waves

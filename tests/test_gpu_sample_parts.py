@@ -136,3 +136,20 @@ def test_whole_rows_in_parts_in_a_graph(device, top_p):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, _one_launch(x, 0.8, 0, top_p, True, u)[0]), i
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k", [50, 56, 57, 60, 61, 64])
+@pytest.mark.parametrize("V", [20000, 81920, 128256])
+def test_ties_of_16_bit_rows(device, V, k, dtype):
+    """Ties of the k-th value beside it, as many as leave the short merge its 64 lanes and more."""
+    x = torch.cat([_rows(V, dtype, device)] * 2)
+    for row, n in enumerate((1, 14, 15, 16, 60, 70)):
+        x[row, :] = x[row, :].clamp(max=5.0)
+        x[row, torch.arange(k - 1, device=device) * 7 + 3] = 9.0
+        x[row, V - 1 - torch.arange(n, device=device) * 5] = 8.0
+    for i in range(4):
+        u = torch.rand(x.shape[0], generator=torch.Generator().manual_seed(i)).to(device)
+        top_p = (1.0, 0.9, 0.999, 0.3)[i]
+        got = ops.sample_tokens(x, 0.8, k, top_p, uniforms=u)
+        assert torch.equal(got, _one_launch(x, 0.8, k, top_p, True, u)[0]), (top_p, i)

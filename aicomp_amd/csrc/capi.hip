@@ -433,8 +433,13 @@ static int rope_decode_impl(void* out, const void* query, int64_t q_token_stride
     a.v_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? v_scale : nullptr;
     a.num_parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, columns, kv_dtype, shape, a.partition_size);
     a.stream = (hipStream_t)stream;
-    // (a batch for the balanced schedule streams for tens of microseconds: the launch saved is lost in it)
-    AICOMP_REQUIRE(vectors && shape && small_call(batch, block_size, columns) && decode_mfma_supported(a),
+    // A batch for the balanced schedule streams for tens of microseconds: the launch saved is lost in it.  So it is in split
+    // rows of more than 512 workgroups (two calls, which the table's width sends to the balanced schedule, / this one, us:
+    // 32 rows of 700, fp8 pool, 32/8 heads, D 128 18.1 / 21.1, D 64 17.2 / 18.7, 64/8 19.4 / 23.6), but for float32 groups
+    // of up to four heads (32 rows of 700, D 128 37.8 / 33.4, D 64 24.4 / 20.2).
+    const bool few = a.num_parts == 1 || (int64_t)batch * num_kv_heads * a.num_parts <= 512 ||
+                     (q_dtype == AICOMP_KV_F32 && num_q_heads <= 4 * num_kv_heads);
+    AICOMP_REQUIRE(vectors && shape && few && small_call(batch, block_size, columns) && decode_mfma_supported(a),
                    AICOMP_KV_EUNSUPPORTED, "%s: not a call of the matrix-core grid schedule", who);
     a.new_key = new_key; a.new_value = new_value;
     a.new_token_stride = kv_token_stride; a.new_head_stride = kv_head_stride;

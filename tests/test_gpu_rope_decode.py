@@ -103,7 +103,7 @@ def test_split_rows_and_odd_slots(device, decode_routing, dtype, kv, d):
 
 
 def test_what_it_declines(device, decode_routing):
-    """Batches for the balanced schedule, other head dims, rows that cannot be read in vectors: None, and nothing written."""
+    """Batches for the balanced schedule, many split rows, other head dims, rows that cannot be read in vectors: None, and nothing written."""
     c = _case(device, torch.bfloat16, torch.bfloat16, 8, 2, 64, CTX, 1)
     prev = ops.set_small_decode_tokens(0)
     try:
@@ -115,6 +115,16 @@ def test_what_it_declines(device, decode_routing):
     c["q"] = odd
     out, kp, vp = _one(c, c["lens"])
     assert out is None and torch.equal(_bits(kp), _bits(c["pools"][0])) and torch.equal(_bits(vp), _bits(c["pools"][1]))
+    # split rows of more than 512 workgroups, but for float32 groups of up to four heads
+    for dtype, kv, hq, rows, one in ((torch.bfloat16, torch.float8_e4m3fn, 8, 21, True), (torch.bfloat16, torch.float8_e4m3fn, 8, 22, False),
+                                     (torch.float32, torch.float32, 32, 22, True), (torch.float32, torch.float32, 40, 22, False)):
+        s = _case(device, dtype, kv, hq, 8, 64, [641] * rows, 3)
+        s["cos"], s["sin"] = ops.rotary_tables(1.0 / 10000 ** (torch.arange(0, 64, 2) / 64).to(device), 700, dtype)
+        got = _one(s, s["lens"])
+        assert (got[0] is not None) == one
+        if one:
+            for a, b in zip(got, _two(s, 41)):
+                assert torch.equal(_bits(a), _bits(b))
     w = _case(device, torch.bfloat16, torch.bfloat16, 4, 2, 256, [5, 20], 2)
     assert _one(w, w["lens"])[0] is None
     w["table"] = w["table"].long()

@@ -576,7 +576,7 @@ PyObject* append_prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs
         }
         const c10::DeviceGuard guard(q->device());
         void* stream = stream_of(*q);
-        const int longest = longest_of(args[15], S);
+        const int longest = dt == AICOMP_KV_F32 ? 0 : longest_of(args[15], S);       // (float32 has no line that looks at it)
         const int rc = unlocked([&] {
             return aicomp_kv_append_prefill_attn_sized(
                 out->data_ptr(), q->data_ptr(), key ? key->data_ptr() : nullptr, key ? value->data_ptr() : nullptr,

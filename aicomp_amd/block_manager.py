@@ -24,8 +24,8 @@ kernels read (``block_table``, ``context_lens``, ``slot_mapping``,
 Row order inside a plan: sequences that ingest more than one token (prompt
 chunks) first, then the one-token sequences; ``paged_attention_step`` below
 runs the append, the chunked-prefill kernel on the first group and the decode
-kernel on the second, or, for a mixed step with a moderate decode part, one
-launch of the chunked-prefill kernel over both (``StepPlan.step_items``).
+kernel on the second, or, for a mixed step without very long decode rows, one
+launch of the chunked-prefill kernel over both (``StepPlan.launch_items``).
 
 Token t of a sequence lives in slot ``block_table[t // BS] * BS + t % BS``.
 """
@@ -267,6 +267,46 @@ class StepPlan:
                     hgroups = hq // gpack
                     cus = torch.cuda.get_device_properties(query.device).multi_processor_count if query.is_cuda else 0
                     items = ops.step_items(self.host_context_lens, self.new_lens, npre, tile, hgroups, cus)
+                    items = torch.from_numpy(items).to(query.device, non_blocking=True)
+            self._prefill_items[key] = items
+        return items
+
+    # Longest decode row of the one launch: a workgroup of it walks a row of its heads alone, 8 us per 1000 keys
+    # (head_dim 128; 5.5 at 64), which the decode kernels split between workgroups, and what takes its time beside it is the
+    # rest of the launch.  Device us, one launch / separate kernels, 32 / 8 heads, bf16, head_dim 128, by workgroups:
+    #     40  one row of 2000 18 / 20, 3000 23 / 20        96  8 rows of 2000 21 / 26, 3000 31 / 31, 4600 46 / 35
+    #    192  8 rows of 3000 33 / 40, 4600 50 / 44         384  8 rows of 4600 60 / 64;  32 of 4600 77 / 88, 8000 122 / 119
+    #    576  32 rows of 4600 96 / 108, 8000 135 / 138     832  100 of 4600 196 / 205, 8000 333 / 332
+    # and fp8 pools, head_dim 64 and 16 / 2, 8 / 8, 64 / 8 heads alike.  A launch has (tiles + rows) x head groups of them.
+    ONE_LAUNCH_KEYS = (2000, 8, 8000)          # at least, more per workgroup, at most
+
+    def launch_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:
+        """What ``paged_attention_step`` and ``attend`` run a mixed step by: the item list of one launch over its chunks and
+        decode rows where that is faster than the prefill and decode kernels one after the other, else ``None``.  The kernel
+        with two column groups streams a one-token row like a decode kernel does, so neither the number of rows nor an fp8
+        pool stands against it; a chunk bound too short for that kernel does, and rows too long for the launch (above).
+        ``ONE_LAUNCH_MAX_ROWS`` of 0 switches it off.  Cached per step."""
+        from . import ops
+        npre, ndec = self.num_prefill_seqs, self.num_decode_seqs
+        if not npre or not ndec or not self.ONE_LAUNCH_MAX_ROWS:
+            return None
+        if query.dtype not in (torch.bfloat16, torch.float16) or k_pool.dtype not in (query.dtype, torch.float8_e4m3fn):
+            return None
+        key = self._list_key(("launch", self.ONE_LAUNCH_KEYS), query, k_pool)
+        if self._prefill_items is None:
+            self._prefill_items = {}
+        items = self._prefill_items.get(key, _UNSEEN)
+        if items is _UNSEEN:
+            items = None
+            hq, (_, hkv, bs, d) = query.shape[1], k_pool.shape
+            tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
+            group = hq // hkv
+            gpack = group if 16 % group == 0 else 1
+            if tile * gpack == 128 and (d == 128 or gpack <= 8):     # (sixteen heads of 64 do not stream)
+                least, more, most = self.ONE_LAUNCH_KEYS
+                wgs = (int((-(-self.new_lens[:npre] // tile)).sum()) + ndec) * (hq // gpack)
+                if int(self.host_context_lens[npre:].max()) <= min(most, least + more * wgs):
+                    items = ops.one_launch_items(self.host_context_lens, self.new_lens, npre, tile)
                     items = torch.from_numpy(items).to(query.device, non_blocking=True)
             self._prefill_items[key] = items
         return items
@@ -674,17 +714,17 @@ def paged_attention_step(plan: StepPlan, out: torch.Tensor, query: torch.Tensor,
     ``query`` / ``out`` are ``[T, Hq, D]``, ``key`` / ``value`` ``[T, Hkv, D]`` in the plan's
     row order (``cu_q_lens``).  The prompt chunks go through the chunked-prefill kernel;
     the one-token rows go through the decode kernel with their append fused into it, or, in a
-    mixed step whose decode part is small enough (``StepPlan.step_items``), through the same
-    launch as the chunks.
+    mixed step whose decode rows are not too long for it (``StepPlan.launch_items``), through the
+    same launch as the chunks.
     Replaces, per sequence, the append + ``.contiguous()`` + SDPA of
     opt_prime/opt_prime/kv_cache.py:385-415.
     """
     from . import ops
     npre, S = plan.num_prefill_seqs, plan.num_seqs
     t_pre = plan.num_prefill_tokens
-    items = plan.step_items(query, k_pool)
+    items = plan.launch_items(query, k_pool)
     if items is not None:
-        # mixed step, decode part within the measured bounds: every new row appended, then one
+        # mixed step, decode rows within the measured bounds: every new row appended, then one
         # launch over all sequences (a decode row is a chunk of one token)
         ops.kv_append(key, value, k_pool, v_pool, plan.slot_mapping, k_scale, v_scale)
         return ops.paged_prefill_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens,

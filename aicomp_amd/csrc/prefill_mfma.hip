@@ -27,6 +27,7 @@
 //              Otherwise: coalesced 16-byte loads into registers ahead of their use, written
 //              to LDS (one padded row per token; fp8 is widened to the query's type on the way).
 // head_dim     128 or 64, one instantiation each.
+// One token    a chunk of one token streams through the decode tiles instead (one_token_row).
 // Per wave     16 or 32 rows (one or two column groups).  S^T = K Q^T with K rows as
 //              the A operand and the wave's query rows as B columns
 //              (v_mfma_f32_16x16x32_bf16 / _f16), the score multiplier folded into Q and the
@@ -48,9 +49,9 @@ namespace aicomp {
 
 namespace {
 
-constexpr int BS = 16;
+#include "decode_tile16.h"
+
 constexpr int ROWS = 64;               // query rows per workgroup and column group (16 per wave)
-constexpr float NEG_BIG = -1.0e30f;
 
 struct PrefillParams {
     void* out;
@@ -70,6 +71,79 @@ struct PrefillParams {
     const int32_t* items;              // (sequence, query tile) pairs; grid.y numbers them (NULL: none)
     int num_seqs;
 };
+
+// A chunk of one token (a decode row of a mixed step): the rows of its workgroup, gpack heads of one position, over the ctx
+// keys of the sequence.  The four waves take every fourth tile of the decode kernels each, no barrier and up to 16 KB in flight
+// per wave, and are merged through LDS like those of the decode grid schedule.  Through the tile loop below such a row paid a
+// barrier and, with one tile of look-ahead, a round trip to memory per 64 keys, 2.2 us, whatever its workgroup's neighbours
+// did; the launch of a mixed step was those round trips on 512 places.  Now it is bound by what the memory gives all of them:
+//   4 chunks of 512 over <= 2048 + 60 rows of 512..4096 tokens, 32 / 8 heads   append + launch 136 -> 116 us (the four
+//   launches that take chunks and rows one after the other: 144)
+//   the same with an fp8 pool 108 (four launches) -> 82, head_dim 64 90 -> 70, both 70 -> 47
+// kt_of(w): 8 KB of LDS for wave w.
+template <typename T, typename Lds>
+__device__ __forceinline__ void one_token_row(const PrefillParams& p, int seq, int q_row, int ctx, int hgroup, Lds kt_of) {
+    constexpr int DQ = T::DQ, TT = T::TT, BPT = T::BPT, NW = NWAVES;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g4 = lane >> 4;
+    const int kvh = (hgroup * p.gpack) / p.group;
+    __shared__ float sm_m[NW][16];
+    __shared__ float sm_l[NW][16];
+    unsigned char* kt = kt_of(w);
+
+    const int32_t* table = p.block_table + (int64_t)seq * p.block_table_stride;
+    int tab_first = 0;
+    int tab = lane < p.max_blocks ? table[lane] : 0;
+    const int64_t row0 = ((int64_t)q_row * p.hq + hgroup * p.gpack) * DQ;
+    typename T::Q qf;
+    T::load_q(qf, (const uint16_t*)p.query + row0, p.gpack, lane);
+    const float cmul = p.qk_mul * (T::FP8 ? p.k_scale[kvh] : 1.f);
+    const int ntiles = (ctx + TT - 1) / TT;
+    typename T::State st;
+    clear_state(st);
+
+    int64_t bb[4] = {0, 0, 0, 0};
+    auto tile_blocks = [&](int tt) {
+        const int i0 = BPT * tt;
+        if (i0 - tab_first >= 64) {
+            tab_first = i0;
+            tab = i0 + lane < p.max_blocks ? table[i0 + lane] : 0;
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0) here, so the common path never waits on `tab`
+        }
+#pragma unroll
+        for (int j = 0; j < BPT; ++j) bb[j] = clamp_block(__builtin_amdgcn_readlane(tab, i0 + j - tab_first), p.num_blocks);
+    };
+    const typename T::Offsets ko = T::offsets(lane);
+    if (w < ntiles) {
+        typename T::Regs kv;
+        tile_blocks(w);
+        T::load(kv, p, bb, kvh, lane);
+        T::q_operand(qf, qf, p.gpack, lane);
+        int tt = w;
+        for (; tt + NW < ntiles; tt += NW) {
+            tile_blocks(tt + NW);
+            T::template process<true, false>(st, kv, qf, kt, ko, p, bb, kvh, lane, tt * TT, ctx, cmul);
+        }
+        T::template process<false, true>(st, kv, qf, kt, ko, p, bb, kvh, lane, tt * TT, ctx, cmul);
+    }
+    float lsum = st.lsum;
+    lsum += __shfl_xor(lsum, 16);
+    lsum += __shfl_xor(lsum, 32);
+    if (r16 < T::NPAR * p.gpack) {
+        T::store_acc((float*)kt + r16 * T::OROW, st, g4);
+        if (g4 == 0) { sm_m[w][r16] = st.m; sm_l[w][r16] = lsum; }
+    }
+    __syncthreads();
+    const float vs = T::FP8 ? p.v_scale[kvh] : 1.f;
+    for (int idx = tid; idx < p.gpack * DQ; idx += 64 * NW) {
+        float mx, num, den;
+        merge_waves<T, NW>(kt_of, sm_m, sm_l, idx / DQ, idx % DQ, mx, num, den);
+        // The weights of a row add up to one at least, or to nothing where every score is -inf: 0 then, as in the decode
+        // kernels.  (No comparison: this file is compiled as if there were no NaN, and a row with one has to stay NaN.)
+        ((uint16_t*)p.out)[row0 + idx] = T::Fmt::from_f32(vs * num / fmaxf(den, 1e-30f));
+    }
+}
 
 // register stage of one K and one V tile: NL loads of the workgroup each
 template <bool FP8, int NL> struct Stage;
@@ -221,6 +295,25 @@ paged_prefill_mfma_kernel(PrefillParams p) {
                 *(uint4*)((uint16_t*)p.out + ((int64_t)(q_begin + pos) * p.hq + hd) * DH + 8 * chunk) = make_uint4(0, 0, 0, 0);
         }
         return;
+    }
+
+    // (one column group, 64 rows a workgroup: 80 to 129 registers, half of what the decode tiles need)
+    if constexpr (R == 2) {
+        if (n == 1 && (DH == 128 || p.gpack <= 8)) {                 // workgroup-uniform (sixteen heads of 64 are 32 columns)
+            typedef Tile16<E, FP8, DH == 64, true, DH == 64> Tile;
+            // The arguments come through a pointer of this path's own: shared with the tile loop below they would be held
+            // in scalar registers across it, whose spills took the vector register that the loop at head_dim 64 then lacked.
+            auto args = __builtin_amdgcn_kernarg_segment_ptr();
+            asm volatile("" : "+s"(args));
+            const PrefillParams& own = *(const PrefillParams*)args;
+            if constexpr (DMA && DH == 128)
+                one_token_row<Tile>(own, seq, q_begin, ctx, hgroup, [&](int wv) { return (wv >> 1 ? dma_v0 : dma_k0) + (wv & 1) * KTILE_BYTES; });
+            else if constexpr (DMA)
+                one_token_row<Tile>(own, seq, q_begin, ctx, hgroup, [&](int wv) { return wv == 0 ? dma_k0 : wv == 1 ? dma_v0 : wv == 2 ? dma_k1 : dma_v1; });
+            else
+                one_token_row<Tile>(own, seq, q_begin, ctx, hgroup, [&](int wv) { return lds + wv * KTILE_BYTES; });
+            return;
+        }
     }
 
     // rows of this lane's columns: row = WROWS*w + CR*c + (column, or column / 2) -> (position, head)

@@ -427,6 +427,24 @@ def step_items(context_lens, new_lens, num_prefill_seqs: int, tile_positions: in
     return np.concatenate([dec[:per_round], pre[:per_round], rest, a[k:], b[k:]]).astype(np.int32)
 
 
+def one_launch_items(context_lens, new_lens, num_prefill_seqs: int, tile_positions: int):
+    """``step_items`` for the kernels whose one-token rows stream (two column groups of 16-bit queries): the item order of
+    ONE launch over a mixed step, ``int32 [n, 2]``.
+
+    Falling time.  A chunk tile of 128 rows takes 2.1 us per 64 keys beside another one, bound by the matrix cores, and a
+    one-token row about 0.7 of that, bound by what the memory gives all of them; equal keys are therefore not equal times.
+    Measured on MI355X, 4 chunks of 512 over priors up to 2048 with 60 rows of 512 to 4096 tokens, 32 / 8 heads, head_dim
+    128 (64): weights 0.5 / 0.6 / 0.7 / 0.8 117.3 / 116.4 / 115.9 / 119.3 us (71.2 / 70.8 / 70.4 / 72.1), ``step_items``
+    121.6 (74.2), falling keys 119.7; rows of 128 to 1024 tokens 57.3 against 60.3.
+    """
+    import numpy as np
+    ctx, new = np.asarray(context_lens, dtype=np.int64), np.asarray(new_lens, dtype=np.int64)
+    base = prefill_items(ctx, new, tile_positions)                              # falling keys
+    keys = np.minimum(ctx[base[:, 0]], ctx[base[:, 0]] - new[base[:, 0]] + (base[:, 1] + 1) * tile_positions)
+    time = np.where(base[:, 0] < num_prefill_seqs, 10 * keys, 7 * keys)
+    return base[np.argsort(-time, kind="stable")]
+
+
 def rope_paged_decode_attn(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                            positions: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, slot_mapping: torch.Tensor,
                            block_table: torch.Tensor, context_lens: torch.Tensor, host_lens, scale: float,

@@ -200,7 +200,7 @@ def run_decode_config(name, steps, warmup, dev, settle_ms=30.0):
         from aicomp_amd.block_manager import paged_attention_step
         plan = plan_of_workload(w)
         out_all = torch.empty_like(w.query)
-        one_launch = plan.step_items(w.query, w.k_pool) is not None
+        one_launch = plan.launch_items(w.query, w.k_pool) is not None
 
         def planned_step(i):
             kp, vp = pools[i % len(pools)]
@@ -845,7 +845,7 @@ def profile_target(which, steps, warmup, dev, settle_ms=30.0):
         w = workloads.make_workload("chunked_prefill_mixed", device=dev)
         plan = plan_of_workload(w)
         out = torch.empty_like(w.query)
-        one = plan.step_items(w.query, w.k_pool) is not None
+        one = plan.launch_items(w.query, w.k_pool) is not None
         how = drive(lambda: paged_attention_step(plan, out, w.query, w.new_key, w.new_value, w.k_pool, w.v_pool, w.scale))
         print(f"mixed_planned (chunked_prefill_mixed): {how}; "
               f"{'append + one launch over chunks and decode rows' if one else 'append + prefill + decode kernels'}")

@@ -478,3 +478,29 @@ def test_step_plan_sends_only_moderate_decode_parts_through_one_launch():
     assert mixed(2000).step_items(q.float(), pool.float()) is None
     assert mixed(2000, chunk=16).step_items(q, pool) is None                              # one-column-group kernel
     assert mixed(2000).step_items(torch.zeros(1, 32, 256, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 256, dtype=torch.bfloat16)) is None
+
+
+def test_launch_items_of_a_mixed_step():
+    """StepPlan.launch_items: one launch however many rows and for fp8 pools too, unless its longest row outlasts the rest of
+    the launch; every tile and row once, in falling time."""
+    import torch
+    from aicomp_amd import ops
+    q, pool = torch.zeros(1, 32, 128, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 128, dtype=torch.bfloat16)
+    mixed = lambda ctx_dec, n_dec=8, chunk=512, npre=2: _mixed_plan([chunk + 100] * npre + [ctx_dec] * n_dec,
+                                                                   [chunk] * npre + [1] * n_dec, npre, chunk)
+    it = mixed(2000).launch_items(q, pool)
+    assert sorted(map(tuple, it.tolist())) == sorted([(s, t) for s in range(2) for t in range(16)] + [(s, 0) for s in range(2, 10)])
+    plan = mixed(2000)
+    assert plan.launch_items(q, pool) is plan.launch_items(q, pool)
+    # (32 tiles + rows) x 8 head groups
+    assert mixed(2000 + 8 * 320).launch_items(q, pool) is not None and mixed(2001 + 8 * 320).launch_items(q, pool) is None
+    assert mixed(8000, n_dec=300).launch_items(q, pool) is not None and mixed(8001, n_dec=300).launch_items(q, pool) is None
+    assert mixed(2000).launch_items(q, pool.to(torch.float8_e4m3fn)) is not None
+    assert mixed(2000, npre=0).launch_items(q, pool) is None and mixed(2000, n_dec=0).launch_items(q, pool) is None
+    assert mixed(2000).launch_items(q.float(), pool.float()) is None
+    assert mixed(2000).launch_items(q, pool.half()) is None
+    assert mixed(2000, chunk=16).launch_items(q, pool) is None                            # one-column-group kernel
+    wide = torch.zeros(1, 16, 64, dtype=torch.bfloat16), torch.zeros(1, 1, 16, 64, dtype=torch.bfloat16)
+    assert mixed(2000).launch_items(*wide) is None                                        # 32 columns of 64
+    items = ops.one_launch_items([300, 300, 500, 400], [64, 64, 1, 1], 2, 32)
+    assert items.tolist() == [[2, 0], [0, 1], [1, 1], [3, 0], [0, 0], [1, 0]]             # 350, 300, 300, 280, 268, 268

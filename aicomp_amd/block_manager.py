@@ -284,7 +284,9 @@ class StepPlan:
         """What ``paged_attention_step`` and ``attend`` run a mixed step by: the item list of one launch over its chunks and
         decode rows where that is faster than the prefill and decode kernels one after the other, else ``None``.  The kernel
         with two column groups streams a one-token row like a decode kernel does, so neither the number of rows nor an fp8
-        pool stands against it; a chunk bound too short for that kernel does, and rows too long for the launch (above).
+        pool stands against it; rows too long for the launch (above) do.  Chunks too short for that kernel go through it all
+        the same (``launch_q_len``; in their own kernel and the rows in theirs: 8 chunks of 30 tokens over 1500 with 8 rows of
+        1000 51 us, 37 so, alone with 32 rows of 500 23 and 15), if there are as many new tokens as it asks for.
         ``ONE_LAUNCH_MAX_ROWS`` of 0 switches it off.  Cached per step."""
         from . import ops
         npre, ndec = self.num_prefill_seqs, self.num_decode_seqs
@@ -299,10 +301,11 @@ class StepPlan:
         if items is _UNSEEN:
             items = None
             hq, (_, hkv, bs, d) = query.shape[1], k_pool.shape
-            tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
+            bound = self.launch_q_len(hq, hkv)
+            tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, bound)
             group = hq // hkv
             gpack = group if 16 % group == 0 else 1
-            if tile * gpack == 128 and (d == 128 or gpack <= 8):     # (sixteen heads of 64 do not stream)
+            if bound <= self.total_new_tokens and tile * gpack == 128 and (d == 128 or gpack <= 8):  # (sixteen heads of 64 do not stream)
                 least, more, most = self.ONE_LAUNCH_KEYS
                 wgs = (int((-(-self.new_lens[:npre] // tile)).sum()) + ndec) * (hq // gpack)
                 if int(self.host_context_lens[npre:].max()) <= min(most, least + more * wgs):
@@ -310,6 +313,11 @@ class StepPlan:
                     items = torch.from_numpy(items).to(query.device, non_blocking=True)
             self._prefill_items[key] = items
         return items
+
+    def launch_q_len(self, hq: int, hkv: int) -> int:
+        """The chunk bound to pass with ``launch_items``: one that the kernel with two column groups takes, 128 rows."""
+        group = hq // hkv
+        return max(self.max_q_len, 128 // (group if 16 % group == 0 else 1))
 
     @property
     def num_seqs(self) -> int:
@@ -728,8 +736,8 @@ def paged_attention_step(plan: StepPlan, out: torch.Tensor, query: torch.Tensor,
         # launch over all sequences (a decode row is a chunk of one token)
         ops.kv_append(key, value, k_pool, v_pool, plan.slot_mapping, k_scale, v_scale)
         return ops.paged_prefill_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens,
-                                      plan.cu_q_lens, scale, max_q_len=plan.max_q_len, k_scale=k_scale,
-                                      v_scale=v_scale, items=items)
+                                      plan.cu_q_lens, scale, max_q_len=plan.launch_q_len(query.shape[1], k_pool.shape[1]),
+                                      k_scale=k_scale, v_scale=v_scale, items=items)
     if plan.only_chunks and t_pre == query.shape[0] == out.shape[0] == key.shape[0] == value.shape[0]:
         # chunks alone: the tensors as they are (a slice costs a microsecond)
         return ops.append_prefill_attn(out, query, key, value, k_pool, v_pool, plan.slot_mapping, plan.block_table,

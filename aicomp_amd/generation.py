@@ -90,7 +90,8 @@ class PagedAttentionBackend:
         items = plan.launch_items(q, kp)
         if items is not None:                      # mixed step: chunks and decode rows in one launch
             return ops.paged_prefill_attn(out, q, kp, vp, plan.block_table, plan.context_lens, plan.cu_q_lens,
-                                          self.scale, max_q_len=plan.max_q_len, k_scale=ks, v_scale=vs, items=items)
+                                          self.scale, max_q_len=plan.launch_q_len(q.shape[1], kp.shape[1]), k_scale=ks,
+                                          v_scale=vs, items=items)
         if plan.only_chunks and t_pre == query.shape[0]:     # chunks alone, rows alone: the plan's tensors as they are
             return ops.append_prefill_attn(out, q, None, None, kp, vp, None, plan.block_table, plan.context_lens,
                                            plan.cu_q_lens, self.scale, plan.max_q_len, ks, vs, plan.prefill_items(q, kp),

@@ -499,7 +499,10 @@ def test_launch_items_of_a_mixed_step():
     assert mixed(2000, npre=0).launch_items(q, pool) is None and mixed(2000, n_dec=0).launch_items(q, pool) is None
     assert mixed(2000).launch_items(q.float(), pool.float()) is None
     assert mixed(2000).launch_items(q, pool.half()) is None
-    assert mixed(2000, chunk=16).launch_items(q, pool) is None                            # one-column-group kernel
+    short = mixed(2000, chunk=16)                                                         # through the same kernel: tiles of 32
+    assert short.launch_q_len(32, 8) == 32 and sorted(map(tuple, short.launch_items(q, pool).tolist())) == [(s, 0) for s in range(10)]
+    assert mixed(300, n_dec=1, chunk=15).launch_items(q, pool) is None                    # 31 new tokens, none of them 32
+    assert mixed(300, n_dec=2, chunk=15).launch_items(q, pool) is not None
     wide = torch.zeros(1, 16, 64, dtype=torch.bfloat16), torch.zeros(1, 1, 16, 64, dtype=torch.bfloat16)
     assert mixed(2000).launch_items(*wide) is None                                        # 32 columns of 64
     items = ops.one_launch_items([300, 300, 500, 400], [64, 64, 1, 1], 2, 32)

@@ -319,6 +319,11 @@ class StepPlan:
         group = hq // hkv
         return max(self.max_q_len, 128 // (group if 16 % group == 0 else 1))
 
+    def few_chunk_lens(self, hq: int, hkv: int):
+        """The chunks' context lengths where a mixed step of separate kernels may run them by the kernel for few chunks: those
+        too short for the one launch's kernel.  (Others are bit for bit what the one launch gives.)"""
+        return self.host_context_lens[:self.num_prefill_seqs] if self.max_q_len < self.launch_q_len(hq, hkv) else None
+
     @property
     def num_seqs(self) -> int:
         return len(self.seq_ids)
@@ -746,14 +751,15 @@ def paged_attention_step(plan: StepPlan, out: torch.Tensor, query: torch.Tensor,
     if S and npre == 0:
         return ops.paged_decode_attn(out, query, k_pool, v_pool, plan.block_table, plan.context_lens, scale, k_scale,
                                      v_scale, new_key=key, new_value=value)
+    if npre and S > npre:
+        return ops.chunks_and_rows_attn(out, query, key, value, k_pool, v_pool, plan.slot_mapping, plan.block_table,
+                                        plan.context_lens, plan.cu_q_lens, scale, plan.max_q_len, npre, t_pre, k_scale,
+                                        v_scale, plan.prefill_items(query, k_pool),
+                                        plan.few_chunk_lens(query.shape[1], k_pool.shape[1]))
     if npre:
         ops.kv_append(key[:t_pre], value[:t_pre], k_pool, v_pool, plan.slot_mapping[:t_pre], k_scale, v_scale)
         ops.paged_prefill_attn(out[:t_pre], query[:t_pre], k_pool, v_pool, plan.block_table[:npre],
                                plan.context_lens[:npre], plan.cu_q_lens[:npre + 1], scale,
                                max_q_len=plan.max_q_len, k_scale=k_scale, v_scale=v_scale,
                                items=plan.prefill_items(query, k_pool))
-    if S > npre:
-        ops.paged_decode_attn(out[t_pre:], query[t_pre:], k_pool, v_pool, plan.block_table[npre:],
-                              plan.context_lens[npre:], scale, k_scale, v_scale,
-                              new_key=key[t_pre:], new_value=value[t_pre:])
     return out

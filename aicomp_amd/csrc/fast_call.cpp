@@ -9,11 +9,12 @@
 //
 //   layer = _aicomp_fast.layer(k_pool, v_pool, block_table, ctx_rows)
 //   out   = _aicomp_fast.decode_step(layer, query, key, value, position, group, scale)
+//   out   = _aicomp_fast.prompt_step(layer, slots, cu, query, key, value, position, group, scale)
 //
 // Same checks, same errors (RuntimeError), same results as the registered operator.
 //
 // Beside it, the plain calls of aicomp_amd.ops (kv_append, rope_kv_append, paged_decode_attn, rope_paged_decode_attn,
-// paged_prefill_attn, append_prefill_attn, sample_tokens): the same checks made here instead of in Python.  A call that
+// paged_prefill_attn, append_prefill_attn, chunks_and_rows, sample_tokens): the same checks made here instead of in Python.  A call that
 // passes them all is launched and returns true; any other returns false without having touched
 // anything, and the Python function goes on to convert what may be converted or to name what is wrong.
 #include <Python.h>
@@ -181,13 +182,6 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
 }
 
-// ---------------------------------------------------------------- the plain calls of aicomp_amd.ops
-// Host time was what bounded these calls: their checks alone, a few dozen attribute reads of Python
-// tensors, cost 15 to 20 us a call, where the kernels of a decode or rotary call of ordinary size
-// need 3 to 12 (measured per call: see the wrappers in ops.py).
-
-int any_dtype_code(at::ScalarType t) { return t == at::kFloat8_e4m3fn ? AICOMP_KV_FP8_E4M3 : dtype_code(t); }
-
 // The tensor behind an argument, or null unless it is a plain strided tensor on a GPU with storage of
 // its own (no subclass, no wrapper of a transform): those go the Python way.
 const at::Tensor* plain(PyObject* o) {
@@ -195,6 +189,73 @@ const at::Tensor* plain(PyObject* o) {
     const at::Tensor& t = THPVariable_Unpack(o);
     return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.has_storage() ? &t : nullptr;
 }
+
+// runs a library call without the interpreter lock (a launch waits while the stream's queue is full)
+template <typename F> int unlocked(F call) {
+    PyThreadState* state = PyEval_SaveThread();
+    const int rc = call();
+    PyEval_RestoreThread(state);
+    return rc;
+}
+
+// A prompt chunk of the operator: append of its rows and causal attention, [B, Hq, n, D] as decode_step returns its row.
+// slots [B, positions]: where sequence b keeps its tokens; cu: int32 [B + 1], the multiples of n.  None, with nothing done,
+// for what is not a plain call; the operator's own way through ops.py goes on from there.
+PyObject* prompt_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        if (nargs != 9) FAIL("prompt_step(layer, slots, cu, query, key, value, position, group, scale)");
+        const Layer* L = (const Layer*)PyCapsule_GetPointer(args[0], "aicomp_amd.layer");
+        if (L == nullptr) return nullptr;
+        const at::Tensor *slots = plain(args[1]), *cu = plain(args[2]), *q_in = plain(args[3]), *k_in = plain(args[4]),
+                         *v_in = plain(args[5]);
+        const int64_t position = PyLong_AsLongLong(args[6]), group = PyLong_AsLongLong(args[7]);
+        const double scale = PyFloat_AsDouble(args[8]);
+        if (PyErr_Occurred()) return nullptr;
+        if (!slots || !cu || !q_in || !k_in || !v_in || q_in->dim() != 4 || k_in->dim() != 4) Py_RETURN_NONE;
+        const int64_t B = L->B, hq = q_in->size(1), n = q_in->size(2), H = k_in->size(1), D = L->d;
+        const int64_t hstep = (group > 1 && H == (int64_t)L->hkv * group) ? group : 1;
+        if (n < 2 || hq <= 0 || hq > INT_MAX || hq % L->hkv || position < 0 || n > INT_MAX || position + n >= L->ctx_count ||
+            q_in->size(0) != B || q_in->size(3) != D || H != L->hkv * hstep || k_in->size(0) != B || k_in->size(2) != n ||
+            k_in->size(3) != D || v_in->sizes() != k_in->sizes() || q_in->scalar_type() != L->st ||
+            k_in->scalar_type() != L->st || v_in->scalar_type() != L->st || q_in->device() != L->dev ||
+            k_in->device() != L->dev || v_in->device() != L->dev || slots->device() != L->dev || cu->device() != L->dev ||
+            slots->scalar_type() != at::kLong || slots->dim() != 2 || slots->size(0) != B || slots->stride(1) != 1 ||
+            slots->size(1) < position + n || cu->scalar_type() != at::kInt || cu->dim() != 1 || cu->size(0) != B + 1 ||
+            !cu->is_contiguous())
+            Py_RETURN_NONE;
+        const c10::DeviceGuard guard(L->dev);
+        // token-major rows: a view where the tensors are projections seen head-major, as attention layers hand them over
+        const at::Tensor q = q_in->permute({0, 2, 1, 3}).contiguous();
+        at::Tensor k = k_in->permute({0, 2, 1, 3}), v = v_in->permute({0, 2, 1, 3});          // [B, n, H, D]
+        if (hstep > 1) { k = k.slice(2, 0, H, hstep); v = v.slice(2, 0, H, hstep); }
+        if (k.stride(3) != 1 || k.strides() != v.strides() || (B > 1 && k.stride(0) != n * k.stride(1))) {
+            k = k.contiguous();
+            v = v.contiguous();
+        }
+        const at::Tensor slot = B == 1 ? *slots : slots->narrow(1, position, n).contiguous();
+        const int64_t* slot_ptr = (const int64_t*)slot.data_ptr() + (B == 1 ? position : 0);
+        at::Tensor out(at::detail::empty_cuda({B, n, hq, D}, L->st, L->dev, c10::MemoryFormat::Contiguous));
+        void* stream = (void*)c10::hip::getCurrentHIPStream(L->dev.index()).stream();
+        const int rc = unlocked([&] {
+            return aicomp_kv_append_prefill_attn_sized(
+                out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(1), k.stride(2), L->kp, L->vp, slot_ptr,
+                L->table, L->table_stride, L->ctx + (position + n) * L->ctx_stride, (const int32_t*)cu->data_ptr(), (int)B,
+                B * n, (int)n, (int)hq, L->hkv, (int)D, L->bs, L->width, L->nb, (float)scale, L->dt, L->dt, nullptr, nullptr,
+                nullptr, 0, (int)(position + n), stream);
+        });
+        if (rc != AICOMP_KV_OK) FAIL("aicomp_kv error %d: %s", rc, aicomp_kv_last_error());
+        return THPVariable_Wrap(out.permute({0, 2, 1, 3}));
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
+// ---------------------------------------------------------------- the plain calls of aicomp_amd.ops
+// Host time was what bounded these calls: their checks alone, a few dozen attribute reads of Python
+// tensors, cost 15 to 20 us a call, where the kernels of a decode or rotary call of ordinary size
+// need 3 to 12 (measured per call: see the wrappers in ops.py).
+
+int any_dtype_code(at::ScalarType t) { return t == at::kFloat8_e4m3fn ? AICOMP_KV_FP8_E4M3 : dtype_code(t); }
 
 bool on(const at::Tensor& t, const at::Tensor& ref) { return t.device() == ref.device(); }
 
@@ -245,14 +306,6 @@ bool as_int(PyObject* o, int& x) {
 }
 
 void* stream_of(const at::Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
-
-// runs a library call without the interpreter lock (a launch waits while the stream's queue is full)
-template <typename F> int unlocked(F call) {
-    PyThreadState* state = PyEval_SaveThread();
-    const int rc = call();
-    PyEval_RestoreThread(state);
-    return rc;
-}
 
 #define DONE(rc)                                                                                     \
     do {                                                                                             \
@@ -592,6 +645,97 @@ PyObject* append_prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t nargs
     }
 }
 
+// A layer's step of prompt chunks (the first `chunks` sequences, t_pre rows) and one-token rows after them, each through
+// their own kernels: append and prefill of the chunks, append and decode of the rows; key, value and slot_mapping None where
+// the new rows are in the pools already.  (Slices of a dozen tensors and three calls through Python were 36 us a step, this is 22.)
+PyObject* chunks_and_rows(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    try {
+        Pools p;
+        const at::Tensor *out, *q, *table, *ctx;
+        int dt, max_q_len, chunks, t_pre;
+        int64_t S;
+        double scale;
+        if (nargs != 18)
+            FAIL("chunks_and_rows(out, query, k_pool, v_pool, block_table, context_lens, cu_q_lens, scale, max_q_len, k_scale, "
+                 "v_scale, items, key, value, slot_mapping, chunks, t_pre, chunk_lens)");
+        if (!attention_args(args, out, q, p, table, ctx, dt, S) || !as_double(args[7], scale) ||
+            !as_int(args[8], max_q_len) || !p.scales(args[9], args[10]) || !as_int(args[15], chunks) || !as_int(args[16], t_pre))
+            Py_RETURN_FALSE;
+        const int64_t T = q->size(0), rows = S - chunks;
+        const at::Tensor* cu = plain(args[6]);
+        if (!vector_of(cu, at::kInt, S + 1, *q) || chunks <= 0 || rows <= 0 || S > INT_MAX || t_pre <= 0 || t_pre + rows != T)
+            Py_RETURN_FALSE;
+        const at::Tensor *items = nullptr, *key = nullptr, *value = nullptr, *slots = nullptr;
+        if (args[11] != Py_None) {
+            items = plain(args[11]);
+            if (!items || items->numel() == 0 || items->scalar_type() != at::kInt || items->dim() != 2 ||
+                items->size(1) != 2 || items->size(0) > INT_MAX || !items->is_contiguous() || !on(*items, *q))
+                Py_RETURN_FALSE;
+        }
+        if (args[12] != Py_None) {
+            key = plain(args[12]); value = plain(args[13]); slots = plain(args[14]);
+            if (!key || !value || !slots || key->dim() != 3 || value->sizes() != key->sizes() ||
+                key->scalar_type() != q->scalar_type() || value->scalar_type() != q->scalar_type() ||
+                key->size(0) != T || key->size(1) != p.hkv || key->size(2) != p.d || slots->dim() != 1 ||
+                !vector_of(slots, at::kLong, T, *q) || !on(*key, *q) || !on(*value, *q) || key->stride(2) != 1 ||
+                key->strides() != value->strides())
+                Py_RETURN_FALSE;
+        }
+        const int hq = (int)q->size(1), width = (int)table->size(1);
+        const c10::DeviceGuard guard(q->device());
+        void* stream = stream_of(*q);
+        at::Tensor scratch;
+        const size_t need = aicomp_paged_decode_workspace_bytes((int)rows, hq, p.hkv, p.d, p.bs, width, dt, p.dt, 0);
+        if (need) scratch = cached_scratch(q->device(), stream, need);
+        // (with the chunks' lengths they may take the kernel for few chunks)
+        const bool few = args[17] != Py_None && dt != AICOMP_KV_F32;
+        const int longest = few ? longest_of(args[17], chunks) : 0;
+        const int rc = unlocked([&] {
+            const int32_t *bt = (const int32_t*)table->data_ptr(), *cl = (const int32_t*)ctx->data_ptr();
+            const int64_t done = (int64_t)t_pre * hq * p.d * q->element_size();            // query and output of the chunks
+            void *kp = p.k->data_ptr(), *vp = p.v->data_ptr();
+            const int64_t* slot = key ? (const int64_t*)slots->data_ptr() : nullptr;
+            const int32_t *off = (const int32_t*)cu->data_ptr(), *list = items ? (const int32_t*)items->data_ptr() : nullptr;
+            const int pairs = items ? (int)items->size(0) : 0;
+            int rc = AICOMP_KV_OK;
+            if (few) {
+                rc = aicomp_kv_append_prefill_attn_sized(
+                    out->data_ptr(), q->data_ptr(), key ? key->data_ptr() : nullptr, key ? value->data_ptr() : nullptr,
+                    key ? key->stride(0) : 0, key ? key->stride(1) : 0, kp, vp, slot, bt, table->stride(0), cl, off, chunks, t_pre,
+                    max_q_len, hq, p.hkv, p.d, p.bs, width, p.nb, (float)scale, dt, p.dt, p.ks, p.vs, list, pairs, longest, stream);
+            } else {
+                if (key)
+                    rc = aicomp_kv_append(key->data_ptr(), value->data_ptr(), key->stride(0), key->stride(1), kp, vp, slot, t_pre,
+                                          p.hkv, p.d, p.bs, p.nb, dt, p.dt, p.ks, p.vs, stream);
+                if (rc == AICOMP_KV_OK)
+                    rc = aicomp_paged_prefill_attn_items(out->data_ptr(), q->data_ptr(), kp, vp, bt, table->stride(0), cl, off, chunks,
+                                                         t_pre, max_q_len, hq, p.hkv, p.d, p.bs, width, p.nb, (float)scale, dt,
+                                                         p.dt, p.ks, p.vs, list, pairs, stream);
+            }
+            if (rc != AICOMP_KV_OK) return rc;
+            std::unique_lock<std::mutex> one_at_a_time(scratch_launches(), std::defer_lock);
+            if (need) one_at_a_time.lock();
+            char *o = (char*)out->data_ptr() + done;
+            const char* qr = (const char*)q->data_ptr() + done;
+            bt += chunks * table->stride(0); cl += chunks;
+            void* ws = need ? scratch.data_ptr() : nullptr;
+            const size_t ws_bytes = need ? (size_t)scratch.numel() : 0;
+            if (key) {
+                const int64_t later = t_pre * key->stride(0) * (int64_t)key->element_size();
+                return aicomp_paged_decode_attn_append(
+                    o, qr, (const char*)key->data_ptr() + later, (const char*)value->data_ptr() + later, key->stride(0),
+                    key->stride(1), kp, vp, bt, table->stride(0), cl, (int)rows, hq, p.hkv, p.d, p.bs, width, p.nb,
+                    (float)scale, dt, p.dt, p.ks, p.vs, 0, ws, ws_bytes, stream);
+            }
+            return aicomp_paged_decode_attn(o, qr, kp, vp, bt, table->stride(0), cl, (int)rows, hq, p.hkv, p.d, p.bs, width, p.nb,
+                                            (float)scale, dt, p.dt, p.ks, p.vs, 0, ws, ws_bytes, stream);
+        });
+        DONE(rc);
+    } catch (const std::exception& e) {
+        FAIL("%s", e.what());
+    }
+}
+
 // (tokens come back as a new tensor; None: take the Python way)
 PyObject* sample_tokens(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     try {
@@ -776,6 +920,8 @@ PyMethodDef methods[] = {
      "layer(k_pool, v_pool, block_table, ctx_rows) -> handle: a layer's static tensors, checked once"},
     {"decode_step", (PyCFunction)(void (*)(void))decode_step, METH_FASTCALL,
      "decode_step(layer, query, key, value, position, group, scale) -> out [B, Hq, 1, D]"},
+    {"prompt_step", FAST(prompt_step),
+     "prompt_step(layer, slots, cu, query, key, value, position, group, scale) -> out [B, Hq, n, D], or None"},
     {"kv_append", FAST(kv_append), "ops.kv_append of a plain call: True once launched, False if it is not one"},
     {"rope_kv_append", FAST(rope_kv_append), "ops.rope_kv_append of a plain call, out given"},
     {"paged_decode_attn", FAST(paged_decode_attn), "ops.paged_decode_attn of a plain call"},
@@ -785,6 +931,7 @@ PyMethodDef methods[] = {
     {"plan_upload", FAST(plan_upload), "the packed plan on its way to the device: its five tensors there"},
     {"paged_prefill_attn", FAST(paged_prefill_attn), "ops.paged_prefill_attn of a plain call, max_q_len given"},
     {"append_prefill_attn", FAST(append_prefill_attn), "ops.append_prefill_attn of a plain call"},
+    {"chunks_and_rows", FAST(chunks_and_rows), "prompt chunks and one-token rows of a step, each through their own kernels"},
     {"sample_tokens", FAST(sample_tokens), "ops.sample_tokens of a plain call: the tokens, or None if it is not one"},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -98,13 +98,14 @@ class PagedAttentionBackend:
                                            plan.host_context_lens)
         if S and npre == 0:
             return ops.paged_decode_attn(out, q, kp, vp, plan.block_table, plan.context_lens, self.scale, ks, vs)
+        if npre and S > npre:
+            return ops.chunks_and_rows_attn(out, q, None, None, kp, vp, None, plan.block_table, plan.context_lens,
+                                            plan.cu_q_lens, self.scale, plan.max_q_len, npre, t_pre, ks, vs,
+                                            plan.prefill_items(q, kp), plan.few_chunk_lens(q.shape[1], kp.shape[1]))
         if npre:
             ops.paged_prefill_attn(out[:t_pre], q[:t_pre], kp, vp, plan.block_table[:npre], plan.context_lens[:npre],
                                    plan.cu_q_lens[:npre + 1], self.scale, max_q_len=plan.max_q_len,
                                    k_scale=ks, v_scale=vs, items=plan.prefill_items(q, kp))
-        if S > npre:
-            ops.paged_decode_attn(out[t_pre:], q[t_pre:], kp, vp, plan.block_table[npre:], plan.context_lens[npre:],
-                                  self.scale, ks, vs)
         return out
 
 

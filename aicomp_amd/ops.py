@@ -558,6 +558,39 @@ def append_prefill_attn(out: torch.Tensor, query: torch.Tensor, key: Optional[to
                               k_scale=k_scale, v_scale=v_scale, items=items)
 
 
+def chunks_and_rows_attn(out: torch.Tensor, query: torch.Tensor, key: Optional[torch.Tensor],
+                         value: Optional[torch.Tensor], k_pool: torch.Tensor, v_pool: torch.Tensor,
+                         slot_mapping: Optional[torch.Tensor], block_table: torch.Tensor, context_lens: torch.Tensor,
+                         cu_q_lens: torch.Tensor, scale: float, max_q_len: int, num_chunks: int, chunk_rows: int,
+                         k_scale: Optional[torch.Tensor] = None, v_scale: Optional[torch.Tensor] = None,
+                         items: Optional[torch.Tensor] = None, chunk_lens=None) -> torch.Tensor:
+    """A layer's step of prompt chunks, the first ``num_chunks`` sequences and ``chunk_rows`` rows, and of one-token rows,
+    through the prefill and the decode kernels one after the other: ``kv_append`` and ``paged_prefill_attn`` of the chunks,
+    ``paged_decode_attn`` of the rows with their append (``key`` None: the new rows are in the pools already).
+    ``chunk_lens``: the chunks' context lengths on the host, with which they may take the kernel for few chunks
+    (``append_prefill_attn``)."""
+    decode = "aicomp_paged_decode_attn" if key is None else "aicomp_paged_decode_attn_append"
+    prefill = "aicomp_paged_prefill_attn" if items is None else "aicomp_paged_prefill_attn_items"
+    if _native(decode) and _lib.untouched(prefill) and _lib.untouched("aicomp_kv_append") \
+            and _lib.untouched("aicomp_kv_append_prefill_attn_sized") \
+            and _FAST.chunks_and_rows(out, query, k_pool, v_pool, block_table, context_lens, cu_q_lens, scale, max_q_len,
+                                      k_scale, v_scale, items, key, value, slot_mapping, num_chunks, chunk_rows, chunk_lens):
+        return out
+    n, t = num_chunks, chunk_rows
+    if chunk_lens is not None:
+        new = (None, None, None) if key is None else (key[:t], value[:t], slot_mapping[:t])
+        append_prefill_attn(out[:t], query[:t], new[0], new[1], k_pool, v_pool, new[2], block_table[:n], context_lens[:n],
+                            cu_q_lens[:n + 1], scale, max_q_len, k_scale, v_scale, items, chunk_lens)
+    else:
+        if key is not None:
+            kv_append(key[:t], value[:t], k_pool, v_pool, slot_mapping[:t], k_scale, v_scale)
+        paged_prefill_attn(out[:t], query[:t], k_pool, v_pool, block_table[:n], context_lens[:n], cu_q_lens[:n + 1], scale,
+                           max_q_len=max_q_len, k_scale=k_scale, v_scale=v_scale, items=items)
+    paged_decode_attn(out[t:], query[t:], k_pool, v_pool, block_table[n:], context_lens[n:], scale, k_scale, v_scale,
+                      new_key=None if key is None else key[t:], new_value=None if key is None else value[t:])
+    return out
+
+
 def rotary_tables(inv_freq: torch.Tensor, num_positions: int, dtype: torch.dtype,
                   attention_scaling: float = 1.0, device=None):
     """cos / sin tables ``[num_positions, D]`` the way the reference's rotary module builds them

@@ -65,13 +65,12 @@ static bool streamk_shape(int batch, int hq, int hkv, int d, int bs, int q_dtype
 // A decode call over few, short rows is a chain of launch and memory latencies, not a stream: the
 // balanced schedule (set up for 256 CUs of work, always followed by its merge kernel) then loses to
 // one workgroup per (row, KV head, partition) on the grid schedule, without any merge kernel when
-// no row can be longer than 768 (head_dim 128) or 1280 (64) tokens of a 16-bit pool, 640 or 448 of
-// another (measured on 1 to 16 rows of 512 and 2048 tokens: 5.4-8.5 against 9-13 us, 8-15 against
+// no row can be longer than whole_row_tokens (measured on 1 to 16 rows of 512 and 2048 tokens: 5.4-8.5 against 9-13 us, 8-15 against
 // 11-17 us).  "Small" is rows x (table width x block size) at or
 // below a process-wide threshold: 32768 by default, or the value of the environment variable
 // AICOMP_KV_SMALL_DECODE_TOKENS when the library first needs it (read once, never again), or what
 // aicomp_kv_set_small_decode_tokens() stored last (0 keeps every automatic call of a supported
-// shape on the balanced schedule).  The sizing helpers and the decode calls read the same word.
+// shape on the balanced schedule).  Larger calls may take it too: see grid_call.  The sizing helpers and the decode calls read the same word.
 static std::atomic<long long>& small_decode_tokens() {
     static std::atomic<long long> limit{[] {
         const char* e = getenv("AICOMP_KV_SMALL_DECODE_TOKENS");
@@ -84,26 +83,58 @@ static bool small_call(int64_t rows, int bs, int max_blocks) {
     return rows * (int64_t)max_blocks * bs <= small_decode_tokens().load(std::memory_order_relaxed);
 }
 
-static int auto_partition(int64_t rows, int hkv, int d, int bs, int max_blocks, int kv_dtype, bool matrix_shape) {
+// Tokens up to which a row of the matrix-core grid schedule is whole in `wgs` (row, KV head) workgroups.
+// Few workgroups: the line lies where the merge's launch (about 3 us of device and 3 us of host time) costs what the longer
+// chain of one workgroup does: 1000 and 1200 tokens at D 64 whole 7.2 and 7.4 us, split 8.0 us, 2000 tokens 9.7 and 7.9;
+// D 128: 760 tokens 7.7 and 8.8, 1000 tokens 9.2 and 8.2 us.  Other pools: 640.  Float32 at D 64: 640 tokens of
+// one row whole 10.1 us, split 9.4 (and 3 us of host time), 768 tokens 11.3 and 9.9.  A float32 row at D 128
+// is as many bytes as two bf16 rows on its CU: whole up to 448 tokens where the split has a CU for each of its
+// workgroups (one row of 448 12.2 whole, 11.5 split; 512 tokens 13.1 and 12.1, 640 15.3
+// and 11.9), otherwise up to 640 (16 rows of 8 KV heads, 640 tokens 19.1 and 21.5, 768 tokens 21.8 and 23.2).
+// At the two float32 lines themselves the split is 0.7 us faster on the device, which is less than the host
+// time that its second launch takes.
+// More workgroups share the memory's bandwidth, a longer row is then hidden behind the others and neither a split nor the
+// balanced schedule has its start and merge to show for it.  Whole / the better of the two, us, 8 KV heads:
+//   bf16 D 128   128 workgroups 768 tokens 11.5 / 13.0, 1168 16.6 / 14.6;  256  1168 19.2 / 22.1, 1536 23.3 / 25.6 (of unlike
+//                lengths 1616 19.5 / 16.7);  512  1200 36.5 / 39.0, 1600 46.4 / 46.0;  1024  1200 64.1 / 68.6, 1600 84.1 / 91.1
+//   bf16 D 64    128  1536 12.7 / 12.6;  256  1600 16.0 / 20.7, 2100 18.1 / 22.0;  512  1168 20.4 / 24.7, 2600 0.94, 3600 0.98
+//   fp8 D 128    128  1168 0.98;  256  1536 0.81, 2100 0.83;  512  1600 0.93, 2672 0.96;  of D 64  256  2672 0.78;  512  3600 0.89
+//   float32 D 64 256  1168 0.87;  384  1200 1.02;  512  1200 0.94, 1600 1.03;  16 / 2 heads, bf16: 128 800 0.86, 256 1200 0.82
+// One head per KV head merges little: 8 / 8 heads, D 128, 384 workgroups 1200 tokens 30.6 / 28.8.  More than 512 workgroups come
+// in rounds: 768 of D 64, 2112 tokens 51.2 / 49.0, of fp8 54.4 / 53.0.
+static int64_t whole_row_tokens(int64_t wgs, int group, int d, int64_t max_ctx, int kv_dtype) {
+    const int64_t more = std::min<int64_t>(std::max<int64_t>(wgs - 64, 0), 448), rounds = wgs > 512 ? 2048 : 4096;
+    if (is_16bit_float(kv_dtype)) return d == 64 ? std::min(1280 + 4 * more, rounds) : 768 + (group > 1 ? 2 : 1) * more;
+    if (kv_dtype == AICOMP_KV_FP8_E4M3) return d == 64 ? std::min<int64_t>(640 + 10 * more, 4096) : std::min(640 + 5 * more, rounds);
+    if (d == 64) return std::min<int64_t>(640 + 3 * more / 2, 1100);
+    return wgs * ((max_ctx + 255) / 256) <= 256 ? 448 : 640;
+}
+
+// Whether an automatic call takes the grid schedule.  Beyond the threshold (one that is at least the default; a lower
+// one pins the schedule) it still does where its rows are whole, and where few (row, KV head) pairs are long: each of the
+// balanced schedule's waves then has so few tiles that its start and flush outweigh them.  Split in 256 tokens / balanced, us,
+// 8 KV heads, by tokens x KV heads:  24 rows of 2096 (402 k) 27.3 / 29.2, 2672 (513 k) 30.3 / 31.6, of unlike lengths 15.9 /
+// 19.0 and 21.2 / 23.3;  32 of 2096 (537 k) 34.3 / 34.7, 48 of 1600 (614 k) 34.9 / 35.8, 2096 (805 k) 45.8 / 45.9;  16 / 2 heads:
+// 64 of 2112 (270 k) 0.95, 3600 (461 k) 1.00, 16 of 3584 (115 k) 0.76;  fp8 pools cross earlier: 16 of 2672 (342 k) 0.94,
+// 24 of 2096 (402 k) 1.02, 2672 (513 k) 1.05;  float32 rows of D 128 at once (48 of 800 46.5 / 37.8).
+static bool grid_call(int64_t rows, int hq, int hkv, int d, int bs, int max_blocks, int kv_dtype) {
+    if (small_call(rows, bs, max_blocks)) return true;
+    const int64_t limit = small_decode_tokens().load(std::memory_order_relaxed), max_ctx = (int64_t)max_blocks * bs;
+    if (limit < 32768 || rows * hkv > 2048) return false;               // (measured up to there)
+    return max_ctx <= whole_row_tokens(rows * hkv, hq / hkv, d, max_ctx, kv_dtype) ||
+           (max_ctx <= 4096 && !(kv_dtype == AICOMP_KV_F32 && d == 128) &&
+            rows * hkv * max_ctx <= (kv_dtype == AICOMP_KV_FP8_E4M3 ? 12 : 16) * std::min<int64_t>(limit, 1 << 20));
+}
+
+static int auto_partition(int64_t rows, int hq, int hkv, int d, int bs, int max_blocks, int kv_dtype, bool matrix_shape) {
     // Longer partitions amortise a workgroup's start-up and merge; shorter ones give the
     // 256 CUs enough workgroups when there are few (sequence, KV head) rows.
     const int64_t max_ctx = (int64_t)max_blocks * bs;
     int ps;
-    if (matrix_shape && small_call(rows, bs, max_blocks)) {
-        // Matrix-core grid schedule: whole rows (a whole number of its 64-token tiles) and no merge
-        // launch, or partitions of 256 tokens.  The line lies where the merge's launch (about 3 us of
-        // device and 3 us of host time) costs what the longer chain of one workgroup does: 1000 and
-        // 1200 tokens at D 64 whole 7.2 and 7.4 us, split 8.0 us, 2000 tokens 9.7 and 7.9; D 128: 760
-        // tokens 7.7 and 8.8, 1000 tokens 9.2 and 8.2 us.  Other pools: 640.  Float32 at D 64: 640 tokens of
-        // one row whole 10.1 us, split 9.4 (and 3 us of host time), 768 tokens 11.3 and 9.9.  A float32 row at D 128
-        // is as many bytes as two bf16 rows on its CU: whole up to 448 tokens where the split has a CU for each of its
-        // workgroups (one row of 448 12.2 whole, 11.5 split; 512 tokens 13.1 and 12.1, 640 15.3
-        // and 11.9), otherwise up to 640 (16 rows of 8 KV heads, 640 tokens 19.1 and 21.5, 768 tokens 21.8 and 23.2).
-        // At the two float32 lines themselves the split is 0.7 us faster on the device, which is less than the host
-        // time that its second launch takes.
-        const bool f32_few = kv_dtype == AICOMP_KV_F32 && d == 128 && rows * hkv * ((max_ctx + 255) / 256) <= 256;
-        const int64_t whole = f32_few ? 448 : !is_16bit_float(kv_dtype) ? 640 : d == 64 ? 1280 : 768;
-        ps = max_ctx <= whole ? (int)((max_ctx + 63) / 64 * 64) : 256;
+    if (matrix_shape && grid_call(rows, hq, hkv, d, bs, max_blocks, kv_dtype)) {
+        // matrix-core grid schedule: whole rows (a whole number of its 64-token tiles) and no merge launch, or partitions of
+        // 256 tokens
+        ps = max_ctx <= whole_row_tokens(rows * hkv, hq / hkv, d, max_ctx, kv_dtype) ? (int)((max_ctx + 63) / 64 * 64) : 256;
     } else {
         ps = 64;       // vector-ALU kernel on few short rows: spread the call wide
         for (int cand : {1024, 512, 256, 128}) {
@@ -237,13 +268,13 @@ int aicomp_paged_decode_partition_size(int batch, int num_q_heads, int num_kv_he
                                        int block_size, int max_blocks_per_seq, int q_dtype,
                                        int kv_dtype) {
     if (batch <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || block_size <= 0 || max_blocks_per_seq <= 0) return 0;
-    return auto_partition(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype,
+    return auto_partition(batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype,
                           streamk_shape(batch, num_q_heads, num_kv_heads, head_dim, block_size, q_dtype, kv_dtype));
 }
 
-static int resolve_parts(int64_t rows, int hkv, int d, int bs, int max_blocks, int kv_dtype, bool matrix_shape,
+static int resolve_parts(int64_t rows, int hq, int hkv, int d, int bs, int max_blocks, int kv_dtype, bool matrix_shape,
                          int& partition_size) {
-    if (partition_size <= 0) partition_size = auto_partition(rows, hkv, d, bs, max_blocks, kv_dtype, matrix_shape);
+    if (partition_size <= 0) partition_size = auto_partition(rows, hq, hkv, d, bs, max_blocks, kv_dtype, matrix_shape);
     const int64_t max_ctx = (int64_t)max_blocks * bs;
     int64_t parts = (max_ctx + partition_size - 1) / partition_size;
     return (int)(parts < 1 ? 1 : parts);
@@ -257,9 +288,10 @@ size_t aicomp_paged_decode_workspace_bytes(int batch, int num_q_heads, int num_k
         return 0;
     const bool automatic = partition_size <= 0;
     const bool matrix_shape = streamk_shape(batch, num_q_heads, num_kv_heads, head_dim, block_size, q_dtype, kv_dtype);
-    const int parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, matrix_shape, partition_size);
+    const int parts = resolve_parts(batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, matrix_shape, partition_size);
     size_t need = parts <= 1 ? 0 : split_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, parts);
-    if (automatic && matrix_shape && !small_call(batch, block_size, max_blocks_per_seq)) {
+    if (automatic && matrix_shape &&
+        !grid_call(batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype)) {
         const size_t sk = decode_streamk_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim);
         if (sk > need) need = sk;
     }
@@ -304,13 +336,14 @@ static int decode_impl(void* out, const void* query, const void* new_key, const 
     a.v_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? v_scale : nullptr;
     a.partition_size = partition_size;
     const bool matrix_shape = streamk_shape(batch, num_q_heads, num_kv_heads, head_dim, block_size, q_dtype, kv_dtype);
-    a.num_parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, matrix_shape, a.partition_size);
+    a.num_parts = resolve_parts(batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, matrix_shape, a.partition_size);
     a.stream = (hipStream_t)stream;
     // the matrix-core kernels append the new rows themselves when they can read them 16 bytes at a time
     const int64_t vec = 16 / dtype_size(q_dtype);
     const bool injectable = fused && kv_token_stride % vec == 0 && kv_head_stride % vec == 0 && (uintptr_t)new_key % 16 == 0 &&
                             (uintptr_t)new_value % 16 == 0;
-    if (partition_size == 0 && decode_streamk_supported(a) && !small_call(batch, block_size, max_blocks_per_seq)) {
+    if (partition_size == 0 && decode_streamk_supported(a) &&
+        !grid_call(batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype)) {
         // balanced schedule: equal tile counts per wave, merged by a second kernel
         const size_t need = decode_streamk_workspace_bytes(a.rows, a.hq, a.hkv, a.d);
         AICOMP_REQUIRE(workspace && workspace_bytes >= need, AICOMP_KV_EWORKSPACE,
@@ -431,13 +464,17 @@ static int rope_decode_impl(void* out, const void* query, int64_t q_token_stride
     a.scale = scale; a.q_dtype = q_dtype; a.kv_dtype = kv_dtype;
     a.k_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? k_scale : nullptr;
     a.v_scale = kv_dtype == AICOMP_KV_FP8_E4M3 ? v_scale : nullptr;
-    a.num_parts = resolve_parts(batch, num_kv_heads, head_dim, block_size, columns, kv_dtype, shape, a.partition_size);
+    a.num_parts = resolve_parts(batch, num_q_heads, num_kv_heads, head_dim, block_size, columns, kv_dtype, shape, a.partition_size);
     a.stream = (hipStream_t)stream;
     // A batch for the balanced schedule streams for tens of microseconds: the launch saved is lost in it.  So it is in split
     // rows of more than 512 workgroups (two calls, which the table's width sends to the balanced schedule, / this one, us:
     // 32 rows of 700, fp8 pool, 32/8 heads, D 128 18.1 / 21.1, D 64 17.2 / 18.7, 64/8 19.4 / 23.6), but for float32 groups
     // of up to four heads (32 rows of 700, D 128 37.8 / 33.4, D 64 24.4 / 20.2).
-    const bool few = a.num_parts == 1 || (int64_t)batch * num_kv_heads * a.num_parts <= 512 ||
+    // (counted by the lines of few workgroups, whatever the call's own partitions are)
+    const int64_t max_ctx = (int64_t)columns * block_size, wgs = (int64_t)batch * num_kv_heads;
+    const int64_t whole = whole_row_tokens(kv_dtype == AICOMP_KV_F32 && head_dim == 128 ? wgs : std::min<int64_t>(wgs, 64),
+                                           num_q_heads / num_kv_heads, head_dim, max_ctx, kv_dtype);
+    const bool few = max_ctx <= whole || wgs * ((max_ctx + 255) / 256) <= 512 ||
                      (q_dtype == AICOMP_KV_F32 && num_q_heads <= 4 * num_kv_heads);
     AICOMP_REQUIRE(vectors && shape && few && small_call(batch, block_size, columns) && decode_mfma_supported(a),
                    AICOMP_KV_EUNSUPPORTED, "%s: not a call of the matrix-core grid schedule", who);
@@ -526,13 +563,19 @@ int aicomp_paged_decode_attn_append_static(void* out, const void* query, const v
         return aicomp_paged_decode_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim, block_size,
                                                    max_blocks_per_seq, q_dtype, kv_dtype, ps);
     };
-    size_t need = scratch_bytes(partition_size);
+    // Which shapes are too large follows from the threshold alone: one above it counts as the balanced schedule would take
+    // it, also where the call keeps to the grid schedule and needs less.
+    const bool balanced = partition_size == 0 && num_kv_heads > 0 && batch > 0 && num_q_heads % num_kv_heads == 0 &&
+                          streamk_shape(batch, num_q_heads, num_kv_heads, head_dim, block_size, q_dtype, kv_dtype) &&
+                          !small_call(batch, block_size, max_blocks_per_seq);
+    size_t need = std::max(scratch_bytes(partition_size),
+                           balanced ? decode_streamk_workspace_bytes(batch, num_q_heads, num_kv_heads, head_dim) : (size_t)0);
     if (partition_size == 0 && need > (size_t)AICOMP_KV_STATIC_SCRATCH_BYTES && q_dtype == AICOMP_KV_F32 &&
         kv_dtype == AICOMP_KV_F32) {
         // The balanced schedule's partials have a fixed part of 4096 slots, 34 MB for sixteen heads of 128 per KV
         // head whatever the batch.  The grid schedule over partitions chosen by the number of workgroups needs
         // less: 32 rows of 2048 tokens, 16 / 1 heads, 8.5 MB.
-        partition_size = auto_partition(batch, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, false);
+        partition_size = auto_partition(batch, num_q_heads, num_kv_heads, head_dim, block_size, max_blocks_per_seq, kv_dtype, false);
         need = scratch_bytes(partition_size);
     }
     AICOMP_REQUIRE(need <= (size_t)AICOMP_KV_STATIC_SCRATCH_BYTES, AICOMP_KV_EWORKSPACE,

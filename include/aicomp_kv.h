@@ -60,8 +60,10 @@ const char* aicomp_kv_last_error(void);
 /*
  * Routing threshold of automatic decode calls (partition_size 0), in tokens: a call with
  * batch * max_blocks_per_seq * block_size at or below it takes the grid schedule (see
- * aicomp_paged_decode_attn), a larger one the balanced schedule; 0 sends every supported shape
- * to the balanced schedule.  Process-wide; the initial value is 32768, or the value of the
+ * aicomp_paged_decode_attn).  A larger one takes the balanced schedule, except that with a
+ * threshold of at least the default, 32768, the grid schedule also keeps the larger calls whose
+ * rows it does not split and those of few long rows (aicomp_paged_decode_attn).  0 sends every
+ * supported shape to the balanced schedule.  Process-wide; the initial value is 32768, or the value of the
  * environment variable AICOMP_KV_SMALL_DECODE_TOKENS at the library's first use of it (the
  * environment is read once, never per call).  Stores `tokens` and returns the previous value; a
  * negative `tokens` only queries.  aicomp_paged_decode_workspace_bytes and
@@ -131,7 +133,14 @@ int aicomp_kv_append(const void* key, const void* value,
  *                   max_blocks_per_seq * block_size <= 768 (head_dim 128) or 1280 (64) over a
  *                   16-bit pool, 640 over another (448 over a float32 pool of head_dim 128 when
  *                   the partitions of all rows and KV heads are at most 256): such a call is bound by launch and memory latency, not
- *                   by bandwidth.  The result is the same to within the tolerance between split sizes (2e-3).
+ *                   by bandwidth.  From 64 to 512 pairs of a row and a KV head that limit grows, to 1664 tokens of
+ *                   bf16 or fp16 at head_dim 128 (1216 with as many KV heads as query heads), 3072 at 64, of fp8
+ *                   2880 and 4096 (2048 of head_dim 128, and of 16 bits at 64, beyond 512 pairs), of float32 1100 at
+ *                   64; and calls above the threshold take this schedule too where rows are whole by it, or, with
+ *                   rows of at most 4096 tokens, where batch * num_kv_heads * max_blocks_per_seq * block_size is at
+ *                   most sixteen times the threshold (fp8: twelve; not float32 at head_dim 128), split in 256 tokens: many rows hide
+ *                   each other's latency, and few give the balanced schedule too little to balance (at most 2048
+ *                   pairs of a row and a KV head).  The result is the same to within the tolerance between split sizes (2e-3).
  *   workspace       device scratch of at least
  *                   aicomp_paged_decode_workspace_bytes(...) bytes (may be NULL
  *                   when that returns 0), 16-byte aligned.  Its contents need

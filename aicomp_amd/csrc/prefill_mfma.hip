@@ -812,9 +812,17 @@ int launch_prefill_mfma(const DecodeArgs& a, int max_q_len) {
         const int64_t wgs = groups * std::min(tiles * a.num_seqs, a.rows / tile_pos + a.num_seqs);
         const int64_t keys = a.longest_context > 0 ? a.longest_context : (int64_t)a.max_blocks * a.bs;
         const int cols = tile_pos * gpack / ROWS;
+        // More workgroups, longer contexts: this kernel walks them at the latency of its loads with up to 512 workgroups, the other
+        // one takes as long as it has rows and keys.  Here / there in us, by column groups (workgroups times cols):
+        //   D 128, 32/8  112: 994 24 / 17, 1973 41 / 23, 3493 70 / 34    144: 301 17 / 18, 1031 29 / 24, 2010 48 / 33, 3530 78 / 48
+        //                192: 411 22 / 25    224: 994 28 / 33, 1973 46 / 49    240: 2014 49 / 46, 3536 82 / 62    288: 2064 50 / 51
+        //          fp8   224: 1973 45 / 40;  16/2  108: 1035 30 / 21    136: 481 19 / 20, 1085 30 / 23    208: 2039 50 / 43
+        //   D 64, one    56: 994 17 / 14, 1973 30 / 17    112: 994 18 / 23, 1973 32 / 29, 3493 46 / 32;  two  144: 2010 36 / 41
         // (sixteen heads of 64 are more rows per position than its workgroups have)
-        const bool rows = a.d == 128 ? wgs <= 64 && (keys >= 256 || (cols == 2 && (wgs <= 32 || a.num_seqs == 1)))
-                                     : wgs <= 32 && group != 16 && (wgs * cols <= 32 ? cols == 2 || keys >= 192 : keys >= 600);
+        const bool rows = a.d == 128 ? (wgs <= 64 && (keys >= 256 || (cols == 2 && (wgs <= 32 || a.num_seqs == 1)))) ||
+                                           (wgs * cols <= 144 && keys >= 640) || (wgs * cols <= 192 && keys >= 2048)
+                                     : group != 16 && ((wgs <= 32 && (wgs * cols <= 32 ? cols == 2 || keys >= 192 : keys >= 600)) ||
+                                                       (cols == 1 && ((wgs <= 64 && keys >= 900) || (wgs <= 112 && keys >= 2048))));
         if (rows) return launch_prefill_rows(a, max_q_len, tile_pos, wgs);
     }
     PrefillParams p;

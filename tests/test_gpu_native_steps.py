@@ -6,7 +6,7 @@ import torch
 import test_gpu_prefill as tp
 from aicomp_amd import kv_cache, ops
 from aicomp_amd.kv_cache import CachedScaledDotProductAttention
-from helpers import assert_close_attn, to_f64
+from helpers import assert_close_attn, kernels_of, to_f64
 
 pytestmark = pytest.mark.gpu
 
@@ -93,3 +93,20 @@ def test_chunks_and_rows(device, monkeypatch, dtype, kv, hq, hkv, d, appended, l
     for x, y in zip(*got):
         assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
     assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("hq,hkv,d,priors,news,longest,rows", [
+    # column groups of the tile kernel: up to 144 from 640 keys on, up to 192 from 2048 (head_dim 64, one per workgroup: 64 from 900, 112 from 2048)
+    (32, 8, 128, [3000, 900, 2000] + [0] * 3, [30] * 6, 3030, True), (32, 8, 128, [607] * 9, [32] * 9, 639, False),
+    (32, 8, 128, [608] * 9, [32] * 9, 640, True), (16, 2, 128, [2100] + [40] * 8, [70] * 9, 2170, True),
+    (16, 2, 128, [1900] + [40] * 8, [70] * 9, 1970, False), (16, 4, 64, [884] * 15, [16] * 15, 900, True),
+    (16, 4, 64, [874] * 15, [16] * 15, 890, False), (16, 4, 64, [2032] + [100] * 24, [16] * 25, 2048, True)])
+@pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, None), (torch.float16, torch.float8_e4m3fn)])
+def test_more_chunks_of_long_contexts(device, dtype, kv, hq, hkv, d, priors, news, longest, rows):
+    c = tp.build_case(device, priors, news, hq, hkv, d, dtype=dtype, kv_dtype=kv, seed=d)
+    out = torch.full_like(c["q"], float("nan"))
+    names = kernels_of(lambda: ops.append_prefill_attn(
+        out, c["q"], None, None, c["k_pool"], c["v_pool"], None, c["table"], c["ctx"], c["cu"], c["scale"], max(news), c["ks"],
+        c["vs"], None, np.full(len(news), longest, dtype=np.int32)))
+    assert any(("paged_prefill_rows" if rows else "paged_prefill_mfma") in n for n in names), names
+    assert_close_attn(to_f64(out), tp.oracle(c), 1e-2, 2e-2, f"{hq}/{hkv} {d}")

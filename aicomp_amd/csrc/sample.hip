@@ -76,7 +76,7 @@ constexpr int PART_MAX = NT * PART_SLOTS;           // 16384
 constexpr int GREEDY_CAP = 256;                     // room per part of a greedy call, which keeps one: 2 KB apart
 constexpr int RAW_CAP = 2048;                       // candidates of a part before the exact test
 constexpr int MAX_PARTS = 16;
-constexpr int MERGE_SLOTS = 8;                      // candidates a lane of the merge takes: NT * 8 per row
+constexpr int MERGE_SLOTS = 16;                     // candidates a lane of the merge takes: 16 lists of 1024 per row
 constexpr int PART_MAX_K = 256;
 constexpr int PART_MAX_BATCH = 1024;
 constexpr unsigned int PART_WHOLE = 0xffffffffu;
@@ -205,10 +205,6 @@ __device__ __forceinline__ uint64_t shfl64(uint64_t v, int src) {
     const uint32_t lo = __shfl((uint32_t)v, src), hi = __shfl((uint32_t)(v >> 32), src);
     return ((uint64_t)hi << 32) | lo;
 }
-__device__ __forceinline__ uint64_t shfl_up64(uint64_t v, int d) {
-    const uint32_t lo = __shfl_up((uint32_t)v, d), hi = __shfl_up((uint32_t)(v >> 32), d);
-    return ((uint64_t)hi << 32) | lo;
-}
 __device__ __forceinline__ uint64_t wave_sum64(uint64_t v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -217,13 +213,26 @@ __device__ __forceinline__ uint64_t wave_sum64(uint64_t v) {
     }
     return v;
 }
-__device__ __forceinline__ uint64_t wave_incl_scan64(uint64_t v, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint64_t o = shfl_up64(v, d);
-        if (lane >= d) v += o;
-    }
-    return v;
+// Sum over the lanes up to and including this one, in the vector ALU (every lane active): four shifts within a
+// row of sixteen lanes, then the rows' last lanes broadcast onwards.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned long long dpp_add64(unsigned long long v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xf, false);
+    return v + ((unsigned long long)hi << 32 | lo);
+}
+__device__ __forceinline__ unsigned long long wave_scan_dpp64(unsigned long long v) {
+    v = dpp_add64<0x111, 0xf>(v);            // row_shr 1, 2, 4, 8
+    v = dpp_add64<0x112, 0xf>(v);
+    v = dpp_add64<0x114, 0xf>(v);
+    v = dpp_add64<0x118, 0xf>(v);
+    v = dpp_add64<0x142, 0xa>(v);            // row_bcast 15: into rows 1 and 3
+    return dpp_add64<0x143, 0xc>(v);         // row_bcast 31: into rows 2 and 3
+}
+__device__ __forceinline__ unsigned long long readlane64(unsigned long long v, int lane) {
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+    return (unsigned long long)hi << 32 | lo;
 }
 
 // The largest key with its low ten bits clear that at least r lanes of the wave reach (0: fewer do).
@@ -332,7 +341,7 @@ __device__ __forceinline__ void pick_by_mass(Shared& s, int nbins, unsigned long
         const int b = nbins - 1 - (lane * per + j);
         if (b >= 0) local += s.mass[b];
     }
-    const unsigned long long incl = wave_incl_scan64(local, lane);
+    const unsigned long long incl = wave_scan_dpp64(local);
     const unsigned long long excl = incl - local;
     // mass above the LAST bin of a lane's range is incl - mass[last]; the walk continues past a
     // lane while even the mass above the first bin of the next lane (= incl) is <= limit
@@ -614,7 +623,7 @@ __device__ __forceinline__ void no_mass(S& s, const SampleParams& p, int row_idx
 // Sum of v over the lanes before this one, and over all.
 __device__ __forceinline__ unsigned long long block_scan(Shared& s, unsigned long long v, unsigned long long& total) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned long long incl = wave_incl_scan64(v, lane);            // -> sum before this lane
+    unsigned long long incl = wave_scan_dpp64(v);            // -> sum before this lane
     if (lane == 63) s.seg_mass[wave] = incl;
     __syncthreads();
     unsigned long long before = 0;
@@ -628,74 +637,78 @@ __device__ __forceinline__ unsigned long long block_scan(Shared& s, unsigned lon
     return before + incl - v;
 }
 
-// At most one candidate per lane.
+// Ranks of the entries wave + NW l (mine, lane l) of a list of n among the 64 G at list_w: those above it, by (key, ~index) and, << 16, by
+// ~index alone.  The entries are in registers, 64 to a compare: a ballot and a scalar count per 64 pairs, where reading
+// them from LDS for every pair was bound by those reads.  The zeros behind the list are above nothing.
+template <int G>
+__device__ __forceinline__ uint32_t list_ranks(const unsigned long long* list_w, int n, unsigned long long mine, int lane, int wave) {
+    unsigned long long x[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) x[g] = list_w[64 * g + lane];
+    uint32_t ranks = 0;
+    for (int l = 0; NW * l + wave < n; ++l) {
+        const unsigned long long me = readlane64(mine, l);
+        int by_key = 0, by_index = 0;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            by_key += __popcll(__ballot(x[g] > me));
+            by_index += __popcll(__ballot((uint32_t)x[g] > (uint32_t)me));
+        }
+        ranks = lane == l ? (uint32_t)(by_key | by_index << 16) : ranks;
+    }
+    return ranks;
+}
+
+// At most one candidate per lane, in list_key and list_idx.
 // No histograms: every candidate is ranked in the descending order a stable sort would give (key, then
 // index) and in index order, by counting; with top-k the one of rank k-1 holds the k-th largest key;
 // the mass before a candidate in the first order decides the nucleus, a scan in the second
 // order the draw.  Exact 64-bit sums.  Without top-k the list is everything above a cut of the
 // whole row and z_row the mass of the whole row.
-// The counting is n^2 compares: a candidate's are shared by as many lanes as there are for it.  (One lane each and a
-// loop over the list for every mass took 10 of the 25 us of a call over 64 rows, k = 50.)
+// A chain of short steps between barriers: four of them, five with top_p.  One launch over 64 rows of 32000 float32: k 65 16.5
+// -> 15.4 us, k 256 23.0 -> 21.9, k 600 58.0 -> 53.9 (eight barriers before, ranks by LDS reads, scans by LDS permutes).
 template <typename T, int U>
 __device__ __forceinline__ void draw_from_small_list(Shared& s, const SampleParams& p, int row_idx, const T* row, bool vec_ok,
                                                      float m, bool has_topk, unsigned long long z_row) {
-    const int tid = threadIdx.x, V = p.vocab;
-    const int n = (int)s.n_list;                                    // 1..NT
-    int sh = 6;                                                     // 2^sh lanes per candidate
-    while (sh > 0 && (n << sh) > NT) --sh;
-    const int mine_e = tid >> sh, step = 1 << sh;
-    // (key, ~index) as one number: two compares and two adds per pair.  The zeros behind the list are
-    // above nothing in either order; a lane reads at most 8 * 64 - 1 of them.
-    if (tid < n) s.list_w[tid] = (unsigned long long)s.list_key[tid] << 32 | ~s.list_idx[tid];
-    if (tid < 512) s.list_w[n + tid] = 0;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), V = p.vocab;
+    const int n = __builtin_amdgcn_readfirstlane((int)s.n_list);    // 1..NT
+    // (key, ~index) as one number: one compare per pair
+    s.list_w[tid] = tid < n ? (unsigned long long)s.list_key[tid] << 32 | ~s.list_idx[tid] : 0ull;
     __syncthreads();
-    uint32_t ranks = 0;                                             // rank | rank by index << 16
-    if (mine_e < n) {
-        const unsigned long long me = s.list_w[mine_e];
-        unsigned int by_key = 0, by_index = 0;
-        for (int i0 = tid & (step - 1); i0 < n; i0 += 8 * step) {
-            unsigned long long e[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) e[u] = s.list_w[i0 + u * step];     // eight independent reads
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                by_key += e[u] > me ? 1u : 0u;
-                by_index += (uint32_t)e[u] > (uint32_t)me ? 1u : 0u;
-            }
-        }
-        ranks = by_key | by_index << 16;
+    unsigned long long* sorted = s.mass;                            // descending; s.cnt: the ranks by index in this order
+    const unsigned long long mine = s.list_w[NW * lane + wave];
+    uint32_t ranks;
+    if (n <= 128) ranks = list_ranks<2>(s.list_w, n, mine, lane, wave);
+    else if (n <= 256) ranks = list_ranks<4>(s.list_w, n, mine, lane, wave);
+    else if (n <= 384) ranks = list_ranks<6>(s.list_w, n, mine, lane, wave);
+    else {                                                          // (1024 at a time: 32 registers)
+        ranks = list_ranks<8>(s.list_w, n, mine, lane, wave);
+        if (n > 512) ranks += list_ranks<8>(s.list_w + 512, n, mine, lane, wave);
     }
-    for (int o = 1; o < step; o <<= 1) ranks += __shfl_xor(ranks, o);
-    if (mine_e < n && (tid & (step - 1)) == 0) {
-        s.cnt[mine_e] = ranks;
-        if (has_topk && (int)(ranks & 0xffffu) == p.top_k - 1) s.sel_digit = s.list_key[mine_e];   // one writer
+    if (NW * lane + wave < n) {
+        sorted[ranks & 0xffffu] = mine;
+        s.cnt[ranks & 0xffffu] = ranks >> 16;
     }
     __syncthreads();
-    const uint32_t kth = has_topk && n >= p.top_k ? s.sel_digit : 0u;       // fewer than k: all of them stay
-    unsigned int idx = 0, by_index = 0, by_key = 0;
+    // lane t takes the t-th entry of the sorted order
+    const uint32_t kth = has_topk && n >= p.top_k ? (uint32_t)(sorted[p.top_k - 1] >> 32) : 0u;   // fewer than k: all of them stay
+    unsigned int by_index = 0, idx = 0;
     uint64_t w = 0;
     if (tid < n) {
-        const uint32_t key = s.list_key[tid];
-        idx = s.list_idx[tid];
-        by_key = s.cnt[tid] & 0xffffu;
-        by_index = s.cnt[tid] >> 16;
-        if (key >= kth) w = weight_of(key_value(key), m);                   // ties at the k-th value all stay
+        const unsigned long long e = sorted[tid];
+        by_index = s.cnt[tid];
+        idx = ~(uint32_t)e;
+        if ((uint32_t)(e >> 32) >= kth) w = weight_of(key_value((uint32_t)(e >> 32)), m);        // ties at the k-th value all stay
     }
     unsigned long long z = 0;
     if (p.top_p < 1.f) {
-        // lane t takes the t-th entry of the sorted order
-        __syncthreads();                        // everyone has read keys and indices
-        if (tid < n) { s.list_w[by_key] = w; s.list_idx[by_key] = idx; s.list_key[by_key] = by_index; }
-        __syncthreads();
-        if (tid < n) { w = s.list_w[tid]; idx = s.list_idx[tid]; by_index = s.list_key[tid]; }
         const unsigned long long before = block_scan(s, w, z);
         // an entry stays while the mass before it is at most top_p of the total (of the row's total
         // when the list is a cut of the whole row rather than its top k)
         const unsigned long long limit = (unsigned long long)((double)fmaxf(p.top_p, 0.f) * (double)(has_topk ? z : z_row));
         if (before > limit) w = 0;
     }
-    __syncthreads();
-    if (tid < n) { s.list_w[by_index] = w; s.list_idx[by_index] = idx; }
+    if (tid < n) { s.list_w[by_index] = w; s.list_idx[by_index] = idx; }    // (both last read before the ranks were written)
     __syncthreads();
     w = 0;
     if (tid < n) { w = s.list_w[tid]; idx = s.list_idx[tid]; }
@@ -944,7 +957,7 @@ __device__ __forceinline__ void sample_row(const SampleParams& p, Shared& s, int
         }
         __syncthreads();
         const unsigned long long mine_b = s.mass[tid];
-        unsigned long long incl = wave_incl_scan64(mine_b, lane);
+        unsigned long long incl = wave_scan_dpp64(mine_b);
         if (lane == 63) s.seg_mass[wave] = incl;
         __syncthreads();
         unsigned long long base = 0;
@@ -1058,7 +1071,7 @@ __device__ __forceinline__ void sample_row(const SampleParams& p, Shared& s, int
     const unsigned int lane_tied_base = my_tied_base + tied_incl - lane_tied;
     if (tie_rule && lane_tied_base < tie_keep)
         lane_mass += (unsigned long long)min(lane_tied, tie_keep - lane_tied_base) * w_t_val;
-    const unsigned long long incl = my_base + wave_incl_scan64(lane_mass, lane);
+    const unsigned long long incl = my_base + wave_scan_dpp64(lane_mass);
     const unsigned long long hit = __ballot(lane_mass != 0 && incl > target);
     if (!hit) return;                                          // cannot happen: the segment holds the target
     const int owner = __ffsll((long long)hit) - 1;
@@ -1073,7 +1086,7 @@ __device__ __forceinline__ void sample_row(const SampleParams& p, Shared& s, int
         const unsigned long long tb = __ballot(tied);
         if (tied && tied_seen + __popcll(tb & ((1ull << lane) - 1ull)) < tie_keep) w = w_t_val;
         tied_seen += __popcll(tb);
-        const unsigned long long sc = wave_incl_scan64(w, lane);
+        const unsigned long long sc = wave_scan_dpp64(w);
         const unsigned long long h2 = __ballot(w != 0 && running + sc > target);
         if (h2) {
             if (lane == __ffsll((long long)h2) - 1) p.out[row_idx] = i;
@@ -1083,26 +1096,79 @@ __device__ __forceinline__ void sample_row(const SampleParams& p, Shared& s, int
     }
 }
 
-// Sum over the lanes up to and including this one, in the vector ALU (every lane active): four shifts within a
-// row of sixteen lanes, then the rows' last lanes broadcast onwards.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ unsigned long long dpp_add64(unsigned long long v) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xf, false);
-    return v + ((unsigned long long)hi << 32 | lo);
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false));      // as in wave_scan_dpp64
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
-__device__ __forceinline__ unsigned long long wave_scan_dpp64(unsigned long long v) {
-    v = dpp_add64<0x111, 0xf>(v);            // row_shr 1, 2, 4, 8
-    v = dpp_add64<0x112, 0xf>(v);
-    v = dpp_add64<0x114, 0xf>(v);
-    v = dpp_add64<0x118, 0xf>(v);
-    v = dpp_add64<0x142, 0xa>(v);            // row_bcast 15: into rows 1 and 3
-    return dpp_add64<0x143, 0xc>(v);         // row_bcast 31: into rows 2 and 3
-}
-__device__ __forceinline__ unsigned long long readlane64(unsigned long long v, int lane) {
-    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, lane);
-    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
-    return (unsigned long long)hi << 32 | lo;
+
+// SLOTS entries per lane of the lists of a row's parts, read while their lengths are still on the way.
+// Lane -> part lane >> lp of 2^(6 - lp) >= parts; a list goes round the waves in pieces of at most eight entries
+// (64 bytes), so that their shares of it are alike.
+template <int SLOTS>
+struct Lists {
+    uint2 e[SLOTS];
+    unsigned int count;                                      // entries of the lane's list
+    int at, stride;
+
+    __device__ __forceinline__ void load(const SampleParams& p, int row_idx, int lane, int wave) {
+        const int lp = __clz(p.parts - 1) - 26, piece = min(lp, 3);
+        const int q = lane >> lp, l = lane & ((1 << lp) - 1);
+        stride = NW << lp;
+        at = ((((l >> piece) * NW) + wave) << piece) + (l & ((1 << piece) - 1));
+        const bool in = q < p.parts;
+        const unsigned int* counts = p.part_count + (int64_t)row_idx * p.parts;
+        const uint2* list = p.part_list + ((int64_t)row_idx * p.parts + (in ? q : 0)) * p.part_cap;
+#pragma unroll
+        for (int u = 0; u < SLOTS; ++u) {
+            e[u] = make_uint2(0u, 0u);
+            if (SLOTS <= 4 || u * stride < p.part_cap) e[u] = list[min(at + u * stride, p.part_cap - 1)];
+        }
+        count = in ? counts[q] : 0u;
+    }
+    // a list is longer than its lanes' SLOTS, or than its room
+    __device__ __forceinline__ bool too_long(const SampleParams& p) const {
+        return __any(count > (unsigned int)min(p.part_cap, SLOTS * stride));
+    }
+    __device__ __forceinline__ bool empty() const { return !__any(count != 0u); }
+    // key 0 (no candidate has it) beyond a list's end; the lane's largest key
+    __device__ __forceinline__ uint32_t trim() {
+        uint32_t top = 0;
+#pragma unroll
+        for (int u = 0; u < SLOTS; ++u) {
+            if ((unsigned int)(at + u * stride) >= count) e[u].x = 0u;
+            top = max(top, e[u].x);
+        }
+        return top;
+    }
+};
+
+// A bound of the row's top_k-th largest key from below, 1 at least, out of the lanes' largest ones: the largest of the waves'
+// bounds that top_k lanes of all waves reach (the smallest of the sixteen always is such a one, but lets several times as
+// many pass).  s.cnt[0 .. NW) is zero before; two barriers.
+__device__ __forceinline__ uint32_t bound_of_lanes(const SampleParams& p, Shared& s, uint32_t top, int lane, int wave) {
+    const uint32_t bound = wave_rth_bound(top, (p.top_k + NW - 1) / NW);
+    if (lane == 0) s.seg_tied[wave] = bound;
+    __syncthreads();
+    const uint32_t t = s.seg_tied[lane & 15];
+    unsigned int reach = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const unsigned int r = (unsigned int)__popcll(__ballot(top >= (uint32_t)__builtin_amdgcn_readlane((int)t, w)));
+        reach = lane == w ? r : reach;
+    }
+    if (lane < NW) atomicAdd(&s.cnt[lane], reach);
+    __syncthreads();
+    uint32_t key_l = s.cnt[lane & 15] >= (unsigned int)p.top_k ? t : 0u;
+    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x128, 0xf, 0xf, false));   // row_ror 8, 4, 2, 1
+    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x124, 0xf, 0xf, false));
+    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x122, 0xf, 0xf, false));
+    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x121, 0xf, 0xf, false));
+    return max(key_l, 1u);
 }
 
 // The usual draw from the candidates of a row's parts, top_k <= FewK: false (for the whole workgroup, nothing written)
@@ -1125,48 +1191,15 @@ constexpr int FEW_SLOTS = 4;               // 512 entries of a list of eight par
 template <typename T>
 __device__ __forceinline__ bool merge_few(const SampleParams& p, Shared& s, int row_idx) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // lane -> part lane >> lp of 2^(6 - lp) >= parts; a list goes round the waves in pieces of at most eight entries
-    // (64 bytes), so that their shares of it are alike
-    const int lp = __clz(p.parts - 1) - 26, piece = min(lp, 3);
-    const int q = lane >> lp, l = lane & ((1 << lp) - 1), stride = NW << lp;
-    const int at = ((((l >> piece) * NW) + wave) << piece) + (l & ((1 << piece) - 1));
-    const bool in = q < p.parts;
-    const unsigned int* counts = p.part_count + (int64_t)row_idx * p.parts;
-    const uint2* list = p.part_list + ((int64_t)row_idx * p.parts + (in ? q : 0)) * p.part_cap;
-    uint2 e[FEW_SLOTS];
-#pragma unroll
-    for (int u = 0; u < FEW_SLOTS; ++u) e[u] = list[min(at + u * stride, p.part_cap - 1)];
-    const unsigned int c = in ? counts[q] : 0u;
+    Lists<FEW_SLOTS> lists;
+    lists.load(p, row_idx, lane, wave);
     if (tid < FEW) s.list_w[tid] = 0;
     if (tid < NW) s.cnt[tid] = 0;
     if (tid == 0) s.n_list = 0;
-    if (__any(c > (unsigned int)min(p.part_cap, FEW_SLOTS * stride)) || !__any(c != 0u)) return false;
-    uint32_t top = 0;
-#pragma unroll
-    for (int u = 0; u < FEW_SLOTS; ++u) {
-        if ((unsigned int)(at + u * stride) >= c) e[u].x = 0u;             // (no candidate has key 0)
-        top = max(top, e[u].x);
-    }
-    const uint32_t bound = wave_rth_bound(top, (p.top_k + NW - 1) / NW);
-    if (lane == 0) s.seg_tied[wave] = bound;
-    __syncthreads();
-    // Each wave's bound, and how many lanes of all waves reach it: the largest one that top_k lanes reach is the
-    // row's (the smallest of the sixteen always is such a one, but lets several times as many pass).
-    const uint32_t t = s.seg_tied[lane & 15];
-    unsigned int reach = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        const unsigned int r = (unsigned int)__popcll(__ballot(top >= (uint32_t)__builtin_amdgcn_readlane((int)t, w)));
-        reach = lane == w ? r : reach;
-    }
-    if (lane < NW) atomicAdd(&s.cnt[lane], reach);
-    __syncthreads();
-    uint32_t key_l = s.cnt[lane & 15] >= (unsigned int)p.top_k ? t : 0u;
-    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x128, 0xf, 0xf, false));   // row_ror 8, 4, 2, 1
-    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x124, 0xf, 0xf, false));
-    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x122, 0xf, 0xf, false));
-    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x121, 0xf, 0xf, false));
-    key_l = max(key_l, 1u);
+    if (lists.too_long(p) || lists.empty()) return false;
+    const uint32_t top = lists.trim();
+    const uint2 (&e)[FEW_SLOTS] = lists.e;
+    const uint32_t key_l = bound_of_lanes(p, s, top, lane, wave);
     unsigned long long pass[FEW_SLOTS];
     unsigned int mine_n = 0;
 #pragma unroll
@@ -1240,77 +1273,60 @@ __device__ __forceinline__ bool merge_few(const SampleParams& p, Shared& s, int 
 }
 
 // The draw from the candidates of a row's parts: those of all parts hold the row's top k, with ties (all finite
-// logits if there are fewer).  The same bound once more, over one maximum per lane, leaves a list a few times k
-// long.  A row that its parts gave up, or whose list is longer than the lanes, is done whole.
+// logits if there are fewer).  Beyond merge_few's the lists are read and bounded as there, which leaves little more than k
+// candidates (230 at k = 200) for draw_from_small_list.  A row that its parts gave up, or with more than a lane's each, is done
+// whole.  16 rows of 128256, parts and merge: k 100 18.6 -> 16.6 us, k 200 24.2 -> 19.0, k 256 27.6 -> 21.6 (before, a list's entry was
+// found by comparisons with all lists' ends, and the smallest of the waves' bounds let in twice as many).
 template <typename T>
 __global__ void __launch_bounds__(NT)
 sample_merge_kernel(SampleParams p) {
     __shared__ Shared s;
     const int row_idx = blockIdx.x;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const T* row = (const T*)p.logits + (int64_t)row_idx * p.row_stride;
     const bool vec_ok = ((uintptr_t)row % 16) == 0;
     if (p.top_k <= FewK<T>::value && p.probs_out == nullptr) {
         if (merge_few<T>(p, s, row_idx)) return;
         __syncthreads();
     }
-    const unsigned int* counts = p.part_count + (int64_t)row_idx * p.parts;
-    unsigned int end[MAX_PARTS], total = 0;
-    bool fits = true;
-#pragma unroll
-    for (int q = 0; q < MAX_PARTS; ++q) {
-        const unsigned int c = q < p.parts ? counts[q] : 0u;
-        fits = fits && c <= (unsigned int)p.part_cap;
-        total += min(c, (unsigned int)p.part_cap);
-        end[q] = total;
-    }
-    if (fits && total == 0) {                // nothing above -inf
-        no_mass<T, 4>(s, p, row_idx, row, vec_ok);
-        return;
-    }
-    if (fits && total <= (unsigned int)(NT * MERGE_SLOTS)) {
-        // candidate j goes to wave j % 16, so that the waves' shares are alike; lanes without one: key 0
-        const uint2* lists = p.part_list + (int64_t)row_idx * p.parts * p.part_cap;
-        uint2 e[MERGE_SLOTS];
-        uint32_t top = 0;
+    Lists<MERGE_SLOTS> lists;
+    lists.load(p, row_idx, lane, wave);
+    if (tid < NW) s.cnt[tid] = 0;
+    if (tid == 0) s.n_list = 0;
+    if (!lists.too_long(p)) {
+        if (lists.empty()) {                 // nothing above -inf
+            no_mass<T, 4>(s, p, row_idx, row, vec_ok);
+            return;
+        }
+        const uint32_t top = lists.trim();
+        const uint2 (&e)[MERGE_SLOTS] = lists.e;
+        const uint32_t largest = wave_max(top);
+        if (lane == 0) s.red_i[wave] = (int)largest;
+        const uint32_t key_l = bound_of_lanes(p, s, top, lane, wave);
+        const uint32_t key_m = wave_max((uint32_t)s.red_i[lane & 15]);
+        unsigned long long pass[MERGE_SLOTS];
+        unsigned int mine_n = 0;
 #pragma unroll
         for (int u = 0; u < MERGE_SLOTS; ++u) {
-            const unsigned int j = (unsigned int)(lane * NW + wave + NT * u);
-            e[u] = make_uint2(0u, 0u);
-            if (j < total) {
-                int q = 0;
-                unsigned int start = 0;
-#pragma unroll
-                for (int c = 0; c < MAX_PARTS - 1; ++c)
-                    if (j >= end[c]) { q = c + 1; start = end[c]; }
-                e[u] = lists[(int64_t)q * p.part_cap + (j - start)];
-            }
-            top = max(top, e[u].x);
+            pass[u] = __ballot(e[u].x >= key_l);
+            mine_n += (unsigned int)__popcll(pass[u]);
         }
-        const uint32_t bound = wave_rth_bound(top, (p.top_k + NW - 1) / NW);
+        unsigned int j = 0;
+        if (lane == 0 && mine_n) j = atomicAdd(&s.n_list, mine_n);
+        j = __builtin_amdgcn_readfirstlane(j);
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) top = max(top, (uint32_t)__shfl_xor(top, o));
-        if (lane == 0) { s.seg_tied[wave] = bound; s.red_i[wave] = (int)top; }
-        if (tid == 0) s.n_list = 0;
-        __syncthreads();
-        uint32_t key_l = s.seg_tied[0], key_m = (uint32_t)s.red_i[0];
-        for (int w = 1; w < NW; ++w) {
-            key_l = min(key_l, s.seg_tied[w]);
-            key_m = max(key_m, (uint32_t)s.red_i[w]);
+        for (int u = 0; u < MERGE_SLOTS; ++u) {
+            const unsigned int at = j + __popcll(pass[u] & ((1ull << lane) - 1ull));
+            if (e[u].x >= key_l && at < NT) { s.list_key[at] = e[u].x; s.list_idx[at] = e[u].y; }
+            j += (unsigned int)__popcll(pass[u]);
         }
-#pragma unroll
-        for (int u = 0; u < MERGE_SLOTS; ++u)
-            if (e[u].x >= key_l && e[u].x) {
-                const unsigned int j = atomicAdd(&s.n_list, 1u);
-                if (j < NT) { s.list_key[j] = e[u].x; s.list_idx[j] = e[u].y; }
-            }
         __syncthreads();
         if (s.n_list <= NT) {
             draw_from_small_list<T, 4>(s, p, row_idx, row, vec_ok, key_value(key_m), true, 0ull);
             return;
         }
-        __syncthreads();
     }
+    __syncthreads();
     sample_row<T, 4>(p, s, row_idx);
 }
 
@@ -1699,7 +1715,7 @@ greedy_kernel(SampleParams p) {
 }  // namespace
 
 // How many parts the rows of a call are cut into (1: none).  A second launch and the merge cost about 5 us for top_k <= FewK
-// (merge_few) and 9 us beyond, so it has to save more.  us per call, one launch -> parts:
+// (merge_few) and 8 to 11 us beyond, so it has to save more.  us per call, one launch -> parts:
 //   few (k 50)          float32  20000, 2 parts: 1 row 14.4 -> 10.0, 64 15.8 -> 11.3, 1024 61.3 -> 44.3
 //                                50256, 4 parts: 1 row 16.0 -> 10.9, 64 16.7 -> 11.7, 128 17.2 -> 13.9, 1024 86.7 -> 66.5
 //                                128256, 8 parts: 1 row 20 -> 10.7, 64 23 -> 14.4, 512 88 -> 61;  262144: 16 rows 29 -> 11.3
@@ -1717,9 +1733,14 @@ greedy_kernel(SampleParams p) {
 //   the whole row       float32  20000, 2 parts: 1 row 14.8 -> 10.9, 1024 62.9 -> 49.3;  50256: 64 rows 26.3 -> 11.7
 //   (top_p off)         128256: 1 row 50.9 -> 11.3, 64 54.9 -> 16.0, 1024 281 -> 203;  262144: 64 rows 106 -> 31.5
 //                       bf16     20000: 64 rows 17.5 -> 12.1, 1024 66.2 -> 42.7;  128256: 64 61.0 -> 16.0, 1024 258 -> 146
-//   other calls from six parts on
-//     k to 256          128256: 1 row 24.3 -> 21.1, 16 25.5 -> 24.6, 64 27.0 -> 30.3: up to 128 parts
-//     greedy            128256: 16 rows 9.1 -> 7.2, 64 10.8 -> 9.8, 128 14.1 -> 17.2: up to 512 parts
+//   k to 256            float32  50256, 4 parts: k 65 1 row 15.1 -> 14.7, 64 16.0 -> 15.6, 128 16.9 -> 18.5;  k 200 18.8 -> 17.8, 20.0 -> 18.8,
+//   from four parts on           21.0 -> 22.2;  81920, 5: 64 rows k 65 19.7 -> 18.0, k 200 24.0 -> 23.2, 128 24.1 -> 23.3, 27.5 -> 29.4
+//                                128256, 8: k 200 64 rows 26.0 -> 23.9, 128 34.5 -> 33.3, 256 50.7 -> 48.0, 512 92 -> 88, k 65 86 -> 72
+//                                262144, 16: k 200 16 rows 32.9 -> 19.7, 256 96 -> 79;  4096 parts: 34 MB of lists
+//                       bf16     50256: k 200 1 row 19.8 -> 17.8, 64 21.0 -> 19.2, 128 21.3 -> 22.1;  128256: 64 rows k 65 21.6 -> 18.8,
+//                                k 200 26.2 -> 23.3, 128 22.0 -> 25.2, 26.6 -> 31.8;  262144: 64 k 200 35.9 -> 32.0, 128 38.6 -> 47.2
+//   greedy, from six parts on
+//                       128256: 16 rows 9.1 -> 7.2, 64 10.8 -> 9.8, 128 14.1 -> 17.2: up to 512 parts
 // A nucleus of the whole row takes four launches, about 22 us of them where a row is short, so it pays from four parts on and
 // while the rows leave CUs idle.  us per call, temperature 0.8, top_p 0.9, one launch -> parts:
 //   float32  32000, 2 parts: 1 row 21.0 -> 22.4;  50256, 4: 1 row 24.3 -> 22.4, 64 25.7 -> 24.8, 128 26.1 -> 34.2;  50257: 64 35.3 -> 25.7
@@ -1747,8 +1768,9 @@ static int sample_parts(int batch, int vocab, int64_t row_stride, float temperat
         if (parts >= 6) return all <= 1024 ? parts : 1;
         return !together || all <= (parts == 5 ? 640 : 512) ? parts : 1;
     }
-    if (parts < 6) return 1;
-    return all <= (greedy || top_k <= FEW_K ? 512 : 128) ? parts : 1;
+    if (greedy) return parts >= 6 && all <= 512 ? parts : 1;
+    if (parts < 4) return 1;
+    return f32 && parts >= 8 ? (all <= 4096 ? parts : 1) : batch <= 64 ? parts : 1;
 }
 
 // Candidates a part has room for.  Of 16384 normally distributed logits about 2.7 k pass the bound of sixteen waves

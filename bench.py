@@ -332,7 +332,7 @@ def run_decode_config(name, steps, warmup, dev, settle_ms=30.0):
     }
     mfma_shape = (w.shape.head_dim in (64, 128) and w.shape.block_size == 16
                   and qd.dtype in (torch.bfloat16, torch.float16, torch.float32))
-    balanced = mfma_shape and (S - npre) <= 1024 and not routed_small        # the library's own routing rule
+    balanced = mfma_shape and (S - npre) <= 1024 and not routed_small        # the library's rule, for rows as long as these
     merge = "" if res["partition_size"] >= mb * w.shape.block_size else " + split_reduce_kernel"
     res["roofline"] = {
         "kernel": ("streamk_decode_kernel + streamk_reduce_kernel" if balanced else

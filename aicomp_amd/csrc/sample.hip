@@ -1135,11 +1135,14 @@ struct Lists {
         return __any(count > (unsigned int)min(p.part_cap, SLOTS * stride));
     }
     __device__ __forceinline__ bool empty() const { return !__any(count != 0u); }
+    // whether any lane of the wave has an entry in slot u
+    __device__ __forceinline__ bool used(int u) const { return SLOTS <= 4 || __any((unsigned int)(u * stride) < count); }
     // key 0 (no candidate has it) beyond a list's end; the lane's largest key
     __device__ __forceinline__ uint32_t trim() {
         uint32_t top = 0;
 #pragma unroll
         for (int u = 0; u < SLOTS; ++u) {
+            if (!used(u)) break;
             if ((unsigned int)(at + u * stride) >= count) e[u].x = 0u;
             top = max(top, e[u].x);
         }
@@ -1275,8 +1278,10 @@ __device__ __forceinline__ bool merge_few(const SampleParams& p, Shared& s, int 
 // The draw from the candidates of a row's parts: those of all parts hold the row's top k, with ties (all finite
 // logits if there are fewer).  Beyond merge_few's the lists are read and bounded as there, which leaves little more than k
 // candidates (230 at k = 200) for draw_from_small_list.  A row that its parts gave up, or with more than a lane's each, is done
-// whole.  16 rows of 128256, parts and merge: k 100 18.6 -> 16.6 us, k 200 24.2 -> 19.0, k 256 27.6 -> 21.6 (before, a list's entry was
-// found by comparisons with all lists' ends, and the smallest of the waves' bounds let in twice as many).
+// whole.  16 rows of 128256, parts and merge: k 100 18.6 -> 15.5 us, k 200 24.2 -> 18.2, k 256 27.6 -> 20.7 (before, a list's entry was
+// found by comparisons with all lists' ends, and the smallest of the waves' bounds let in twice as many; slots that no lane
+// has an entry for took 1.1).  Bounding a part's own list as tightly leaves fewer than k lanes with entries to bound the row by: such rows
+// were done whole, k 50 12.3 -> 24.6.
 template <typename T>
 __global__ void __launch_bounds__(NT)
 sample_merge_kernel(SampleParams p) {
@@ -1304,21 +1309,22 @@ sample_merge_kernel(SampleParams p) {
         if (lane == 0) s.red_i[wave] = (int)largest;
         const uint32_t key_l = bound_of_lanes(p, s, top, lane, wave);
         const uint32_t key_m = wave_max((uint32_t)s.red_i[lane & 15]);
-        unsigned long long pass[MERGE_SLOTS];
         unsigned int mine_n = 0;
 #pragma unroll
         for (int u = 0; u < MERGE_SLOTS; ++u) {
-            pass[u] = __ballot(e[u].x >= key_l);
-            mine_n += (unsigned int)__popcll(pass[u]);
+            if (!lists.used(u)) break;
+            mine_n += (unsigned int)__popcll(__ballot(e[u].x >= key_l));
         }
         unsigned int j = 0;
         if (lane == 0 && mine_n) j = atomicAdd(&s.n_list, mine_n);
         j = __builtin_amdgcn_readfirstlane(j);
 #pragma unroll
         for (int u = 0; u < MERGE_SLOTS; ++u) {
-            const unsigned int at = j + __popcll(pass[u] & ((1ull << lane) - 1ull));
+            if (!lists.used(u)) break;
+            const unsigned long long pass = __ballot(e[u].x >= key_l);
+            const unsigned int at = j + __popcll(pass & ((1ull << lane) - 1ull));
             if (e[u].x >= key_l && at < NT) { s.list_key[at] = e[u].x; s.list_idx[at] = e[u].y; }
-            j += (unsigned int)__popcll(pass[u]);
+            j += (unsigned int)__popcll(pass);
         }
         __syncthreads();
         if (s.n_list <= NT) {
@@ -1715,7 +1721,7 @@ greedy_kernel(SampleParams p) {
 }  // namespace
 
 // How many parts the rows of a call are cut into (1: none).  A second launch and the merge cost about 5 us for top_k <= FewK
-// (merge_few) and 8 to 11 us beyond, so it has to save more.  us per call, one launch -> parts:
+// (merge_few) and 7 to 10 us beyond, so it has to save more.  us per call, one launch -> parts:
 //   few (k 50)          float32  20000, 2 parts: 1 row 14.4 -> 10.0, 64 15.8 -> 11.3, 1024 61.3 -> 44.3
 //                                50256, 4 parts: 1 row 16.0 -> 10.9, 64 16.7 -> 11.7, 128 17.2 -> 13.9, 1024 86.7 -> 66.5
 //                                128256, 8 parts: 1 row 20 -> 10.7, 64 23 -> 14.4, 512 88 -> 61;  262144: 16 rows 29 -> 11.3
@@ -1733,12 +1739,15 @@ greedy_kernel(SampleParams p) {
 //   the whole row       float32  20000, 2 parts: 1 row 14.8 -> 10.9, 1024 62.9 -> 49.3;  50256: 64 rows 26.3 -> 11.7
 //   (top_p off)         128256: 1 row 50.9 -> 11.3, 64 54.9 -> 16.0, 1024 281 -> 203;  262144: 64 rows 106 -> 31.5
 //                       bf16     20000: 64 rows 17.5 -> 12.1, 1024 66.2 -> 42.7;  128256: 64 61.0 -> 16.0, 1024 258 -> 146
-//   k to 256            float32  50256, 4 parts: k 65 1 row 15.1 -> 14.7, 64 16.0 -> 15.6, 128 16.9 -> 18.5;  k 200 18.8 -> 17.8, 20.0 -> 18.8,
-//   from four parts on           21.0 -> 22.2;  81920, 5: 64 rows k 65 19.7 -> 18.0, k 200 24.0 -> 23.2, 128 24.1 -> 23.3, 27.5 -> 29.4
-//                                128256, 8: k 200 64 rows 26.0 -> 23.9, 128 34.5 -> 33.3, 256 50.7 -> 48.0, 512 92 -> 88, k 65 86 -> 72
-//                                262144, 16: k 200 16 rows 32.9 -> 19.7, 256 96 -> 79;  4096 parts: 34 MB of lists
-//                       bf16     50256: k 200 1 row 19.8 -> 17.8, 64 21.0 -> 19.2, 128 21.3 -> 22.1;  128256: 64 rows k 65 21.6 -> 18.8,
-//                                k 200 26.2 -> 23.3, 128 22.0 -> 25.2, 26.6 -> 31.8;  262144: 64 k 200 35.9 -> 32.0, 128 38.6 -> 47.2
+//   k to 256            float32  40000, 3 parts: k 65 1 row 15.4 -> 13.3, 64 15.7 -> 14.4, 96 15.8 -> 16.5;  k 200 18.9 -> 16.4, 19.5 -> 17.6,
+//   from three parts on          19.6 -> 20.4;  50256, 4: k 200 64 rows 20.0 -> 17.6, 96 20.0 -> 20.2, 128 20.9 -> 21.2
+//                                81920, 5: 96 rows k 65 20.0 -> 17.5, k 200 24.0 -> 23.4, 128 24.2 -> 22.1, 27.7 -> 28.2
+//                                128256, 8: k 200 64 rows 26.0 -> 23.0, 128 34.5 -> 31.9, 256 50.7 -> 47, 512 92 -> 87, k 65 86 -> 70
+//                                262144, 16: k 200 16 rows 32.9 -> 19.3, 256 96 -> 79;  4096 parts: 34 MB of lists
+//                       bf16     40000: k 200 64 rows 20.3 -> 17.9, 128 20.7 -> 21.1;  50256: 64 21.0 -> 17.9, 128 21.1 -> 21.0
+//                                128256: 64 rows k 65 21.6 -> 17.5, k 200 26.2 -> 22.2, 128 22.1 -> 24.3, 27.2 -> 30.8
+//                                262144: 64 rows k 200 35.9 -> 31.3, 128 38.0 -> 47.3
+//                       (32000, 2 parts, whose calls ask for no scratch: 64 rows k 65 15.6 -> 14.6, k 200 19.2 -> 17.1)
 //   greedy, from six parts on
 //                       128256: 16 rows 9.1 -> 7.2, 64 10.8 -> 9.8, 128 14.1 -> 17.2: up to 512 parts
 // A nucleus of the whole row takes four launches, about 22 us of them where a row is short, so it pays from four parts on and
@@ -1769,7 +1778,7 @@ static int sample_parts(int batch, int vocab, int64_t row_stride, float temperat
         return !together || all <= (parts == 5 ? 640 : 512) ? parts : 1;
     }
     if (greedy) return parts >= 6 && all <= 512 ? parts : 1;
-    if (parts < 4) return 1;
+    if (parts < 3) return 1;
     return f32 && parts >= 8 ? (all <= 4096 ? parts : 1) : batch <= 64 ? parts : 1;
 }
 

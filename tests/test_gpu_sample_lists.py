@@ -27,7 +27,7 @@ def test_equal_logits_are_drawn_in_index_order(device, V, n):
 
 
 @pytest.mark.parametrize("dtype,name", [(torch.float32, "f32"), (torch.bfloat16, "bf16"), (torch.float16, "f16")])
-@pytest.mark.parametrize("V,k", [(20000, 65), (20000, 129), (20000, 300), (20000, 700), (65536, 100), (131072, 66), (131072, 130),
+@pytest.mark.parametrize("V,k", [(20000, 65), (20000, 129), (20000, 300), (20000, 700), (40000, 90), (65536, 100), (131072, 66), (131072, 130),
                                  (131072, 200), (131072, 256), (262144, 256)])
 def test_lists_of_distinct_logits(device, V, k, dtype, name):
     """Kept set, masses and the inverse CDF in index order against the oracle.  A mass is rounded to 2^-40 of the largest, its

@@ -123,6 +123,10 @@ PyObject* layer_new(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
 }
 
+// Elements between the heads of new rows.  One head's stride is never taken, and is 0 in what is left of an expanded view
+// (repeated heads, every group-th taken), which the library refuses.
+int64_t head_stride(int hkv, int d, int64_t stride) { return hkv == 1 ? d : stride; }
+
 PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     try {
         if (nargs != 7) FAIL("decode_step(layer, query, key, value, position, group, scale)");
@@ -171,7 +175,8 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         std::unique_lock<std::mutex> one_at_a_time(scratch_launches(), std::defer_lock);
         if (ws) one_at_a_time.lock();
         const int rc = aicomp_paged_decode_attn_append(
-            out.data_ptr(), query.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1) * hstep, L->kp, L->vp,
+            out.data_ptr(), query.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(0),
+            head_stride(L->hkv, L->d, k.stride(1) * hstep), L->kp, L->vp,
             L->table, L->table_stride, L->ctx + (position + 1) * L->ctx_stride, L->B, hq, L->hkv, L->d, L->bs, width,
             L->nb, (float)scale, L->dt, L->dt, nullptr, nullptr, 0, ws, ws_bytes, stream);
         if (ws) one_at_a_time.unlock();
@@ -238,7 +243,8 @@ PyObject* prompt_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         void* stream = (void*)c10::hip::getCurrentHIPStream(L->dev.index()).stream();
         const int rc = unlocked([&] {
             return aicomp_kv_append_prefill_attn_sized(
-                out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(1), k.stride(2), L->kp, L->vp, slot_ptr,
+                out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(1),
+                head_stride(L->hkv, L->d, k.stride(2)), L->kp, L->vp, slot_ptr,
                 L->table, L->table_stride, L->ctx + (position + n) * L->ctx_stride, (const int32_t*)cu->data_ptr(), (int)B,
                 B * n, (int)n, (int)hq, L->hkv, (int)D, L->bs, L->width, L->nb, (float)scale, L->dt, L->dt, nullptr, nullptr,
                 nullptr, 0, (int)(position + n), stream);

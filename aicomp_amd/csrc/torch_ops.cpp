@@ -277,7 +277,7 @@ at::Tensor decode_step(const at::Tensor& query_in, const at::Tensor& key, const 
     void* ws = decode_workspace(workspace, own, query, B, hq, p, width, qd, kd, 0, ws_bytes);
     at::Tensor out = at::empty_like(query);
     check_rc(aicomp_paged_decode_attn_append(out.data_ptr(), query.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(0),
-                                             k.stride(1) * hstep, k_pool.data_ptr(), v_pool.data_ptr(),
+                                             p.hkv == 1 ? p.d : k.stride(1) * hstep, k_pool.data_ptr(), v_pool.data_ptr(),
                                              block_table.data_ptr<int32_t>(), block_table.stride(0),
                                              ctx_rows.data_ptr<int32_t>() + (position + 1) * ctx_rows.stride(0), B, hq,
                                              p.hkv, p.d, p.bs, width, p.nb, (float)scale, qd, kd,

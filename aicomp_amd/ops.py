@@ -345,7 +345,7 @@ class PreparedDecode:
             tail = tail[:5] + (width,) + tail[6:]
         rc = self.lib.aicomp_paged_decode_attn_append(
             out.data_ptr(), query.data_ptr(), key.data_ptr(), value.data_ptr(),
-            key.stride(0), key.stride(1) * hstep, *self._head,
+            key.stride(0), D if hkv == 1 else key.stride(1) * hstep, *self._head,     # (one head's stride may be 0, and is not taken)
             context_lens if isinstance(context_lens, int) else context_lens.data_ptr(), *tail,
             ws_ptr, ws_bytes, stream)
         _lib.check(rc, self.lib)

@@ -53,6 +53,31 @@ def test_prompt_chunks_of_the_operator(device, monkeypatch, dtype, B, hkv, group
                 assert_close_attn(to_f64(x), to_f64(y), *tol, f"{expanded} {kind}")
 
 
+@pytest.mark.parametrize("route", ["fast", "torch_op", "ctypes"])
+@pytest.mark.parametrize("B,D", [(1, 64), (3, 128)])
+def test_one_kv_head_repeated_by_a_view(device, monkeypatch, route, B, D):
+    """One KV head repeated over the query heads without a copy, as ``repeat_kv`` does: what is kept of the view has a head
+    stride of 0.  Prompt and decode against the same rows repeated by a copy."""
+    hq, g, got = 8, torch.Generator().manual_seed(D), []
+    monkeypatch.setattr(kv_cache, "_route", route)
+    calls = [[torch.randn(B, n, h, D, generator=g).to(torch.bfloat16).to(device).transpose(1, 2) for h in (hq, 1, 1)]
+             for n in (20, 3, 1, 1)]
+    for copied in (False, True):
+        op = CachedScaledDotProductAttention(0, max_seq_len=64, dtype=torch.bfloat16, num_kv_groups=hq)
+        op.enable()
+        outs = []
+        for q, k, v in calls:
+            n = q.shape[2]
+            k, v = (x[:, :, None].expand(B, 1, hq, n, D).reshape(B, hq, n, D) for x in (k, v))
+            assert k.stride(1) == 0
+            if copied:
+                k, v = k.contiguous(), v.contiguous()
+            outs.append(op(q, k, v, is_causal=n > 1))
+        got.append(outs + [op._store.k_pool, op._store.v_pool])
+    for x, y in zip(*got):
+        assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
 def test_prompt_chunks_that_are_refused(device):
     op = CachedScaledDotProductAttention(0, max_seq_len=32, dtype=torch.bfloat16)
     op.enable()

@@ -116,14 +116,15 @@ static int64_t whole_row_tokens(int64_t wgs, int group, int d, int64_t max_ctx, 
 // 8 KV heads, by tokens x KV heads:  24 rows of 2096 (402 k) 27.3 / 29.2, 2672 (513 k) 30.3 / 31.6, of unlike lengths 15.9 /
 // 19.0 and 21.2 / 23.3;  32 of 2096 (537 k) 34.3 / 34.7, 48 of 1600 (614 k) 34.9 / 35.8, 2096 (805 k) 45.8 / 45.9;  16 / 2 heads:
 // 64 of 2112 (270 k) 0.95, 3600 (461 k) 1.00, 16 of 3584 (115 k) 0.76;  fp8 pools cross earlier: 16 of 2672 (342 k) 0.94,
-// 24 of 2096 (402 k) 1.02, 2672 (513 k) 1.05;  float32 rows of D 128 at once (48 of 800 46.5 / 37.8).
+// 24 of 2096 (402 k) 1.02, 2672 (513 k) 1.05;  float32 rows of D 128 at once (48 of 800 46.5 / 37.8).  A raised threshold does
+// not move that line: the split would need more scratch than the balanced schedule (64 rows of 4096, 64 / 8 heads 34 MB, 19).
 static bool grid_call(int64_t rows, int hq, int hkv, int d, int bs, int max_blocks, int kv_dtype) {
     if (small_call(rows, bs, max_blocks)) return true;
     const int64_t limit = small_decode_tokens().load(std::memory_order_relaxed), max_ctx = (int64_t)max_blocks * bs;
     if (limit < 32768 || rows * hkv > 2048) return false;               // (measured up to there)
     return max_ctx <= whole_row_tokens(rows * hkv, hq / hkv, d, max_ctx, kv_dtype) ||
            (max_ctx <= 4096 && !(kv_dtype == AICOMP_KV_F32 && d == 128) &&
-            rows * hkv * max_ctx <= (kv_dtype == AICOMP_KV_FP8_E4M3 ? 12 : 16) * std::min<int64_t>(limit, 1 << 20));
+            rows * hkv * max_ctx <= (kv_dtype == AICOMP_KV_FP8_E4M3 ? 393216 : 524288));
 }
 
 static int auto_partition(int64_t rows, int hq, int hkv, int d, int bs, int max_blocks, int kv_dtype, bool matrix_shape) {

@@ -138,7 +138,7 @@ int aicomp_kv_append(const void* key, const void* value,
  *                   2880 and 4096 (2048 of head_dim 128, and of 16 bits at 64, beyond 512 pairs), of float32 1100 at
  *                   64; and calls above the threshold take this schedule too where rows are whole by it, or, with
  *                   rows of at most 4096 tokens, where batch * num_kv_heads * max_blocks_per_seq * block_size is at
- *                   most sixteen times the threshold (fp8: twelve; not float32 at head_dim 128), split in 256 tokens: many rows hide
+ *                   most 524288 (fp8: 393216; not float32 at head_dim 128), split in 256 tokens: many rows hide
  *                   each other's latency, and few give the balanced schedule too little to balance (at most 2048
  *                   pairs of a row and a KV head).  The result is the same to within the tolerance between split sizes (2e-3).
  *   workspace       device scratch of at least

@@ -70,3 +70,20 @@ def test_no_call_needs_more_scratch_than_on_the_balanced_schedule(lib):
                         most = lib.aicomp_paged_decode_workspace_bytes(*args)
                         lib.aicomp_kv_set_small_decode_tokens(DEFAULT)
                         assert lib.aicomp_paged_decode_workspace_bytes(*args) <= most, args
+
+
+@pytest.mark.parametrize("threshold", [DEFAULT + 1, 131072, 262144, 1 << 20, 1 << 24])
+def test_nor_under_a_raised_threshold(lib, threshold):
+    """Calls above the threshold in force; the first two outgrew the library's own 32 MiB where the line of the split rose with it."""
+    shapes = [(64, 64, 8, 128, BF16, BF16, 4096), (128, 32, 8, 128, BF16, BF16, 4096)]
+    shapes += [(rows, hq, hkv, d, q, kv, tokens) for hq, hkv in ((32, 8), (64, 8), (16, 1), (8, 8)) for d in (64, 128)
+               for q, kv in ((BF16, BF16), (F16, FP8), (F32, F32)) for rows in (16, 33, 65, 129, 300, 1024)
+               for tokens in (784, 1680, 2064, 3088, 4096, 4112, 20000)]
+    for rows, hq, hkv, d, q, kv, tokens in shapes:
+        if rows * tokens <= threshold:
+            continue
+        args = rows, hq, hkv, d, 16, tokens // 16, q, kv, 0
+        lib.aicomp_kv_set_small_decode_tokens(0)
+        most = lib.aicomp_paged_decode_workspace_bytes(*args)
+        lib.aicomp_kv_set_small_decode_tokens(threshold)
+        assert lib.aicomp_paged_decode_workspace_bytes(*args) <= most, args

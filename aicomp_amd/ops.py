@@ -445,6 +445,31 @@ def one_launch_items(context_lens, new_lens, num_prefill_seqs: int, tile_positio
     return base[np.argsort(-time, kind="stable")]
 
 
+def one_launch_times(context_lens, new_lens, num_prefill_seqs: int, tile_positions: int, num_q_heads: int, num_kv_heads: int,
+                     head_dim: int, kv_bytes: int):
+    """Estimated device us of a mixed step in one launch (``one_launch_items``) and by the prefill and decode kernels one
+    after the other, for the choice between them: fitted to 1951 steps of 16 geometries with 1 to 300 rows of 60 to 16000 tokens.
+
+    Chunk tiles keep the matrix cores busy, 48 us (head_dim 64: 30) per 1000 keys of 512 tiles, the places of a launch, and one
+    alone takes 19 (13) us per 1000 keys; rows are read at what the memory gives.  The decode kernels read a row once per
+    KV head, the one launch once per head group, which is once per QUERY head where the group does not divide 16: 28 / 4
+    heads, a chunk of 512 with 32 rows of up to 4500 tokens 207 us together, 59 apart, with one row of 500 20 and 29.
+    (Groups that the matrix-core decode kernels do not take are read half as often apart as together.)
+    """
+    import numpy as np
+    ctx, new = np.asarray(context_lens, dtype=np.int64), np.asarray(new_lens, dtype=np.int64)
+    group, wide = num_q_heads // num_kv_heads, head_dim > 64
+    hgroups = num_q_heads // (group if 16 % group == 0 else 1)
+    once = num_kv_heads if group <= (16 if wide else 8) else num_q_heads / 2
+    n, rows = new[:num_prefill_seqs], ctx[num_prefill_seqs:]
+    tiles = -(-n // tile_positions)
+    keys = tiles * (ctx[:num_prefill_seqs] - n) + tile_positions * tiles * (tiles + 1) // 2 - (tiles * tile_positions - n)
+    work = int(keys.sum()) * hgroups / 512 * (0.048 if wide else 0.030)
+    chunks = max(work, int(ctx[:num_prefill_seqs].max()) * (0.019 if wide else 0.013))
+    read = int(rows.sum()) * 2 * head_dim * kv_bytes / 7e6                       # of one head
+    return work + read * hgroups, chunks + read * once + 10 + 0.0007 * int(rows.max())
+
+
 def rope_paged_decode_attn(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                            positions: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, slot_mapping: torch.Tensor,
                            block_table: torch.Tensor, context_lens: torch.Tensor, host_lens, scale: float,

@@ -507,3 +507,20 @@ def test_launch_items_of_a_mixed_step():
     assert mixed(2000).launch_items(*wide) is None                                        # 32 columns of 64
     items = ops.one_launch_items([300, 300, 500, 400], [64, 64, 1, 1], 2, 32)
     assert items.tolist() == [[2, 0], [0, 1], [1, 1], [3, 0], [0, 0], [1, 0]]             # 350, 300, 300, 280, 268, 268
+
+
+@pytest.mark.parametrize("hq,hkv,d,fp8", [(28, 4, 128, False), (28, 4, 128, True), (40, 8, 128, False), (24, 8, 64, False),
+                                          (12, 1, 128, False)])
+def test_rows_that_one_launch_reads_once_per_query_head(hq, hkv, d, fp8):
+    """A group that does not divide 16: many rows, or long ones, are for the decode kernels, which read them once per KV head; a
+    short row beside a chunk is not worth their launches."""
+    import torch
+    q = torch.zeros(1, hq, d, dtype=torch.bfloat16)
+    pool = torch.zeros(1, hkv, 16, d, dtype=torch.bfloat16)
+    pool = pool.to(torch.float8_e4m3fn) if fp8 else pool
+    mixed = lambda rows, chunk=512: _mixed_plan([chunk] + rows, [chunk] + [1] * len(rows), 1, chunk)
+    assert mixed([500]).launch_items(q, pool) is not None
+    for rows in ([4500] * 32, [1000] * 100, [2500] * 60, [4000] * 200):
+        assert mixed(rows).launch_items(q, pool) is None, rows
+    group4 = torch.zeros(1, 4 * hkv, d, dtype=torch.bfloat16)
+    assert mixed([1000] * 100).launch_items(group4, pool) is not None

@@ -271,21 +271,13 @@ class StepPlan:
             self._prefill_items[key] = items
         return items
 
-    # Longest decode row of the one launch: a workgroup of it walks a row of its heads alone, 8 us per 1000 keys
-    # (head_dim 128; 5.5 at 64), which the decode kernels split between workgroups, and what takes its time beside it is the
-    # rest of the launch.  Device us, one launch / separate kernels, 32 / 8 heads, bf16, head_dim 128, by workgroups:
-    #     40  one row of 2000 18 / 20, 3000 23 / 20        96  8 rows of 2000 21 / 26, 3000 31 / 31, 4600 46 / 35
-    #    192  8 rows of 3000 33 / 40, 4600 50 / 44         384  8 rows of 4600 60 / 64;  32 of 4600 77 / 88, 8000 122 / 119
-    #    576  32 rows of 4600 96 / 108, 8000 135 / 138     832  100 of 4600 196 / 205, 8000 333 / 332
-    # and fp8 pools, head_dim 64 and 16 / 2, 8 / 8, 64 / 8 heads alike.  A launch has (tiles + rows) x KV heads of them (more
-    # where the group does not divide 16: those of one KV head read the same rows, and hide nothing).
-    ONE_LAUNCH_KEYS = (2000, 8, 8000)          # at least, more per workgroup, at most
+    ONE_LAUNCH_LONGEST = 16000                 # tokens of a decode row, as far as the two ways were measured
 
     def launch_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:
         """What ``paged_attention_step`` and ``attend`` run a mixed step by: the item list of one launch over its chunks and
         decode rows where that is faster than the prefill and decode kernels one after the other, else ``None``.  The kernel
         with two column groups streams a one-token row like a decode kernel does, so neither the number of rows nor an fp8
-        pool stands against it; rows too long for the launch (above) do, and rows that it reads several times over
+        pool stands against it; rows that would outlast the separate kernels do, and rows that it reads several times over
         (``ops.one_launch_times``).  Chunks too short for that kernel go through it all
         the same (``launch_q_len``; in their own kernel and the rows in theirs: 8 chunks of 30 tokens over 1500 with 8 rows of
         1000 51 us, 37 so, alone with 32 rows of 500 23 and 15), if there are as many new tokens as it asks for.
@@ -296,7 +288,7 @@ class StepPlan:
             return None
         if query.dtype not in (torch.bfloat16, torch.float16) or k_pool.dtype not in (query.dtype, torch.float8_e4m3fn):
             return None
-        key = self._list_key(("launch", self.ONE_LAUNCH_KEYS), query, k_pool)
+        key = self._list_key(("launch", self.ONE_LAUNCH_LONGEST), query, k_pool)
         if self._prefill_items is None:
             self._prefill_items = {}
         items = self._prefill_items.get(key, _UNSEEN)
@@ -308,11 +300,9 @@ class StepPlan:
             group = hq // hkv
             gpack = group if 16 % group == 0 else 1
             if bound <= self.total_new_tokens and tile * gpack == 128 and (d == 128 or gpack <= 8):  # (sixteen heads of 64 do not stream)
-                least, more, most = self.ONE_LAUNCH_KEYS
-                wgs = (int((-(-self.new_lens[:npre] // tile)).sum()) + ndec) * hkv
                 together, apart = ops.one_launch_times(self.host_context_lens, self.new_lens, npre, tile, hq, hkv, d,
                                                        k_pool.element_size())
-                if together < apart and int(self.host_context_lens[npre:].max()) <= min(most, least + more * wgs):
+                if together < apart and int(self.host_context_lens[npre:].max()) <= self.ONE_LAUNCH_LONGEST:
                     items = ops.one_launch_items(self.host_context_lens, self.new_lens, npre, tile)
                     items = torch.from_numpy(items).to(query.device, non_blocking=True)
             self._prefill_items[key] = items

@@ -455,19 +455,28 @@ def one_launch_times(context_lens, new_lens, num_prefill_seqs: int, tile_positio
     KV head, the one launch once per head group, which is once per QUERY head where the group does not divide 16: 28 / 4
     heads, a chunk of 512 with 32 rows of up to 4500 tokens 207 us together, 59 apart, with one row of 500 20 and 29.
     (Groups that the matrix-core decode kernels do not take are read half as often apart as together.)
+
+    A row is walked by one workgroup per head group, 10 (5) us per 1000 keys, 0.7 of that from an fp8 pool, and by a third of
+    the launch's time more beside other work, where the decode kernels split it: no row may outlast the separate kernels.
+    32 / 8 heads, head_dim 128, bf16, together / apart: a chunk of 128 with one row of 1000 15 / 20, 8 rows of which one is of
+    2000 25 / 24, of 4600 48 / 31, 100 rows of up to 4600 209 / 223, 100 of which one is of 8000 and the others of up to 300
+    86 / 44; 4 chunks of 300 over 1000 with 8 rows of which one is of 4600 63 / 64, of 8000 94 / 67.  Over all 1951 steps the choice
+    costs 1 % more than the faster way of each, at most 1.4 times (1.75 where the few-chunk kernel is the separate way).
     """
-    import numpy as np
-    ctx, new = np.asarray(context_lens, dtype=np.int64), np.asarray(new_lens, dtype=np.int64)
+    # (plain numbers: a step has a few chunks, and array calls on so few cost 15 us a step, this 5)
+    ctx, new = (x.tolist() if hasattr(x, "tolist") else list(x) for x in (context_lens, new_lens))
     group, wide = num_q_heads // num_kv_heads, head_dim > 64
     hgroups = num_q_heads // (group if 16 % group == 0 else 1)
     once = num_kv_heads if group <= (16 if wide else 8) else num_q_heads / 2
-    n, rows = new[:num_prefill_seqs], ctx[num_prefill_seqs:]
-    tiles = -(-n // tile_positions)
-    keys = tiles * (ctx[:num_prefill_seqs] - n) + tile_positions * tiles * (tiles + 1) // 2 - (tiles * tile_positions - n)
-    work = int(keys.sum()) * hgroups / 512 * (0.048 if wide else 0.030)
-    chunks = max(work, int(ctx[:num_prefill_seqs].max()) * (0.019 if wide else 0.013))
-    read = int(rows.sum()) * 2 * head_dim * kv_bytes / 7e6                       # of one head
-    return work + read * hgroups, chunks + read * once + 10 + 0.0007 * int(rows.max())
+    rows, keys = ctx[num_prefill_seqs:], 0
+    for c, n in zip(ctx[:num_prefill_seqs], new):
+        tiles = -(-n // tile_positions)
+        keys += tiles * (c - n) + tile_positions * tiles * (tiles + 1) // 2 - (tiles * tile_positions - n)
+    work = keys * hgroups / 512 * (0.048 if wide else 0.030)
+    chunks = max(work, max(ctx[:num_prefill_seqs]) * (0.019 if wide else 0.013))
+    read, longest = sum(rows) * 2 * head_dim * kv_bytes / 7e6, max(rows)          # of one head
+    together, walk = work + read * hgroups, longest * (0.010 if wide else 0.005) * (0.7 if kv_bytes == 1 else 1)
+    return max(together, walk + 0.3 * together), chunks + read * once + 10 + 0.0007 * longest
 
 
 def rope_paged_decode_attn(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,

@@ -492,9 +492,11 @@ def test_launch_items_of_a_mixed_step():
     assert sorted(map(tuple, it.tolist())) == sorted([(s, t) for s in range(2) for t in range(16)] + [(s, 0) for s in range(2, 10)])
     plan = mixed(2000)
     assert plan.launch_items(q, pool) is plan.launch_items(q, pool)
-    # (32 tiles + rows) x 8 head groups
-    assert mixed(2000 + 8 * 320).launch_items(q, pool) is not None and mixed(2001 + 8 * 320).launch_items(q, pool) is None
-    assert mixed(8000, n_dec=300).launch_items(q, pool) is not None and mixed(8001, n_dec=300).launch_items(q, pool) is None
+    # 32 tiles, then 8 rows and more that are as long as each other, or one of them alone: the memory's time, or the longest row's
+    skewed = lambda ctx_dec, n_dec, rest=200: _mixed_plan([612] * 2 + [ctx_dec] + [rest] * (n_dec - 1), [512] * 2 + [1] * n_dec, 2, 512)
+    for plan_of, n_dec, last in ((mixed, 8, 3146), (mixed, 60, 16000), (skewed, 1, 2131), (skewed, 8, 2195), (skewed, 300, 4886)):
+        assert plan_of(last, n_dec).launch_items(q, pool) is not None and plan_of(last + 1, n_dec).launch_items(q, pool) is None
+    assert skewed(8000, 100, 100).launch_items(q, pool) is None                            # many short rows hide no long one
     assert mixed(2000).launch_items(q, pool.to(torch.float8_e4m3fn)) is not None
     assert mixed(2000, npre=0).launch_items(q, pool) is None and mixed(2000, n_dec=0).launch_items(q, pool) is None
     assert mixed(2000).launch_items(q.float(), pool.float()) is None

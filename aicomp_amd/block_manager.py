@@ -238,7 +238,7 @@ class StepPlan:
     # tokens; a row of 8192 and more tokens, walked by a single workgroup row, makes it up to
     # twice as slow, and beyond ~128 rows the decode kernel's faster streaming wins)
     ONE_LAUNCH_MAX_CONTEXT = 4608
-    ONE_LAUNCH_MAX_ROWS = 128
+    ONE_LAUNCH_MAX_ROWS = 1 << 30              # decode rows of the one launch: a caller's cap, 0 switches it off
 
     def step_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:
         """Item list over ALL sequences of a mixed step (chunks and one-token rows) for one launch
@@ -248,7 +248,7 @@ class StepPlan:
         two-column-group kernel, or a decode part outside the bounds above.  Cached per step."""
         from . import ops
         npre, ndec = self.num_prefill_seqs, self.num_decode_seqs
-        if not npre or not ndec or ndec > self.ONE_LAUNCH_MAX_ROWS:
+        if not npre or not ndec or ndec > min(128, self.ONE_LAUNCH_MAX_ROWS):
             return None
         if query.dtype not in (torch.bfloat16, torch.float16) or k_pool.dtype != query.dtype:
             return None
@@ -281,10 +281,10 @@ class StepPlan:
         (``ops.one_launch_times``).  Chunks too short for that kernel go through it all
         the same (``launch_q_len``; in their own kernel and the rows in theirs: 8 chunks of 30 tokens over 1500 with 8 rows of
         1000 51 us, 37 so, alone with 32 rows of 500 23 and 15), if there are as many new tokens as it asks for.
-        ``ONE_LAUNCH_MAX_ROWS`` of 0 switches it off.  Cached per step."""
+        No step of more than ``ONE_LAUNCH_MAX_ROWS`` decode rows takes it.  Cached per step."""
         from . import ops
         npre, ndec = self.num_prefill_seqs, self.num_decode_seqs
-        if not npre or not ndec or not self.ONE_LAUNCH_MAX_ROWS:
+        if not npre or not ndec or ndec > self.ONE_LAUNCH_MAX_ROWS:
             return None
         if query.dtype not in (torch.bfloat16, torch.float16) or k_pool.dtype not in (query.dtype, torch.float8_e4m3fn):
             return None

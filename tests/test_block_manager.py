@@ -480,6 +480,18 @@ def test_step_plan_sends_only_moderate_decode_parts_through_one_launch():
     assert mixed(2000).step_items(torch.zeros(1, 32, 256, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 256, dtype=torch.bfloat16)) is None
 
 
+@pytest.mark.parametrize("cap", [0, 1, 8, 64])
+def test_cap_on_the_rows_of_the_one_launch(monkeypatch, cap):
+    import torch
+
+    from aicomp_amd.block_manager import StepPlan
+    monkeypatch.setattr(StepPlan, "ONE_LAUNCH_MAX_ROWS", cap)
+    q, pool = torch.zeros(1, 32, 128, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 128, dtype=torch.bfloat16)
+    for rows in (1, 8, 9, 64, 65, 200):
+        plan = _mixed_plan([612] + [500] * rows, [512] + [1] * rows, 1, 512)
+        assert (plan.launch_items(q, pool) is not None) == (rows <= cap)
+
+
 def test_launch_items_of_a_mixed_step():
     """StepPlan.launch_items: one launch however many rows and for fp8 pools too, unless its longest row outlasts the rest of
     the launch; every tile and row once, in falling time."""

@@ -247,6 +247,14 @@ __device__ __forceinline__ uint32_t wave_rth_bound(uint32_t key, int r) {
     return t;
 }
 
+// The largest over the lanes of a row of sixteen.
+__device__ __forceinline__ uint32_t largest_of_16(uint32_t v) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));   // row_ror 8, 4, 2, 1
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false));
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false));
+}
+
 // What a raw logit has to reach so that its scaled key can be key_ls = the scaled key of key_l: a
 // prefilter of one compare per element (it lets through whatever the key order would, -0.0 next to +0.0,
 // and everything when the bound lies below -inf, whose key decodes to a NaN).
@@ -467,9 +475,9 @@ __device__ __forceinline__ Nucleus nucleus_threshold(Shared& s, Src src, uint32_
 // row's top k leaves it.  Each wave finds the r-th largest of its 64 lane maxima, r = ceil(k / 16); at
 // least 16 r >= k elements of the part reach the smallest of the sixteen, so whatever lies below it (in
 // scaled order, ties stay) is not among the part's top k, nor the row's.  About 2.6 k of 16384 pass at
-// k = 50.  A logit of -inf has no mass and is left out; a part with a NaN, or one
-// with more than part_cap candidates (masses of equal logits), sends its row the whole way.  Greedy: the part's
-// argmax is its one candidate.
+// k = 50 (the tight bound of the merge would leave it too few lanes with entries there, k 50 12.3 -> 24.6).  A logit of -inf has no mass and
+// is left out; a part with a NaN, or one with more than part_cap candidates (masses of equal logits), sends its row the whole way.
+// Greedy: the part's argmax is its one candidate.
 //
 // Bound by latency: one round of loads, 22 ballots, three barriers, a few dozen appends.  64 rows of 128256
 // float32, k = 50: 8.8 us here and 5.2 us in sample_merge_kernel as traced, where one launch took 25.5 us.
@@ -1108,11 +1116,12 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
 
 // SLOTS entries per lane of the lists of a row's parts, read while their lengths are still on the way.
 // Lane -> part lane >> lp of 2^(6 - lp) >= parts; a list goes round the waves in pieces of at most eight entries
-// (64 bytes), so that their shares of it are alike.
-template <int SLOTS>
+// (64 bytes), so that their shares of it are alike.  TURN: each slot goes to the lanes of the next part, so that a list longer
+// than its lanes has the other parts' too: the row's top may be in one part.
+template <int SLOTS, bool TURN>
 struct Lists {
     uint2 e[SLOTS];
-    unsigned int count;                                      // entries of the lane's list
+    unsigned int count;                                      // entries of the list of the lane's part
     int at, stride;
 
     __device__ __forceinline__ void load(const SampleParams& p, int row_idx, int lane, int wave) {
@@ -1120,15 +1129,16 @@ struct Lists {
         const int q = lane >> lp, l = lane & ((1 << lp) - 1);
         stride = NW << lp;
         at = ((((l >> piece) * NW) + wave) << piece) + (l & ((1 << piece) - 1));
-        const bool in = q < p.parts;
         const unsigned int* counts = p.part_count + (int64_t)row_idx * p.parts;
-        const uint2* list = p.part_list + ((int64_t)row_idx * p.parts + (in ? q : 0)) * p.part_cap;
+        const uint2* lists = p.part_list + (int64_t)row_idx * p.parts * p.part_cap;
+        auto part = [&](int u) { return TURN ? (q + u) & ((64 >> lp) - 1) : q; };
 #pragma unroll
         for (int u = 0; u < SLOTS; ++u) {
             e[u] = make_uint2(0u, 0u);
-            if (SLOTS <= 4 || u * stride < p.part_cap) e[u] = list[min(at + u * stride, p.part_cap - 1)];
+            if (SLOTS <= 4 || u * stride < p.part_cap)
+                e[u] = lists[(part(u) < p.parts ? part(u) : 0) * p.part_cap + min(at + u * stride, p.part_cap - 1)];
         }
-        count = in ? counts[q] : 0u;
+        count = q < p.parts ? counts[q] : 0u;
     }
     // a list is longer than its lanes' SLOTS, or than its room
     __device__ __forceinline__ bool too_long(const SampleParams& p) const {
@@ -1138,12 +1148,13 @@ struct Lists {
     // whether any lane of the wave has an entry in slot u
     __device__ __forceinline__ bool used(int u) const { return SLOTS <= 4 || __any((unsigned int)(u * stride) < count); }
     // key 0 (no candidate has it) beyond a list's end; the lane's largest key
-    __device__ __forceinline__ uint32_t trim() {
+    __device__ __forceinline__ uint32_t trim(int lane) {
         uint32_t top = 0;
 #pragma unroll
         for (int u = 0; u < SLOTS; ++u) {
             if (!used(u)) break;
-            if ((unsigned int)(at + u * stride) >= count) e[u].x = 0u;
+            const unsigned int c = TURN && u ? __shfl(count, (lane + u * (stride / NW)) & 63) : count;
+            if ((unsigned int)(at + u * stride) >= c) e[u].x = 0u;
             top = max(top, e[u].x);
         }
         return top;
@@ -1166,12 +1177,7 @@ __device__ __forceinline__ uint32_t bound_of_lanes(const SampleParams& p, Shared
     }
     if (lane < NW) atomicAdd(&s.cnt[lane], reach);
     __syncthreads();
-    uint32_t key_l = s.cnt[lane & 15] >= (unsigned int)p.top_k ? t : 0u;
-    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x128, 0xf, 0xf, false));   // row_ror 8, 4, 2, 1
-    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x124, 0xf, 0xf, false));
-    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x122, 0xf, 0xf, false));
-    key_l = max(key_l, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key_l, 0x121, 0xf, 0xf, false));
-    return max(key_l, 1u);
+    return max(largest_of_16(s.cnt[lane & 15] >= (unsigned int)p.top_k ? t : 0u), 1u);
 }
 
 // The usual draw from the candidates of a row's parts, top_k <= FewK: false (for the whole workgroup, nothing written)
@@ -1194,13 +1200,13 @@ constexpr int FEW_SLOTS = 4;               // 512 entries of a list of eight par
 template <typename T>
 __device__ __forceinline__ bool merge_few(const SampleParams& p, Shared& s, int row_idx) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    Lists<FEW_SLOTS> lists;
+    Lists<FEW_SLOTS, false> lists;
     lists.load(p, row_idx, lane, wave);
     if (tid < FEW) s.list_w[tid] = 0;
     if (tid < NW) s.cnt[tid] = 0;
     if (tid == 0) s.n_list = 0;
     if (lists.too_long(p) || lists.empty()) return false;
-    const uint32_t top = lists.trim();
+    const uint32_t top = lists.trim(lane);
     const uint2 (&e)[FEW_SLOTS] = lists.e;
     const uint32_t key_l = bound_of_lanes(p, s, top, lane, wave);
     unsigned long long pass[FEW_SLOTS];
@@ -1276,12 +1282,13 @@ __device__ __forceinline__ bool merge_few(const SampleParams& p, Shared& s, int 
 }
 
 // The draw from the candidates of a row's parts: those of all parts hold the row's top k, with ties (all finite
-// logits if there are fewer).  Beyond merge_few's the lists are read and bounded as there, which leaves little more than k
-// candidates (230 at k = 200) for draw_from_small_list.  A row that its parts gave up, or with more than a lane's each, is done
-// whole.  16 rows of 128256, parts and merge: k 100 18.6 -> 15.5 us, k 200 24.2 -> 18.2, k 256 27.6 -> 20.7 (before, a list's entry was
-// found by comparisons with all lists' ends, and the smallest of the waves' bounds let in twice as many; slots that no lane
-// has an entry for took 1.1).  Bounding a part's own list as tightly leaves fewer than k lanes with entries to bound the row by: such rows
-// were done whole, k 50 12.3 -> 24.6.
+// logits if there are fewer).  Beyond merge_few's the lists are read and bounded as there, but turned, which leaves little more than
+// k candidates (230 at k = 200) for draw_from_small_list.  A row that its parts gave up, or with more than a lane's each, is done
+// whole.  16 rows of 128256, parts and merge, by replayed graphs: k 100 21.2 -> 18.4 us, k 200 27.1 -> 21.0, k 256 32.5 -> 23.6 (before, a
+// list's entry was found by comparisons with all lists' ends, and the smallest of the waves' bounds let in twice as many; slots
+// that no lane has an entry for took 1.1).  A language model's rows have their top in few parts: logits of deviation 2.5 less
+// ln(1 + index), 64 rows of 128256, k 200 30.2 -> 27.2, k 256 33.1 -> 30.6; with lists that keep to their part's lanes, fewer than k of
+// them then, such rows were done whole, 33.5 and 51.2.
 template <typename T>
 __global__ void __launch_bounds__(NT)
 sample_merge_kernel(SampleParams p) {
@@ -1294,7 +1301,7 @@ sample_merge_kernel(SampleParams p) {
         if (merge_few<T>(p, s, row_idx)) return;
         __syncthreads();
     }
-    Lists<MERGE_SLOTS> lists;
+    Lists<MERGE_SLOTS, true> lists;
     lists.load(p, row_idx, lane, wave);
     if (tid < NW) s.cnt[tid] = 0;
     if (tid == 0) s.n_list = 0;
@@ -1303,7 +1310,7 @@ sample_merge_kernel(SampleParams p) {
             no_mass<T, 4>(s, p, row_idx, row, vec_ok);
             return;
         }
-        const uint32_t top = lists.trim();
+        const uint32_t top = lists.trim(lane);
         const uint2 (&e)[MERGE_SLOTS] = lists.e;
         const uint32_t largest = wave_max(top);
         if (lane == 0) s.red_i[wave] = (int)largest;

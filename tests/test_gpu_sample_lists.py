@@ -37,11 +37,32 @@ def test_lists_of_distinct_logits(device, V, k, dtype, name):
     x[1, torch.randperm(V, generator=g)[:k // 2]] += 9
     x[2, V // 3:V // 3 + k] += 9
     u = torch.rand(3, generator=g)
+    check_draws(device, x, u, k, name)
+
+
+@pytest.mark.parametrize("dtype,name", [(torch.float32, "f32"), (torch.bfloat16, "bf16")])
+@pytest.mark.parametrize("V,k", [(40000, 65), (131072, 50), (131072, 65), (131072, 100), (131072, 256), (262144, 64), (262144, 200)])
+def test_lists_of_clustered_logits(device, V, k, dtype, name):
+    """Rows whose top is in few parts, or in few waves of a part: likelier tokens of lower index, as a language model's (lists longer
+    than their room at first, k 256), all of it in the last part but one, and clusters of 256 (rows done whole)."""
+    g = torch.Generator().manual_seed(V + k)
+    fall = torch.log1p(torch.arange(V, dtype=torch.float32))
+    x = torch.randn(5, V, generator=g)
+    x[0] = x[0] * 1.5 - fall
+    x[1] -= fall
+    x[2] = x[2] * 2.5 - 2 * fall
+    part = 16384 * ((V - 1) // 16384 - 1)
+    x[3, part + torch.randperm(16384, generator=g)[:2 * k]] += 30
+    x[4] += torch.randn((V + 255) // 256, generator=g).mul(2).repeat_interleave(256)[:V]
+    check_draws(device, x.to(dtype), torch.rand(5, generator=g), k, name)
+
+
+def check_draws(device, x, u, k, name):
     for top_p in (1.0, 0.9):
         tokens, probs = ops.sample_tokens(x.to(device), 0.8, k, top_p, uniforms=u.to(device), return_probs=True)
         plain = ops.sample_tokens(x.to(device), 0.8, k, top_p, uniforms=u.to(device))
         assert torch.equal(plain, tokens)
-        for b in range(3):
+        for b in range(len(x)):
             row, p = x[b].float().numpy(), probs[b].cpu().double().numpy()
             want = S.filtered_probs(row, 0.8, k, top_p, name)
             if top_p < 1:                                   # entries at the threshold may fall on either side

@@ -255,6 +255,39 @@ __device__ __forceinline__ uint32_t largest_of_16(uint32_t v) {
     return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false));
 }
 
+// A bound of the top_k-th largest of all lanes' entries, N each (0: none), from below: each wave's r-th largest entry, r =
+// ceil(top_k / 16), and of these the largest one that top_k entries reach (0: none does).  Any lane may hold any number of
+// the top; the waves' shares of it should be alike.  reach[0 .. NW) is zero before the first of two barriers.
+template <int N>
+__device__ __forceinline__ uint32_t bound_of_entries(const uint32_t (&key)[N], int top_k, uint32_t* bounds, unsigned int* reach, int lane,
+                                                     int wave) {
+    const int r = (top_k + NW - 1) / NW;
+    uint32_t mine = 0;
+#pragma unroll 1
+    for (int bit = 31; bit >= 10; --bit) {
+        const uint32_t cand = mine | (1u << bit);
+        int n = 0;
+#pragma unroll
+        for (int u = 0; u < N; ++u) n += __popcll(__ballot(key[u] >= cand));
+        if (n >= r) mine = cand;
+    }
+    if (lane == 0) bounds[wave] = mine;
+    __syncthreads();
+    const uint32_t t = bounds[lane & 15];
+    unsigned int entries = 0;
+#pragma unroll 1
+    for (int w = 0; w < NW; ++w) {
+        const uint32_t cand = (uint32_t)__builtin_amdgcn_readlane((int)t, w);
+        unsigned int n = 0;
+#pragma unroll
+        for (int u = 0; u < N; ++u) n += (unsigned int)__popcll(__ballot(key[u] >= cand));
+        entries = lane == w ? n : entries;
+    }
+    if (lane < NW) atomicAdd(&reach[lane], entries);
+    __syncthreads();
+    return largest_of_16(reach[lane & 15] >= (unsigned int)top_k ? t : 0u);
+}
+
 // What a raw logit has to reach so that its scaled key can be key_ls = the scaled key of key_l: a
 // prefilter of one compare per element (it lets through whatever the key order would, -0.0 next to +0.0,
 // and everything when the bound lies below -inf, whose key decodes to a NaN).
@@ -475,9 +508,12 @@ __device__ __forceinline__ Nucleus nucleus_threshold(Shared& s, Src src, uint32_
 // row's top k leaves it.  Each wave finds the r-th largest of its 64 lane maxima, r = ceil(k / 16); at
 // least 16 r >= k elements of the part reach the smallest of the sixteen, so whatever lies below it (in
 // scaled order, ties stay) is not among the part's top k, nor the row's.  About 2.6 k of 16384 pass at
-// k = 50 (the tight bound of the merge would leave it too few lanes with entries there, k 50 12.3 -> 24.6).  A logit of -inf has no mass and
-// is left out; a part with a NaN, or one with more than part_cap candidates (masses of equal logits), sends its row the whole way.
-// Greedy: the part's argmax is its one candidate.
+// k = 50.  Where likely tokens are neighbours, and so in few waves, more pass than there is room for: then the tight bound of
+// bound_of_entries, from what passed (64 rows of 128256, logits of deviation 1 less ln(1 + index), k 50 38.9 -> 26.5 us; of 2.5 less
+// twice that, k 256 51.2 -> 32.3).  At once it would leave a usual row's merge too few lanes with entries, k 50 12.3 -> 24.6.  A logit of -inf has
+// no mass and is left out; a part with a NaN, or with more than RAW_CAP that pass (2000 neighbours far above all others), or with
+// more than part_cap candidates all the same (masses of equal logits), sends its row the whole way.  Greedy: the part's
+// argmax is its one candidate.
 //
 // Bound by latency: one round of loads, 22 ballots, three barriers, a few dozen appends.  64 rows of 128256
 // float32, k = 50: 8.8 us here and 5.2 us in sample_merge_kernel as traced, where one launch took 25.5 us.
@@ -589,6 +625,26 @@ sample_parts_kernel(SampleParams p) {
         }
     }
     __syncthreads();
+    if (__builtin_expect(nr > (unsigned int)p.part_cap, 0) && nr <= RAW_CAP && n_list > (unsigned int)p.part_cap && !whole) {
+        // some waves have next to nothing of the top, and the smallest of the bounds is theirs
+        uint32_t key[RAW_CAP / NT];
+#pragma unroll
+        for (int j = 0; j < RAW_CAP / NT; ++j) {
+            const unsigned int i = lane * NW + wave + NT * j;
+            key[j] = i < nr ? order_key(apply_temperature<T>(raw_x[i], p.temperature)) : 0u;
+        }
+        if (tid < NW) red_idx[tid] = 0;
+        __syncthreads();                                          // (n_list is read above by all)
+        if (tid == 0) n_list = 0;
+        const uint32_t least = max(max(key_ls, 1u), bound_of_entries(key, p.top_k, red_key, red_idx, lane, wave));
+#pragma unroll
+        for (int j = 0; j < RAW_CAP / NT; ++j)
+            if (key[j] >= least) {
+                const unsigned int at = atomicAdd(&n_list, 1u);
+                if (at < (unsigned int)p.part_cap) list[at] = make_uint2(key[j], raw_i[lane * NW + wave + NT * j]);
+            }
+        __syncthreads();
+    }
     if (tid == 0) p.part_count[slot] = whole || nr > RAW_CAP || n_list > (unsigned int)p.part_cap ? PART_WHOLE : n_list;
 }
 

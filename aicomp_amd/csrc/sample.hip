@@ -74,7 +74,7 @@ struct SampleParams {
 constexpr int PART_SLOTS = 16;                      // logits a lane of a part holds in registers
 constexpr int PART_MAX = NT * PART_SLOTS;           // 16384
 constexpr int GREEDY_CAP = 256;                     // room per part of a greedy call, which keeps one: 2 KB apart
-constexpr int RAW_CAP = 2048;                       // candidates of a part before the exact test
+constexpr int RAW_CAP = 4096;                       // candidates of a part before the exact test
 constexpr int MAX_PARTS = 16;
 constexpr int MERGE_SLOTS = 16;                     // candidates a lane of the merge takes: 16 lists of 1024 per row
 constexpr int PART_MAX_K = 256;
@@ -509,10 +509,11 @@ __device__ __forceinline__ Nucleus nucleus_threshold(Shared& s, Src src, uint32_
 // least 16 r >= k elements of the part reach the smallest of the sixteen, so whatever lies below it (in
 // scaled order, ties stay) is not among the part's top k, nor the row's.  About 2.6 k of 16384 pass at
 // k = 50.  Where likely tokens are neighbours, and so in few waves, more pass than there is room for: then the tight bound of
-// bound_of_entries, from what passed (64 rows of 128256, logits of deviation 1 less ln(1 + index), k 50 38.9 -> 26.5 us; of 2.5 less
-// twice that, k 256 51.2 -> 32.3).  At once it would leave a usual row's merge too few lanes with entries, k 50 12.3 -> 24.6.  A logit of -inf has
-// no mass and is left out; a part with a NaN, or with more than RAW_CAP that pass (2000 neighbours far above all others), or with
-// more than part_cap candidates all the same (masses of equal logits), sends its row the whole way.  Greedy: the part's
+// bound_of_entries, from what passed (64 rows of 128256, logits of deviation 1 less ln(1 + index), k 50 38.9 -> 27.2 us, k 256
+// 50.0 -> 32.7; 2000 neighbours 20 above all others, k 50 39.4 -> 25.1, which with room for 2048 that pass went the whole way).  At
+// once it would leave a usual row's merge too few lanes with entries, k 50 12.3 -> 24.6.  A logit of -inf has no mass and is
+// left out; a part with a NaN, or with more than RAW_CAP that pass, or with more than part_cap candidates all the same (masses of
+// equal logits: sorted bf16 rows, 64 of 128256, k 50 40 -> 47), sends its row the whole way.  Greedy: the part's
 // argmax is its one candidate.
 //
 // Bound by latency: one round of loads, 22 ballots, three barriers, a few dozen appends.  64 rows of 128256

@@ -231,46 +231,7 @@ class StepPlan:
             self._prefill_items[key] = items
         return items
 
-    # Longest decode row and largest decode batch for which a mixed step goes through one launch
-    # (measured on MI355X, 32 / 8 and 64 / 8 heads, head_dim 64 and 128, 1 to 16 chunks of 128 to
-    # 2048 tokens with 16 to 250 rows: within these bounds the one launch takes 0.95 to 1.65 times
-    # less than chunks and rows through their own kernels, 1.06 on 4 x 512 + 60 rows of up to 4096
-    # tokens; a row of 8192 and more tokens, walked by a single workgroup row, makes it up to
-    # twice as slow, and beyond ~128 rows the decode kernel's faster streaming wins)
-    ONE_LAUNCH_MAX_CONTEXT = 4608
     ONE_LAUNCH_MAX_ROWS = 1 << 30              # decode rows of the one launch: a caller's cap, 0 switches it off
-
-    def step_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:
-        """Item list over ALL sequences of a mixed step (chunks and one-token rows) for one launch
-        of the chunked-prefill kernel, or ``None`` when the step should go through the prefill
-        and decode kernels separately: no chunk or no decode row in it, pools of another type
-        than the 16-bit queries, a kernel that takes no list, a chunk bound too short for the
-        two-column-group kernel, or a decode part outside the bounds above.  Cached per step."""
-        from . import ops
-        npre, ndec = self.num_prefill_seqs, self.num_decode_seqs
-        if not npre or not ndec or ndec > min(128, self.ONE_LAUNCH_MAX_ROWS):
-            return None
-        if query.dtype not in (torch.bfloat16, torch.float16) or k_pool.dtype != query.dtype:
-            return None
-        key = self._list_key(("step", self.ONE_LAUNCH_MAX_CONTEXT), query, k_pool)
-        if self._prefill_items is None:
-            self._prefill_items = {}
-        items = self._prefill_items.get(key, _UNSEEN)
-        if items is _UNSEEN:
-            items = None
-            if int(self.host_context_lens[npre:].max()) <= self.ONE_LAUNCH_MAX_CONTEXT:
-                hq, (_, hkv, bs, d) = query.shape[1], k_pool.shape
-                tile = ops.prefill_tile_positions(hq, hkv, d, bs, query.dtype, k_pool.dtype, self.max_q_len)
-                group = hq // hkv
-                gpack = group if 16 % group == 0 else 1
-                if tile * gpack == 128:               # (0: no list; 64: the one-column-group kernel)
-                    hgroups = hq // gpack
-                    cus = torch.cuda.get_device_properties(query.device).multi_processor_count if query.is_cuda else 0
-                    items = ops.step_items(self.host_context_lens, self.new_lens, npre, tile, hgroups, cus)
-                    items = torch.from_numpy(items).to(query.device, non_blocking=True)
-            self._prefill_items[key] = items
-        return items
-
     ONE_LAUNCH_LONGEST = 16000                 # tokens of a decode row, as far as the two ways were measured
 
     def launch_items(self, query: torch.Tensor, k_pool: torch.Tensor) -> Optional[torch.Tensor]:

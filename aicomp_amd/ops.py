@@ -393,49 +393,17 @@ def prefill_items(context_lens, new_lens, tile_positions: int, num_head_groups: 
     return np.stack([seq[order], q[order]], axis=1).astype(np.int32)
 
 
-def step_items(context_lens, new_lens, num_prefill_seqs: int, tile_positions: int,
-               num_head_groups: int = 1, num_cus: int = 0):
-    """Item order for ONE prefill launch over a whole mixed step: the first ``num_prefill_seqs``
-    sequences are prompt chunks, the others one-token decode rows (chunks of one token, which the
-    kernel handles), ``int32 [n, 2]`` for ``paged_prefill_attn(items=...)``.
-
-    A chunk tile is bound by the matrix cores, a decode row by the latency of its loads; two
-    workgroups share a CU, and the launch is shortest when they are one of each kind.  When the
-    decode rows are the longer items the list therefore opens with one CU-round of decode rows
-    (longest first), then one of chunk tiles, which land beside them, and hands the rest out
-    alternately, each kind longest first.  When the chunk tiles are the longer items the order is
-    simply falling cost: the short rows then fill the launch's tail.  Measured on 32 / 8 heads,
-    head_dim 128: 4 chunks of 512 with 60 rows of 512 to 4096 tokens 138 us against 144 us in
-    falling order and 174 us chunks first; with rows of 128 to 1024 tokens falling order wins,
-    78 against 93 us.
-    """
-    import numpy as np
-    ctx = np.asarray(context_lens, dtype=np.int64)
-    new = np.asarray(new_lens, dtype=np.int64)
-    base = prefill_items(ctx, new, tile_positions, num_head_groups, 0)          # falling cost
-    pre, dec = base[base[:, 0] < num_prefill_seqs], base[base[:, 0] >= num_prefill_seqs]
-    per_round = num_cus // num_head_groups if num_cus > 0 and num_head_groups > 0 else 0
-    if not len(pre) or not len(dec) or per_round <= 0:
-        return base
-    cost = lambda it: np.minimum(ctx[it[:, 0]], ctx[it[:, 0]] - new[it[:, 0]] + (it[:, 1] + 1) * tile_positions)
-    if cost(dec).mean() < cost(pre).mean():
-        return base
-    a, b = dec[per_round:], pre[per_round:]
-    k = min(len(a), len(b))
-    rest = np.empty((2 * k, 2), dtype=base.dtype)
-    rest[0::2], rest[1::2] = a[:k], b[:k]
-    return np.concatenate([dec[:per_round], pre[:per_round], rest, a[k:], b[k:]]).astype(np.int32)
-
-
 def one_launch_items(context_lens, new_lens, num_prefill_seqs: int, tile_positions: int):
-    """``step_items`` for the kernels whose one-token rows stream (two column groups of 16-bit queries): the item order of
-    ONE launch over a mixed step, ``int32 [n, 2]``.
+    """The item order of ONE launch over a whole mixed step, whose first ``num_prefill_seqs`` sequences are prompt chunks and the
+    others one-token rows (chunks of one token, which stream in the kernels with two column groups): ``int32 [n, 2]`` for
+    ``paged_prefill_attn(items=...)``, every tile and every row once.
 
     Falling time.  A chunk tile of 128 rows takes 2.1 us per 64 keys beside another one, bound by the matrix cores, and a
     one-token row about 0.7 of that, bound by what the memory gives all of them; equal keys are therefore not equal times.
-    Measured on MI355X, 4 chunks of 512 over priors up to 2048 with 60 rows of 512 to 4096 tokens, 32 / 8 heads, head_dim
-    128 (64): weights 0.5 / 0.6 / 0.7 / 0.8 117.3 / 116.4 / 115.9 / 119.3 us (71.2 / 70.8 / 70.4 / 72.1), ``step_items``
-    121.6 (74.2), falling keys 119.7; rows of 128 to 1024 tokens 57.3 against 60.3.
+    Measured on MI355X, 4 chunks of 512 over priors up to 2048 with 60 rows of 512 to 4096 tokens, 32 / 8 heads, 16-bit pools,
+    head_dim 128 (64): weights 0.5 / 0.6 / 0.7 / 0.8 117.3 / 116.4 / 115.9 / 119.3 us (71.2 / 70.8 / 70.4 / 72.1), falling keys
+    119.7; rows of 128 to 1024 tokens 57.3 against 60.3.  (An order: other steps and fp8 pools, whose rows are half the
+    bytes, go by it unswept.)
     """
     import numpy as np
     ctx, new = np.asarray(context_lens, dtype=np.int64), np.asarray(new_lens, dtype=np.int64)

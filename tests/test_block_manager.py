@@ -410,14 +410,14 @@ def test_item_lists_follow_the_plan_as_it_is(how):
 
     import torch
     q, pool = torch.zeros(1, 32, 128, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 128, dtype=torch.bfloat16)
-    first = dict(ctx=[300, 300, 2000], new=[64, 64, 1], npre=2, max_q=64)          # tiles of 32 positions
+    first = dict(ctx=[300, 300, 1000], new=[64, 64, 1], npre=2, max_q=64)          # tiles of 32 positions
     others = [dict(first, max_q=16),                                                # tiles of 16
-              dict(first, ctx=[300, 400, 2000], new=[64, 128, 1]),
+              dict(first, ctx=[300, 400, 1000], new=[64, 128, 1]),
               dict(first, ctx=[300, 300, 5000]),                                    # a decode row beyond the one launch
-              dict(first, ctx=[300, 300, 2000, 2000], new=[64, 64, 1, 1])]
+              dict(first, ctx=[300, 300, 1000, 1000], new=[64, 64, 1, 1])]
     for other in others:
         plan, want = (_mixed_plan(*(c[k] for k in ("ctx", "new", "npre", "max_q"))) for c in (first, other))
-        used = [plan.prefill_items(q, pool), plan.step_items(q, pool)]
+        used = [plan.prefill_items(q, pool), plan.launch_items(q, pool)]
         assert all(x is not None for x in used) and plan.prefill_items(q, pool) is used[0]
         changes = {f.name: getattr(want, f.name) for f in dataclasses.fields(want) if not f.name.startswith("_")}
         if how == "replaced":
@@ -426,58 +426,27 @@ def test_item_lists_follow_the_plan_as_it_is(how):
             for name, value in changes.items():
                 setattr(plan, name, value)
         for got, ref in ((plan.prefill_items(q, pool), want.prefill_items(q, pool)),
-                         (plan.step_items(q, pool), want.step_items(q, pool))):
+                         (plan.launch_items(q, pool), want.launch_items(q, pool))):
             assert (got is None) == (ref is None) and (got is None or torch.equal(got, ref)), other
 
 
-def test_step_item_list_orders_a_mixed_step_for_one_launch():
-    """ops.step_items: every chunk tile and every decode row exactly once; decode rows that are the
-    longer items open the list (one CU-round of them, then one of chunk tiles, then alternating,
-    each kind longest first); shorter decode rows leave the list in falling cost."""
+def test_one_launch_list_orders_a_mixed_step_by_time():
+    """ops.one_launch_items: every chunk tile and every decode row exactly once, in falling time: a tile's keys, seven tenths
+    of a row's."""
     from aicomp_amd import ops
     rng = np.random.default_rng(5)
     npre, ndec, tile = 4, 60, 32
     new = [512] * npre + [1] * ndec
-    ctx = [int(p) + 512 for p in rng.integers(0, 2049, npre)] + [int(c) for c in rng.integers(513, 4098, ndec)]
-    items = ops.step_items(ctx, new, npre, tile, num_head_groups=8, num_cus=256)
-    want = {(s, q) for s in range(npre) for q in range(16)} | {(s, 0) for s in range(npre, npre + ndec)}
-    got = [tuple(x) for x in items.tolist()]
-    assert len(got) == len(set(got)) and set(got) == want and items.dtype == np.int32
-    assert all(s >= npre for s, _ in got[:32]) and all(s < npre for s, _ in got[32:64])
-    dec_keys = [ctx[s] for s, _ in got if s >= npre]
-    assert dec_keys == sorted(dec_keys, reverse=True)                       # each kind longest first
-    pre_keys = [min(ctx[s], ctx[s] - 512 + (q + 1) * tile) for s, q in got if s < npre]
-    assert pre_keys == sorted(pre_keys, reverse=True)
-    kinds = [s >= npre for s, _ in got[64:64 + 2 * min(ndec - 32, 64 - 32)]]
-    assert kinds == [True, False] * (len(kinds) // 2)                       # then alternating
-    # short decode rows: falling cost over both kinds
-    ctx2 = ctx[:npre] + [int(c) for c in rng.integers(2, 300, ndec)]
-    items2 = ops.step_items(ctx2, new, npre, tile, num_head_groups=8, num_cus=256)
-    keys2 = [min(ctx2[s], ctx2[s] - new[s] + (q + 1) * tile) for s, q in items2.tolist()]
-    assert keys2 == sorted(keys2, reverse=True) and {tuple(x) for x in items2.tolist()} == want
-    # no decode rows, or no chunks: the chunk order
-    assert (ops.step_items(ctx[:npre], new[:npre], npre, tile, 8, 256) == ops.prefill_items(ctx[:npre], new[:npre], tile, 8, 0)).all()
-
-
-def test_step_plan_sends_only_moderate_decode_parts_through_one_launch():
-    """StepPlan.step_items: a list for a mixed step of 16-bit pools whose decode part is within
-    the measured bounds, None otherwise (the step then goes through the prefill and decode kernels)."""
-    import torch
-    q = torch.zeros(1, 32, 128, dtype=torch.bfloat16)
-    pool = torch.zeros(1, 8, 16, 128, dtype=torch.bfloat16)
-    mixed = lambda ctx_dec, n_dec=8, chunk=512, npre=2: _mixed_plan([chunk + 100] * npre + [ctx_dec] * n_dec,
-                                                                   [chunk] * npre + [1] * n_dec, npre, chunk)
-    it = mixed(2000).step_items(q, pool)
-    assert it is not None and it.shape == (2 * 16 + 8, 2)
-    plan = mixed(2000)
-    assert plan.step_items(q, pool) is plan.step_items(q, pool)                           # built once per step
-    assert mixed(4608).step_items(q, pool) is not None and mixed(4609).step_items(q, pool) is None   # a long decode row
-    assert mixed(2000, n_dec=128).step_items(q, pool) is not None and mixed(2000, n_dec=129).step_items(q, pool) is None
-    assert mixed(2000, npre=0).step_items(q, pool) is None and mixed(2000, n_dec=0).step_items(q, pool) is None
-    assert mixed(2000).step_items(q, pool.to(torch.float8_e4m3fn)) is None                # fp8 pools: own kernels
-    assert mixed(2000).step_items(q.float(), pool.float()) is None
-    assert mixed(2000, chunk=16).step_items(q, pool) is None                              # one-column-group kernel
-    assert mixed(2000).step_items(torch.zeros(1, 32, 256, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 256, dtype=torch.bfloat16)) is None
+    for longest in (4098, 300):
+        ctx = [int(p) + 512 for p in rng.integers(0, 2049, npre)] + [int(c) for c in rng.integers(2, longest, ndec)]
+        items = ops.one_launch_items(ctx, new, npre, tile)
+        got = [tuple(x) for x in items.tolist()]
+        assert len(got) == len(set(got)) and items.dtype == np.int32
+        assert set(got) == {(s, q) for s in range(npre) for q in range(16)} | {(s, 0) for s in range(npre, npre + ndec)}
+        time = [(7 if s >= npre else 10) * min(ctx[s], ctx[s] - new[s] + (q + 1) * tile) for s, q in got]
+        assert time == sorted(time, reverse=True)
+    # no decode rows: the chunk order
+    assert (ops.one_launch_items(ctx[:npre], new[:npre], npre, tile) == ops.prefill_items(ctx[:npre], new[:npre], tile, 8, 0)).all()
 
 
 @pytest.mark.parametrize("cap", [0, 1, 8, 64])
@@ -513,6 +482,7 @@ def test_launch_items_of_a_mixed_step():
     assert mixed(2000, npre=0).launch_items(q, pool) is None and mixed(2000, n_dec=0).launch_items(q, pool) is None
     assert mixed(2000).launch_items(q.float(), pool.float()) is None
     assert mixed(2000).launch_items(q, pool.half()) is None
+    assert mixed(2000).launch_items(torch.zeros(1, 32, 256, dtype=torch.bfloat16), torch.zeros(1, 8, 16, 256, dtype=torch.bfloat16)) is None
     short = mixed(2000, chunk=16)                                                         # through the same kernel: tiles of 32
     assert short.launch_q_len(32, 8) == 32 and sorted(map(tuple, short.launch_items(q, pool).tolist())) == [(s, 0) for s in range(10)]
     assert mixed(300, n_dec=1, chunk=15).launch_items(q, pool) is None                    # 31 new tokens, none of them 32

@@ -13,7 +13,7 @@ import torch
 from aicomp_amd import ops
 from aicomp_amd.block_manager import StepPlanner, paged_attention_step
 from oracle import paged_kv_oracle as orc
-from helpers import assert_close_attn, raw, to_f64
+from helpers import assert_close_attn, kernels_of, raw, to_f64
 
 pytestmark = pytest.mark.gpu
 BF16_ATOL, BF16_RTOL = 1e-2, 2e-2
@@ -169,9 +169,11 @@ def test_mixed_step_one_launch_equals_separate_kernels_random_mixes(device, monk
             plan._prefill_items = None
             k_pool, v_pool = pools()
             out = torch.full((T, hq, d), float("nan"), dtype=dtype, device=device)
-            used = plan.step_items(q, k_pool) is not None
+            used = plan.launch_items(q, k_pool) is not None
             assert used == one
-            paged_attention_step(plan, out, q, kn, vn, k_pool, v_pool, 1 / math.sqrt(d))
+            names = kernels_of(lambda: paged_attention_step(plan, out, q, kn, vn, k_pool, v_pool, 1 / math.sqrt(d)))
+            assert any("paged_prefill" in n for n in names)
+            assert any("paged_decode" in n or "streamk_decode" in n for n in names) != one, names
             torch.cuda.synchronize()
             outs.append((out, k_pool, v_pool))
         took_one += 1

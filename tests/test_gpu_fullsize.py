@@ -106,7 +106,7 @@ def test_full_chunked_prefill_mixed(device):
                     max_q_len=512, total_new_tokens=int(w.query.shape[0]), block_table=w.block_table,
                     context_lens=w.context_lens, cu_q_lens=w.cu_q_lens, slot_mapping=w.slot_mapping, positions=None,
                     preempted=[], host_context_lens=np.asarray(w.ctx_list), host_cu_q_lens=w.cu_q_lens.cpu().numpy())
-    items = plan.step_items(w.query, w.k_pool)
+    items = plan.launch_items(w.query, w.k_pool)
     assert items is not None and items.shape == (4 * 16 + 60, 2)
     assert sorted(map(tuple, items.cpu().tolist())) == sorted([(s, q) for s in range(4) for q in range(16)] +
                                                               [(s, 0) for s in range(4, 64)])

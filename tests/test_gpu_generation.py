@@ -92,7 +92,7 @@ def test_backend_attend_mixed_step_one_launch_equals_separate_kernels(device, mo
             v = (torch.randn(T, hkv, d, device=device) * 0.5).to(torch.bfloat16)
             backend.begin_step(plan)
             outs.append((plan.num_prefill_seqs, plan.num_prefill_tokens, backend.attend(0, q, k, v)))
-            routes.append(plan.step_items(q, backend.k_pools[0]) is not None)
+            routes.append(plan.launch_items(q, backend.k_pools[0]) is not None)
         torch.cuda.synchronize()
         return outs, routes, backend.k_pools[0].clone(), backend.v_pools[0].clone()
 

@@ -303,7 +303,6 @@ def run_decode_config(name, steps, warmup, dev, settle_ms=30.0):
     # call's duration on the GPU, inside the replayed graph, is reported beside them.
     host_bound = (not npre) and t_graph is not None and t_enqueue / steps > 0.9 * region
     mb = btd.shape[1]
-    routed_small = (S - npre) * mb * w.shape.block_size <= ops.set_small_decode_tokens(-1)
     res = {
         "workload": name, "ms_per_step": (planned["wall"] if planned else wall) / steps * 1e3,
         "pools_in_rotation": len(pools), "settle_ms": settle_ms,
@@ -332,8 +331,13 @@ def run_decode_config(name, steps, warmup, dev, settle_ms=30.0):
     }
     mfma_shape = (w.shape.head_dim in (64, 128) and w.shape.block_size == 16
                   and qd.dtype in (torch.bfloat16, torch.float16, torch.float32))
-    balanced = mfma_shape and (S - npre) <= 1024 and not routed_small        # the library's rule, for rows as long as these
-    merge = "" if res["partition_size"] >= mb * w.shape.block_size else " + split_reduce_kernel"
+    # the schedule, by what the library reports: the grid schedule has whole rows or partitions of 256 tokens, and scratch for
+    # their partials alone
+    parts = -(-mb * w.shape.block_size // res["partition_size"])
+    partials = (S - npre) * w.shape.num_q_heads * parts * (w.shape.head_dim + 2) * 4 if parts > 1 else 0
+    balanced = mfma_shape and ((parts > 1 and res["partition_size"] != 256) or partials != ops.decode_workspace_bytes(
+        S - npre, w.shape.num_q_heads, w.shape.num_kv_heads, w.shape.head_dim, w.shape.block_size, mb, qd.dtype, w.k_pool.dtype))
+    merge = "" if parts == 1 else " + split_reduce_kernel"
     res["roofline"] = {
         "kernel": ("streamk_decode_kernel + streamk_reduce_kernel" if balanced else
                    "paged_decode_mfma_kernel" + merge if mfma_shape else

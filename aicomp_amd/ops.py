@@ -421,7 +421,8 @@ def one_launch_times(context_lens, new_lens, num_prefill_seqs: int, tile_positio
     Chunk tiles keep the matrix cores busy, 48 us (head_dim 64: 30) per 1000 keys of 512 tiles, the places of a launch, and one
     alone takes 19 (13) us per 1000 keys; rows are read at what the memory gives.  The decode kernels read a row once per
     KV head, the one launch once per head group, which is once per QUERY head where the group does not divide 16: 28 / 4
-    heads, a chunk of 512 with 32 rows of up to 4500 tokens 207 us together, 59 apart, with one row of 500 20 and 29.
+    heads, a chunk of 512 with 32 rows of up to 4500 tokens 207 us together, 59 apart, with one row of 500 20 and 29.  The launch's
+    additional workgroups take 3 us a round to start: 12 / 2 heads, D 64, 14 chunks of up to 50 with 162 rows of up to 143 18 and 13.
     (Groups that the matrix-core decode kernels do not take are read half as often apart as together.)
 
     A row is walked by one workgroup per head group, 10 (5) us per 1000 keys, 0.7 of that from an fp8 pool, and by a third of
@@ -443,7 +444,8 @@ def one_launch_times(context_lens, new_lens, num_prefill_seqs: int, tile_positio
     work = keys * hgroups / 512 * (0.048 if wide else 0.030)
     chunks = max(work, max(ctx[:num_prefill_seqs]) * (0.019 if wide else 0.013))
     read, longest = sum(rows) * 2 * head_dim * kv_bytes / 7e6, max(rows)          # of one head
-    together, walk = work + read * hgroups, longest * (0.010 if wide else 0.005) * (0.7 if kv_bytes == 1 else 1)
+    together = work + read * hgroups + 3 * len(rows) * (hgroups - once) / 512
+    walk = longest * (0.010 if wide else 0.005) * (0.7 if kv_bytes == 1 else 1)
     return max(together, walk + 0.3 * together), chunks + read * once + 10 + 0.0007 * longest
 
 

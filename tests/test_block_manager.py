@@ -508,3 +508,12 @@ def test_rows_that_one_launch_reads_once_per_query_head(hq, hkv, d, fp8):
         assert mixed(rows).launch_items(q, pool) is None, rows
     group4 = torch.zeros(1, 4 * hkv, d, dtype=torch.bfloat16)
     assert mixed([1000] * 100).launch_items(group4, pool) is not None
+
+
+def test_many_short_rows_of_such_a_group():
+    """Their workgroups' start is what the one launch would pay for."""
+    import torch
+    q, pool = torch.zeros(1, 12, 64, dtype=torch.bfloat16), torch.zeros(1, 2, 16, 64, dtype=torch.bfloat16)
+    for rows, one in ((162, False), (40, True)):
+        plan = _mixed_plan([40] * 14 + [80] * rows, [40] * 14 + [1] * rows, 14, 40)
+        assert (plan.launch_items(q, pool) is not None) == one

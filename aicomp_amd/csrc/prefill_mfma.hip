@@ -818,9 +818,12 @@ int launch_prefill_mfma(const DecodeArgs& a, int max_q_len) {
         //                192: 411 22 / 25    224: 994 28 / 33, 1973 46 / 49    240: 2014 49 / 46, 3536 82 / 62    288: 2064 50 / 51
         //          fp8   224: 1973 45 / 40;  16/2  108: 1035 30 / 21    136: 481 19 / 20, 1085 30 / 23    208: 2039 50 / 43
         //   D 64, one    56: 994 17 / 14, 1973 30 / 17    112: 994 18 / 23, 1973 32 / 29, 3493 46 / 32;  two  144: 2010 36 / 41
+        // Those are of unlike contexts.  Where all are as long as the longest, single column groups beyond 144, which share no
+        // keys in L2, take longer there: 168 (28/4) 2064 52 / 78, 192 (8/8) 2064 60 / 105, 192 (32/8) 3516 93 / 173, unlike 82 / 87;
+        // pairs of them, which do, hardly: 192 (32/8) 2064 52 / 49, 3564 82 / 82;  144 single ones 3530 81 / 88, unlike 78 / 52.
         // (sixteen heads of 64 are more rows per position than its workgroups have)
         const bool rows = a.d == 128 ? (wgs <= 64 && (keys >= 256 || (cols == 2 && (wgs <= 32 || a.num_seqs == 1)))) ||
-                                           (wgs * cols <= 144 && keys >= 640) || (wgs * cols <= 192 && keys >= 2048)
+                                           (wgs * cols <= 144 && keys >= 640) || (cols == 2 && wgs <= 96 && keys >= 2048)
                                      : group != 16 && ((wgs <= 32 && (wgs * cols <= 32 ? cols == 2 || keys >= 192 : keys >= 600)) ||
                                                        (cols == 1 && ((wgs <= 64 && keys >= 900) || (wgs <= 112 && keys >= 2048))));
         if (rows) return launch_prefill_rows(a, max_q_len, tile_pos, wgs);

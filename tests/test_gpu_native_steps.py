@@ -121,10 +121,10 @@ def test_chunks_and_rows(device, monkeypatch, dtype, kv, hq, hkv, d, appended, l
 
 
 @pytest.mark.parametrize("hq,hkv,d,priors,news,longest,rows", [
-    # column groups of the tile kernel: up to 144 from 640 keys on, up to 192 from 2048 (head_dim 64, one per workgroup: 64 from 900, 112 from 2048)
+    # column groups of the tile kernel: up to 144 from 640 keys on, up to 192 in pairs from 2048 (head_dim 64, one per workgroup: 64 from 900, 112 from 2048)
     (32, 8, 128, [3000, 900, 2000] + [0] * 3, [30] * 6, 3030, True), (32, 8, 128, [607] * 9, [32] * 9, 639, False),
     (32, 8, 128, [608] * 9, [32] * 9, 640, True), (16, 2, 128, [2100] + [40] * 8, [70] * 9, 2170, True),
-    (16, 2, 128, [1900] + [40] * 8, [70] * 9, 1970, False), (16, 4, 64, [884] * 15, [16] * 15, 900, True),
+    (16, 2, 128, [1900] + [40] * 8, [70] * 9, 1970, False), (8, 8, 128, [2036] + [100] * 20, [12] * 21, 2048, False), (16, 4, 64, [884] * 15, [16] * 15, 900, True),
     (16, 4, 64, [874] * 15, [16] * 15, 890, False), (16, 4, 64, [2032] + [100] * 24, [16] * 25, 2048, True)])
 @pytest.mark.parametrize("dtype,kv", [(torch.bfloat16, None), (torch.float16, torch.float8_e4m3fn)])
 def test_more_chunks_of_long_contexts(device, dtype, kv, hq, hkv, d, priors, news, longest, rows):

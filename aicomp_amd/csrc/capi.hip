@@ -102,6 +102,8 @@ static bool small_call(int64_t rows, int bs, int max_blocks) {
 //   float32 D 64 256  1168 0.87;  384  1200 1.02;  512  1200 0.94, 1600 1.03;  16 / 2 heads, bf16: 128 800 0.86, 256 1200 0.82
 // One head per KV head merges little: 8 / 8 heads, D 128, 384 workgroups 1200 tokens 30.6 / 28.8.  More than 512 workgroups come
 // in rounds: 768 of D 64, 2112 tokens 51.2 / 49.0, of fp8 54.4 / 53.0.
+// The table's width is all that is known here.  One row as long as it among rows a tenth of that, and rows alike, at the ends of the lines:
+// bf16 D 128 64 rows of 1648 22.8 / 19.3, 70.0 / 76.4;  D 64 64 of 3072 20.9 / 17.8, 67.3 / 72.1;  fp8 D 128 64 of 2560 23.7 / 20.9, 60.3 / 64.6.
 static int64_t whole_row_tokens(int64_t wgs, int group, int d, int64_t max_ctx, int kv_dtype) {
     const int64_t more = std::min<int64_t>(std::max<int64_t>(wgs - 64, 0), 448), rounds = wgs > 512 ? 2048 : 4096;
     if (is_16bit_float(kv_dtype)) return d == 64 ? std::min(1280 + 4 * more, rounds) : 768 + (group > 1 ? 2 : 1) * more;
@@ -118,6 +120,9 @@ static int64_t whole_row_tokens(int64_t wgs, int group, int d, int64_t max_ctx, 
 // 64 of 2112 (270 k) 0.95, 3600 (461 k) 1.00, 16 of 3584 (115 k) 0.76;  fp8 pools cross earlier: 16 of 2672 (342 k) 0.94,
 // 24 of 2096 (402 k) 1.02, 2672 (513 k) 1.05;  float32 rows of D 128 at once (48 of 800 46.5 / 37.8).  A raised threshold does
 // not move that line: the split would need more scratch than the balanced schedule (64 rows of 4096, 64 / 8 heads 34 MB, 19).
+// With pools that take turns (every call reads cold rows), partitions turned, one long row / lengths spread evenly / rows alike, split to
+// balanced: 16 / 2 heads 128 rows of 2048 0.81 / 1.01 / 1.04, 1648 0.72 / 1.03 / 1.09;  32 / 8 24 of 2048 0.74 / 0.99 / 1.00;  fp8 24 of
+// 2048 0.73 / 1.07 / 1.06, 16 of 2560 0.82 / 0.95 / 1.08, D 64 0.87 / 0.93 / 1.10.
 static bool grid_call(int64_t rows, int hq, int hkv, int d, int bs, int max_blocks, int kv_dtype) {
     if (small_call(rows, bs, max_blocks)) return true;
     const int64_t limit = small_decode_tokens().load(std::memory_order_relaxed), max_ctx = (int64_t)max_blocks * bs;

@@ -121,7 +121,7 @@ static int64_t whole_row_tokens(int64_t wgs, int group, int d, int64_t max_ctx, 
 // 24 of 2096 (402 k) 1.02, 2672 (513 k) 1.05;  float32 rows of D 128 at once (48 of 800 46.5 / 37.8).  A raised threshold does
 // not move that line: the split would need more scratch than the balanced schedule (64 rows of 4096, 64 / 8 heads 34 MB, 19).
 // With pools that take turns (every call reads cold rows), partitions turned, one long row / lengths spread evenly / rows alike, split to
-// balanced: 16 / 2 heads 128 rows of 2048 0.81 / 1.01 / 1.04, 1648 0.72 / 1.03 / 1.09;  32 / 8 24 of 2048 0.74 / 0.99 / 1.00;  fp8 24 of
+// balanced: 16 / 2 heads 128 rows of 2048 0.81 / 1.01 / 1.04, 1648 0.72 / 1.03 / 1.09;  32 / 8 24 of 2048 0.74 / 1.00 / 0.99;  fp8 24 of
 // 2048 0.73 / 1.07 / 1.06, 16 of 2560 0.82 / 0.95 / 1.08, D 64 0.87 / 0.93 / 1.10.
 static bool grid_call(int64_t rows, int hq, int hkv, int d, int bs, int max_blocks, int kv_dtype) {
     if (small_call(rows, bs, max_blocks)) return true;

@@ -102,10 +102,16 @@ static bool small_call(int64_t rows, int bs, int max_blocks) {
 //   float32 D 64 256  1168 0.87;  384  1200 1.02;  512  1200 0.94, 1600 1.03;  16 / 2 heads, bf16: 128 800 0.86, 256 1200 0.82
 // One head per KV head merges little: 8 / 8 heads, D 128, 384 workgroups 1200 tokens 30.6 / 28.8.  More than 512 workgroups come
 // in rounds: 768 of D 64, 2112 tokens 51.2 / 49.0, of fp8 54.4 / 53.0.
+// Between 256 and 512 workgroups some CUs have two, and two long rows on one of them wait for each other's loads while others idle: the
+// limit grows half as fast there, and at 512, two on every CU, is whole again.  384 workgroups, lengths lognormal (median an eighth of the table; of five draws the mean and the worst) /
+// spread evenly / alike, whole to balanced: bf16 D 128 1216 tokens 0.97, 1.19 / 1.06 / 0.95, 1344 1.06, 1.38 / 1.04 / 0.94;  D 64 1920 0.89, 0.96 /
+// 1.06 / 0.91, 2560 1.07, 1.33 / 1.07 / 0.98;  fp8 1920 0.99, 1.10 / 1.05 / 0.96, 2240 1.07, 1.13 / 1.03 / 1.01;  512: bf16 D 128 1472 0.95, 1.15 /
+// 0.92 / 0.90, D 64 2560 0.96, 1.17 / 0.93 / 0.90, 3072 1.03, 1.10 / 1.02 / 0.91, fp8 1920 0.95, 1.13 / 0.90 / 0.88, 2880 1.10, 1.19 / 0.97 / 0.94.
 // The table's width is all that is known here.  One row as long as it among rows a tenth of that, and rows alike, at the ends of the lines:
 // bf16 D 128 64 rows of 1648 22.8 / 19.3, 70.0 / 76.4;  D 64 64 of 3072 20.9 / 17.8, 67.3 / 72.1;  fp8 D 128 64 of 2560 23.7 / 20.9, 60.3 / 64.6.
 static int64_t whole_row_tokens(int64_t wgs, int group, int d, int64_t max_ctx, int kv_dtype) {
-    const int64_t more = std::min<int64_t>(std::max<int64_t>(wgs - 64, 0), 448), rounds = wgs > 512 ? 2048 : 4096;
+    const int64_t uneven = wgs > 256 && wgs < 512 ? (wgs - 256) / 2 : 0;
+    const int64_t more = std::min<int64_t>(std::max<int64_t>(wgs - uneven - 64, 0), 448), rounds = wgs > 512 ? 2048 : 4096;
     if (is_16bit_float(kv_dtype)) return d == 64 ? std::min(1280 + 4 * more, rounds) : 768 + (group > 1 ? 2 : 1) * more;
     if (kv_dtype == AICOMP_KV_FP8_E4M3) return d == 64 ? std::min<int64_t>(640 + 10 * more, 4096) : std::min(640 + 5 * more, rounds);
     if (d == 64) return std::min<int64_t>(640 + 3 * more / 2, 1100);

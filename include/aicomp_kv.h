@@ -133,7 +133,8 @@ int aicomp_kv_append(const void* key, const void* value,
  *                   max_blocks_per_seq * block_size <= 768 (head_dim 128) or 1280 (64) over a
  *                   16-bit pool, 640 over another (448 over a float32 pool of head_dim 128 when
  *                   the partitions of all rows and KV heads are at most 256): such a call is bound by launch and memory latency, not
- *                   by bandwidth.  From 64 to 512 pairs of a row and a KV head that limit grows, to 1664 tokens of
+ *                   by bandwidth.  From 64 to 512 pairs of a row and a KV head that limit grows
+ *                   (beyond 256 half as fast until 512 is reached), to 1664 tokens of
  *                   bf16 or fp16 at head_dim 128 (1216 with as many KV heads as query heads), 3072 at 64, of fp8
  *                   2880 and 4096 (2048 of head_dim 128, and of 16 bits at 64, beyond 512 pairs), of float32 1100 at
  *                   64; and calls above the threshold take this schedule too where rows are whole by it, or, with

@@ -34,6 +34,7 @@ def route(lib, rows, hq, hkv, d, tokens, q, kv):
     (32, 32, 8, 64, BF16, BF16, 2048, None), (64, 32, 8, 64, BF16, BF16, 3072, None), (128, 32, 8, 64, BF16, BF16, 2048, None),
     (32, 32, 8, 128, BF16, FP8, 1600, None), (64, 32, 8, 128, BF16, FP8, 2880, None), (128, 32, 8, 128, BF16, FP8, 2048, None),
     (96, 16, 2, 64, F16, FP8, 1920, 256), (64, 32, 8, 64, BF16, FP8, 4096, None),
+    (48, 32, 8, 128, BF16, BF16, 1280, 256), (48, 32, 8, 64, F16, F16, 2304, None), (48, 64, 8, 128, BF16, FP8, 1920, None),     # 1.5 to a CU
     (32, 32, 8, 64, F32, F32, 928, 256), (64, 32, 8, 64, F32, F32, 1088, None), (64, 32, 8, 128, F32, F32, 640, None),
     (1, 64, 8, 128, F32, F32, 448, 256)])
 def test_whole_rows(lib, rows, hq, hkv, d, q, kv, longest, beyond):
